@@ -143,13 +143,14 @@ void Ccsd::form_integrals() {
   make(w.Vpphh, "pphh");
   make(w.Vhhhh, "hhhh");
   make(w.Vhhhp, "hhhp");
+  w.hermitian = is_hermitian(E_.stream(), f, gamma_, s_.NG, s_.Np());
+  // conj(V_cdkl) = sum_G Gamma[G,k,c] conj Gamma[G,d,l]
+  //             = sum_G conj(Gamma[G,c,k]) Gamma[G,l,d] = V_klcd
+  if (w.hermitian) w.Vhhpp_view = w.Vpphh.v.transposed({2, 3, 0, 1});
   if (f == Field::Complex) {
     make(w.Vphhh, "phhh");
-    w.hermitian = is_hermitian(E_.stream(), gamma_, s_.NG, s_.Np());
     if (w.hermitian) {
-      // conj(V_cdkl) = sum_G Gamma[G,k,c] conj Gamma[G,d,l]
-      //             = sum_G conj(Gamma[G,c,k]) Gamma[G,l,d] = V_klcd
-      w.Vhhpp_view = w.Vpphh.v.transposed({2, 3, 0, 1}).conjugated();
+      w.Vhhpp_view = w.Vhhpp_view.conjugated();
     } else {
       make(w.Vhhpp, "hhpp");
       w.Vhhpp_view = w.Vhhpp.v;
@@ -162,10 +163,12 @@ void Ccsd::form_integrals() {
 
 bool Ccsd::vertex_is_hermitian() const { return w_->hermitian; }
 
-void Ccsd::get_residuum(const void *T, void *R) {
+void Ccsd::get_residuum(const void *T, void *R, bool symmetric) {
   auto t0 = std::chrono::steady_clock::now();
   if (opt_.method == Method::Drccd)
     residuum_drccd(T, R);
+  else if (T && symmetric && w_->hermitian && !E_.mixed())
+    residuum_symmetric(T, R);
   else if (s_.field == Field::Complex)
     residuum_complex(T, R);
   else
@@ -350,6 +353,137 @@ void Ccsd::residuum_drccd(const void *Tp, void *Rp) {
     E.contract(1.0, Vlkcd, T2.as("acik"), 0.0, Q);
     E.contract(-2.0, Q, T2.as("dblj"), 1.0, R2);
   }
+}
+
+// The residuum of both fields for a vertex with Gamma_qp = conj(Gamma_pq) and
+// amplitudes with T_abij = T_baji, in FP64: the statements of Ccsd.cxx:381-633
+// regrouped so that the o^3 v^3 products fall from five (complex; seven in the
+// real field's order, :76-378) to four and every operand combination is formed
+// once.  What the two symmetries allow:
+//   - crossed rings (:516-517): with X the intermediate, Y_cbkj = 2 T_cbkj - T_bckj
+//     and Z_abij = sum_kc X_bkci T_ackj,
+//       sum_kc X_akci T_cbkj = 1/2 sum_kc X_akci Y_cbkj + 1/2 Z_baij,
+//     so the first crossed product joins the ring product over Y (:502) as
+//     Xakic - 1/2 Xakci and only Z is left;
+//   - Wt_cdkl = V_klcd - 1/2 V_kldc serves :465-466, :472-473, :497-499 and
+//     :613-614, and 2 tau - tau~ serves :622-625 and :627-628;
+//   - the products with one occupied index summed (:490-491) act on one Q_akij.
+// Measured (one pass and the amplitudes read back, before -> after): complex
+// No=32, Nv=256, NG=1500 1.045 -> 0.968 s, No=12, Nv=60, NG=300 4.79 -> 4.18 ms;
+// real No=31, Nv=243, NG=1201 0.663 -> 0.578 s.
+// Split (mixed) passes, other vertices and other amplitudes keep the reference's
+// statements: residuum_complex and residuum_real.
+void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
+  auto &w = *w_;
+  auto &E = E_;
+  const Field f = s_.field;
+  const bool cplx = f == Field::Complex;
+  const int64_t o = s_.No, v = s_.Nv;
+  const hipStream_t st = E.stream();
+  const View R1 = dense_view(Rp, f, "ai", {v, o});
+  const View R2 = dense_view(offset_ptr(Rp, s_.n1(), f), f, "abij", {v, v, o, o});
+  const View T1 = dense_view(const_cast<void *>(Tp), f, "ai", {v, o});
+  const View T2 = dense_view(offset_ptr(Tp, s_.n1(), f), f, "abij", {v, v, o, o});
+  const View Vpphh = w.Vpphh("abij");
+  auto C = [&](double al, const View &A, const View &B, double be, const View &Cv) {
+    E.contract(al, A, B, be, Cv);
+  };
+  auto S = [&](double al, const View &A, double be, const View &Cv) {
+    E.sum(al, A, be, Cv);
+  };
+  auto Vhhpp = [&w](const std::string &names) { return w.Vhhpp_view.as(names); };
+  auto &Vhhhp = w.Vhhhp;
+  // two o^2 v^2 buffers hold every intermediate of that size in turn
+  auto A = [&](const std::string &names) { return w.X(names); };
+  const View Bv = dense_view(w.Xakic.buf.get(), f, "abij", {v, v, o, o});
+  auto B = [&](const std::string &names) { return Bv.as(names); };
+  auto X = [&](const std::string &names) { return w.Xakic(names); };  // [v,o,o,v]
+  auto combine = [&](const View &out, const View &in, double al, double be, double ga,
+                     bool conj = false) {
+    exchange_combination(st, f, out.ptr, in.ptr, al, be, ga, conj, o, v);
+  };
+
+  // one-particle intermediates; A = tau, B = Wt
+  tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 1.0, o, v);         // :460-461
+  combine(Bv, Vpphh, 1.0, -0.5, 0.0, cplx);
+  C(-2.0, B("cdkl"), A("adkl"), 0.0, w.Kac("ac"));              // :465-466
+  C(2.0, B("cdkl"), A("cdil"), 0.0, w.Kki("ki"));               // :472-473
+  C(2.0, B("cdkl"), T1.as("dl"), 0.0, w.Kck("ck"));             // :613-614
+  S(1.0, w.Kac("ac"), 0.0, w.Lac("ac"));                        // :468
+  C(1.0, gam("hp", "Gkd"), T1.as("dk"), 0.0, w.wG("G"));        // :469
+  C(2.0, gam("pp", "Gac", true), w.wG("G"), 1.0, w.Lac("ac"));
+  C(1.0, gam("pp", "Gad", true), T1.as("dk"), 0.0, w.Zgvo("Gak"));  // :470
+  C(-1.0, w.Zgvo("Gak"), gam("hp", "Gkc"), 1.0, w.Lac("ac"));
+  S(1.0, w.Kki("ki"), 0.0, w.Lki("ki"));                        // :476
+  C(2.0, Vhhhp("klic"), T1.as("cl"), 1.0, w.Lki("ki"));         // :477
+  C(-1.0, Vhhhp("lkic"), T1.as("cl"), 1.0, w.Lki("ki"));        // :478
+  C(1.0, w.Lac("ac"), T2.as("cbij"), 0.0, R2);                  // :481
+  C(-1.0, w.Lki("ki"), T2.as("abkj"), 1.0, R2);                 // :484
+  S(1.0, gam("ph", "Gai", true), 0.0, w.DGph("Gai"));           // :487
+  C(-1.0, gam("hh", "Gki", true), T1.as("ak"), 1.0, w.DGph("Gai"));  // :488
+  C(1.0, gam("pp", "Gbc"), T1.as("cj"), 0.0, w.Wgvo("Gbj"));    // :489
+  C(1.0, w.DGph("Gai"), w.Wgvo("Gbj"), 1.0, R2);
+  // Q_akij = V_akij + V_akic T_cj (:490-491); complex: V_akic = sum_G
+  // cTGamma_ph[G,a,i] Gamma_hp[G,k,c] (slice phhp) through G; real: V_akic is V_acik
+  if (cplx) {
+    C(1.0, gam("hp", "Gkc"), T1.as("cj"), 0.0, w.Zgoo("Gkj"));
+    C(1.0, gam("ph", "Gai", true), w.Zgoo("Gkj"), 0.0, w.Wvooo("akij"));
+    S(1.0, w.Vphhh("akij"), 1.0, w.Wvooo("akij"));
+  } else {
+    C(1.0, Vpphh.as("acik"), T1.as("cj"), 0.0, w.Wvooo("akij"));
+    S(1.0, Vhhhp("jika"), 1.0, w.Wvooo("akij"));
+  }
+  C(-1.0, w.Wvooo("akij"), T1.as("bk"), 1.0, R2);
+  // A = T2 + 2 T1 T1
+  tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 2.0, o, v);         // :462-463
+  S(1.0, w.Zgvo("Gai"), 1.0, w.DGph("Gai"));                    // :494
+  C(-0.5, gam("hp", "Gld", true), A("dail"), 1.0, w.DGph("Gai"));   // :495
+  // crossed ring, its intermediate Xakci stored as [a,k,i,c]; A = Z
+  S(1.0, gam("pp", "Gab", true), 0.0, w.DGpp("Gab"));           // :509
+  C(-1.0, gam("hp", "Glc", true), T1.as("al"), 1.0, w.DGpp("Gac"));  // :510
+  S(1.0, gam("hh", "Gij"), 0.0, w.DGhh("Gij"));                 // :511
+  C(1.0, gam("hp", "Gkd"), T1.as("di"), 1.0, w.DGhh("Gki"));    // :512
+  C(1.0, w.DGpp("Gac"), w.DGhh("Gki"), 0.0, X("akic"));         // :514
+  C(-0.5, Vhhpp("lkcd"), T2.as("dail"), 1.0, X("akic"));        // :515
+  C(1.0, X("bkic"), T2.as("ackj"), 0.0, A("abij"));             // :517
+  combine(R2, w.X.v, -1.0, -0.5, 1.0);
+  // ring over Xakic - 1/2 Xakci; A = Wt, then 2 T - T~
+  C(1.0, w.DGph("Gai"), gam("hp", "Gkc"), -0.5, X("akic"));     // :496
+  combine(w.X.v, Vpphh, 1.0, -0.5, 0.0, cplx);                  // :497-498
+  C(1.0, A("dclk"), T2.as("adil"), 1.0, X("akic"));             // :499
+  combine(w.X.v, T2, 2.0, -1.0, 0.0);                           // :500-501
+  C(1.0, X("akic"), A("cbkj"), 1.0, R2);                        // :502, :516
+  C(1.0, w.Kck("ck"), A("caki"), 0.0, R1);                      // :617-618
+  symmetrize_pairs(st, f, R2.ptr, o, v);                        // :520
+  S(1.0, Vpphh, 1.0, R2);                                       // :529
+  // hole ladder; A = tau
+  tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 1.0, o, v);
+  S(1.0, w.Vhhhh("klij"), 0.0, w.Xklij("klij"));                // :534
+  C(1.0, Vhhhp("klic"), T1.as("cj"), 1.0, w.Xklij("klij"));     // :535
+  C(1.0, Vhhhp("lkjc"), T1.as("ci"), 1.0, w.Xklij("klij"));     // :536
+  if (opt_.ppl) {
+    C(1.0, w.Xklij("klij"), A("abkl"), 1.0, R2);                // :538
+    C(1.0, Vhhpp("klcd"), A("cdij"), 0.0, w.Xklij("klij"));     // :541
+    C(1.0, w.Xklij("klij"), T2.as("abkl"), 1.0, R2);            // :542-546
+    // with Gamma_qp = conj Gamma_pq, Gamma_pp[G,a,b] - Gamma_hp[G,k,b] T_ak
+    // (:560-561) equals cTDGamma_pp[G,a,b] of :509-510 term by term
+    ladder(w.DGpp.v, w.DGpp.v, w.X.v, R2);                      // :564-600
+  } else {
+    C(1.0, Vhhpp("klcd"), A("cdij"), 1.0, w.Xklij("klij"));     // :541
+    C(1.0, w.Xklij("klij"), A("abkl"), 1.0, R2);                // :538, :542-546
+  }
+  // singles; B = 2 tau - tau~
+  combine(Bv, w.X.v, 2.0, -1.0, 0.0);
+  C(1.0, w.Kac("ac"), T1.as("ci"), 1.0, R1);                    // :609
+  C(1.0, w.Kck("ck"), T1.as("ci"), -1.0, w.Kki("ki"));          // :610, :619
+  C(1.0, w.Kki("ki"), T1.as("ak"), 1.0, R1);
+  // :620, V_akic T_ck = sum_G cTGamma_ph[G,a,i] (sum_kc Gamma_hp[G,k,c] T_ck)
+  C(2.0, gam("ph", "Gai", true), w.wG("G"), 1.0, R1);
+  // :621-625, all of the form cTGamma_pp[G,a,c] W[G,c,i]
+  C(-1.0, gam("hh", "Gki"), T1.as("ck"), 0.0, w.Wgvo("Gci"));
+  C(1.0, gam("hp", "Gkd"), B("cdik"), 1.0, w.Wgvo("Gci"));
+  C(1.0, gam("pp", "Gac", true), w.Wgvo("Gci"), 1.0, R1);
+  C(-1.0, Vhhhp("klic"), B("ackl"), 1.0, R1);                   // :627-628
 }
 
 void Ccsd::residuum_complex(const void *Tp, void *Rp) {

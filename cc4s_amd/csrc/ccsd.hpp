@@ -56,8 +56,10 @@ class Ccsd {
   // (VertexCoulombIntegrals.cxx:55-197)
   void form_integrals();
 
-  // R = residuum(T); T == nullptr is the first iteration (R1 = 0, R2 = V)
-  void get_residuum(const void *T, void *R);
+  // R = residuum(T); T == nullptr is the first iteration (R1 = 0, R2 = V).
+  // `symmetric` tells that T_abij = T_baji holds exactly (the iteration's own
+  // amplitudes always satisfy it).
+  void get_residuum(const void *T, void *R, bool symmetric);
 
   const View &Vpphh() const;
 
@@ -65,12 +67,14 @@ class Ccsd {
   // cxx:55-180, cT off); eps_h, eps_p on the device.  V_ppph (No*Nv^3) is
   // formed for the call and released afterwards.
   double triples(const void *T, const double *eps_h, const double *eps_p);
-  // Gamma^G_qp == conj(Gamma^G_pq) bit for bit (checked on the device)
+  // Gamma^G_qp == conj(Gamma^G_pq) (real field: == Gamma^G_pq) bit for bit
+  // (checked on the device)
   bool vertex_is_hermitian() const;
   CcsdTimings timings;
   bool profile = false;
 
  private:
+  void residuum_symmetric(const void *T, void *R);
   void residuum_complex(const void *T, void *R);
   void residuum_real(const void *T, void *R);
   void residuum_drccd(const void *T, void *R);

@@ -408,9 +408,17 @@ void CoupledCluster::download_set(const void *src, double *T1, double *T2) {
   CC4S_HIP(hipStreamSynchronize(stream_));
 }
 
+bool CoupledCluster::pairs_symmetric(const void *T) {
+  const auto &s = p_.shape;
+  return cc4s_amd::pairs_symmetric(
+      stream_, s.field, static_cast<const char *>(T) + s.n1() * scalar_bytes(s.field), s.No,
+      s.Nv);
+}
+
 void CoupledCluster::set_amplitudes(const double *T1, const double *T2) {
   CC4S_HIP(hipSetDevice(device_));
   upload_set(T_.get(), T1, T2);
+  symmetric_ = pairs_symmetric(T_.get());
   have_amplitudes_ = true;
 }
 
@@ -448,10 +456,10 @@ IterationReport CoupledCluster::iterate() {
     // holds no split residua
     defect_.reserve(packed_set_size(s.No, s.Nv) * scalar_bytes(s.field));
     engine_->set_mixed(true);
-    ccsd_->get_residuum(T, R_.get());
+    ccsd_->get_residuum(T, R_.get(), symmetric_);
     engine_->set_mixed(false);
     pack_axpby(stream_, s.field, R_.get(), -1.0, defect_.get(), 0.0, s.No, s.Nv);
-    ccsd_->get_residuum(T, R_.get());                   // :136
+    ccsd_->get_residuum(T, R_.get(), symmetric_);                   // :136
     pack_axpby(stream_, s.field, R_.get(), 1.0, defect_.get(), 1.0, s.No, s.Nv);
     mixer_->restart(0);
     rep.mixed = false;
@@ -460,7 +468,7 @@ IterationReport CoupledCluster::iterate() {
     rep.mixed = phase_ == Phase::Mixed || phase_ == Phase::Corrected;
     rep.kind = phase_ == Phase::Mixed ? 1 : phase_ == Phase::Corrected ? 3 : 0;
     engine_->set_mixed(rep.mixed);
-    ccsd_->get_residuum(T, R_.get());                   // :136
+    ccsd_->get_residuum(T, R_.get(), symmetric_);                   // :136
     engine_->set_mixed(false);
     if (phase_ == Phase::Corrected)
       unpack_accumulate(stream_, s.field, defect_.get(), 0, packed_set_size(s.No, s.Nv),
@@ -474,6 +482,7 @@ IterationReport CoupledCluster::iterate() {
   const bool is_second_order = !have_amplitudes_;
   mixer_->append(T_.get());                             // :145-147
   have_amplitudes_ = true;
+  symmetric_ = true;  // the mixer's history is pair-packed
   CC4S_HIP(hipStreamSynchronize(stream_));
   const auto t2 = std::chrono::steady_clock::now();
   rep.residuum_seconds = std::chrono::duration<double>(t1 - t0).count();
@@ -566,9 +575,10 @@ void CoupledCluster::residuum(const double *T1, const double *T2, double *R1,
     upload_set(scratch_.get(), T1, T2);
     T = scratch_.get();
   }
+  const bool symmetric = T && pairs_symmetric(T);
   // a context created for mixed precision evaluates its residuum that way
   engine_->set_mixed(p_.mixed);
-  ccsd_->get_residuum(T, R_.get());
+  ccsd_->get_residuum(T, R_.get(), symmetric);
   engine_->set_mixed(false);
   download_set(R_.get(), R1, R2);
 }

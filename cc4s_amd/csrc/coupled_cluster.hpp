@@ -156,6 +156,7 @@ class CoupledCluster {
 
  private:
   void energy(const void *T, cplx *E, cplx *D, cplx *X);
+  bool pairs_symmetric(const void *T);
   void upload_set(void *dst, const double *T1, const double *T2);
   void download_set(const void *src, double *T1, double *T2);
   void create_mixer();
@@ -175,6 +176,7 @@ class CoupledCluster {
   // transition structure factor: singular vectors, grid vertex blocks, Y
   DeviceBuffer fsc_u_, fsc_ph_, fsc_hp_, fsc_y_;
   bool have_amplitudes_ = false;
+  bool symmetric_ = true;  // T_ satisfies T_abij = T_baji (set_amplitudes may not)
   bool inputs_set_ = false;
   enum class Phase { Fp64, Mixed, Anchor, Corrected };
   Phase phase_ = Phase::Fp64;

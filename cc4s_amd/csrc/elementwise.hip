@@ -102,6 +102,56 @@ __global__ __launch_bounds__(kBlock) void symmetrize_kernel(typename Sc<CPLX>::T
   }
 }
 
+// out_abij = alpha in_abij + beta in_baij + gamma out_abij at fixed (i, j).
+// HBM-bound: a block takes the tile pair {(A, B), (B, A)}, so `in` is read once,
+// along its contiguous index, and serves both elements.
+template <bool CPLX>
+__global__ __launch_bounds__(kBlock) void exchange_kernel(
+    typename Sc<CPLX>::T *__restrict__ out, const typename Sc<CPLX>::T *__restrict__ in,
+    double alpha, double beta, double gamma, double sign, int64_t No, int64_t Nv) {
+  using S = Sc<CPLX>;
+  using T = typename S::T;
+  constexpr int kt = kPairTile;
+  __shared__ T xs[kt][kt + 1], ys[kt][kt + 1];
+  const int64_t nt = (Nv + kt - 1) / kt;
+  const int64_t ntiles = nt * nt * No * No;
+  for (int64_t tid = blockIdx.x; tid < ntiles; tid += gridDim.x) {
+    const int64_t ta = tid % nt, tb = (tid / nt) % nt, ij = tid / (nt * nt);
+    if (ta > tb) continue;  // the partner's block does it (uniform per block)
+    const int64_t a0 = ta * kt, b0 = tb * kt, off = Nv * Nv * ij;
+    __syncthreads();  // the previous pair's LDS reads are done
+    for (int e = threadIdx.x; e < kt * kt; e += kBlock) {
+      const int u = e % kt, w = e / kt;
+      // xs[a - a0][b - b0] = in_abij, ys[b - b0][a - a0] = in_baij
+      const bool ox = a0 + u < Nv && b0 + w < Nv, oy = b0 + u < Nv && a0 + w < Nv;
+      T x = ox ? in[off + (a0 + u) + Nv * (b0 + w)] : S::zero();
+      T y = oy ? in[off + (b0 + u) + Nv * (a0 + w)] : S::zero();
+      if constexpr (CPLX) {
+        x.y *= sign;
+        y.y *= sign;
+      }
+      xs[u][w] = x;
+      ys[u][w] = y;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < kt * kt; e += kBlock) {
+      const int u = e % kt, w = e / kt;
+      if (a0 + u < Nv && b0 + w < Nv) {
+        const int64_t o = off + (a0 + u) + Nv * (b0 + w);
+        T r = S::add(S::scale(xs[u][w], alpha), S::scale(ys[w][u], beta));
+        if (gamma != 0.0) r = S::add(r, S::scale(out[o], gamma));
+        out[o] = r;
+      }
+      if (ta != tb && b0 + u < Nv && a0 + w < Nv) {
+        const int64_t o = off + (b0 + u) + Nv * (a0 + w);
+        T r = S::add(S::scale(ys[u][w], alpha), S::scale(xs[w][u], beta));
+        if (gamma != 0.0) r = S::add(r, S::scale(out[o], gamma));
+        out[o] = r;
+      }
+    }
+  }
+}
+
 template <bool CPLX>
 __global__ __launch_bounds__(kBlock) void update_kernel(
     const typename Sc<CPLX>::T *R, const typename Sc<CPLX>::T *T,
@@ -318,6 +368,23 @@ void symmetrize_pairs(hipStream_t s, Field f, void *R2, int64_t No, int64_t Nv) 
     symmetrize_kernel<true><<<kReduceBlocks, kBlock, 0, s>>>(static_cast<double2 *>(R2), No, Nv);
   else
     symmetrize_kernel<false><<<kReduceBlocks, kBlock, 0, s>>>(static_cast<double *>(R2), No, Nv);
+  CC4S_HIP(hipGetLastError());
+}
+
+void exchange_combination(hipStream_t s, Field f, void *out, const void *in, double alpha,
+                          double beta, double gamma, bool conj, int64_t No, int64_t Nv) {
+  CC4S_ASSERT(out != in, "exchange combination in place");
+  const int64_t nt = (Nv + kPairTile - 1) / kPairTile;
+  const int blocks = static_cast<int>(std::min<int64_t>(nt * nt * No * No, 256 * 32));
+  const double sign = conj ? -1.0 : 1.0;
+  if (f == Field::Complex)
+    exchange_kernel<true><<<blocks, kBlock, 0, s>>>(static_cast<double2 *>(out),
+                                                    static_cast<const double2 *>(in), alpha,
+                                                    beta, gamma, sign, No, Nv);
+  else
+    exchange_kernel<false><<<blocks, kBlock, 0, s>>>(static_cast<double *>(out),
+                                                     static_cast<const double *>(in), alpha,
+                                                     beta, gamma, sign, No, Nv);
   CC4S_HIP(hipGetLastError());
 }
 
@@ -809,7 +876,8 @@ double combine_packed(hipStream_t s, Field f, const void *const *A,
 namespace {
 
 // per-block count of (G,p,q), p <= q, with Gamma[G,q,p] != conj Gamma[G,p,q]
-__global__ __launch_bounds__(kBlock) void hermitian_kernel(const double2 *g,
+// (sign -1) or != Gamma[G,p,q] (sign 1)
+__global__ __launch_bounds__(kBlock) void hermitian_kernel(const double2 *g, double sign,
                                                            int64_t NG, int64_t Np,
                                                            double2 *partials) {
   __shared__ double2 sh[kBlock];
@@ -823,26 +891,85 @@ __global__ __launch_bounds__(kBlock) void hermitian_kernel(const double2 *g,
     if (p > q) continue;
     const double2 a = g[e];
     const double2 b = g[G + NG * (q + Np * p)];
-    if (!(b.x == a.x && b.y == -a.y)) bad += 1.0;
+    if (!(b.x == a.x && b.y == sign * a.y)) bad += 1.0;
   }
   const double2 s = block_sum(make_double2(bad, 0.0), sh);
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
-}  // namespace
+// per-block count of elements with T_abij != T_baji: tile pairs
+// {(A, B, i, j), (B, A, j, i)} through LDS, as symmetrize_kernel
+template <bool CPLX>
+__global__ __launch_bounds__(kBlock) void asymmetry_kernel(const typename Sc<CPLX>::T *T2,
+                                                           int64_t No, int64_t Nv,
+                                                           double2 *partials) {
+  using S = Sc<CPLX>;
+  using T = typename S::T;
+  constexpr int kt = kPairTile;
+  __shared__ double2 sh[kBlock];
+  __shared__ T ys[kt][kt + 1];
+  const int64_t nt = (Nv + kt - 1) / kt;
+  const int64_t ntiles = nt * nt * No * No;
+  double bad = 0.0;
+  for (int64_t tid = blockIdx.x; tid < ntiles; tid += gridDim.x) {
+    const int64_t ta = tid % nt, tb = (tid / nt) % nt, ij = tid / (nt * nt);
+    const int64_t i = ij % No, j = ij / No;
+    if (i * nt + ta > j * nt + tb) continue;  // uniform per block
+    const int64_t a0 = ta * kt, b0 = tb * kt;
+    const int64_t offX = Nv * Nv * (i + No * j), offY = Nv * Nv * (j + No * i);
+    __syncthreads();
+    for (int e = threadIdx.x; e < kt * kt; e += kBlock) {
+      const int u = e % kt, w = e / kt;
+      ys[u][w] = (b0 + u < Nv && a0 + w < Nv) ? T2[offY + (b0 + u) + Nv * (a0 + w)] : S::zero();
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < kt * kt; e += kBlock) {
+      const int u = e % kt, w = e / kt;
+      if (a0 + u >= Nv || b0 + w >= Nv) continue;
+      const T x = T2[offX + (a0 + u) + Nv * (b0 + w)], y = ys[w][u];
+      if constexpr (CPLX) {
+        if (!(x.x == y.x && x.y == y.y)) bad += 1.0;
+      } else {
+        if (!(x == y)) bad += 1.0;
+      }
+    }
+  }
+  const double2 s = block_sum(make_double2(bad, 0.0), sh);
+  if (threadIdx.x == 0) partials[blockIdx.x] = s;
+}
 
-bool is_hermitian(hipStream_t s, const void *gamma, int64_t NG, int64_t Np) {
-  DeviceBuffer part((kReduceBlocks + 1) * sizeof(double2));
-  double2 *p = part.as<double2>();
-  hermitian_kernel<<<kReduceBlocks, kBlock, 0, s>>>(
-      static_cast<const double2 *>(gamma), NG, Np, p);
-  CC4S_HIP(hipGetLastError());
+// sums kReduceBlocks partials and reads the total back
+double finish_count(hipStream_t s, double2 *p) {
   finish_kernel<<<1, kBlock, 0, s>>>(p, 1, kReduceBlocks, p + kReduceBlocks);
   CC4S_HIP(hipGetLastError());
   double2 h;
   CC4S_HIP(hipMemcpyAsync(&h, p + kReduceBlocks, sizeof(h), hipMemcpyDeviceToHost, s));
   CC4S_HIP(hipStreamSynchronize(s));
-  return h.x == 0.0;
+  return h.x;
+}
+
+}  // namespace
+
+bool is_hermitian(hipStream_t s, Field f, const void *gamma, int64_t NG, int64_t Np) {
+  DeviceBuffer part((kReduceBlocks + 1) * sizeof(double2));
+  double2 *p = part.as<double2>();
+  hermitian_kernel<<<kReduceBlocks, kBlock, 0, s>>>(
+      static_cast<const double2 *>(gamma), f == Field::Complex ? -1.0 : 1.0, NG, Np, p);
+  CC4S_HIP(hipGetLastError());
+  return finish_count(s, p) == 0.0;
+}
+
+bool pairs_symmetric(hipStream_t s, Field f, const void *T2, int64_t No, int64_t Nv) {
+  DeviceBuffer part((kReduceBlocks + 1) * sizeof(double2));
+  double2 *p = part.as<double2>();
+  if (f == Field::Complex)
+    asymmetry_kernel<true><<<kReduceBlocks, kBlock, 0, s>>>(static_cast<const double2 *>(T2),
+                                                            No, Nv, p);
+  else
+    asymmetry_kernel<false><<<kReduceBlocks, kBlock, 0, s>>>(static_cast<const double *>(T2),
+                                                             No, Nv, p);
+  CC4S_HIP(hipGetLastError());
+  return finish_count(s, p) == 0.0;
 }
 
 void copy(hipStream_t s, void *y, const void *x, size_t bytes) {

@@ -17,6 +17,16 @@ void tau(hipStream_t s, Field f, void *X, const void *T2, const void *T1,
 // R_abij += R_baji with the old values on both sides (Ccsd.cxx:256, 520)
 void symmetrize_pairs(hipStream_t s, Field f, void *R2, int64_t No, int64_t Nv);
 
+// out_abij = alpha in_abij + beta in_baij + gamma out_abij (gamma 0: out is not
+// read), `in` conjugated first with conj; out and in are different [v,v,o,o]
+// tensors.  One kernel for the spin-adapted combinations V_lkdc - 1/2 V_lkcd,
+// 2 T_cbkj - T_bckj (Ccsd.cxx:497-501) and the crossed ring's two orientations.
+void exchange_combination(hipStream_t s, Field f, void *out, const void *in, double alpha,
+                          double beta, double gamma, bool conj, int64_t No, int64_t Nv);
+
+// T_abij == T_baji for every element, exactly
+bool pairs_symmetric(hipStream_t s, Field f, const void *T2, int64_t No, int64_t Nv);
+
 // New amplitudes and amplitude change of one amplitude set [T1; T2]
 // (CoupledCluster.cxx:137-144, 255-317):
 //   R' = R - shift*T (only when T is given and shift != 0)
@@ -87,9 +97,10 @@ double norm_packed_range(hipStream_t s, Field f, const void *const *R,
                          const std::vector<double> &c, int64_t t0, int64_t len,
                          int64_t No, int64_t Nv, void *partials);
 
-// true when the complex vertex [NG, Np, Np] satisfies
-// Gamma[G,q,p] == conj(Gamma[G,p,q]) exactly for every G, p, q
-bool is_hermitian(hipStream_t s, const void *gamma, int64_t NG, int64_t Np);
+// true when the vertex [NG, Np, Np] satisfies Gamma[G,q,p] == conj(Gamma[G,p,q])
+// (complex field) or Gamma[G,q,p] == Gamma[G,p,q] (real field: the real and the
+// imaginary part are two real vertices) exactly for every G, p, q
+bool is_hermitian(hipStream_t s, Field f, const void *gamma, int64_t NG, int64_t Np);
 
 // y = x (device copy on the stream)
 void copy(hipStream_t s, void *y, const void *x, size_t bytes);

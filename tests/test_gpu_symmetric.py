@@ -1,0 +1,75 @@
+"""The residuum's symmetric form (Hermitian or symmetric vertex, amplitudes with
+T_abij = T_baji, FP64) against the FP64 oracle of the reference's statements,
+and the calls that must keep the reference's own statements.
+
+Tolerance: every element is a sum of at most o v^2 + G products of magnitude
+below one, so the relative rounding of two summation orders stays under
+sqrt(n) 2^-53 ~ 1e-13 for the sizes below; 1e-12 of the largest element is
+asserted, as everywhere for one FP64 residuum."""
+
+import numpy as np
+import pytest
+
+from cc4s_amd import api
+from cc4s_amd import synthetic as syn
+from oracle import ccsd_oracle as O
+from tests.conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+
+R_TOL = 1e-12
+
+# Nv around the 32 x 32 tiles of the pair kernels, odd sizes, No above Nv
+SHAPES = [(2, 3, 4), (2, 31, 9), (3, 32, 17), (3, 33, 40), (4, 65, 21), (7, 50, 33),
+          (11, 5, 13), (17, 20, 23)]
+
+
+def _check(field, shape, T, **kw):
+    No, Nv, NG = shape
+    inp = syn.generate(No, Nv, NG, field, 21)
+    P = O.CcsdProblem(inp.gamma, inp.eps, No, field, ppl=kw.get("ppl", True),
+                      integrals_slice_size=kw.get("integralsSliceSize") or None)
+    Q1, Q2 = P.residuum(T)
+    with api.CoupledCluster(No, Nv, NG, field=field, **kw) as cc:
+        cc.set_inputs(inp.gamma, inp.eps)
+        for _ in range(2):  # the second call finds every plan and buffer made
+            R1, R2 = cc.residuum(T)
+            assert rel_err(R1, Q1) < R_TOL
+            assert rel_err(R2, Q2) < R_TOL
+
+
+@pytest.mark.parametrize("ppl", [True, False])
+@pytest.mark.parametrize("field", ["complex", "real"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_symmetric_residuum(field, shape, ppl):
+    print(f"symmetric residuum {field} {shape} ppl {ppl}", flush=True)
+    T = syn.random_amplitudes(shape[0], shape[1], field, 13, t1_scale=0.05, t2_scale=0.05)
+    _check(field, shape, T, ppl=ppl)
+
+
+@pytest.mark.parametrize("shape", [(3, 9, 12), (4, 33, 20)])
+def test_amplitudes_without_pair_symmetry(shape):
+    """Real field: T_abij != T_baji follows the reference's statements."""
+    print(f"amplitudes without pair symmetry {shape}", flush=True)
+    No, Nv, NG = shape
+    T1, T2 = syn.random_amplitudes(No, Nv, "real", 13, t1_scale=0.05, t2_scale=0.05)
+    T2 = T2.copy(order="F")
+    T2[1, 0, 0, 1] += 1e-3
+    _check("real", shape, (T1, T2))
+
+
+@pytest.mark.parametrize("shape", [(3, 9, 12), (4, 33, 20)])
+def test_real_vertex_without_symmetry(shape):
+    print(f"real vertex without symmetry {shape}", flush=True)
+    No, Nv, NG = shape
+    inp = syn.generate(No, Nv, NG, "real", 21)
+    rng = np.random.default_rng(4)
+    g = inp.gamma + 0.003 * rng.standard_normal(inp.gamma.shape)
+    T = syn.random_amplitudes(No, Nv, "real", 13, t1_scale=0.05, t2_scale=0.05)
+    P = O.CcsdProblem(g, inp.eps, No, "real")
+    Q1, Q2 = P.residuum(T)
+    with api.CoupledCluster(No, Nv, NG, field="real") as cc:
+        cc.set_inputs(g, inp.eps)
+        R1, R2 = cc.residuum(T)
+    assert rel_err(R1, Q1) < R_TOL
+    assert rel_err(R2, Q2) < R_TOL
