@@ -38,6 +38,10 @@ struct Ccsd::Work {
   Tensor wG, Zgvo, Wgvo, Wvooo, Woo, Zgoo;
   Tensor slab, Rxy, Rpm;  // Rpm: the paired ladder's Rp and Rm of a chunk
   FusedLadderTable fused;  // pair blocks of the fused ladder
+  // resident ladder: pair integrals S, A and the products Rp, Rm; formed at
+  // the first pass that can use them
+  enum class Resident { Unknown, Ready, Off } resident = Resident::Unknown;
+  Tensor VS, VA, Rp, Rm;
   int64_t NGe = 0;  // length of the G index of the real-path vertex views
   bool hermitian = false;
 };
@@ -46,7 +50,8 @@ Ccsd::Ccsd(ContractionEngine &E, const CcsdShape &shape, const CcsdOptions &opt,
            void *gamma, bool gamma_real)
     : E_(E), s_(shape), opt_(opt), gamma_(gamma), gamma_real_(gamma_real),
       w_(new Work) {
-  if (opt_.integrals_slice_size <= 0) opt_.integrals_slice_size = s_.No;
+  opt_.default_slices = opt_.integrals_slice_size <= 0;
+  if (opt_.default_slices) opt_.integrals_slice_size = s_.No;
   const Field f = s_.field;
   const int64_t o = s_.No, v = s_.Nv;
   // the real path sees Re and Im of Gamma as one real index of length 2 NG
@@ -226,7 +231,7 @@ void Ccsd::ladder(const View &left, const View &right, const View &tauv,
     CC4S_HIP(hipEventCreate(&e1));
     CC4S_HIP(hipEventRecord(e0, E_.stream()));
   }
-  if (paired) ladder_tau_pairs(tauv.ptr, Tp, Tm, v, o, E_.stream());
+  if (paired) ladder_tau_pairs(f, tauv.ptr, Tp, Tm, 1.0, v, o, E_.stream());
   const double flops0 = E_.stats.flops;
   if (fused) {
     E_.stats.flops += ladder_fused(left.as("Gxc"), right.as("Gyd"), tauv.as("cdij"),
@@ -291,6 +296,113 @@ void Ccsd::ladder(const View &left, const View &right, const View &tauv,
     }
   }
   E_.clear_operand_cache();
+  if (profile) {
+    CC4S_HIP(hipEventRecord(e1, E_.stream()));
+    CC4S_HIP(hipEventSynchronize(e1));
+    float ms = 0;
+    CC4S_HIP(hipEventElapsedTime(&ms, e0, e1));
+    timings.ladder_ms += ms;
+    timings.ladder_flops += E_.stats.flops - flops0;
+    timings.ladder_calls += 1;
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+  }
+}
+
+// The ladder's pair integrals S and A (ladder_pairs.hip), formed from Gamma on
+// first use and kept for the run like the other integral slices.  They are kept
+// when they take at most half of the device memory that is free then (less what
+// the pass itself may still allocate), so that other contexts and the caller
+// keep room; other runs use the slab ladder.  An explicit integralsSliceSize
+// asks for the slab, whose memory it bounds, and so do the other ladder modes.
+bool Ccsd::resident_integrals() {
+  auto &w = *w_;
+  if (w.resident != Work::Resident::Unknown) return w.resident == Work::Resident::Ready;
+  w.resident = Work::Resident::Off;
+  const Field f = s_.field;
+  const int64_t o = s_.No, v = s_.Nv;
+  if (!opt_.ladder_paired || !opt_.default_slices || v < 2) return false;
+  const int64_t Kp = v * (v + 1) / 2, Km = v * (v - 1) / 2;
+  const int64_t Np = o * (o + 1) / 2, Nm = o * (o - 1) / 2;
+  const double es = static_cast<double>(scalar_bytes(f));
+  const double need = es * (double(Kp) * double(Kp + o * v) + double(Km) * double(Km + o * v) +
+                            double(Np) * double(Kp + o * v) + double(Nm) * double(Km + o * v));
+  size_t free_b = 0, total_b = 0;
+  CC4S_HIP(hipMemGetInfo(&free_b, &total_b));
+  const double avail = static_cast<double>(free_b) - 6.0 * (1 << 30);
+  if (need > 0.5 * avail) return false;
+  // slab of nx x values: at most 2 GiB; wider slices form more of the square
+  // d < x1 than the triangle needs, narrower ones launch more
+  const double per_x = es * double(v) * double(v) * double(v);
+  const int64_t fit = static_cast<int64_t>((2.0 * (1 << 30)) / per_x);
+  if (fit < 1 || v > 65535) return false;
+  const int64_t nx = std::min(std::min<int64_t>(fit, std::max<int64_t>(16, v / 16)), 65535 / v);
+  if (nx < 1) return false;
+  Tensor slab;
+  try {
+    w.VS.reset(f, "km", {Kp, Kp + o * v});
+    w.VA.reset(f, "km", {Km, Km + o * v});
+    w.Rp.reset(f, "nm", {Np, Kp + o * v});
+    w.Rm.reset(f, "nm", {Nm, Km + o * v});
+    slab.reset(f, "cxdy", {v, nx, v, v});
+  } catch (const Error &) {  // no room after all
+    (void)hipGetLastError();
+    w.VS = Tensor();
+    w.VA = Tensor();
+    w.Rp = Tensor();
+    w.Rm = Tensor();
+    return false;
+  }
+  const hipStream_t st = E_.stream();
+  const View left = gam("pp", "Gxc", true), right = gam("pp", "Gyd");
+  for (int64_t x0 = 0; x0 < v; x0 += nx) {
+    const int64_t x1 = std::min(v, x0 + nx), cx = x1 - x0;
+    const View V = dense_view(slab.buf.get(), f, "cxdy", {x1, cx, x1, x1});
+    E_.contract(1.0, left.sliced(1, x0, x1).sliced(2, 0, x1),
+                right.sliced(1, 0, x1).sliced(2, 0, x1), 0.0, V);
+    resident_fold(f, true, V.ptr, w.VS.buf.get(), w.VA.buf.get(), x1, cx, x1, x0, v, st);
+  }
+  resident_mirror(f, w.VS.buf.get(), Kp, st);
+  resident_mirror(f, w.VA.buf.get(), Km, st);
+  const View hole = gam("hp", "Gxc", true);
+  for (int64_t x0 = 0; x0 < o; x0 += nx) {
+    const int64_t cx = std::min(nx, o - x0);
+    const View V = dense_view(slab.buf.get(), f, "cxdy", {v, cx, v, v});
+    E_.contract(1.0, hole.sliced(1, x0, x0 + cx), right, 0.0, V);
+    resident_fold(f, false, V.ptr, w.VS.buf.get(), w.VA.buf.get(), v, cx, v, x0, v, st);
+  }
+  CC4S_HIP(hipStreamSynchronize(st));  // the slab is released here
+  w.resident = Work::Resident::Ready;
+  return true;
+}
+
+// Rp and Rm of the resident ladder; tau's combinations go to Xakic's buffer
+void Ccsd::resident_products(const View &tauv) {
+  auto &w = *w_;
+  const Field f = s_.field;
+  const int64_t o = s_.No, v = s_.Nv;
+  const int64_t Kp = v * (v + 1) / 2, Km = v * (v - 1) / 2;
+  const int64_t Np = o * (o + 1) / 2, Nm = o * (o - 1) / 2;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (profile) {
+    CC4S_HIP(hipEventCreate(&e0));
+    CC4S_HIP(hipEventCreate(&e1));
+    CC4S_HIP(hipEventRecord(e0, E_.stream()));
+  }
+  void *Tp = w.Xakic.buf.get();
+  void *Tm = offset_ptr(Tp, Kp * Np, f);
+  ladder_tau_pairs(f, tauv.ptr, Tp, Tm, 0.5, v, o, E_.stream());
+  const double flops0 = E_.stats.flops;
+  E_.contract(1.0, w.VS("km"), dense_view(Tp, f, "kn", {Kp, Np}), 0.0, w.Rp("nm"));
+  E_.contract(1.0, w.VA("km"), dense_view(Tm, f, "kn", {Km, Nm}), 0.0, w.Rm("nm"));
+  // credited as the contractions of the reference that it replaces: every pair
+  // x, y of the slice pairs over v^2 k and o^2 columns (the integrals' formation
+  // is credited where it is done, once)
+  const int64_t s = opt_.integrals_slice_size;
+  double pairs = 0;
+  for (int64_t b = 0; b < v; b += s)
+    pairs += static_cast<double>(std::min(s, v - b)) * static_cast<double>(v - b);
+  E_.stats.flops = flops0 + (f == Field::Complex ? 8.0 : 2.0) * pairs * v * v * o * o;
   if (profile) {
     CC4S_HIP(hipEventRecord(e1, E_.stream()));
     CC4S_HIP(hipEventSynchronize(e1));
@@ -403,8 +515,11 @@ void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
     exchange_combination(st, f, out.ptr, in.ptr, al, be, ga, conj, o, v);
   };
 
-  // one-particle intermediates; A = tau, B = Wt
+  // A = tau; the resident ladder's products
   tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 1.0, o, v);         // :460-461
+  const bool resident = opt_.ppl && resident_integrals();
+  if (resident) resident_products(w.X.v);
+  // one-particle intermediates; B = Wt
   combine(Bv, Vpphh, 1.0, -0.5, 0.0, cplx);
   C(-2.0, B("cdkl"), A("adkl"), 0.0, w.Kac("ac"));              // :465-466
   C(2.0, B("cdkl"), A("cdil"), 0.0, w.Kki("ki"));               // :472-473
@@ -433,6 +548,10 @@ void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
     C(1.0, Vpphh.as("acik"), T1.as("cj"), 0.0, w.Wvooo("akij"));
     S(1.0, Vhhhp("jika"), 1.0, w.Wvooo("akij"));
   }
+  // the resident ladder (half of it: R2 is symmetrised below) and, with U_kaji
+  // in Q_akij, the T1 dressing of its left or right vertex
+  if (resident)
+    resident_unpack(f, w.Rp.buf.get(), w.Rm.buf.get(), R2.ptr, w.Wvooo.buf.get(), 0.5, v, o, st);
   C(-1.0, w.Wvooo("akij"), T1.as("bk"), 1.0, R2);
   // A = T2 + 2 T1 T1
   tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 2.0, o, v);         // :462-463
@@ -461,7 +580,7 @@ void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
   S(1.0, w.Vhhhh("klij"), 0.0, w.Xklij("klij"));                // :534
   C(1.0, Vhhhp("klic"), T1.as("cj"), 1.0, w.Xklij("klij"));     // :535
   C(1.0, Vhhhp("lkjc"), T1.as("ci"), 1.0, w.Xklij("klij"));     // :536
-  if (opt_.ppl) {
+  if (opt_.ppl && !resident) {
     C(1.0, w.Xklij("klij"), A("abkl"), 1.0, R2);                // :538
     C(1.0, Vhhpp("klcd"), A("cdij"), 0.0, w.Xklij("klij"));     // :541
     C(1.0, w.Xklij("klij"), T2.as("abkl"), 1.0, R2);            // :542-546
@@ -469,6 +588,8 @@ void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
     // (:560-561) equals cTDGamma_pp[G,a,b] of :509-510 term by term
     ladder(w.DGpp.v, w.DGpp.v, w.X.v, R2);                      // :564-600
   } else {
+    // over tau: :542-546 without ppl, or with the dressing T_ak T_bl V_klcd tau_cdij
+    // of the resident ladder
     C(1.0, Vhhpp("klcd"), A("cdij"), 1.0, w.Xklij("klij"));     // :541
     C(1.0, w.Xklij("klij"), A("abkl"), 1.0, R2);                // :538, :542-546
   }

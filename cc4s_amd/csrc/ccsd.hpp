@@ -26,6 +26,7 @@ struct CcsdOptions {
   Method method = Method::Ccsd;      // CoupledCluster.cxx:77-84
   bool ppl = true;                   // Ccsd.cxx:95,402
   int64_t integrals_slice_size = 0;  // 0: No (Ccsd.cxx:287-289)
+  bool default_slices = true;        // it was 0
   bool linearized = false;           // Drccd.cxx:53-55
   bool adjacent_pairs_exchange = false;  // Drccd.cxx:56-58
   // FP64 complex ladder as one fused kernel (V formed in LDS, never in HBM)
@@ -79,6 +80,8 @@ class Ccsd {
   void residuum_real(const void *T, void *R);
   void residuum_drccd(const void *T, void *R);
   void form_slice(Tensor &V, const char *name);
+  bool resident_integrals();
+  void resident_products(const View &tauv);
   void ladder(const View &left, const View &right, const View &tauv,
               const View &R2);
   View gam(const char *part, const std::string &names, bool conjT = false) const;

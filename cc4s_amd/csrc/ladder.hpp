@@ -32,17 +32,33 @@ double ladder_fused(const View &left, const View &right, const View &tau,
 // diagonal), Vm = V_xycd - V_xydc; R_xyij = Rp + Rm, R_xyji = Rp - Rm: half
 // the multiply-adds.  Pair indices c <= d -> c + d(d+1)/2, c < d ->
 // c + d(d-1)/2 (the same for i, j).
-//   ladder_tau_pairs:    tau [c,d,i,j] dense -> tau+ [Kp][Np], tau- [Km][Nm]
+//   ladder_tau_pairs:    tau [c,d,i,j] dense -> tau+ [Kp][Np] (its c = d
+//                        elements times `diag`), tau- [Km][Nm]
 //   ladder_vertex_pairs: slab [c,x,d,y] dense (v, cx, v, Ny) -> Vp [Kp][x][y],
 //                        Vm [Km][x][y]
 //   ladder_unpack_pairs: Rp [xy][Np], Rm [xy][Nm] -> R [xy][i][j]
 // with Kp = v(v+1)/2, Km = v(v-1)/2, Np = o(o+1)/2, Nm = o(o-1)/2, k or xy
 // fastest.
-void ladder_tau_pairs(const void *tau, void *Tp, void *Tm, int64_t v, int64_t o,
-                      hipStream_t s);
+void ladder_tau_pairs(Field f, const void *tau, void *Tp, void *Tm, double diag, int64_t v,
+                      int64_t o, hipStream_t s);
 void ladder_vertex_pairs(const void *slab, void *Vp, void *Vm, int64_t v, int64_t cx,
                          int64_t Ny, hipStream_t s);
 void ladder_unpack_pairs(const void *Rp, const void *Rm, void *R, int64_t nxy, int64_t o,
                          hipStream_t s);
+
+// Resident pair integrals (ladder_pairs.hip), both fields:
+//   S [Kp][Kp + o v], A [Km][Km + o v], first index fastest; the first Kp (Km)
+//   columns are the particle pairs, column Kp + v k + a the hole k, particle a.
+//   resident_fold:   columns of S and A from a slab V[c,x,d,y] (n, cx, n, Ny):
+//                    particle pairs X = x0 + x >= y (rows d < n), or holes
+//                    X = x0 + x (n = v)
+//   resident_mirror: lower triangle of an n x n Hermitian matrix from the upper
+//   resident_unpack: Rp [Np][Kp + o v], Rm [Nm][Km + o v] of the two products:
+//                    R2[a,b,i,j] += factor R_abij, Q[a,k,i,j] += U_kaji
+void resident_fold(Field f, bool particles, const void *slab, void *S, void *A, int64_t n,
+                   int64_t cx, int64_t Ny, int64_t x0, int64_t v, hipStream_t s);
+void resident_mirror(Field f, void *M, int64_t n, hipStream_t s);
+void resident_unpack(Field f, const void *Rp, const void *Rm, void *R2, void *Q, double factor,
+                     int64_t v, int64_t o, hipStream_t s);
 
 }  // namespace cc4s_amd

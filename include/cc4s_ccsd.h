@@ -105,7 +105,14 @@ typedef struct {
                                      pairs c <= d, i <= j of tau's symmetric and
                                      antisymmetric combinations, half its multiply-adds;
                                      FP64 and split passes); same results to rounding.
-                                     The real field always uses the slab. */
+                                     With PAIRED, integrals_slice_size 0, a vertex with
+                                     Gamma_qp = conj(Gamma_pq) (real field: Gamma_pq) and
+                                     amplitudes with T_abij = T_baji, FP64 passes of both
+                                     fields keep the pair integrals of the ladder on the
+                                     device instead (about Nv^4 scalars), formed in the
+                                     first such pass, where they take at most half of the
+                                     free device memory.  The real field otherwise uses
+                                     the slab. */
 } cc4s_ccsd_params;
 
 /* Values of cc4s_ccsd_params.ladder. */
