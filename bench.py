@@ -54,7 +54,7 @@ FP64_MFMA_PEAK_TFLOPS = 78.6      # MI355X dense FP64 matrix
 METRIC = ("s per CCSD iteration + % MFMA peak, mixed vs FP64 GPU at "
           "|ΔE|≤1 µEh")
 VARIANTS = [f"gett_{t}_{a}_{b}{k}" for t in ("c64", "f64") for a in ("ak", "am")
-            for b in ("bk", "bn") for k in ("", "_shortk")]
+            for b in ("bk", "bn") for k in ("", "_t64", "_t32")]
 
 
 def measured_traffic(kernel, cfg):

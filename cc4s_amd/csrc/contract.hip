@@ -37,15 +37,15 @@ struct KArgs {
   double f2, signA2, signB2;
 };
 
-// Workgroup tile BM x BN, K staged BK at a time through LDS; 4 waves in a
+// Complex GETT, first generation: workgroup tile BM x BN, K staged BK at a time through LDS; 4 waves in a
 // (BM/WM) x (BN/WN) grid, each owning WM x WN of C as 16x16 MFMA blocks.
 // A is read either along K (AKC: consecutive lanes -> consecutive k) or along
 // M; B along K (BKC) or along N.  LDS holds A as [k][m] and B as [k][n] (one
 // plane per real/imaginary part), which is exactly the lane order of the
 // MFMA operands (lane l reads row l%16 at k = l/16).
-template <bool CPLX, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC>
+template <int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC>
 __global__ __launch_bounds__(kThreads, 2) void gett_kernel(KArgs p) {
-  constexpr int NPL = CPLX ? 2 : 1;
+  constexpr int NPL = 2;
   constexpr int MB = WM / 16, NB = WN / 16;
   constexpr int WAVES_N = BN / WN;
   static_assert((BM / WM) * (BN / WN) == 4, "four waves per workgroup");
@@ -128,28 +128,20 @@ __global__ __launch_bounds__(kThreads, 2) void gett_kernel(KArgs p) {
       const int ir = AKC ? i : 0, ik = AKC ? 0 : i;
       const bool ok = aRowOk[ir] && aKok[ik];
       const int64_t off = aRow[ir] + aK[ik];
-      if constexpr (CPLX) {
-        double2 v = ok ? *reinterpret_cast<const double2 *>(p.A + 2 * off)
-                       : make_double2(0.0, 0.0);
-        ra[i][0] = v.x;
-        ra[i][1] = v.y * p.signA;
-      } else {
-        ra[i][0] = ok ? p.A[off] : 0.0;
-      }
+      double2 v = ok ? *reinterpret_cast<const double2 *>(p.A + 2 * off)
+                     : make_double2(0.0, 0.0);
+      ra[i][0] = v.x;
+      ra[i][1] = v.y * p.signA;
     }
 #pragma unroll
     for (int i = 0; i < EB; ++i) {
       const int ir = BKC ? i : 0, ik = BKC ? 0 : i;
       const bool ok = bColOk[ir] && bKok[ik];
       const int64_t off = bCol[ir] + bK[ik];
-      if constexpr (CPLX) {
-        double2 v = ok ? *reinterpret_cast<const double2 *>(p.B + 2 * off)
-                       : make_double2(0.0, 0.0);
-        rb[i][0] = v.x;
-        rb[i][1] = v.y * p.signB;
-      } else {
-        rb[i][0] = ok ? p.B[off] : 0.0;
-      }
+      double2 v = ok ? *reinterpret_cast<const double2 *>(p.B + 2 * off)
+                     : make_double2(0.0, 0.0);
+      rb[i][0] = v.x;
+      rb[i][1] = v.y * p.signB;
     }
   };
   auto store_lds = [&]() {
@@ -205,37 +197,35 @@ __global__ __launch_bounds__(kThreads, 2) void gett_kernel(KArgs p) {
 #pragma unroll
       for (int i = 0; i < MB; ++i) {
         ar[i] = As[0][kr][wm * WM + i * 16 + (lane & 15)];
-        if constexpr (CPLX) ai[i] = As[NPL - 1][kr][wm * WM + i * 16 + (lane & 15)];
+        ai[i] = As[1][kr][wm * WM + i * 16 + (lane & 15)];
       }
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
         br[j] = Bs[0][kr][wn * WN + j * 16 + (lane & 15)];
-        if constexpr (CPLX) bi[j] = Bs[NPL - 1][kr][wn * WN + j * 16 + (lane & 15)];
+        bi[j] = Bs[1][kr][wn * WN + j * 16 + (lane & 15)];
       }
 #pragma unroll
       for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j)
           accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], br[j], accR[i][j], 0, 0, 0);
-      if constexpr (CPLX) {
 #pragma unroll
-        for (int i = 0; i < MB; ++i)
+      for (int i = 0; i < MB; ++i)
 #pragma unroll
-          for (int j = 0; j < NB; ++j)
-            accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], bi[j], accI[i][j], 0, 0, 0);
+        for (int j = 0; j < NB; ++j)
+          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], bi[j], accI[i][j], 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < MB; ++i) {
-          const double nai = -ai[i];
+      for (int i = 0; i < MB; ++i) {
+        const double nai = -ai[i];
 #pragma unroll
-          for (int j = 0; j < NB; ++j)
-            accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai, bi[j], accR[i][j], 0, 0, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-            accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[i], br[j], accI[i][j], 0, 0, 0);
+        for (int j = 0; j < NB; ++j)
+          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai, bi[j], accR[i][j], 0, 0, 0);
       }
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[i], br[j], accI[i][j], 0, 0, 0);
     }
     if (more) {
       __syncthreads();
@@ -269,39 +259,39 @@ __global__ __launch_bounds__(kThreads, 2) void gett_kernel(KArgs p) {
         const double vi = accI[i][j][r];
         if (p.W) {
           const int64_t o = (static_cast<int64_t>(blockIdx.y) * p.M + m) * p.N + n;
-          if constexpr (CPLX) {
-            reinterpret_cast<double2 *>(p.W)[o] = make_double2(vr, vi);
-          } else {
-            p.W[o] = vr;
-          }
+          reinterpret_cast<double2 *>(p.W)[o] = make_double2(vr, vi);
         } else {
           const int64_t o = rc + cCol[j];
-          if constexpr (CPLX) {
-            double2 *c = reinterpret_cast<double2 *>(p.C) + o;
-            double2 out = make_double2(p.alpha * vr, p.alpha * vi);
-            if (p.beta != 0.0) {
-              const double2 old = *c;
-              out.x += p.beta * old.x;
-              out.y += p.beta * old.y;
-            }
-            *c = out;
-          } else {
-            double *c = p.C + o;
-            double out = p.alpha * vr;
-            if (p.beta != 0.0) out += p.beta * *c;
-            *c = out;
+          double2 *c = reinterpret_cast<double2 *>(p.C) + o;
+          double2 out = make_double2(p.alpha * vr, p.alpha * vi);
+          if (p.beta != 0.0) {
+            const double2 old = *c;
+            out.x += p.beta * old.x;
+            out.y += p.beta * old.y;
           }
+          *c = out;
         }
       }
     }
   }
 }
 
-// Complex GETT, second generation: NT/64 waves on a BM x BN complex tile,
-// one workgroup per CU.  LDS holds two K-stages (double buffer) with (re, im)
-// interleaved, so an MFMA operand pair is one 128-bit LDS read and a K-stage
-// needs one barrier.  Global loads for stage s+2 are issued while stage s is
-// multiplied; their K offsets were fetched a stage earlier still.
+// The GETT kernel of both fields: NT/64 waves on a BM x BN tile.  LDS holds two
+// K-stages (double buffer), complex elements with (re, im) interleaved, so an
+// MFMA operand pair is one 128-bit LDS read and a K-stage needs one barrier.
+// Global loads for stage s+2 are issued while stage s is multiplied; their K
+// offsets were fetched a stage earlier still.
+//
+// Bound by the FP64 matrix pipe.  What kept it from that was the vector work
+// between the MFMAs, which share their issue: the address of an operand element
+// is one add (row pointers and K offsets in registers, no bounds: padded K
+// tables, the last row repeated), conjugation is a sign-bit flip and elements
+// past K are zeroed in their one stage only, 35 vector instructions per stage
+// and wave of 32 x 32 instead of 82; and LDS reads and stores waited for in
+// place (fragments one k step ahead, no branch around the stores).  Measured
+// before -> after: complex ring (8192^3) 55.2 -> 51.9 ms, 85 TFLOP/s of 8 flops
+// per complex MAC; real ring (7533^3), which ran on a single-buffered kernel
+// with loads under branches, 19.8 -> 15.6 ms (55 TFLOP/s).
 //
 // M3 selects the three-product complex multiply (Gauss/Karatsuba):
 //   P1 = ar br, P2 = ai bi, P3 = (ar + ai)(br + bi),
@@ -319,13 +309,15 @@ constexpr int kZThreads = 512;
 // SEG2 adds a second K segment with its own operands (two contractions with
 // the same result index partition, e.g. a particle and a hole term of (T),
 // accumulated in one pass over C); a K-stage lies in one segment.
-template <int NT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC, bool M3,
-          bool DEEP, int MINW = 1, bool SEG2 = false>
+template <bool CPLX, int NT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC,
+          bool M3, bool DEEP, int MINW = 1, bool SEG2 = false>
 __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
+  using T = std::conditional_t<CPLX, double2, double>;
+  static_assert(CPLX || (!M3 && !SEG2), "complex forms");
   constexpr int MB = WM / 16, NB = WN / 16;
   constexpr int WAVES_N = BN / WN;
   static_assert((BM / WM) * (BN / WN) * 64 == NT, "one wave per WM x WN block");
-  static_assert(BK % 4 == 0, "BK multiple of the MFMA k");
+  static_assert(BK % 8 == 0, "an even number of MFMA k steps per stage");
   constexpr int EA = BM * BK / NT;
   constexpr int EB = BN * BK / NT;
   static_assert(EA >= 1 && EB >= 1, "tile too small");
@@ -335,20 +327,27 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
   constexpr int NRA = AKC ? EA : 1;
   constexpr int NKB = BKC ? 1 : EB;
   constexpr int NRB = BKC ? EB : 1;
-  // complex elements per LDS row: BM+1 shifts consecutive k-rows by one
+  // elements per LDS row.  Complex: BM+1 shifts consecutive k-rows by one
   // 16-byte bank group, so the column-wise stores of K-contiguous operands
   // and the row-wise 128-bit operand reads are both conflict-free per
-  // 16-lane pass
-  constexpr int LDA = BM + 1, LDB = BN + 1;
+  // 16-lane pass.  Real: a shift of 18 8-byte banks (of 32) spreads the 16
+  // k-rows of a column-wise store over all even banks and leaves two of 32
+  // lanes of a row-wise read in conflict.
+  constexpr int PAD = CPLX ? 1 : 18;
+  constexpr int LDA = BM + PAD, LDB = BN + PAD;
 
-  __shared__ double2 As[2][BK][LDA];
-  __shared__ double2 Bs[2][BK][LDB];
+  __shared__ T As[2][BK][LDA];
+  __shared__ T Bs[2][BK][LDB];
 
   const int t = threadIdx.x;
   const int ntiles = p.tilesM * p.tilesN;
+  // workgroups go round the 8 XCDs: each XCD takes a contiguous run of tiles
   int g = blockIdx.x;
-  if ((ntiles & 7) == 0) g = (g & 7) * (ntiles >> 3) + (g >> 3);
-  constexpr int GM = 8;
+  {
+    const int x = g & 7, q = ntiles >> 3, r = ntiles & 7;
+    g = x * q + min(x, r) + (g >> 3);
+  }
+  constexpr int GM = 1024 / BM;  // M-tiles of a group: 1024 rows
   const int per_group = GM * p.tilesN;
   const int first_m = (g / per_group) * GM;
   const int gsize = min(p.tilesM - first_m, GM);
@@ -365,123 +364,119 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
   auto b_n = [&](int i) { return BKC ? (t / BK + i * (NT / BK)) : (t % BN); };
   auto b_k = [&](int i) { return BKC ? (t % BK) : (t / BN + i * (NT / BN)); };
 
-  int64_t aRow[NRA], aRow2[SEG2 ? NRA : 1];
-  bool aRowOk[NRA];
+  // byte addresses of this thread's rows of A and columns of B; one past the
+  // edge reads the last row (its products are never stored)
+  const char *aRow[NRA], *aRow2[SEG2 ? NRA : 1];
 #pragma unroll
   for (int i = 0; i < NRA; ++i) {
-    const int64_t m = m0 + a_m(i);
-    aRowOk[i] = m < p.M;
-    aRow[i] = aRowOk[i] ? p.rowA[m] : 0;
-    if constexpr (SEG2) aRow2[i] = aRowOk[i] ? p.rowA2[m] : 0;
+    const int64_t m = min(m0 + a_m(i), p.M - 1);
+    aRow[i] = reinterpret_cast<const char *>(p.A) + p.rowA[m] * static_cast<int64_t>(sizeof(T));
+    if constexpr (SEG2)
+      aRow2[i] = reinterpret_cast<const char *>(p.A2) + p.rowA2[m] * static_cast<int64_t>(sizeof(T));
   }
-  int64_t bCol[NRB], bCol2[SEG2 ? NRB : 1];
-  bool bColOk[NRB];
+  const char *bCol[NRB], *bCol2[SEG2 ? NRB : 1];
 #pragma unroll
   for (int i = 0; i < NRB; ++i) {
-    const int64_t n = n0 + b_n(i);
-    bColOk[i] = n < p.N;
-    bCol[i] = bColOk[i] ? p.colB[n] : 0;
-    if constexpr (SEG2) bCol2[i] = bColOk[i] ? p.colB2[n] : 0;
+    const int64_t n = min(n0 + b_n(i), p.N - 1);
+    bCol[i] = reinterpret_cast<const char *>(p.B) + p.colB[n] * static_cast<int64_t>(sizeof(T));
+    if constexpr (SEG2)
+      bCol2[i] = reinterpret_cast<const char *>(p.B2) + p.colB2[n] * static_cast<int64_t>(sizeof(T));
   }
 
-  // K offsets of two stages: stage t's in buffer t & 1, indexed by
-  // constants (the loop below is unrolled by two), so no register copies
-  // wait for a load
-  int64_t aK[2][NKA], bK[2][NKB];
-  bool aKok[2][NKA], bKok[2][NKB];
-  bool segK[2] = {false, false};  // SEG2: the stage lies in the second segment
-  // every load is unconditional (out-of-range lanes read a valid element,
-  // kbeg < kend or offset 0, and are zeroed when stored to LDS): a load
-  // under a branch makes the compiler wait for it at the branch's end, which
-  // would stall the wave a whole K-stage early
-  auto load_koff = [&](int s, auto par_c) {
-    constexpr int pb = decltype(par_c)::value;
-    int64_t *ak = aK[pb], *bk = bK[pb];
-    bool *akok = aKok[pb], *bkok = bKok[pb];
-    const int64_t kb = kbeg + static_cast<int64_t>(s) * BK;
+  // K offsets of the next stage to load: its loads take them from the
+  // registers as they are issued, and the following stage's offsets are then
+  // loaded into the same registers, a whole stage before their use.  The K tables are padded with a valid offset (kTablePad
+  // entries past whole stages), so neither these loads nor the operand loads
+  // they address need a bound; what lies past K is zeroed when it is stored to
+  // LDS, in the one stage that holds K's end
+  int64_t aK[NKA], bK[NKB];
+  bool segK = false;  // SEG2: the stage lies in the second segment
+  auto load_koff = [&](int s) {
+    int64_t kb = kbeg + static_cast<int64_t>(s) * BK;
+    const int64_t *ca = p.colA, *rb = p.rowB;
     if constexpr (SEG2) {
       const bool sg = kb >= p.K1p;
-      segK[pb] = sg;
-      const int64_t k0 = sg ? p.K1p : 0, klen = sg ? p.K2 : p.K1;
-      const int64_t *ca = sg ? p.colA2 : p.colA, *rb = sg ? p.rowB2 : p.rowB;
-#pragma unroll
-      for (int i = 0; i < NKA; ++i) {
-        const int64_t k = kb + a_k(i);
-        akok[i] = k < kend && k - k0 < klen;
-        ak[i] = ca[akok[i] ? k - k0 : 0];
-      }
-#pragma unroll
-      for (int i = 0; i < NKB; ++i) {
-        const int64_t k = kb + b_k(i);
-        bkok[i] = k < kend && k - k0 < klen;
-        bk[i] = rb[bkok[i] ? k - k0 : 0];
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < NKA; ++i) {
-        const int64_t k = kb + a_k(i);
-        akok[i] = k < kend;
-        ak[i] = p.colA[akok[i] ? k : kbeg];
-      }
-#pragma unroll
-      for (int i = 0; i < NKB; ++i) {
-        const int64_t k = kb + b_k(i);
-        bkok[i] = k < kend;
-        bk[i] = p.rowB[bkok[i] ? k : kbeg];
-      }
+      segK = sg;
+      ca = sg ? p.colA2 : ca;
+      rb = sg ? p.rowB2 : rb;
+      kb = sg ? kb - p.K1p : kb;
     }
+#pragma unroll
+    for (int i = 0; i < NKA; ++i) aK[i] = ca[kb + a_k(i)];
+#pragma unroll
+    for (int i = 0; i < NKB; ++i) bK[i] = rb[kb + b_k(i)];
   };
 
   // staging registers; DEEP uses two sets, always indexed by constants
   constexpr int NSET = DEEP ? 2 : 1;
-  double2 ra[NSET][EA], rb[NSET][EB];
-  bool oka[NSET][EA], okb[NSET][EB];
+  T ra[NSET][EA], rb[NSET][EB];
   bool segS[NSET];  // SEG2: the registers hold a second-segment stage
-  auto load_data = [&](auto set_c, auto par_c) {
+  auto load_data = [&](auto set_c) {
     constexpr int q = decltype(set_c)::value;
-    constexpr int pb = decltype(par_c)::value;
     bool sg = false;
-    if constexpr (SEG2) sg = segK[pb];
+    if constexpr (SEG2) sg = segK;
     segS[q] = sg;
-    const double2 *A = reinterpret_cast<const double2 *>(sg ? p.A2 : p.A);
-    const double2 *B = reinterpret_cast<const double2 *>(sg ? p.B2 : p.B);
 #pragma unroll
     for (int i = 0; i < EA; ++i) {
       const int ir = AKC ? i : 0, ik = AKC ? 0 : i;
-      oka[q][i] = aRowOk[ir] && aKok[pb][ik];
-      int64_t row = aRow[ir];
+      const char *row = aRow[ir];
       if constexpr (SEG2) row = sg ? aRow2[ir] : row;
-      ra[q][i] = A[oka[q][i] ? row + aK[pb][ik] : 0];
+      ra[q][i] = reinterpret_cast<const T *>(row)[aK[ik]];
     }
 #pragma unroll
     for (int i = 0; i < EB; ++i) {
       const int ir = BKC ? i : 0, ik = BKC ? 0 : i;
-      okb[q][i] = bColOk[ir] && bKok[pb][ik];
-      int64_t col = bCol[ir];
+      const char *col = bCol[ir];
       if constexpr (SEG2) col = sg ? bCol2[ir] : col;
-      rb[q][i] = B[okb[q][i] ? col + bK[pb][ik] : 0];
+      rb[q][i] = reinterpret_cast<const T *>(col)[bK[ik]];
     }
   };
-  // out-of-range elements are zeroed and the conjugation signs (and the
-  // second segment's factor) applied here, a stage after the loads were
-  // issued
-  auto store_lds = [&](int buf, auto set_c) {
+  // conjugation flips the sign bit of the imaginary part (an integer operation:
+  // FP64 multiplies would take the MFMAs' cycles)
+  const int flipA = p.signA < 0.0 ? static_cast<int>(0x80000000u) : 0;
+  const int flipB = p.signB < 0.0 ? static_cast<int>(0x80000000u) : 0;
+  auto flip = [](double x, int mask) {
+    return __hiloint2double(__double2hiint(x) ^ mask, __double2loint(x));
+  };
+  // stage s from its registers to LDS: conjugation (and the second segment's
+  // factor) applied, elements past K zeroed
+  auto store_lds = [&](int s, int buf, auto set_c) {
     constexpr int q = decltype(set_c)::value;
-    const double2 zero = make_double2(0.0, 0.0);
-    double fa = 1.0, sa = p.signA, sb = p.signB;
-    if constexpr (SEG2) {
-      fa = segS[q] ? p.f2 : 1.0;
-      sa = segS[q] ? p.signA2 : sa;
-      sb = segS[q] ? p.signB2 : sb;
+    int64_t left = p.K - kbeg - static_cast<int64_t>(s) * BK;  // k of this stage within K
+    if constexpr (SEG2) left = segS[q] ? left : p.K1 - kbeg - static_cast<int64_t>(s) * BK;
+    if (left < BK) {
+#pragma unroll
+      for (int i = 0; i < EA; ++i)
+        if (a_k(i) >= left) ra[q][i] = T{};
+#pragma unroll
+      for (int i = 0; i < EB; ++i)
+        if (b_k(i) >= left) rb[q][i] = T{};
     }
+    if constexpr (CPLX) {
+      int fa = flipA, fb = flipB;
+      if constexpr (SEG2) {
+        fa = segS[q] ? (p.signA2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fa;
+        fb = segS[q] ? (p.signB2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fb;
+      }
 #pragma unroll
-    for (int i = 0; i < EA; ++i)
-      As[buf][a_k(i)][a_m(i)] =
-          oka[q][i] ? make_double2(fa * ra[q][i].x, fa * ra[q][i].y * sa) : zero;
+      for (int i = 0; i < EA; ++i) {
+        double x = ra[q][i].x, y = flip(ra[q][i].y, fa);
+        if constexpr (SEG2) {
+          const double f = segS[q] ? p.f2 : 1.0;
+          x *= f;
+          y *= f;
+        }
+        As[buf][a_k(i)][a_m(i)] = make_double2(x, y);
+      }
 #pragma unroll
-    for (int i = 0; i < EB; ++i)
-      Bs[buf][b_k(i)][b_n(i)] =
-          okb[q][i] ? make_double2(rb[q][i].x, rb[q][i].y * sb) : zero;
+      for (int i = 0; i < EB; ++i)
+        Bs[buf][b_k(i)][b_n(i)] = make_double2(rb[q][i].x, flip(rb[q][i].y, fb));
+    } else {
+#pragma unroll
+      for (int i = 0; i < EA; ++i) As[buf][a_k(i)][a_m(i)] = ra[q][i];
+#pragma unroll
+      for (int i = 0; i < EB; ++i) Bs[buf][b_k(i)][b_n(i)] = rb[q][i];
+    }
   };
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, DEEP ? 1 : 0>;
@@ -491,112 +486,132 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
   const int lane = t & 63;
   const int w = t >> 6;
   const int wm = w / WAVES_N, wn = w % WAVES_N;
-  // four-product: accR = re, accI = im; M3: accR = P1, accI = P2, accS = P3
-  dbl4 accR[MB][NB], accI[MB][NB], accS[M3 ? MB : 1][M3 ? NB : 1];
+  // real: accR; four-product: accR = re, accI = im; M3: accR = P1, accI = P2,
+  // accS = P3
+  dbl4 accR[MB][NB], accI[CPLX ? MB : 1][CPLX ? NB : 1], accS[M3 ? MB : 1][M3 ? NB : 1];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       accR[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
-      accI[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+      if constexpr (CPLX) accI[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
       if constexpr (M3) accS[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
     }
 
   // prologue: stage 0 in LDS buffer 0; stage 1 in registers (DEEP: stage 1
-  // in set 1, stage 2 in set 0)
+  // in set 1, stage 2 in set 0), the offsets of the stage after it under way
   if (nstages > 0) {
-    load_koff(0, P0{});
-    if (nstages > 1) load_koff(1, P1{});
-    load_data(S0{}, P0{});
-    store_lds(0, S0{});
-    if (nstages > 1) {
-      if (nstages > 2) load_koff(2, P0{});
-      load_data(S1{}, P1{});
-      if (DEEP && nstages > 2) {
-        if (nstages > 3) load_koff(3, P1{});
-        load_data(S0{}, P0{});
-      }
+    load_koff(0);
+    load_data(S0{});
+    load_koff(1);
+    if constexpr (DEEP) {
+      load_data(S1{});
+      load_koff(2);
     }
+    store_lds(0, 0, S0{});
+    load_data(S0{});
+    load_koff(DEEP ? 3 : 2);
     __syncthreads();
   }
-  // one K-stage: multiply LDS buffer s&1, then move stage s+1 from its
-  // registers to the other buffer and load the next stage into them
+  // operand fragments of two k steps: step kq + 1 is read from LDS before the
+  // MFMAs of step kq are issued, so a wave does not wait for LDS between them
+  constexpr int KQ = BK / 4;
+  T fa[2][MB], fb[2][NB];
+  auto load_frag = [&](int buf, int kq, int q) {
+    const int kr = kq * 4 + (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) fa[q][i] = As[buf][kr][wm * WM + i * 16 + (lane & 15)];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) fb[q][j] = Bs[buf][kr][wn * WN + j * 16 + (lane & 15)];
+  };
+  auto multiply = [&](int q) {
+    const T(&a)[MB] = fa[q];
+    const T(&b)[NB] = fb[q];
+    if constexpr (!CPLX) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], accR[i][j], 0, 0, 0);
+    } else if constexpr (M3) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].x, accR[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, b[j].y, accI[i][j], 0, 0, 0);
+      double bs[NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) bs[j] = b[j].x + b[j].y;
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const double as = a[i].x + a[i].y;
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          accS[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(as, bs[j], accS[i][j], 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].x, accR[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].y, accI[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const double nai = -a[i].y;
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai, b[j].y, accR[i][j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, b[j].x, accI[i][j], 0, 0, 0);
+    }
+  };
+  // one K-stage: multiply LDS buffer s&1, move stage s+1 from its
+  // registers to the other buffer and load a later stage into them, half way
+  // through this stage's MFMAs so that the wave keeps issuing MFMAs around its
+  // memory instructions.  Nothing here stands under a branch (a stage past the
+  // end reads valid elements that are never used): at a branch's end the
+  // compiler would wait for every LDS operation in flight.  The stage's one
+  // barrier stands before the MFMAs of its last k step, whose fragments are in
+  // registers: behind it the other buffer is complete, so the next stage's
+  // first fragments are read under those MFMAs, and this stage's buffer is
+  // free, every wave having read its last step
   auto stage = [&](int s, auto set_c, auto par_c) {
     constexpr int par = decltype(par_c)::value;  // s & 1
-    const int buf = s & 1;
     constexpr int AHEAD = DEEP ? 3 : 2;  // stage loaded into the freed registers
-    using PD = std::integral_constant<int, (par + AHEAD) & 1>;      // stage s+AHEAD
-    using PN = std::integral_constant<int, (par + AHEAD + 1) & 1>;  // stage s+AHEAD+1
-    // stage s+1 moves from its registers to the other LDS buffer (read in
-    // stage s-1, released by that stage's barrier) and stage s+AHEAD is
-    // loaded half way through this stage's MFMAs, so the wave keeps issuing
-    // MFMAs around its memory instructions
-    auto advance = [&]() {
-      if (s + 1 < nstages) {
-        store_lds(buf ^ 1, set_c);  // stage s+1
-        if (s + AHEAD < nstages) {
-          if (s + AHEAD + 1 < nstages) load_koff(s + AHEAD + 1, PN{});
-          load_data(set_c, PD{});
-        }
-      }
-    };
 #pragma unroll
-    for (int kq = 0; kq < BK / 4; ++kq) {
-      if (kq == BK / 8) advance();
-      const int kr = kq * 4 + (lane >> 4);
-      double2 a[MB], b[NB];
-#pragma unroll
-      for (int i = 0; i < MB; ++i) a[i] = As[buf][kr][wm * WM + i * 16 + (lane & 15)];
-#pragma unroll
-      for (int j = 0; j < NB; ++j) b[j] = Bs[buf][kr][wn * WN + j * 16 + (lane & 15)];
-      if constexpr (M3) {
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-            accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].x, accR[i][j], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-            accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, b[j].y, accI[i][j], 0, 0, 0);
-        double bs[NB];
-#pragma unroll
-        for (int j = 0; j < NB; ++j) bs[j] = b[j].x + b[j].y;
-#pragma unroll
-        for (int i = 0; i < MB; ++i) {
-          const double as = a[i].x + a[i].y;
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-            accS[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(as, bs[j], accS[i][j], 0, 0, 0);
-        }
+    for (int kq = 0; kq < KQ; ++kq) {
+      if (kq + 1 < KQ) {
+        load_frag(par, kq + 1, (kq + 1) & 1);
       } else {
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-            accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].x, accR[i][j], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-            accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].x, b[j].y, accI[i][j], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < MB; ++i) {
-          const double nai = -a[i].y;
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-            accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(nai, b[j].y, accR[i][j], 0, 0, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-            accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].y, b[j].x, accI[i][j], 0, 0, 0);
+        __syncthreads();
+        load_frag(par ^ 1, 0, 0);
+      }
+      // the scheduler would sink the reads below the MFMAs to their uses, and
+      // raise what waits for the loads above them
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(kq & 1);
+      if (kq == KQ / 2 - 1) {
+        store_lds(s + 1, par ^ 1, set_c);
+        load_data(set_c);           // stage s+AHEAD
+        load_koff(s + AHEAD + 1);
       }
     }
-    __syncthreads();
   };
+  if (nstages > 0) load_frag(0, 0, 0);
   // stage s+1 sits in set (s+1)&1 (DEEP) or in the single set
   for (int s = 0; s < nstages; s += 2) {
     stage(s, S1{}, P0{});
@@ -622,64 +637,103 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
       for (int j = 0; j < NB; ++j) {
         if (!cColOk[j]) continue;
         const int64_t n = n0 + wn * WN + j * 16 + (lane & 15);
-        double vr = accR[i][j][r];
-        double vi = accI[i][j][r];
-        if constexpr (M3) {
-          const double p1 = vr, p2 = vi;
-          vr = p1 - p2;
-          vi = accS[i][j][r] - (p1 + p2);
-        }
-        if (p.W) {
-          const int64_t o = (static_cast<int64_t>(blockIdx.y) * p.M + m) * p.N + n;
-          reinterpret_cast<double2 *>(p.W)[o] = make_double2(vr, vi);
-        } else {
-          double2 *c = reinterpret_cast<double2 *>(p.C) + rc + cCol[j];
-          double2 out = make_double2(p.alpha * vr, p.alpha * vi);
-          if (p.beta != 0.0) {
-            const double2 old = *c;
-            out.x += p.beta * old.x;
-            out.y += p.beta * old.y;
+        if constexpr (CPLX) {
+          double vr = accR[i][j][r];
+          double vi = accI[i][j][r];
+          if constexpr (M3) {
+            const double p1 = vr, p2 = vi;
+            vr = p1 - p2;
+            vi = accS[i][j][r] - (p1 + p2);
           }
-          *c = out;
+          if (p.W) {
+            const int64_t o = (static_cast<int64_t>(blockIdx.y) * p.M + m) * p.N + n;
+            reinterpret_cast<double2 *>(p.W)[o] = make_double2(vr, vi);
+          } else {
+            double2 *c = reinterpret_cast<double2 *>(p.C) + rc + cCol[j];
+            double2 out = make_double2(p.alpha * vr, p.alpha * vi);
+            if (p.beta != 0.0) {
+              const double2 old = *c;
+              out.x += p.beta * old.x;
+              out.y += p.beta * old.y;
+            }
+            *c = out;
+          }
+        } else {
+          const double vr = accR[i][j][r];
+          if (p.W) {
+            p.W[(static_cast<int64_t>(blockIdx.y) * p.M + m) * p.N + n] = vr;
+          } else {
+            double *c = p.C + rc + cCol[j];
+            double out = p.alpha * vr;
+            if (p.beta != 0.0) out += p.beta * *c;
+            *c = out;
+          }
         }
       }
     }
   }
 }
 
-// C[rowC[m] + colC[n]] = alpha * sum_s W[s][m][n] + beta * C, fixed order
-template <bool CPLX>
+// C[rowC[m] + colC[n]] = alpha * sum_s W[s][m][n] + beta * C.  Bound by the
+// partials' HBM (or L2) reads, or, for few elements and many splits, by their
+// latency: a block takes 256 / G consecutive elements and G interleaved groups
+// of splits, four loads in flight per thread; the group sums are added in LDS.
+// Both orders are fixed, so the result is reproducible.
+template <bool CPLX, int G>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(
-    const double *W, double *C, const int64_t *rowC, const int64_t *colC,
-    int64_t M, int64_t N, int splits, double alpha, double beta) {
-  const int64_t total = M * N;
-  for (int64_t e = blockIdx.x * 256ll + threadIdx.x; e < total;
-       e += static_cast<int64_t>(gridDim.x) * 256) {
-    const int64_t m = e / N, n = e - m * N;
-    const int64_t o = rowC[m] + colC[n];
-    if constexpr (CPLX) {
-      const double2 *w = reinterpret_cast<const double2 *>(W);
-      double sr = 0.0, si = 0.0;
-      for (int s = 0; s < splits; ++s) {
-        const double2 v = w[s * total + e];
-        sr += v.x;
-        si += v.y;
+    const double *W, double *C, const int64_t *rowC, const int64_t *colC, uint32_t total,
+    uint32_t N, int splits, double alpha, double beta) {
+  using T = std::conditional_t<CPLX, double2, double>;
+  constexpr uint32_t E = 256 / G;
+  __shared__ T part[G][E];
+  const uint32_t u = threadIdx.x % E, g = threadIdx.x / E;
+  const T *w = reinterpret_cast<const T *>(W);
+  for (uint32_t e0 = blockIdx.x * E; e0 < total; e0 += gridDim.x * E) {
+    const uint32_t e = e0 + u;
+    const uint32_t ec = e < total ? e : total - 1;
+    T acc[4] = {};
+    auto add = [](T &a, const T &b) {
+      if constexpr (CPLX) {
+        a.x += b.x;
+        a.y += b.y;
+      } else {
+        a += b;
       }
-      double2 *c = reinterpret_cast<double2 *>(C) + o;
-      double2 out = make_double2(alpha * sr, alpha * si);
-      if (beta != 0.0) {
-        const double2 old = *c;
-        out.x += beta * old.x;
-        out.y += beta * old.y;
+    };
+    int s = g;
+    for (; s + 3 * G < splits; s += 4 * G)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) add(acc[q], w[static_cast<int64_t>(s + q * G) * total + ec]);
+    for (; s < splits; s += G) add(acc[0], w[static_cast<int64_t>(s) * total + ec]);
+    add(acc[0], acc[1]);
+    add(acc[2], acc[3]);
+    add(acc[0], acc[2]);
+    if constexpr (G > 1) {
+      part[g][u] = acc[0];
+      __syncthreads();
+      if (g == 0)
+#pragma unroll
+        for (int q = 1; q < G; ++q) add(acc[0], part[q][u]);
+    }
+    if (g == 0 && e < total) {
+      const uint32_t m = e / N, n = e - m * N;
+      const int64_t o = rowC[m] + colC[n];
+      T *c = reinterpret_cast<T *>(C) + o;
+      T out;
+      if constexpr (CPLX) {
+        out = make_double2(alpha * acc[0].x, alpha * acc[0].y);
+        if (beta != 0.0) {
+          const T old = *c;
+          out.x += beta * old.x;
+          out.y += beta * old.y;
+        }
+      } else {
+        out = alpha * acc[0];
+        if (beta != 0.0) out += beta * *c;
       }
       *c = out;
-    } else {
-      double sr = 0.0;
-      for (int s = 0; s < splits; ++s) sr += W[s * total + e];
-      double out = alpha * sr;
-      if (beta != 0.0) out += beta * C[o];
-      C[o] = out;
     }
+    if constexpr (G > 1) __syncthreads();  // part is written again
   }
 }
 
@@ -727,64 +781,65 @@ __global__ __launch_bounds__(256) void sum_kernel(SumArgs p) {
   }
 }
 
-template <bool CPLX, int BM, int BN, int BK, int WM, int WN>
+template <int BM, int BN, int BK, int WM, int WN>
 void dispatch_gett(const GettLaunch &L, const KArgs &args, dim3 grid, hipStream_t s) {
   if (L.a_kcontig && L.b_kcontig)
-    gett_kernel<CPLX, BM, BN, BK, WM, WN, true, true><<<grid, kThreads, 0, s>>>(args);
+    gett_kernel<BM, BN, BK, WM, WN, true, true><<<grid, kThreads, 0, s>>>(args);
   else if (L.a_kcontig)
-    gett_kernel<CPLX, BM, BN, BK, WM, WN, true, false><<<grid, kThreads, 0, s>>>(args);
+    gett_kernel<BM, BN, BK, WM, WN, true, false><<<grid, kThreads, 0, s>>>(args);
   else if (L.b_kcontig)
-    gett_kernel<CPLX, BM, BN, BK, WM, WN, false, true><<<grid, kThreads, 0, s>>>(args);
+    gett_kernel<BM, BN, BK, WM, WN, false, true><<<grid, kThreads, 0, s>>>(args);
   else
-    gett_kernel<CPLX, BM, BN, BK, WM, WN, false, false><<<grid, kThreads, 0, s>>>(args);
+    gett_kernel<BM, BN, BK, WM, WN, false, false><<<grid, kThreads, 0, s>>>(args);
 }
 
-template <int NT, int BM, int BN, int BK, int WM, int WN, bool M3, bool DEEP = false,
-          int MINW = 1, bool SEG2 = false>
+template <bool CPLX, int NT, int BM, int BN, int BK, int WM, int WN, bool M3,
+          bool DEEP = false, int MINW = 1, bool SEG2 = false>
 void dispatch_zgett(const GettLaunch &L, const KArgs &args, dim3 grid, hipStream_t s) {
   if (L.a_kcontig && L.b_kcontig)
-    zgett_kernel<NT, BM, BN, BK, WM, WN, true, true, M3, DEEP, MINW, SEG2>
+    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, true, true, M3, DEEP, MINW, SEG2>
         <<<grid, NT, 0, s>>>(args);
   else if (L.a_kcontig)
-    zgett_kernel<NT, BM, BN, BK, WM, WN, true, false, M3, DEEP, MINW, SEG2>
+    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, true, false, M3, DEEP, MINW, SEG2>
         <<<grid, NT, 0, s>>>(args);
   else if (L.b_kcontig)
-    zgett_kernel<NT, BM, BN, BK, WM, WN, false, true, M3, DEEP, MINW, SEG2>
+    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, false, true, M3, DEEP, MINW, SEG2>
         <<<grid, NT, 0, s>>>(args);
   else
-    zgett_kernel<NT, BM, BN, BK, WM, WN, false, false, M3, DEEP, MINW, SEG2>
+    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, false, false, M3, DEEP, MINW, SEG2>
         <<<grid, NT, 0, s>>>(args);
 }
 
-// tile shapes (complex elements): first generation 128x64; second 128x128;
-// three-product kernels 128x64 with 8 waves of 32x32 (generation 3) or 4
-// waves of 64x32 (generation 4); real 128x128
+// Tiles of the GETT kernel (complex: generation 3).  The waves of a workgroup
+// own 32 x 32 (complex) or 64 x 64 (real) of a large tile, 32 x 32 of a medium
+// and 16 x 16 of a small one; `cap` workgroups share a CU (LDS and registers),
+// so one's barriers, first loads and epilogue pass under another's MFMAs.
+// Measured times in microseconds: `stage`, one 16-k stage of one workgroup on a
+// CU that is full of them (its MFMAs alone take 64 cycles per 16x16x4 block,
+// three per complex block, on four SIMDs); `lone`, the same where it has the CU
+// to itself and nothing hides a stage's latencies; `ends`, the first loads and
+// the epilogue.
+enum class Tile : int { Large = 0, Medium = 1, Small = 2 };
+struct TileShape {
+  int BM, BN, cap;
+  double stage, lone, ends;
+};
+constexpr int kZ3BK = 16;  // K-stage of every tile
+constexpr TileShape kComplexTiles[3] = {
+    {128, 64, 1, 3.3, 3.3, 8.0}, {64, 64, 2, 1.72, 2.0, 6.0}, {32, 32, 4, 0.55, 0.45, 4.0}};
+constexpr TileShape kRealTiles[3] = {
+    {128, 128, 2, 2.4, 4.5, 8.0}, {64, 64, 3, 0.63, 0.76, 5.7}, {32, 32, 4, 0.28, 0.3, 4.0}};
+// other complex generations: first 128x64; second 128x128; fourth and fifth 128x64
 constexpr int kCBM = 128, kCBN = 64, kCBK = 16, kCWM = 64, kCWN = 32;
 constexpr int kZBM = 128, kZBN = 128, kZBK = 16, kZWM = 64, kZWN = 32;
-constexpr int kZ3BM = 128, kZ3BN = 64, kZ3BK = 16;
-// short K (at most kShortK): generation 3's 32x32 wave tiles, 4 waves on a
-// 64x64 tile, two workgroups per CU (66.5 KB of LDS each)
-constexpr int kZSBM = 64, kZSBN = 64, kShortK = 256;
-constexpr int kRBM = 128, kRBN = 128, kRBK = 16, kRWM = 64, kRWN = 64;
 
 int g_complex_generation = 3;
 
-bool short_k(Field f, int64_t K, bool two_segments = false) {
-  return f == Field::Complex && g_complex_generation == 3 && K <= kShortK && !two_segments;
-}
-
-void tile_of(Field f, int64_t K, int &BM, int &BN, int &BK) {
-  if (f == Field::Real) {
-    BM = kRBM; BN = kRBN; BK = kRBK;
-  } else if (g_complex_generation == 1) {
-    BM = kCBM; BN = kCBN; BK = kCBK;
-  } else if (short_k(f, K)) {
-    BM = kZSBM; BN = kZSBN; BK = kZ3BK;
-  } else if (g_complex_generation >= 3) {
-    BM = kZ3BM; BN = kZ3BN; BK = kZ3BK;
-  } else {
-    BM = kZBM; BN = kZBN; BK = kZBK;
-  }
+TileShape tile_shape(Field f, Tile t) {
+  if (f == Field::Real) return kRealTiles[static_cast<int>(t)];
+  if (g_complex_generation == 2) return {kZBM, kZBN, 1, 6.6, 6.6, 10.0};
+  if (g_complex_generation == 1) return {kCBM, kCBN, 2, 4.0, 4.0, 10.0};
+  return kComplexTiles[static_cast<int>(t)];
 }
 
 inline int grid_for(int64_t n) {
@@ -801,7 +856,8 @@ std::string gett_variant(const GettLaunch &L) {
   std::string n = L.field == Field::Complex ? "gett_c64" : "gett_f64";
   n += L.a_kcontig ? "_ak" : "_am";
   n += L.b_kcontig ? "_bk" : "_bn";
-  if (short_k(L.field, L.K, L.A2 != nullptr)) n += "_shortk";
+  if (L.tile == 1) n += "_t64";
+  if (L.tile == 2) n += "_t32";
   if (L.A2) n += "_seg2";
   return n;
 }
@@ -812,8 +868,9 @@ void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
   const bool seg2 = L.A2 != nullptr;
   CC4S_ASSERT(!seg2 || (cplx && g_complex_generation == 3),
               "two-segment contractions need the complex generation-3 kernel");
-  int BM, BN, BK;
-  tile_of(L.field, seg2 ? kShortK + 1 : L.K, BM, BN, BK);
+  const Tile tile = static_cast<Tile>(L.tile);
+  const TileShape shape = tile_shape(L.field, tile);
+  const int BM = shape.BM, BN = shape.BN, BK = kZ3BK;
   KArgs a;
   a.A = static_cast<const double *>(L.A);
   a.B = static_cast<const double *>(L.B);
@@ -840,23 +897,34 @@ void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
   a.signB2 = L.conjB2 ? -1.0 : 1.0;
   dim3 grid(a.tilesM * a.tilesN, L.splits);
   if (start) CC4S_HIP(hipEventRecord(start, s));
-  if (seg2)
-    dispatch_zgett<512, kZ3BM, kZ3BN, kZ3BK, 32, 32, true, false, 1, true>(L, a, grid, s);
-  else if (cplx && g_complex_generation == 2)
-    dispatch_zgett<kZThreads, kZBM, kZBN, kZBK, kZWM, kZWN, false>(L, a, grid, s);
-  else if (short_k(L.field, L.K))
-    dispatch_zgett<256, kZSBM, kZSBN, kZ3BK, 32, 32, true, false, 2>(L, a, grid, s);
-
-  else if (cplx && g_complex_generation == 3)
-    dispatch_zgett<512, kZ3BM, kZ3BN, kZ3BK, 32, 32, true>(L, a, grid, s);
-  else if (cplx && g_complex_generation == 4)
-    dispatch_zgett<256, kZ3BM, kZ3BN, kZ3BK, 64, 32, true>(L, a, grid, s);
-  else if (cplx && g_complex_generation == 5)
-    dispatch_zgett<512, kZ3BM, kZ3BN, kZ3BK, 32, 32, true, true>(L, a, grid, s);
-  else if (cplx)
-    dispatch_gett<true, kCBM, kCBN, kCBK, kCWM, kCWN>(L, a, grid, s);
-  else
-    dispatch_gett<false, kRBM, kRBN, kRBK, kRWM, kRWN>(L, a, grid, s);
+  if (cplx && g_complex_generation == 3) {
+    if (seg2 && tile == Tile::Large)
+      dispatch_zgett<true, 512, 128, 64, 16, 32, 32, true, false, 1, true>(L, a, grid, s);
+    else if (seg2 && tile == Tile::Medium)
+      dispatch_zgett<true, 256, 64, 64, 16, 32, 32, true, false, 2, true>(L, a, grid, s);
+    else if (seg2)
+      dispatch_zgett<true, 256, 32, 32, 16, 16, 16, true, false, 4, true>(L, a, grid, s);
+    else if (tile == Tile::Large)
+      dispatch_zgett<true, 512, 128, 64, 16, 32, 32, true>(L, a, grid, s);
+    else if (tile == Tile::Medium)
+      dispatch_zgett<true, 256, 64, 64, 16, 32, 32, true, false, 2>(L, a, grid, s);
+    else
+      dispatch_zgett<true, 256, 32, 32, 16, 16, 16, true, false, 4>(L, a, grid, s);
+  } else if (cplx && g_complex_generation == 2) {
+    dispatch_zgett<true, kZThreads, kZBM, kZBN, kZBK, kZWM, kZWN, false>(L, a, grid, s);
+  } else if (cplx && g_complex_generation == 4) {
+    dispatch_zgett<true, 256, 128, 64, 16, 64, 32, true>(L, a, grid, s);
+  } else if (cplx && g_complex_generation == 5) {
+    dispatch_zgett<true, 512, 128, 64, 16, 32, 32, true, true>(L, a, grid, s);
+  } else if (cplx) {
+    dispatch_gett<kCBM, kCBN, kCBK, kCWM, kCWN>(L, a, grid, s);
+  } else if (tile == Tile::Large) {
+    dispatch_zgett<false, 256, 128, 128, 16, 64, 64, false, false, 2>(L, a, grid, s);
+  } else if (tile == Tile::Medium) {
+    dispatch_zgett<false, 256, 64, 64, 16, 32, 32, false, false, 3>(L, a, grid, s);
+  } else {
+    dispatch_zgett<false, 256, 32, 32, 16, 16, 16, false, false, 4>(L, a, grid, s);
+  }
   CC4S_HIP(hipGetLastError());
   if (stop) CC4S_HIP(hipEventRecord(stop, s));
   if (L.splits > 1)
@@ -868,13 +936,21 @@ void launch_splitk_reduce(Field f, const double *W, double *C,
                           const int64_t *rowC, const int64_t *colC, int64_t M,
                           int64_t N, int splits, double alpha, double beta,
                           hipStream_t s) {
-  const int64_t total = M * N;
-  if (f == Field::Complex)
-    splitk_reduce_kernel<true><<<grid_for(total), 256, 0, s>>>(
-        W, C, rowC, colC, M, N, splits, alpha, beta);
+  CC4S_ASSERT(M * N < (int64_t(1) << 31), "split-K result too large");
+  const uint32_t total = static_cast<uint32_t>(M * N), n32 = static_cast<uint32_t>(N);
+  auto run = [&](auto kernel, int G) {
+    kernel<<<grid_for(static_cast<int64_t>(total) * G), 256, 0, s>>>(W, C, rowC, colC, total, n32,
+                                                                   splits, alpha, beta);
+  };
+  // groups of splits while the elements alone leave the chip idle (under 64 K
+  // threads) and every group still has several splits
+  const bool c = f == Field::Complex;
+  if (total < 16384 && splits >= 32)
+    c ? run(splitk_reduce_kernel<true, 16>, 16) : run(splitk_reduce_kernel<false, 16>, 16);
+  else if (total < 65536 && splits >= 8)
+    c ? run(splitk_reduce_kernel<true, 4>, 4) : run(splitk_reduce_kernel<false, 4>, 4);
   else
-    splitk_reduce_kernel<false><<<grid_for(total), 256, 0, s>>>(
-        W, C, rowC, colC, M, N, splits, alpha, beta);
+    c ? run(splitk_reduce_kernel<true, 1>, 1) : run(splitk_reduce_kernel<false, 1>, 1);
   CC4S_HIP(hipGetLastError());
 }
 
@@ -886,6 +962,7 @@ struct GettPlan {
   int64_t M = 0, N = 0, K = 0;
   bool swap = false, a_kc = true, b_kc = true;
   int splits = 1;
+  Tile tile = Tile::Large;
   DeviceBuffer tables;
   const int64_t *rowA, *colA, *rowB, *colB, *rowC, *colC;
   // two-segment plans: the second contraction's tables; swap2 tells that
@@ -986,6 +1063,14 @@ std::string plan_key(const View &A, const View &B, const View &C) {
   return k.str();
 }
 
+// K offset tables are padded with their first entry, a valid offset, to whole
+// K-stages and past them: a kernel reads its table up to four stages ahead
+constexpr int64_t kTablePad = 5 * kZ3BK;
+void pad_k(std::vector<int64_t> &v) {
+  if (v.empty()) return;
+  v.resize((v.size() + kZ3BK - 1) / kZ3BK * kZ3BK + kTablePad, v.front());
+}
+
 // offsets of every multi-index of `group` (first listed index fastest)
 std::vector<int64_t> offsets(const View &v, const std::string &group,
                              const View &shape) {
@@ -999,6 +1084,59 @@ std::vector<int64_t> offsets(const View &v, const std::string &group,
     block *= L;
   }
   return out;
+}
+
+}  // namespace
+
+namespace {
+
+// Tile and split count with the smallest estimated time (microseconds):
+//   - workgroups run in waves of 256 CUs x cap; a wave takes its K-stages at the
+//     full CU's rate for the workgroups that share a CU, or at a lone
+//     workgroup's latency where that is longer, and its ends, half of them under
+//     another workgroup where several share a CU;
+//   - split-K adds a reduction launch and its partials' traffic (4 TB/s).
+// Measured over the statements of one pass, fixed choice (128 x 64 complex,
+// 128 x 128 real, split to four workgroups per slot) -> this one; the fixed
+// choice stays the better one only where it is also this one's:
+//   complex No=4 Nv=16 221 -> 103 us, No=12 Nv=60 774 -> 605 us, No=20 Nv=150
+//   21.7 -> 19.4 ms; real No=8 Nv=40 346 -> 167 us, No=20 Nv=150 10.4 -> 9.1 ms.
+void choose_tile(Field f, int64_t M, int64_t N, int64_t K, size_t max_workspace, Tile &tile,
+                 int &splits) {
+  constexpr double kReduce = 3.5, kBytesPerUs = 4e6;
+  tile = Tile::Large;
+  splits = 1;
+  if (M <= 0 || N <= 0 || K <= 0) return;
+  const int64_t kstages = (K + kZ3BK - 1) / kZ3BK;
+  const double es = static_cast<double>(scalar_bytes(f));
+  const bool fixed_tile = f == Field::Complex && g_complex_generation != 3;
+  double best = -1;
+  for (int t = 0; t < (fixed_tile ? 1 : 3); ++t) {
+    const TileShape s = tile_shape(f, static_cast<Tile>(t));
+    const int64_t tiles = ((M + s.BM - 1) / s.BM) * ((N + s.BN - 1) / s.BN);
+    if (tiles >= (int64_t(1) << 31)) continue;
+    const int64_t per = 256 * s.cap;
+    // every count to 16, then steps of about 6 %
+    for (int64_t sp = 1; sp <= std::min<int64_t>(1024, std::max<int64_t>(1, kstages / 2));
+         sp += std::max<int64_t>(1, sp / 16)) {
+      if (sp > 1 && (static_cast<double>(sp) * M * N * es > static_cast<double>(max_workspace) ||
+                     M * N >= (int64_t(1) << 31) || tiles * sp > 4 * per))
+        break;
+      const double n = static_cast<double>((kstages + sp - 1) / sp);
+      auto wave = [&](double c) {
+        return n * std::max(c * s.stage, s.lone) + (s.cap > 1 && c > 1 ? 0.5 : 1.0) * s.ends;
+      };
+      const int64_t W = tiles * sp, full = W / per, rem = W % per;
+      double cost = static_cast<double>(full) * wave(s.cap);
+      if (rem) cost += wave(static_cast<double>((rem + 255) / 256));
+      if (sp > 1) cost += kReduce + 2.0 * static_cast<double>(sp) * M * N * es / kBytesPerUs;
+      if (best < 0 || cost < best) {
+        best = cost;
+        tile = static_cast<Tile>(t);
+        splits = static_cast<int>(sp);
+      }
+    }
+  }
 }
 
 }  // namespace
@@ -1065,6 +1203,8 @@ GettPlan &ContractionEngine::plan_for(const View &A0, const View &B0,
   plan->K = static_cast<int64_t>(colA.size());
   if (Ki.empty()) plan->K = 1;  // outer product: one k with offset 0
 
+  pad_k(colA);
+  pad_k(rowB);
   std::vector<int64_t> all;
   auto append = [&all](const std::vector<int64_t> &v) {
     all.insert(all.end(), v.begin(), v.end());
@@ -1081,24 +1221,7 @@ GettPlan &ContractionEngine::plan_for(const View &A0, const View &B0,
   plan->rowC = base; base += rowC.size();
   plan->colC = base;
 
-  // split K when the tile grid cannot fill the 256 CUs twice over
-  int BM, BN, BK;
-  tile_of(C.field, plan->K, BM, BN, BK);
-  // workgroups per CU: one for the 512-thread complex kernels, two otherwise
-  const int slots = 256 * ((C.field == Field::Complex && g_complex_generation >= 2 &&
-                            !short_k(C.field, plan->K)) ? 1 : 2);
-  const int64_t tiles = ((plan->M + BM - 1) / BM) * ((plan->N + BN - 1) / BN);
-  const int64_t kstages = (plan->K + BK - 1) / BK;
-  int64_t splits = 1;
-  if (tiles < 2 * slots) {
-    splits = std::min<int64_t>((4 * slots + tiles - 1) / tiles, kstages / 4);
-    const size_t es = scalar_bytes(C.field);
-    while (splits > 1 &&
-           static_cast<size_t>(splits) * plan->M * plan->N * es > max_workspace)
-      --splits;
-    splits = std::max<int64_t>(1, std::min<int64_t>(splits, 256));
-  }
-  plan->splits = static_cast<int>(splits);
+  choose_tile(C.field, plan->M, plan->N, plan->K, max_workspace, plan->tile, plan->splits);
 
   auto &ref = *plan;
   plans_.emplace(key, std::move(plan));
@@ -1165,6 +1288,8 @@ GettPlan &ContractionEngine::plan_for2(const View &A1, const View &B1, const Vie
   plan->K1p = (P1.K + kZ3BK - 1) / kZ3BK * kZ3BK;
   plan->K2 = static_cast<int64_t>(colA.size());
   plan->K = plan->K1p + plan->K2;
+  pad_k(colA);
+  pad_k(rowB);
   std::vector<int64_t> all;
   all.insert(all.end(), rowA.begin(), rowA.end());
   all.insert(all.end(), colA.begin(), colA.end());
@@ -1180,18 +1305,7 @@ GettPlan &ContractionEngine::plan_for2(const View &A1, const View &B1, const Vie
   plan->colB2 = base;
   plan->rowA = P1.rowA; plan->colA = P1.colA; plan->rowB = P1.rowB; plan->colB = P1.colB;
   plan->rowC = P1.rowC; plan->colC = P1.colC;
-  // split K when the tile grid cannot fill the CUs twice over (one
-  // workgroup per CU)
-  const int64_t tiles = ((plan->M + kZ3BM - 1) / kZ3BM) * ((plan->N + kZ3BN - 1) / kZ3BN);
-  const int64_t kstages = plan->K / kZ3BK + 1;
-  int64_t splits = 1;
-  if (tiles < 512) {
-    splits = std::min<int64_t>((1024 + tiles - 1) / tiles, kstages / 4);
-    while (splits > 1 && static_cast<size_t>(splits) * plan->M * plan->N * 16 > max_workspace)
-      --splits;
-    splits = std::max<int64_t>(1, std::min<int64_t>(splits, 256));
-  }
-  plan->splits = static_cast<int>(splits);
+  choose_tile(C.field, plan->M, plan->N, plan->K, max_workspace, plan->tile, plan->splits);
   auto &ref = *plan;
   plans_.emplace(key, std::move(plan));
   return ref;
@@ -1229,6 +1343,7 @@ void ContractionEngine::contract2(double alpha, const View &A1, const View &B1,
   L.K1 = P.K1; L.K1p = P.K1p; L.K2 = P.K2;
   L.f2 = alpha2 / alpha;
   L.splits = P.splits;
+  L.tile = static_cast<int>(P.tile);
   L.alpha = alpha; L.beta = beta;
   L.a_kcontig = P.a_kc; L.b_kcontig = P.b_kc;
   L.W = nullptr;
@@ -1266,6 +1381,7 @@ void ContractionEngine::contract(double alpha, const View &A, const View &B,
   L.rowC = P.rowC; L.colC = P.colC;
   L.M = P.M; L.N = P.N; L.K = P.K;
   L.splits = P.splits;
+  L.tile = static_cast<int>(P.tile);
   L.alpha = alpha; L.beta = beta;
   L.a_kcontig = P.a_kc; L.b_kcontig = P.b_kc;
   L.W = nullptr;

@@ -9,7 +9,7 @@
 // (v_mfma_f64_16x16x4_f64), tiles staged through LDS, operands addressed
 // through per-mode offset tables so that any index permutation is read in
 // place (no transpose kernels), optional split-K with a deterministic
-// reduction.  Complex operands use four real MFMA products per complex MAC.
+// reduction.  Complex operands use three real MFMA products per complex MAC.
 #pragma once
 
 #include "tensor.hpp"
@@ -151,6 +151,7 @@ struct GettLaunch {
   const int64_t *rowA, *colA, *rowB, *colB, *rowC, *colC;
   int64_t M, N, K;
   int splits;
+  int tile;  // 0 large, 1 medium (64 x 64), 2 small (32 x 32) workgroup tile
   double alpha, beta;
   bool conjA, conjB;
   bool a_kcontig, b_kcontig;
@@ -170,9 +171,10 @@ void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start = nullptr,
 std::string gett_variant(const GettLaunch &L);
 // selects the complex kernel generation (1: 4 waves, 128x64 tile, single
 // LDS buffer; 2: 8 waves, 128x128 tile, double-buffered LDS, four MFMA
-// products per complex MAC; 3 (default): 8 waves of 32x32 on a 128x64 tile,
-// three products per complex MAC; 4: as 3 with 4 waves of 64x32); plans
-// created afterwards use its tile shape
+// products per complex MAC; 3 (default): 128x64, 64x64 and 32x32 tiles chosen
+// per plan, three products per complex MAC; 4: as 3, always 128x64 with 4 waves
+// of 64x32; 5: as 3, always 128x64 with the loads two stages ahead); plans
+// created afterwards use its tile shapes
 void set_complex_gett_generation(int generation);
 
 // split-K reduction shared by both kernel families:

@@ -116,3 +116,32 @@ def test_contract_rejects_bad_indices():
     A = np.ones((3, 4))
     with pytest.raises(api.CcsdError, match="only in one operand"):
         api.contract(1.0, A, "ab", A, "cd", 0.0, np.ones((3, 3)), "ac")
+
+
+# M, N, K at the edges of the 32, 64 and 128 workgroup tiles and of the 16-k
+# stage, one stage and fewer, split-K with few and with many result elements,
+# and sizes at which the planner takes each tile.  Tolerance: K products of
+# standard normals in two summation orders, sqrt(K) 2^-53 relative to the
+# largest element's sqrt(K): 1e-13 as above.
+TILE_CASES = [(1, 1, 1), (2, 3, 15), (31, 33, 16), (32, 32, 17), (65, 31, 33), (63, 65, 64),
+              (129, 127, 48), (1, 700, 31), (700, 1, 257), (5, 6, 40000), (40, 33, 9000),
+              (257, 130, 2000), (1030, 1100, 100), (2000, 2100, 33)]
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("orient", ["mk,kn", "km,kn", "mk,nk", "km,nk"])
+@pytest.mark.parametrize("shape", TILE_CASES)
+def test_contract_tile_edges(shape, orient, cplx):
+    M, N, K = shape
+    ia, ib = orient.split(",")
+    rng = np.random.default_rng(M + 7 * N + 11 * K)
+
+    def draw(*s):
+        x = rng.standard_normal(s)
+        return x + 1j * rng.standard_normal(s) if cplx else x
+
+    A, B, C = draw(M, K), draw(K, N), draw(M, N)
+    ref = 0.75 * (A @ B) - 0.5 * C
+    out = api.contract(0.75, A if ia == "mk" else A.T, ia, B if ib == "kn" else B.T, ib, -0.5, C,
+                       "mn")
+    assert rel_err(out, ref) < 1e-13
