@@ -391,21 +391,16 @@ void CoupledCluster::set_inputs(const double *gamma, bool on_device,
 void CoupledCluster::upload_set(void *dst, const double *T1, const double *T2) {
   const auto &s = p_.shape;
   const size_t es = scalar_bytes(s.field);
-  CC4S_HIP(hipMemcpyAsync(dst, T1, s.n1() * es, hipMemcpyHostToDevice, stream_));
-  CC4S_HIP(hipMemcpyAsync(static_cast<char *>(dst) + s.n1() * es, T2, s.n2() * es,
-                          hipMemcpyHostToDevice, stream_));
-  CC4S_HIP(hipStreamSynchronize(stream_));
+  transfer_.upload(dst, T1, s.n1() * es, stream_);
+  transfer_.upload(static_cast<char *>(dst) + s.n1() * es, T2, s.n2() * es, stream_);
 }
 
 void CoupledCluster::download_set(const void *src, double *T1, double *T2) {
   const auto &s = p_.shape;
   const size_t es = scalar_bytes(s.field);
-  if (T1)
-    CC4S_HIP(hipMemcpyAsync(T1, src, s.n1() * es, hipMemcpyDeviceToHost, stream_));
+  if (T1) transfer_.download(T1, src, s.n1() * es, stream_);
   if (T2)
-    CC4S_HIP(hipMemcpyAsync(T2, static_cast<const char *>(src) + s.n1() * es,
-                            s.n2() * es, hipMemcpyDeviceToHost, stream_));
-  CC4S_HIP(hipStreamSynchronize(stream_));
+    transfer_.download(T2, static_cast<const char *>(src) + s.n1() * es, s.n2() * es, stream_);
 }
 
 bool CoupledCluster::pairs_symmetric(const void *T) {

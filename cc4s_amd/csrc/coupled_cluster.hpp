@@ -4,6 +4,7 @@
 #pragma once
 
 #include "ccsd.hpp"
+#include "host_transfer.hpp"
 #include "elementwise.hpp"
 
 #include <limits>
@@ -171,6 +172,7 @@ class CoupledCluster {
   std::unique_ptr<Ccsd> ccsd_;
   std::unique_ptr<DiisMixer> mixer_;
   DeviceBuffer T_, R_, scratch_, energy_partials_;
+  HostTransfer transfer_;
   // energy adjoint: uploaded vertex, gradient blocks, FP32 operands, dots
   DeviceBuffer adj_gamma_, adj_hp_, adj_ph_, adj_partials_, adj_S_;
   // transition structure factor: singular vectors, grid vertex blocks, Y
