@@ -1,8 +1,7 @@
-// Energy adjoint kernels: the gradient products with the energy weights
-// recomputed from the amplitudes inside the product (FP64 or FP32 MFMA,
-// G*No^2*Nv^2 complex MACs per block, small next to one CCSD iteration), the
-// energy weights as a tensor (for the structure factor of the finite-size
-// correction), and the per-G block dots of the structure factor.
+// Energy adjoint kernels: the energy weights as a tensor (the FP64 gradient
+// products and the structure factor contract it on the GETT), the FP32 gradient
+// products with the weights recomputed from the amplitudes inside the product,
+// and the per-G block dots of the structure factor.
 #include "adjoint.hpp"
 
 #include <type_traits>
@@ -14,73 +13,81 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kDotChunks = 64;  // fixed: deterministic reduction order
 
-inline int grid_for(int64_t n) {
-  return static_cast<int>(std::min<int64_t>((n + kBlock - 1) / kBlock, 256 * 32));
-}
-
 __device__ inline double2 cmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
-// tau_abij = T2_abij + T1_ai T1_bj (CoupledCluster.cxx:223-231)
-template <bool CPLX>
-struct Amp;
-template <>
-struct Amp<true> {
-  const double2 *T1, *T2;
-  int64_t No, Nv;
-  __device__ double2 tau(int64_t a, int64_t b, int64_t i, int64_t j) const {
-    const double2 t = T2[a + Nv * (b + Nv * (i + No * j))];
-    const double2 s = cmul(T1[a + Nv * i], T1[b + Nv * j]);
-    return make_double2(t.x + s.x, t.y + s.y);
-  }
-  // Z_abij = 2 tau_abij - tau_baij
-  __device__ double2 z(int64_t a, int64_t b, int64_t i, int64_t j) const {
-    const double2 p = tau(a, b, i, j), q = tau(b, a, i, j);
-    return make_double2(2.0 * p.x - q.x, 2.0 * p.y - q.y);
-  }
-};
-template <>
-struct Amp<false> {
-  const double *T1, *T2;
-  int64_t No, Nv;
-  __device__ double tau(int64_t a, int64_t b, int64_t i, int64_t j) const {
-    return T2[a + Nv * (b + Nv * (i + No * j))] + T1[a + Nv * i] * T1[b + Nv * j];
-  }
-  __device__ double z(int64_t a, int64_t b, int64_t i, int64_t j) const {
-    return 2.0 * tau(a, b, i, j) - tau(b, a, i, j);
-  }
-  // weight of the real vertex: Z_abij + Z_baji
-  __device__ double zs(int64_t a, int64_t b, int64_t i, int64_t j) const {
-    return z(a, b, i, j) + z(b, a, j, i);
-  }
-};
+// Z from T1 and T2 [a,b,i,j] (CoupledCluster.cxx:223-231): complex
+// Z_abij = 2 tau_abij - tau_baij, real Z_abij + Z_baji, tau = T2 + T1 T1.
+// HBM-bound: a block takes the (a, b) tile pair {(A, B), (B, A)} at fixed
+// (i, j), reads T2 along its contiguous index and meets the transposed element
+// in LDS (real: also the tiles at (j, i), whose pair is read once more).
+constexpr int kTile = 32;
 
 template <bool CPLX>
-__global__ __launch_bounds__(kBlock) void weights_kernel(Amp<CPLX> t, void *Zout) {
-  const int64_t No = t.No, Nv = t.Nv;
-  const int64_t n = Nv * Nv * No * No;
-  for (int64_t e = blockIdx.x * int64_t(kBlock) + threadIdx.x; e < n;
-       e += int64_t(gridDim.x) * kBlock) {
-    int64_t r = e;
-    const int64_t a = r % Nv; r /= Nv;
-    const int64_t b = r % Nv; r /= Nv;
-    const int64_t i = r % No;
-    const int64_t j = r / No;
-    if constexpr (CPLX)
-      static_cast<double2 *>(Zout)[e] = t.z(a, b, i, j);
-    else
-      static_cast<double *>(Zout)[e] = t.zs(a, b, i, j);
+__global__ __launch_bounds__(kBlock) void weights_kernel(
+    const std::conditional_t<CPLX, double2, double> *__restrict__ T1,
+    const std::conditional_t<CPLX, double2, double> *__restrict__ T2,
+    std::conditional_t<CPLX, double2, double> *__restrict__ Z, int64_t No, int64_t Nv) {
+  using T = std::conditional_t<CPLX, double2, double>;
+  // [0]: (A, B), [1]: (B, A) at (i, j); [2], [3]: the same at (j, i)
+  __shared__ T t[CPLX ? 2 : 4][kTile][kTile + 1];
+  const int64_t nt = (Nv + kTile - 1) / kTile;
+  const int64_t ntiles = nt * nt * No * No;
+  for (int64_t tid = blockIdx.x; tid < ntiles; tid += gridDim.x) {
+    const int64_t ta = tid % nt, tb = (tid / nt) % nt, ij = tid / (nt * nt);
+    if (ta > tb) continue;  // the partner's block does it (uniform per block)
+    const int64_t i = ij % No, j = ij / No;
+    const int64_t a0 = ta * kTile, b0 = tb * kTile;
+    const int64_t off = Nv * Nv * ij, offT = Nv * Nv * (j + No * i);
+    __syncthreads();
+    for (int e = threadIdx.x; e < kTile * kTile; e += kBlock) {
+      const int u = e % kTile, w = e / kTile;
+      const bool ox = a0 + u < Nv && b0 + w < Nv, oy = b0 + u < Nv && a0 + w < Nv;
+      const int64_t x = (a0 + u) + Nv * (b0 + w), y = (b0 + u) + Nv * (a0 + w);
+      t[0][u][w] = ox ? T2[off + x] : T{};
+      t[1][u][w] = oy ? T2[off + y] : T{};
+      if constexpr (!CPLX) {
+        t[2][u][w] = ox ? T2[offT + x] : T{};
+        t[3][u][w] = oy ? T2[offT + y] : T{};
+      }
+    }
+    __syncthreads();
+    // element (f0 + u, s0 + w) from its own tile p and the transposed one q
+    auto put = [&](int64_t f0, int64_t s0, int p, int q, int u, int w) {
+      const int64_t a = f0 + u, b = s0 + w;
+      if (a >= Nv || b >= Nv) return;
+      const T ai = T1[a + Nv * i], bj = T1[b + Nv * j], bi = T1[b + Nv * i], aj = T1[a + Nv * j];
+      T z;
+      if constexpr (CPLX) {
+        const double2 d = cmul(ai, bj), x = cmul(bi, aj);
+        z.x = 2.0 * (t[p][u][w].x + d.x) - (t[q][w][u].x + x.x);
+        z.y = 2.0 * (t[p][u][w].y + d.y) - (t[q][w][u].y + x.y);
+      } else {
+        const double d = ai * bj, x = bi * aj;
+        z = 2.0 * (t[p][u][w] + d) - (t[q][w][u] + x) + 2.0 * (t[q + 2][w][u] + d) -
+            (t[p + 2][u][w] + x);
+      }
+      Z[off + a + Nv * b] = z;
+    };
+    for (int e = threadIdx.x; e < kTile * kTile; e += kBlock) {
+      const int u = e % kTile, w = e / kTile;
+      put(a0, b0, 0, 1, u, w);
+      if (ta != tb) put(b0, a0, 1, 0, u, w);
+    }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Fused gradient products: C[G, n] = sum_k Gamma_blk[G, k] W(k, n), with the
+// FP32 gradient products: C[G, n] = sum_k Gamma_blk[G, k] W(k, n), with the
 // energy weights W recomputed from T1 and T2 for every tile as it is staged
 // into LDS (no Z tensor exists).  Tile 128 (G) x 64 (n), 16 k per stage,
-// double-buffered LDS, 8 waves of 32 x 32 on 16x16x4 MFMA; FP64 uses the
-// three-product complex multiply, FP32 the four-product one (FP32 sums
-// cancel too much in P3 - P1 - P2).  C is complex FP64, G fastest.
+// double-buffered LDS, 8 waves of 32 x 32 on 16x16x4 MFMA, the four-product
+// complex multiply (FP32 sums cancel too much in the three-product form's
+// P3 - P1 - P2).  C is complex FP64, G fastest.  The FP64 products, which ran on
+// this kernel at 55 % of the matrix rate (four amplitude reads and two complex
+// multiplies per weight, once per 128 G), run on the GETT over Z instead: No=24,
+// Nv=192, NG=1100 4.2 -> 2.4 ms per product, Z itself 0.3 ms.
 //   kHP (complex): k = (b,j), n = (a,i), A = Gamma[G, No+b, j],
 //                  W = conj Z_abij, C at G + NG (i + No a)
 //   kPH (complex): k = (a,i), n = (b,j), A = Gamma[G, i, No+a],
@@ -90,34 +97,11 @@ __global__ __launch_bounds__(kBlock) void weights_kernel(Amp<CPLX> t, void *Zout
 //                  C at G + NG (a + Nv i)
 enum { kHP = 0, kPH = 1, kRE = 2 };
 
-typedef double dbl4 __attribute__((ext_vector_type(4)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
 
-template <typename T>
-struct Mfma;
-template <>
-struct Mfma<double> {
-  using acc = dbl4;
-  using pair = double2;
-  __device__ static acc mma(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  // row of register r of the 16x16 block held by `lane`
-  __device__ static int row(int r, int lane) { return 4 * r + (lane >> 4); }
-  __device__ static pair make(double x, double y) { return make_double2(x, y); }
-};
-template <>
-struct Mfma<float> {
-  using acc = flt4;
-  using pair = float2;
-  __device__ static acc mma(float a, float b, acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  __device__ static int row(int r, int lane) { return 4 * (lane >> 4) + r; }
-  __device__ static pair make(double x, double y) {
-    return make_float2(static_cast<float>(x), static_cast<float>(y));
-  }
-};
+__device__ inline flt4 mma(float a, float b, flt4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
 
 struct GradArgs {
   const double2 *gamma;  // [NG, Np, Np]
@@ -131,12 +115,9 @@ constexpr int kAT = 512;                  // 8 waves
 constexpr int kABM = 128, kABN = 64, kABK = 16;
 constexpr int kALA = kABM + 1, kALW = kABN + 1;
 
-template <typename T, int MODE>
+template <int MODE>
 __global__ __launch_bounds__(kAT, 1) void grad_kernel(GradArgs p) {
-  using M = Mfma<T>;
-  using P = typename M::pair;
-  using Acc = typename M::acc;
-  constexpr bool M3 = std::is_same<T, double>::value && MODE != kRE;
+  using P = float2;
   __shared__ P As[2][kABK][kALA];
   __shared__ P Ws[2][kABK][kALW];
 
@@ -225,7 +206,7 @@ __global__ __launch_bounds__(kAT, 1) void grad_kernel(GradArgs p) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const bool ok = gOk && kaOk[e];
-      As[buf][4 * e + ak][ag] = M::make(ok ? ra[e].x : 0.0, ok ? ra[e].y : 0.0);
+      As[buf][4 * e + ak][ag] = make_float2(ok ? ra[e].x : 0.0, ok ? ra[e].y : 0.0);
     }
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
@@ -242,19 +223,18 @@ __global__ __launch_bounds__(kAT, 1) void grad_kernel(GradArgs p) {
         zr = 2.0 * (r2a[e] + p1) - (r2c[e] + p2) + 2.0 * (r2b[e] + p1) - (r2d[e] + p2);
         zi = 0.0;
       }
-      Ws[buf][8 * e + wk][wn] = M::make(kwOk[e] ? zr : 0.0, kwOk[e] ? zi : 0.0);
+      Ws[buf][8 * e + wk][wn] = make_float2(kwOk[e] ? zr : 0.0, kwOk[e] ? zi : 0.0);
     }
   };
 
   const int wr = w / 2, wc = w % 2;  // the wave's 32 x 32 part of the tile
-  Acc a1[2][2], a2[2][2], a3[2][2];
+  flt4 a1[2][2], a2[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      a1[i][j] = Acc{0, 0, 0, 0};
-      a2[i][j] = Acc{0, 0, 0, 0};
-      a3[i][j] = Acc{0, 0, 0, 0};
+      a1[i][j] = flt4{0, 0, 0, 0};
+      a2[i][j] = flt4{0, 0, 0, 0};
     }
   load(0);
   store(0);
@@ -276,38 +256,24 @@ __global__ __launch_bounds__(kAT, 1) void grad_kernel(GradArgs p) {
         for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
-            a1[i][j] = M::mma(x[i].x, y[j].x, a1[i][j]);
-            a2[i][j] = M::mma(x[i].y, y[j].x, a2[i][j]);
+            a1[i][j] = mma(x[i].x, y[j].x, a1[i][j]);
+            a2[i][j] = mma(x[i].y, y[j].x, a2[i][j]);
           }
-      } else if constexpr (M3) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) a1[i][j] = M::mma(x[i].x, y[j].x, a1[i][j]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) a2[i][j] = M::mma(x[i].y, y[j].y, a2[i][j]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            a3[i][j] = M::mma(x[i].x + x[i].y, y[j].x + y[j].y, a3[i][j]);
       } else {
         // four products: a1 = re, a2 = im
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
-            a1[i][j] = M::mma(x[i].x, y[j].x, a1[i][j]);
-            a2[i][j] = M::mma(x[i].x, y[j].y, a2[i][j]);
+            a1[i][j] = mma(x[i].x, y[j].x, a1[i][j]);
+            a2[i][j] = mma(x[i].x, y[j].y, a2[i][j]);
           }
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
-            a1[i][j] = M::mma(-x[i].y, y[j].y, a1[i][j]);
-            a2[i][j] = M::mma(x[i].y, y[j].x, a2[i][j]);
+            a1[i][j] = mma(-x[i].y, y[j].y, a1[i][j]);
+            a2[i][j] = mma(x[i].y, y[j].x, a2[i][j]);
           }
       }
     }
@@ -327,17 +293,9 @@ __global__ __launch_bounds__(kAT, 1) void grad_kernel(GradArgs p) {
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t G = g0 + wr * 32 + i * 16 + M::row(r, lane);
+        const int64_t G = g0 + wr * 32 + i * 16 + 4 * (lane >> 4) + r;
         if (G >= NG) continue;
-        double re, im;
-        if constexpr (M3) {
-          const double p1 = a1[i][j][r], p2 = a2[i][j][r];
-          re = p1 - p2;
-          im = a3[i][j][r] - (p1 + p2);
-        } else {
-          re = a1[i][j][r];
-          im = a2[i][j][r];
-        }
+        const double re = a1[i][j][r], im = a2[i][j][r];
         p.C[G + NG * col] = make_double2(re, im);
       }
   }
@@ -375,22 +333,23 @@ __global__ __launch_bounds__(kBlock) void block_dots_finish_kernel(
 
 void energy_weights(hipStream_t s, Field f, const void *T, int64_t No,
                     int64_t Nv, void *Z) {
-  const int64_t n = Nv * Nv * No * No;
+  const int64_t nt = (Nv + kTile - 1) / kTile;
+  const int blocks = static_cast<int>(std::min<int64_t>(nt * nt * No * No, 256 * 32));
   if (f == Field::Complex) {
-    Amp<true> t{static_cast<const double2 *>(T), static_cast<const double2 *>(T) + Nv * No,
-                No, Nv};
-    weights_kernel<true><<<grid_for(n), kBlock, 0, s>>>(t, Z);
+    const double2 *t = static_cast<const double2 *>(T);
+    weights_kernel<true><<<blocks, kBlock, 0, s>>>(t, t + Nv * No, static_cast<double2 *>(Z), No,
+                                                   Nv);
   } else {
-    Amp<false> t{static_cast<const double *>(T), static_cast<const double *>(T) + Nv * No,
-                 No, Nv};
-    weights_kernel<false><<<grid_for(n), kBlock, 0, s>>>(t, Z);
+    const double *t = static_cast<const double *>(T);
+    weights_kernel<false><<<blocks, kBlock, 0, s>>>(t, t + Nv * No, static_cast<double *>(Z), No,
+                                                    Nv);
   }
   CC4S_HIP(hipGetLastError());
 }
 
-void energy_gradient_product(hipStream_t s, Field f, bool fp32, GradientBlock blk,
-                             const void *gamma, const void *T, int64_t NG, int64_t No,
-                             int64_t Nv, void *C) {
+void energy_gradient_product_fp32(hipStream_t s, Field f, GradientBlock blk,
+                                  const void *gamma, const void *T, int64_t NG, int64_t No,
+                                  int64_t Nv, void *C) {
   CC4S_ASSERT(NG > 0 && No > 0 && Nv > 0, "empty gradient product");
   CC4S_ASSERT(f == Field::Complex || blk == GradientBlock::PH,
               "the real field has the ph gradient block only");
@@ -412,17 +371,12 @@ void energy_gradient_product(hipStream_t s, Field f, bool fp32, GradientBlock bl
   CC4S_ASSERT(gy <= 65535 && No * Nv < (int64_t(1) << 31), "gradient product too wide");
   const dim3 grid(static_cast<unsigned>((NG + kABM - 1) / kABM), static_cast<unsigned>(gy));
   const int mode = f == Field::Real ? kRE : (blk == GradientBlock::HP ? kHP : kPH);
-#define CC4S_GRAD(T_, M_) grad_kernel<T_, M_><<<grid, dim3(kAT), 0, s>>>(a)
-  if (fp32) {
-    if (mode == kHP) CC4S_GRAD(float, kHP);
-    else if (mode == kPH) CC4S_GRAD(float, kPH);
-    else CC4S_GRAD(float, kRE);
-  } else {
-    if (mode == kHP) CC4S_GRAD(double, kHP);
-    else if (mode == kPH) CC4S_GRAD(double, kPH);
-    else CC4S_GRAD(double, kRE);
-  }
-#undef CC4S_GRAD
+  if (mode == kHP)
+    grad_kernel<kHP><<<grid, dim3(kAT), 0, s>>>(a);
+  else if (mode == kPH)
+    grad_kernel<kPH><<<grid, dim3(kAT), 0, s>>>(a);
+  else
+    grad_kernel<kRE><<<grid, dim3(kAT), 0, s>>>(a);
   CC4S_HIP(hipGetLastError());
 }
 

@@ -23,18 +23,17 @@ namespace cc4s_amd {
 void energy_weights(hipStream_t s, Field f, const void *T, int64_t No,
                     int64_t Nv, void *Z);
 
-// One block of the energy gradient, with the weights recomputed from the
+// One block of the energy gradient in FP32, with the weights recomputed from the
 // amplitude set T = [T1; T2] tile by tile inside the product (no Z tensor):
 //   complex HP: C[G, i, a] = sum_bj conj(Z_abij) Gamma^G_bj
 //   complex PH: C[G, b, j] = sum_ai Z_abij Gamma^G_ia
 //   real    PH: C[G, a, i] = sum_bj (Z_abij + Z_baji) Gamma^G_bj
 // (complex FP64 output, G fastest; for the real field Re and Im of C are the
-// gradient of the two real vertex components).  FP64 (fp32 false) or FP32
-// MFMA arithmetic with FP32 accumulation.
+// gradient of the two real vertex components).  FP32 MFMA operands and sums.
 enum class GradientBlock { HP, PH };
-void energy_gradient_product(hipStream_t s, Field f, bool fp32, GradientBlock blk,
-                             const void *gamma, const void *T, int64_t NG, int64_t No,
-                             int64_t Nv, void *C);
+void energy_gradient_product_fp32(hipStream_t s, Field f, GradientBlock blk,
+                                  const void *gamma, const void *T, int64_t NG, int64_t No,
+                                  int64_t Nv, void *C);
 
 // Per-G dots over one block: out[G] (=, or += when accumulate) factor *
 // Re sum_{x<rows, y<cols} conj(Gamma[G, row0+x, col0+y]) g[G + NG*(x + rows*y)]

@@ -682,11 +682,31 @@ void CoupledCluster::transition_structure_factor(const double *U, int64_t NGg,
   for (int64_t G = 0; G < NGg; ++G) S[G] /= V[G];  // (1 / sqrt V)^2, :87-102
 }
 
-// E = sum_G Re sum_ia conj(Gamma^G_ia) g^G_ia with g^G_ia = sum_bj conj(Z_abij)
-// Gamma^G_bj (complex), or 1/2 sum_G sum_ai Re(conj Gamma^G_ai g^G_ai) with
-// g^G_ai = sum_bj Zs_abij Gamma^G_bj (real): the pphh integrals are never
-// formed, and Z exists only tile by tile inside the product kernel, rebuilt
-// from the amplitudes.
+// Gradient blocks in FP64: the energy weights as a tensor (in the residuum's
+// buffer, which the next pass overwrites) contracted with the vertex blocks.
+//   complex: g_hp^G_ia = sum_bj conj(Z_abij) Gamma^G_bj,
+//            g_ph^G_bj = sum_ai Z_abij Gamma^G_ia;
+//   real:    g_ph^G_ai = sum_bj (Z_abij + Z_baji) Gamma^G_bj
+void CoupledCluster::gradient_blocks(const void *gamma, bool hp, bool ph) {
+  const auto &s = p_.shape;
+  const int64_t No = s.No, Nv = s.Nv;
+  const bool cplx_field = s.field == Field::Complex;
+  const int64_t G = cplx_field ? s.NG : 2 * s.NG;
+  energy_weights(stream_, s.field, T_.get(), No, Nv, R_.get());
+  const View Z = dense_view(R_.get(), s.field, "abij", {Nv, Nv, No, No});
+  if (hp)
+    engine_->contract(1.0, vertex_block(gamma, false, "Gbj"), Z.conjugated(), 0.0,
+                      dense_view(adj_hp_.get(), s.field, "Gia", {G, No, Nv}));
+  if (ph && cplx_field)
+    engine_->contract(1.0, vertex_block(gamma, true, "Gia"), Z, 0.0,
+                      dense_view(adj_ph_.get(), s.field, "Gbj", {G, Nv, No}));
+  else if (ph)
+    engine_->contract(1.0, vertex_block(gamma, false, "Gbj"), Z, 0.0,
+                      dense_view(adj_ph_.get(), s.field, "Gai", {G, Nv, No}));
+}
+
+// E = sum_G Re sum_ia conj(Gamma^G_ia) g^G_ia (complex), or 1/2 sum_G sum_ai
+// Re(conj Gamma^G_ai g^G_ai) (real): the pphh integrals are never formed.
 double CoupledCluster::energy_forward(const double *gamma, bool gamma_on_device) {
   CC4S_ASSERT(inputs_set_, "inputs not set");
   CC4S_ASSERT(have_amplitudes_, "no amplitudes yet");
@@ -699,14 +719,12 @@ double CoupledCluster::energy_forward(const double *gamma, bool gamma_on_device)
   adj_S_.reserve(NG * sizeof(double));
   if (s.field == Field::Complex) {
     adj_hp_.reserve(block_bytes);
-    energy_gradient_product(stream_, s.field, false, GradientBlock::HP, g, T_.get(), NG,
-                            No, Nv, adj_hp_.get());
+    gradient_blocks(g, true, false);
     block_dots(stream_, g, NG, s.Np(), 0, No, No, Nv, adj_hp_.get(), 1.0, false,
                adj_partials_.get(), adj_S_.as<double>());
   } else {
     adj_ph_.reserve(block_bytes);
-    energy_gradient_product(stream_, s.field, false, GradientBlock::PH, g, T_.get(), NG,
-                            No, Nv, adj_ph_.get());
+    gradient_blocks(g, false, true);
     block_dots(stream_, g, NG, s.Np(), No, Nv, 0, No, adj_ph_.get(), 0.5, false,
                adj_partials_.get(), adj_S_.as<double>());
   }
@@ -719,9 +737,7 @@ double CoupledCluster::energy_forward(const double *gamma, bool gamma_on_device)
   return E;
 }
 
-// Complex field: g_hp^G_ia = sum_bj conj(Z_abij) Gamma^G_bj and
-// g_ph^G_bj = sum_ai Z_abij Gamma^G_ia; real field: g_ph^G_ai =
-// sum_bj Zs_abij Gamma^G_bj; every other block of the gradient is zero.
+// Every block of the gradient other than gradient_blocks' is zero.
 void CoupledCluster::energy_backward(const double *gamma, bool gamma_on_device,
                                      double *grad, bool grad_on_device, double *S,
                                      bool fp32) {
@@ -735,13 +751,16 @@ void CoupledCluster::energy_backward(const double *gamma, bool gamma_on_device,
   const size_t block_bytes = static_cast<size_t>(NG) * No * Nv * 16;
   if (cplx_field) adj_hp_.reserve(block_bytes);
   adj_ph_.reserve(block_bytes);
-  // the energy weights are rebuilt from the amplitudes tile by tile inside
-  // the products (FP64 or FP32 MFMA)
-  if (cplx_field)
-    energy_gradient_product(stream_, s.field, fp32, GradientBlock::HP, g, T_.get(), NG, No,
-                            Nv, adj_hp_.get());
-  energy_gradient_product(stream_, s.field, fp32, GradientBlock::PH, g, T_.get(), NG, No, Nv,
-                          adj_ph_.get());
+  if (fp32) {
+    // the weights are rebuilt from the amplitudes tile by tile inside the products
+    if (cplx_field)
+      energy_gradient_product_fp32(stream_, s.field, GradientBlock::HP, g, T_.get(), NG, No, Nv,
+                                   adj_hp_.get());
+    energy_gradient_product_fp32(stream_, s.field, GradientBlock::PH, g, T_.get(), NG, No, Nv,
+                                 adj_ph_.get());
+  } else {
+    gradient_blocks(g, cplx_field, true);
+  }
   if (S) {
     adj_partials_.reserve(block_dots_partials_size(NG));
     adj_S_.reserve(NG * sizeof(double));

@@ -161,6 +161,7 @@ class CoupledCluster {
   void upload_set(void *dst, const double *T1, const double *T2);
   void download_set(const void *src, double *T1, double *T2);
   void create_mixer();
+  void gradient_blocks(const void *gamma, bool hp, bool ph);
   const void *adjoint_vertex(const double *gamma, bool on_device);
   View vertex_block(const void *gamma, bool hp, const std::string &names) const;
 
