@@ -411,25 +411,25 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
   constexpr int NSET = DEEP ? 2 : 1;
   T ra[NSET][EA], rb[NSET][EB];
   bool segS[NSET];  // SEG2: the registers hold a second-segment stage
+  bool segOn = false;  // SEG2: the row pointers are the second segment's
   auto load_data = [&](auto set_c) {
     constexpr int q = decltype(set_c)::value;
-    bool sg = false;
-    if constexpr (SEG2) sg = segK;
-    segS[q] = sg;
+    if constexpr (SEG2) {
+      segS[q] = segK;
+      if (segK && !segOn) {  // once, at the first stage of the second segment
+        segOn = true;
 #pragma unroll
-    for (int i = 0; i < EA; ++i) {
-      const int ir = AKC ? i : 0, ik = AKC ? 0 : i;
-      const char *row = aRow[ir];
-      if constexpr (SEG2) row = sg ? aRow2[ir] : row;
-      ra[q][i] = reinterpret_cast<const T *>(row)[aK[ik]];
+        for (int i = 0; i < NRA; ++i) aRow[i] = aRow2[i];
+#pragma unroll
+        for (int i = 0; i < NRB; ++i) bCol[i] = bCol2[i];
+      }
     }
 #pragma unroll
-    for (int i = 0; i < EB; ++i) {
-      const int ir = BKC ? i : 0, ik = BKC ? 0 : i;
-      const char *col = bCol[ir];
-      if constexpr (SEG2) col = sg ? bCol2[ir] : col;
-      rb[q][i] = reinterpret_cast<const T *>(col)[bK[ik]];
-    }
+    for (int i = 0; i < EA; ++i)
+      ra[q][i] = reinterpret_cast<const T *>(aRow[AKC ? i : 0])[aK[AKC ? 0 : i]];
+#pragma unroll
+    for (int i = 0; i < EB; ++i)
+      rb[q][i] = reinterpret_cast<const T *>(bCol[BKC ? i : 0])[bK[BKC ? 0 : i]];
   };
   // conjugation flips the sign bit of the imaginary part (an integer operation:
   // FP64 multiplies would take the MFMAs' cycles)
@@ -453,21 +453,21 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
         if (b_k(i) >= left) rb[q][i] = T{};
     }
     if constexpr (CPLX) {
-      int fa = flipA, fb = flipB;
+      int fa = flipA, fb = flipB, fx = 0;
       if constexpr (SEG2) {
-        fa = segS[q] ? (p.signA2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fa;
+        // the second segment's factor: its sign as bits, its size where it is not 1
+        fx = segS[q] && p.f2 < 0.0 ? static_cast<int>(0x80000000u) : 0;
+        fa = fx ^ (segS[q] ? (p.signA2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fa);
         fb = segS[q] ? (p.signB2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fb;
+        const double f = fabs(p.f2);
+        if (segS[q] && f != 1.0)
+#pragma unroll
+          for (int i = 0; i < EA; ++i) ra[q][i] = make_double2(f * ra[q][i].x, f * ra[q][i].y);
       }
 #pragma unroll
-      for (int i = 0; i < EA; ++i) {
-        double x = ra[q][i].x, y = flip(ra[q][i].y, fa);
-        if constexpr (SEG2) {
-          const double f = segS[q] ? p.f2 : 1.0;
-          x *= f;
-          y *= f;
-        }
-        As[buf][a_k(i)][a_m(i)] = make_double2(x, y);
-      }
+      for (int i = 0; i < EA; ++i)
+        As[buf][a_k(i)][a_m(i)] = make_double2(SEG2 ? flip(ra[q][i].x, fx) : ra[q][i].x,
+                                               flip(ra[q][i].y, fa));
 #pragma unroll
       for (int i = 0; i < EB; ++i)
         Bs[buf][b_k(i)][b_n(i)] = make_double2(rb[q][i].x, flip(rb[q][i].y, fb));

@@ -100,10 +100,14 @@ __global__ __launch_bounds__(256) void maxabs_kernel(const double2 *X, const int
     const int64_t i0 = (item - l * nseg) * kSegment;
     const int64_t i1 = min(len, i0 + kSegment);
     const int64_t base = lineOff[l];
-#pragma unroll 4
-    for (int64_t i = i0 + lane; i < i1; i += 64) {
-      const double2 x = X[base + inOff[i]];
-      m = fmax(m, sumabs ? fabs(x.x) + fabs(x.y) : fmax(fabs(x.x), fabs(x.y)));
+    // eight reads in flight (past the end the last element once more)
+    for (int64_t i = i0 + lane; i < i1; i += 64 * 8) {
+      double2 x[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) x[q] = X[base + inOff[min(i + 64 * q, i1 - 1)]];
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        m = fmax(m, sumabs ? fabs(x[q].x) + fabs(x[q].y) : fmax(fabs(x[q].x), fabs(x[q].y)));
     }
   }
   m = wave_max(m);
@@ -167,25 +171,37 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs p) {
     oMN[t - kPackTile] = mn < p.MN ? p.offMN[mn] : -1;
   }
   __syncthreads();
-  for (int e = t; e < kPackTile * kPackTile; e += 256) {
-    const int a = e % kPackTile, b = e / kPackTile;
-    const int kk = p.kcontig ? a : b, mm = p.kcontig ? b : a;
-    uint2 v = make_uint2(0u, 0u);
-    unsigned int vs = 0u;
-    const int64_t ok = oK[kk], om = oMN[mm];
-    if (ok >= 0 && om >= 0) {
-      const double2 x = p.X[om + ok];
-      if constexpr (FP16) {
-        v.x = split_part_f16(sc * x.x);
-        v.y = split_part_f16(sc * p.sign * x.y);
-        if constexpr (SUMS) vs = split_part_f16(sc * (x.x + p.sign * x.y));
-      } else {
-        v.x = split_part(x.x);
-        v.y = split_part(p.sign * x.y);
-      }
+  // HBM-bound: eight reads of a thread are in flight together (outside the
+  // operand its first element is read and dropped): a 576 x 18336 operand is
+  // packed at 4.2 TB/s, the rate of a large copy
+  constexpr int kBatch = 8;
+  for (int e0 = t; e0 < kPackTile * kPackTile; e0 += 256 * kBatch) {
+    double2 x[kBatch];
+#pragma unroll
+    for (int q = 0; q < kBatch; ++q) {
+      const int e = e0 + 256 * q, a = e % kPackTile, b = e / kPackTile;
+      const int64_t ok = oK[p.kcontig ? a : b], om = oMN[p.kcontig ? b : a];
+      x[q] = p.X[ok >= 0 && om >= 0 ? om + ok : 0];
     }
-    tile[kk][mm] = v;
-    if constexpr (SUMS) tile_s[kk][mm] = vs;
+#pragma unroll
+    for (int q = 0; q < kBatch; ++q) {
+      const int e = e0 + 256 * q, a = e % kPackTile, b = e / kPackTile;
+      const int kk = p.kcontig ? a : b, mm = p.kcontig ? b : a;
+      uint2 v = make_uint2(0u, 0u);
+      unsigned int vs = 0u;
+      if (oK[kk] >= 0 && oMN[mm] >= 0) {
+        if constexpr (FP16) {
+          v.x = split_part_f16(sc * x[q].x);
+          v.y = split_part_f16(sc * p.sign * x[q].y);
+          if constexpr (SUMS) vs = split_part_f16(sc * (x[q].x + p.sign * x[q].y));
+        } else {
+          v.x = split_part(x[q].x);
+          v.y = split_part(p.sign * x[q].y);
+        }
+      }
+      tile[kk][mm] = v;
+      if constexpr (SUMS) tile_s[kk][mm] = vs;
+    }
   }
   __syncthreads();
   // kb and Kc are even: a pair never straddles the chunk's end

@@ -19,12 +19,14 @@
 // most CUs idle while it runs).
 #include "triples.hpp"
 
+#include <type_traits>
+
 namespace cc4s_amd {
 
 namespace {
 
 constexpr int kBlock = 512;
-constexpr int kComplexBlocks = 768;
+constexpr int kComplexBlocks = 512;
 
 template <bool CPLX>
 struct TS;
@@ -33,9 +35,7 @@ struct TS<false> {
   using T = double;
   __device__ static T mul(T a, T b) { return a * b; }
   __device__ static double re_mul(T a, T b) { return a * b; }
-  __device__ static T lin(double x, T a, double y, T b, double z, T c) {
-    return x * a + y * b + z * c;
-  }
+  __device__ static T add_scaled(T a, double y, T b) { return a + y * b; }
   __device__ static T plus(T a, T b) { return a + b; }
 };
 template <>
@@ -45,8 +45,8 @@ struct TS<true> {
     return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
   }
   __device__ static double re_mul(T a, T b) { return a.x * b.x - a.y * b.y; }
-  __device__ static T lin(double x, T a, double y, T b, double z, T c) {
-    return make_double2(x * a.x + y * b.x + z * c.x, x * a.y + y * b.y + z * c.y);
+  __device__ static T add_scaled(T a, double y, T b) {
+    return make_double2(a.x + y * b.x, a.y + y * b.y);
   }
   __device__ static T plus(T a, T b) { return make_double2(a.x + b.x, a.y + b.y); }
 };
@@ -62,18 +62,34 @@ constexpr int kTileElems = kTile * kTile * kTile;
 
 // ordering p = abc, bac, cba, acb, bca, cab: position d of (x1, x2, x3) holds
 // particle kOrder[p][d] of (a, b, c); kCoef[p] is its weight in Zs
-__constant__ int kOrder[6][3] = {{0, 1, 2}, {1, 0, 2}, {2, 1, 0},
-                                 {0, 2, 1}, {1, 2, 0}, {2, 0, 1}};
-__constant__ double kCoef[6] = {8.0, -4.0, -4.0, -4.0, 2.0, 2.0};
+constexpr int kOrder[6][3] = {{0, 1, 2}, {1, 0, 2}, {2, 1, 0}, {0, 2, 1}, {1, 2, 0}, {2, 0, 1}};
+constexpr double kCoef[6] = {8.0, -4.0, -4.0, -4.0, 2.0, 2.0};
 // kCompose[s][p] = q with kOrder[q][d] = kOrder[s][kOrder[p][d]]: in the
 // output tile whose (a, b, c) ranges are the canonical ranges kOrder[s],
 // ordering p reads the LDS tile formed for ordering q
-__constant__ int kCompose[6][6] = {{0, 1, 2, 3, 4, 5}, {1, 0, 5, 4, 3, 2},
-                                   {2, 4, 0, 5, 1, 3}, {3, 5, 4, 0, 2, 1},
-                                   {4, 2, 3, 1, 5, 0}, {5, 3, 1, 2, 0, 4}};
+constexpr int kCompose[6][6] = {{0, 1, 2, 3, 4, 5}, {1, 0, 5, 4, 3, 2}, {2, 4, 0, 5, 1, 3},
+                                {3, 5, 4, 0, 2, 1}, {4, 2, 3, 1, 5, 0}, {5, 3, 1, 2, 0, 4}};
 
+// f(std::integral_constant<int, 0>{}), ..., <5>: the six orderings with their
+// tables as constants
+template <typename F>
+__device__ __forceinline__ void six(F &&f) {
+  f(std::integral_constant<int, 0>{});
+  f(std::integral_constant<int, 1>{});
+  f(std::integral_constant<int, 2>{});
+  f(std::integral_constant<int, 3>{});
+  f(std::integral_constant<int, 4>{});
+  f(std::integral_constant<int, 5>{});
+}
+
+// A thread owns one position t of the tile at all six orderings: it reads W
+// there once, keeps it in registers for the energy of the same element, and its
+// reads of W, V and T1 are in flight together (two blocks per CU with 128
+// registers; three with 80 spill and take 4.1 ms below).  Blocks walk the
+// canonical triples only, so they share them evenly.  Measured over the 55
+// launches of (T) at No=10, Nv=96: 5.6 -> 2.4 ms.
 template <bool CPLX>
-__global__ __launch_bounds__(kBlock) void triples_energy_kernel(
+__global__ __launch_bounds__(kBlock, 4) void triples_energy_kernel(
     const typename TS<CPLX>::T *__restrict__ W, const typename TS<CPLX>::T *__restrict__ V,
     const typename TS<CPLX>::T *__restrict__ T1, const double *__restrict__ eh,
     const double *__restrict__ ep, int64_t No, int64_t Nv, int64_t i, int64_t j,
@@ -83,67 +99,75 @@ __global__ __launch_bounds__(kBlock) void triples_energy_kernel(
   // S at the six orderings of the canonical tile triple's index ranges
   __shared__ T tile[6][kTileElems];
   __shared__ double sh[kBlock / 64];
+  static_assert(kBlock == kTileElems, "one thread per tile position");
   const int64_t v = Nv, o = No;
   const int64_t nt = (v + kTile - 1) / kTile;
-  const int64_t ntiles = nt * nt * nt * kc;
+  const int64_t nc = nt * (nt + 1) * (nt + 2) / 6;  // canonical tile triples
+  const int64_t ntiles = nc * kc;
   // V_pphh[p,q,s,r] at p + v (q + v (s + o r)); T1[a,i] at a + v i
-  auto Vx = [&](int64_t p, int64_t q, int64_t s, int64_t r) {
-    return V[p + v * (q + v * (s + o * r))];
-  };
-  T zero;
-  if constexpr (CPLX) zero = make_double2(0.0, 0.0); else zero = 0.0;
+  const T *Vjk = V + v * v * j, *Vij = V + v * v * (i + o * j);
+  const int t = threadIdx.x;
+  const int l[3] = {t % kTile, (t / kTile) % kTile, t / (kTile * kTile)};
   double sum = 0.0;
   for (int64_t tid = blockIdx.x; tid < ntiles; tid += gridDim.x) {
-    const int64_t ti[3] = {tid % nt, (tid / nt) % nt, (tid / (nt * nt)) % nt};
-    if (ti[0] > ti[1] || ti[1] > ti[2]) continue;  // not canonical (uniform per block)
-    const int64_t r0[3] = {ti[0] * kTile, ti[1] * kTile, ti[2] * kTile};
-    const int64_t kl = tid / (nt * nt * nt);
+    const int64_t kl = tid / nc;
+    // r = tetrahedral(tC) + triangular(tB) + tA, tA <= tB <= tC
+    int64_t r = tid - kl * nc;
+    int64_t tC = 0, tB = 0;
+    while ((tC + 1) * (tC + 2) * (tC + 3) / 6 <= r) ++tC;
+    r -= tC * (tC + 1) * (tC + 2) / 6;
+    while ((tB + 1) * (tB + 2) / 2 <= r) ++tB;
+    const int64_t tA = r - tB * (tB + 1) / 2;
+    const int64_t ti[3] = {tA, tB, tC};
+    const int64_t r0[3] = {tA * kTile, tB * kTile, tC * kTile};
     const int64_t base = v * v * v * kl;
     const int64_t k = k0 + kl;
+    const T *Vik = V + v * v * (i + o * k), *Vjkk = Vjk + v * v * o * k;
     __syncthreads();  // the previous tile's LDS reads are done
     // S at the ordering (x1, x2, x3) and the holes (i, j, k): W plus the
     // disconnected part; x1 runs fastest, so the V and T1 reads along x1 are
-    // coalesced and the others are broadcasts
-    for (int e = threadIdx.x; e < 6 * kTileElems; e += kBlock) {
-      const int p = e / kTileElems, t = e % kTileElems;
-      const int64_t x1 = r0[kOrder[p][0]] + t % kTile;
-      const int64_t x2 = r0[kOrder[p][1]] + (t / kTile) % kTile;
-      const int64_t x3 = r0[kOrder[p][2]] + t / (kTile * kTile);
-      T sv = zero;
-      if (x1 < v && x2 < v && x3 < v)
-        sv = S::plus(W[base + x1 + v * (x2 + v * x3)],
-                     S::plus(S::mul(T1[x1 + v * i], Vx(x2, x3, j, k)),
-                             S::plus(S::mul(T1[x2 + v * j], Vx(x1, x3, i, k)),
-                                     S::mul(T1[x3 + v * k], Vx(x1, x2, i, j)))));
-      tile[p][t] = sv;
-    }
+    // coalesced and the others are broadcasts.  Past the edge the last element
+    // is read and S left zero
+    T w[6];
+    six([&](auto pc) {
+      constexpr int p = decltype(pc)::value;
+      const int64_t y1 = r0[kOrder[p][0]] + l[0], y2 = r0[kOrder[p][1]] + l[1],
+                    y3 = r0[kOrder[p][2]] + l[2];
+      const bool in = y1 < v && y2 < v && y3 < v;
+      const int64_t x1 = min(y1, v - 1), x2 = min(y2, v - 1), x3 = min(y3, v - 1);
+      w[p] = W[base + x1 + v * (x2 + v * x3)];
+      const T s = S::plus(w[p], S::plus(S::mul(T1[x1 + v * i], Vjkk[x2 + v * x3]),
+                                        S::plus(S::mul(T1[x2 + v * j], Vik[x1 + v * x3]),
+                                                S::mul(T1[x3 + v * k], Vij[x1 + v * x2]))));
+      tile[p][t] = in ? s : T{};
+    });
     __syncthreads();
     const double weight = (i == j && j == k) ? 1.0 / 6.0 : (i == j || j == k) ? 0.5 : 1.0;
-    for (int e = threadIdx.x; e < 6 * kTileElems; e += kBlock) {
-      const int sg = e / kTileElems, t = e % kTileElems;
+    const double eo = (eh[i] + eh[j]) + eh[k];
+    six([&](auto sc) {
+      constexpr int sg = decltype(sc)::value;
       // output tile: (a, b, c) over the canonical ranges kOrder[sg]; a
       // permutation that repeats an earlier tile triple is skipped
       bool repeat = false;
+#pragma unroll
       for (int s2 = 0; s2 < sg; ++s2)
         repeat = repeat || (ti[kOrder[s2][0]] == ti[kOrder[sg][0]] &&
                             ti[kOrder[s2][1]] == ti[kOrder[sg][1]] &&
                             ti[kOrder[s2][2]] == ti[kOrder[sg][2]]);
-      if (repeat) continue;
-      const int l[3] = {t % kTile, (t / kTile) % kTile, t / (kTile * kTile)};
+      if (repeat) return;
       const int64_t x[3] = {r0[kOrder[sg][0]] + l[0], r0[kOrder[sg][1]] + l[1],
                             r0[kOrder[sg][2]] + l[2]};
-      if (x[0] >= v || x[1] >= v || x[2] >= v) continue;
-      T zs = zero;
+      if (x[0] >= v || x[1] >= v || x[2] >= v) return;
+      T zs = T{};
 #pragma unroll
       for (int p = 0; p < 6; ++p) {
         const int q0 = kOrder[p][0], q1 = kOrder[p][1], q2 = kOrder[p][2];
-        zs = S::lin(1.0, zs, kCoef[p],
-                    tile[kCompose[sg][p]][l[q0] + kTile * (l[q1] + kTile * l[q2])], 0.0, zero);
+        zs = S::add_scaled(zs, kCoef[p],
+                           tile[kCompose[sg][p]][l[q0] + kTile * (l[q1] + kTile * l[q2])]);
       }
-      const double d = ((eh[i] + eh[j]) + eh[k]) - ((ep[x[0]] + ep[x[1]]) + ep[x[2]]);
-      const T w = W[base + x[0] + v * (x[1] + v * x[2])];
-      sum += weight * S::re_mul(w, zs) / d;
-    }
+      const double d = eo - ((ep[x[0]] + ep[x[1]]) + ep[x[2]]);
+      sum += weight * S::re_mul(w[sg], zs) / d;
+    });
   }
   // wavefront sums, then the wave sums in wave order
   sum = wave_sum(sum);
