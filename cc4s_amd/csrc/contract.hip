@@ -35,7 +35,30 @@ struct KArgs {
   const int64_t *rowA2, *colA2, *rowB2, *colB2;
   int64_t K1, K1p, K2;
   double f2, signA2, signB2;
+  // tiles [0, fullTiles) run over all of K; the others, the last partial wave of
+  // workgroups, are cut into tailSplits parts of tailChunk k each, whose sums go
+  // to Wt [part][tile][BM][BN] (fullTiles is the tile count where nothing is cut)
+  double *Wt;
+  int fullTiles, tailTiles, tailSplits;
+  int64_t tailChunk;
 };
+
+// index in a contiguous run of `n` items per XCD: workgroups go round the 8 XCDs
+__device__ __forceinline__ int xcd_run(int g, int n) {
+  const int x = g & 7, q = n >> 3, r = n & 7;
+  return x * q + min(x, r) + (g >> 3);
+}
+
+// (tm, tn) of tile g: groups of GM tile rows are walked column by column, so that
+// concurrently running tiles share A rows and B columns in L2
+__device__ __forceinline__ void tile_of(int g, int tilesM, int tilesN, int GM, int &tm,
+                                        int &tn) {
+  const int per_group = GM * tilesN;
+  const int first_m = (g / per_group) * GM;
+  const int gsize = min(tilesM - first_m, GM);
+  tm = first_m + (g % per_group) % gsize;
+  tn = (g % per_group) / gsize;
+}
 
 // Complex GETT, first generation: workgroup tile BM x BN, K staged BK at a time through LDS; 4 waves in a
 // (BM/WM) x (BN/WN) grid, each owning WM x WN of C as 16x16 MFMA blocks.
@@ -340,23 +363,26 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
   __shared__ T Bs[2][BK][LDB];
 
   const int t = threadIdx.x;
-  const int ntiles = p.tilesM * p.tilesN;
-  // workgroups go round the 8 XCDs: each XCD takes a contiguous run of tiles
   int g = blockIdx.x;
-  {
-    const int x = g & 7, q = ntiles >> 3, r = ntiles & 7;
-    g = x * q + min(x, r) + (g >> 3);
+  int64_t kbeg = static_cast<int64_t>(blockIdx.y) * p.kChunk, klen = p.kChunk;
+  const bool tail = g >= p.fullTiles;
+  int part = 0;  // (cut, tile) of a tail workgroup
+  if (tail) {
+    part = g - p.fullTiles;
+    const int cut = part / p.tailTiles, r = xcd_run(part - cut * p.tailTiles, p.tailTiles);
+    part = cut * p.tailTiles + r;
+    g = p.fullTiles + r;
+    kbeg = cut * p.tailChunk;
+    klen = p.tailChunk;
+  } else {
+    g = xcd_run(g, p.fullTiles);
   }
   constexpr int GM = 1024 / BM;  // M-tiles of a group: 1024 rows
-  const int per_group = GM * p.tilesN;
-  const int first_m = (g / per_group) * GM;
-  const int gsize = min(p.tilesM - first_m, GM);
-  const int tm = first_m + (g % per_group) % gsize;
-  const int tn = (g % per_group) / gsize;
+  int tm, tn;
+  tile_of(g, p.tilesM, p.tilesN, GM, tm, tn);
   const int64_t m0 = static_cast<int64_t>(tm) * BM;
   const int64_t n0 = static_cast<int64_t>(tn) * BN;
-  const int64_t kbeg = static_cast<int64_t>(blockIdx.y) * p.kChunk;
-  const int64_t kend = min(p.K, kbeg + p.kChunk);
+  const int64_t kend = min(p.K, kbeg + klen);
   const int nstages = kend > kbeg ? static_cast<int>((kend - kbeg + BK - 1) / BK) : 0;
 
   auto a_m = [&](int i) { return AKC ? (t / BK + i * (NT / BK)) : (t % BM); };
@@ -618,6 +644,27 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
     if (s + 1 < nstages) stage(s + 1, S0{}, P1{});
   }
 
+  if (tail) {
+    T *w = reinterpret_cast<T *>(p.Wt) + static_cast<int64_t>(part) * (BM * BN);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          T x;
+          if constexpr (!CPLX) {
+            x = accR[i][j][r];
+          } else if constexpr (M3) {
+            const double p1 = accR[i][j][r], p2 = accI[i][j][r];
+            x = make_double2(p1 - p2, accS[i][j][r] - (p1 + p2));
+          } else {
+            x = make_double2(accR[i][j][r], accI[i][j][r]);
+          }
+          w[(wm * WM + i * 16 + 4 * r + (lane >> 4)) * BN + wn * WN + j * 16 + (lane & 15)] = x;
+        }
+    return;
+  }
   int64_t cCol[NB];
   bool cColOk[NB];
 #pragma unroll
@@ -734,6 +781,49 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(
       *c = out;
     }
     if constexpr (G > 1) __syncthreads();  // part is written again
+  }
+}
+
+// Results of the tail tiles from their parts, in order.  One block takes 256
+// elements of one tile; HBM-bound by the parts, which are a few per cent of the
+// launch's traffic
+template <bool CPLX>
+__global__ __launch_bounds__(256) void tail_reduce_kernel(KArgs p, int BM, int BN, int GM) {
+  using T = std::conditional_t<CPLX, double2, double>;
+  const int per = BM * BN / 256;  // blocks of a tile
+  const int r = blockIdx.x / per;
+  const int e = (blockIdx.x - r * per) * 256 + threadIdx.x;
+  int tm, tn;
+  tile_of(p.fullTiles + r, p.tilesM, p.tilesN, GM, tm, tn);
+  const int64_t m = static_cast<int64_t>(tm) * BM + e / BN;
+  const int64_t n = static_cast<int64_t>(tn) * BN + e % BN;
+  if (m >= p.M || n >= p.N) return;
+  const int64_t stride = static_cast<int64_t>(p.tailTiles) * BM * BN;
+  const T *w = reinterpret_cast<const T *>(p.Wt) + static_cast<int64_t>(r) * BM * BN + e;
+  T acc = w[0];
+#pragma unroll 4
+  for (int s = 1; s < p.tailSplits; ++s) {
+    const T x = w[s * stride];
+    if constexpr (CPLX) {
+      acc.x += x.x;
+      acc.y += x.y;
+    } else {
+      acc += x;
+    }
+  }
+  T *c = reinterpret_cast<T *>(p.C) + p.rowC[m] + p.colC[n];
+  if constexpr (CPLX) {
+    T out = make_double2(p.alpha * acc.x, p.alpha * acc.y);
+    if (p.beta != 0.0) {
+      const T old = *c;
+      out.x += p.beta * old.x;
+      out.y += p.beta * old.y;
+    }
+    *c = out;
+  } else {
+    T out = p.alpha * acc;
+    if (p.beta != 0.0) out += p.beta * *c;
+    *c = out;
   }
 }
 
@@ -899,7 +989,15 @@ void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
   a.f2 = L.f2;
   a.signA2 = L.conjA2 ? -1.0 : 1.0;
   a.signB2 = L.conjB2 ? -1.0 : 1.0;
-  dim3 grid(a.tilesM * a.tilesN, L.splits);
+  const int ntiles = a.tilesM * a.tilesN;
+  a.fullTiles = L.tail_splits > 1 ? static_cast<int>(L.full_tiles) : ntiles;
+  a.tailTiles = ntiles - a.fullTiles;
+  a.tailSplits = L.tail_splits;
+  a.Wt = static_cast<double *>(L.W);
+  a.tailChunk = L.tail_splits > 1 ? (kstages + L.tail_splits - 1) / L.tail_splits * BK : 0;
+  CC4S_ASSERT(L.tail_splits <= 1 || (L.splits == 1 && L.W && a.fullTiles > 0 && a.tailTiles > 0),
+              "tail split without its workspace");
+  dim3 grid(a.fullTiles + a.tailTiles * std::max(1, L.tail_splits), L.splits);
   if (start) CC4S_HIP(hipEventRecord(start, s));
   if (cplx && g_complex_generation == 3) {
     if (seg2 && tile == Tile::Large)
@@ -931,6 +1029,15 @@ void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
   }
   CC4S_HIP(hipGetLastError());
   if (stop) CC4S_HIP(hipEventRecord(stop, s));
+  if (L.tail_splits > 1) {
+    const int GM = 1024 / BM;
+    const unsigned blocks = static_cast<unsigned>(a.tailTiles) * (BM * BN / 256);
+    if (cplx)
+      tail_reduce_kernel<true><<<blocks, 256, 0, s>>>(a, BM, BN, GM);
+    else
+      tail_reduce_kernel<false><<<blocks, 256, 0, s>>>(a, BM, BN, GM);
+    CC4S_HIP(hipGetLastError());
+  }
   if (L.splits > 1)
     launch_splitk_reduce(L.field, a.W, a.C, L.rowC, L.colC, L.M, L.N, L.splits,
                          L.alpha, L.beta, s);
@@ -965,7 +1072,8 @@ void launch_splitk_reduce(Field f, const double *W, double *C,
 struct GettPlan {
   int64_t M = 0, N = 0, K = 0;
   bool swap = false, a_kc = true, b_kc = true;
-  int splits = 1;
+  int splits = 1, tail_splits = 1;
+  int64_t full_tiles = 0;
   Tile tile = Tile::Large;
   DeviceBuffer tables;
   const int64_t *rowA, *colA, *rowB, *colB, *rowC, *colC;
@@ -1105,11 +1213,17 @@ namespace {
 // choice stays the better one only where it is also this one's:
 //   complex No=4 Nv=16 221 -> 103 us, No=12 Nv=60 774 -> 605 us, No=20 Nv=150
 //   21.7 -> 19.4 ms; real No=8 Nv=40 346 -> 167 us, No=20 Nv=150 10.4 -> 9.1 ms.
-void choose_tile(Field f, int64_t M, int64_t N, int64_t K, size_t max_workspace, Tile &tile,
-                 int &splits) {
+//   - where whole waves are followed by a partial one, the partial wave's tiles
+//     can be cut along K instead, so that their parts fill the chip: the same
+//     reduction costs for them alone.  Ladder products 37179 x 496 x 29646: real
+//     21.0 -> 18.1 ms, complex 57.7 -> 52.7 ms; ring 2227^3 complex 1.19 -> 1.15
+//     ms; energy and gradient of No=24, Nv=192, NG=1100 (4608 x 1100 x 4608) 9.2
+//     -> 8.2 ms.
+void choose_tile(Field f, int64_t M, int64_t N, int64_t K, size_t max_workspace, GettPlan &plan) {
   constexpr double kReduce = 3.5, kBytesPerUs = 4e6;
-  tile = Tile::Large;
-  splits = 1;
+  plan.tile = Tile::Large;
+  plan.splits = plan.tail_splits = 1;
+  plan.full_tiles = 0;
   if (M <= 0 || N <= 0 || K <= 0) return;
   const int64_t kstages = (K + kZ3BK - 1) / kZ3BK;
   const double es = static_cast<double>(scalar_bytes(f));
@@ -1120,6 +1234,11 @@ void choose_tile(Field f, int64_t M, int64_t N, int64_t K, size_t max_workspace,
     const int64_t tiles = ((M + s.BM - 1) / s.BM) * ((N + s.BN - 1) / s.BN);
     if (tiles >= (int64_t(1) << 31)) continue;
     const int64_t per = 256 * s.cap;
+    // one wave of c workgroups per CU over n stages
+    auto wave = [&](double n, double c) {
+      return n * std::max(c * s.stage, s.lone) + std::min(n, 8.0) * s.cold +
+             (s.cap > 1 && c > 1 ? 0.5 : 1.0) * s.ends;
+    };
     // every count to 16, then steps of about 6 %
     for (int64_t sp = 1; sp <= std::min<int64_t>(1024, std::max<int64_t>(1, kstages / 2));
          sp += std::max<int64_t>(1, sp / 16)) {
@@ -1127,18 +1246,35 @@ void choose_tile(Field f, int64_t M, int64_t N, int64_t K, size_t max_workspace,
                      M * N >= (int64_t(1) << 31) || tiles * sp > 4 * per))
         break;
       const double n = static_cast<double>((kstages + sp - 1) / sp);
-      auto wave = [&](double c) {
-        return n * std::max(c * s.stage, s.lone) + std::min(n, 8.0) * s.cold +
-               (s.cap > 1 && c > 1 ? 0.5 : 1.0) * s.ends;
-      };
       const int64_t W = tiles * sp, full = W / per, rem = W % per;
-      double cost = static_cast<double>(full) * wave(s.cap);
-      if (rem) cost += wave(static_cast<double>((rem + 255) / 256));
+      double cost = static_cast<double>(full) * wave(n, s.cap);
+      if (rem) cost += wave(n, static_cast<double>((rem + 255) / 256));
       if (sp > 1) cost += kReduce + 2.0 * static_cast<double>(sp) * M * N * es / kBytesPerUs;
       if (best < 0 || cost < best) {
         best = cost;
-        tile = static_cast<Tile>(t);
-        splits = static_cast<int>(sp);
+        plan.tile = static_cast<Tile>(t);
+        plan.splits = static_cast<int>(sp);
+        plan.tail_splits = 1;
+      }
+    }
+    // whole waves, and the rest cut along K
+    const int64_t full = tiles / per, rem = tiles % per;
+    if (fixed_tile || full == 0 || rem == 0) continue;
+    for (int64_t cut = 2; cut <= std::min<int64_t>(32, kstages / 4); ++cut) {
+      const double n = static_cast<double>((kstages + cut - 1) / cut);
+      const double bytes = static_cast<double>(cut * rem) * s.BM * s.BN * es;
+      if (bytes > static_cast<double>(max_workspace)) break;
+      const int64_t W = rem * cut, waves = W / per, last = W % per;
+      double cost = static_cast<double>(full) * wave(static_cast<double>(kstages), s.cap) +
+                    static_cast<double>(waves) * wave(n, s.cap) + kReduce +
+                    2.0 * bytes / kBytesPerUs;
+      if (last) cost += wave(n, static_cast<double>((last + 255) / 256));
+      if (cost < best) {
+        best = cost;
+        plan.tile = static_cast<Tile>(t);
+        plan.splits = 1;
+        plan.tail_splits = static_cast<int>(cut);
+        plan.full_tiles = full * per;
       }
     }
   }
@@ -1226,11 +1362,26 @@ GettPlan &ContractionEngine::plan_for(const View &A0, const View &B0,
   plan->rowC = base; base += rowC.size();
   plan->colC = base;
 
-  choose_tile(C.field, plan->M, plan->N, plan->K, max_workspace, plan->tile, plan->splits);
+  choose_tile(C.field, plan->M, plan->N, plan->K, max_workspace, *plan);
 
   auto &ref = *plan;
   plans_.emplace(key, std::move(plan));
   return ref;
+}
+
+// the workspace for a plan's partial sums, or null
+void *ContractionEngine::reserve_partials(const GettPlan &P, Field f) {
+  size_t elements = 0;
+  if (P.splits > 1) {
+    elements = static_cast<size_t>(P.splits) * P.M * P.N;
+  } else if (P.tail_splits > 1) {
+    const TileShape t = tile_shape(f, P.tile);
+    const int64_t tiles = ((P.M + t.BM - 1) / t.BM) * ((P.N + t.BN - 1) / t.BN);
+    elements = static_cast<size_t>(P.tail_splits) * (tiles - P.full_tiles) * t.BM * t.BN;
+  }
+  if (elements == 0) return nullptr;
+  workspace_.reserve(elements * scalar_bytes(f));
+  return workspace_.get();
 }
 
 GettPlan &ContractionEngine::plan_for2(const View &A1, const View &B1, const View &A2,
@@ -1310,7 +1461,7 @@ GettPlan &ContractionEngine::plan_for2(const View &A1, const View &B1, const Vie
   plan->colB2 = base;
   plan->rowA = P1.rowA; plan->colA = P1.colA; plan->rowB = P1.rowB; plan->colB = P1.colB;
   plan->rowC = P1.rowC; plan->colC = P1.colC;
-  choose_tile(C.field, plan->M, plan->N, plan->K, max_workspace, plan->tile, plan->splits);
+  choose_tile(C.field, plan->M, plan->N, plan->K, max_workspace, *plan);
   auto &ref = *plan;
   plans_.emplace(key, std::move(plan));
   return ref;
@@ -1349,13 +1500,11 @@ void ContractionEngine::contract2(double alpha, const View &A1, const View &B1,
   L.f2 = alpha2 / alpha;
   L.splits = P.splits;
   L.tile = static_cast<int>(P.tile);
+  L.full_tiles = P.full_tiles;
+  L.tail_splits = P.tail_splits;
   L.alpha = alpha; L.beta = beta;
   L.a_kcontig = P.a_kc; L.b_kcontig = P.b_kc;
-  L.W = nullptr;
-  if (P.splits > 1) {
-    workspace_.reserve(static_cast<size_t>(P.splits) * P.M * P.N * 16);
-    L.W = workspace_.get();
-  }
+  L.W = reserve_partials(P, C.field);
   const double flops = 8.0 * double(P.M) * double(P.N) * double(P.K1 + P.K2);
   if (profiling_) {
     Pending p{take_event(), take_event(), gett_variant(L), flops};
@@ -1387,14 +1536,11 @@ void ContractionEngine::contract(double alpha, const View &A, const View &B,
   L.M = P.M; L.N = P.N; L.K = P.K;
   L.splits = P.splits;
   L.tile = static_cast<int>(P.tile);
+  L.full_tiles = P.full_tiles;
+  L.tail_splits = P.tail_splits;
   L.alpha = alpha; L.beta = beta;
   L.a_kcontig = P.a_kc; L.b_kcontig = P.b_kc;
-  L.W = nullptr;
-  if (P.splits > 1) {
-    workspace_.reserve(static_cast<size_t>(P.splits) * P.M * P.N *
-                       scalar_bytes(C.field));
-    L.W = workspace_.get();
-  }
+  L.W = reserve_partials(P, C.field);
   const double flops = (C.field == Field::Complex ? 8.0 : 2.0) * double(P.M) *
                        double(P.N) * double(P.K);
   if (mixed_ && C.field == Field::Complex && flops >= mixed_min_flops) {

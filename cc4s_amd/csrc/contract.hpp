@@ -116,6 +116,7 @@ class ContractionEngine {
   GettPlan &plan_for(const View &A, const View &B, const View &C);
   GettPlan &plan_for2(const View &A1, const View &B1, const View &A2, const View &B2,
                       const View &C);
+  void *reserve_partials(const GettPlan &P, Field f);
   void contract_mixed(GettPlan &P, double alpha, const View &A, const View &B,
                       double beta, const View &C, double flops);
   bool mixed_ = false;
@@ -147,10 +148,12 @@ struct GettLaunch {
   Field field;
   const void *A, *B;
   void *C;
-  void *W;  // split-K partials, splits * M * N elements, or null
+  void *W;  // split-K partials, splits * M * N elements (tail_splits > 1: parts of whole tiles), or null
   const int64_t *rowA, *colA, *rowB, *colB, *rowC, *colC;
   int64_t M, N, K;
   int splits;
+  int64_t full_tiles = 0;  // tiles of whole waves where the others are cut along K
+  int tail_splits = 1;     // parts of each of those others (> 1: partials in W)
   int tile;  // 0 large, 1 medium (64 x 64), 2 small (32 x 32) workgroup tile
   double alpha, beta;
   bool conjA, conjB;

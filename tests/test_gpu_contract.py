@@ -125,7 +125,9 @@ def test_contract_rejects_bad_indices():
 # largest element's sqrt(K): 1e-13 as above.
 TILE_CASES = [(1, 1, 1), (2, 3, 15), (31, 33, 16), (32, 32, 17), (65, 31, 33), (63, 65, 64),
               (129, 127, 48), (1, 700, 31), (700, 1, 257), (5, 6, 40000), (40, 33, 9000),
-              (257, 130, 2000), (1030, 1100, 100), (2000, 2100, 33)]
+              (257, 130, 2000), (1030, 1100, 100), (2000, 2100, 33),
+              # whole waves of tiles and a partial one that is cut along K
+              (1650, 1601, 700), (2300, 1111, 1000)]
 
 
 @pytest.mark.parametrize("cplx", [False, True])
