@@ -436,26 +436,35 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
   // staging registers; DEEP uses two sets, always indexed by constants
   constexpr int NSET = DEEP ? 2 : 1;
   T ra[NSET][EA], rb[NSET][EB];
-  bool segS[NSET];  // SEG2: the registers hold a second-segment stage
   bool segOn = false;  // SEG2: the row pointers are the second segment's
-  auto load_data = [&](auto set_c) {
+  // the stage's EA + EB elements in PARTS parts, part q in [lo(q), lo(q + 1))
+  constexpr int PARTS = BK / 4 - 1;
+  auto lo = [](int q) { return q * (EA + EB) / PARTS; };
+  auto load_part = [&](auto set_c, int part) {
     constexpr int q = decltype(set_c)::value;
     if constexpr (SEG2) {
-      segS[q] = segK;
-      if (segK && !segOn) {  // once, at the first stage of the second segment
-        segOn = true;
+      if (part == 0) {
+        if (segK && !segOn) {  // once, at the first stage of the second segment
+          segOn = true;
 #pragma unroll
-        for (int i = 0; i < NRA; ++i) aRow[i] = aRow2[i];
+          for (int i = 0; i < NRA; ++i) aRow[i] = aRow2[i];
 #pragma unroll
-        for (int i = 0; i < NRB; ++i) bCol[i] = bCol2[i];
+          for (int i = 0; i < NRB; ++i) bCol[i] = bCol2[i];
+        }
       }
     }
 #pragma unroll
     for (int i = 0; i < EA; ++i)
-      ra[q][i] = reinterpret_cast<const T *>(aRow[AKC ? i : 0])[aK[AKC ? 0 : i]];
+      if (i >= lo(part) && i < lo(part + 1))
+        ra[q][i] = reinterpret_cast<const T *>(aRow[AKC ? i : 0])[aK[AKC ? 0 : i]];
 #pragma unroll
     for (int i = 0; i < EB; ++i)
-      rb[q][i] = reinterpret_cast<const T *>(bCol[BKC ? i : 0])[bK[BKC ? 0 : i]];
+      if (EA + i >= lo(part) && EA + i < lo(part + 1))
+        rb[q][i] = reinterpret_cast<const T *>(bCol[BKC ? i : 0])[bK[BKC ? 0 : i]];
+  };
+  auto load_data = [&](auto set_c) {
+#pragma unroll
+    for (int part = 0; part < PARTS; ++part) load_part(set_c, part);
   };
   // conjugation flips the sign bit of the imaginary part (an integer operation:
   // FP64 multiplies would take the MFMAs' cycles)
@@ -466,43 +475,53 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
   };
   // stage s from its registers to LDS: conjugation (and the second segment's
   // factor) applied, elements past K zeroed
-  auto store_lds = [&](int s, int buf, auto set_c) {
+  auto store_part = [&](int s, int buf, auto set_c, int part) {
     constexpr int q = decltype(set_c)::value;
-    int64_t left = p.K - kbeg - static_cast<int64_t>(s) * BK;  // k of this stage within K
-    if constexpr (SEG2) left = segS[q] ? left : p.K1 - kbeg - static_cast<int64_t>(s) * BK;
-    if (left < BK) {
+    const bool seg2 = SEG2 && kbeg + static_cast<int64_t>(s) * BK >= p.K1p;
+    if (part == 0) {
+      int64_t left = p.K - kbeg - static_cast<int64_t>(s) * BK;  // k of this stage within K
+      if constexpr (SEG2) left = seg2 ? left : p.K1 - kbeg - static_cast<int64_t>(s) * BK;
+      if (left < BK) {
 #pragma unroll
-      for (int i = 0; i < EA; ++i)
-        if (a_k(i) >= left) ra[q][i] = T{};
+        for (int i = 0; i < EA; ++i)
+          if (a_k(i) >= left) ra[q][i] = T{};
 #pragma unroll
-      for (int i = 0; i < EB; ++i)
-        if (b_k(i) >= left) rb[q][i] = T{};
+        for (int i = 0; i < EB; ++i)
+          if (b_k(i) >= left) rb[q][i] = T{};
+      }
     }
-    if constexpr (CPLX) {
-      int fa = flipA, fb = flipB, fx = 0;
-      if constexpr (SEG2) {
-        // the second segment's factor: its sign as bits, its size where it is not 1
-        fx = segS[q] && p.f2 < 0.0 ? static_cast<int>(0x80000000u) : 0;
-        fa = fx ^ (segS[q] ? (p.signA2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fa);
-        fb = segS[q] ? (p.signB2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fb;
-        const double f = fabs(p.f2);
-        if (segS[q] && f != 1.0)
+    int fa = flipA, fb = flipB, fx = 0;
+    if constexpr (SEG2) {
+      // the second segment's factor: its sign as bits, its size where it is not 1
+      fx = seg2 && p.f2 < 0.0 ? static_cast<int>(0x80000000u) : 0;
+      fa = fx ^ (seg2 ? (p.signA2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fa);
+      fb = seg2 ? (p.signB2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fb;
+      const double f = fabs(p.f2);
+      if (part == 0 && seg2 && f != 1.0)
 #pragma unroll
-          for (int i = 0; i < EA; ++i) ra[q][i] = make_double2(f * ra[q][i].x, f * ra[q][i].y);
+        for (int i = 0; i < EA; ++i) ra[q][i] = make_double2(f * ra[q][i].x, f * ra[q][i].y);
+    }
+#pragma unroll
+    for (int i = 0; i < EA; ++i)
+      if (i >= lo(part) && i < lo(part + 1)) {
+        if constexpr (CPLX)
+          As[buf][a_k(i)][a_m(i)] = make_double2(SEG2 ? flip(ra[q][i].x, fx) : ra[q][i].x,
+                                                 flip(ra[q][i].y, fa));
+        else
+          As[buf][a_k(i)][a_m(i)] = ra[q][i];
       }
 #pragma unroll
-      for (int i = 0; i < EA; ++i)
-        As[buf][a_k(i)][a_m(i)] = make_double2(SEG2 ? flip(ra[q][i].x, fx) : ra[q][i].x,
-                                               flip(ra[q][i].y, fa));
+    for (int i = 0; i < EB; ++i)
+      if (EA + i >= lo(part) && EA + i < lo(part + 1)) {
+        if constexpr (CPLX)
+          Bs[buf][b_k(i)][b_n(i)] = make_double2(rb[q][i].x, flip(rb[q][i].y, fb));
+        else
+          Bs[buf][b_k(i)][b_n(i)] = rb[q][i];
+      }
+  };
+  auto store_lds = [&](int s, int buf, auto set_c) {
 #pragma unroll
-      for (int i = 0; i < EB; ++i)
-        Bs[buf][b_k(i)][b_n(i)] = make_double2(rb[q][i].x, flip(rb[q][i].y, fb));
-    } else {
-#pragma unroll
-      for (int i = 0; i < EA; ++i) As[buf][a_k(i)][a_m(i)] = ra[q][i];
-#pragma unroll
-      for (int i = 0; i < EB; ++i) Bs[buf][b_k(i)][b_n(i)] = rb[q][i];
-    }
+    for (int part = 0; part < PARTS; ++part) store_part(s, buf, set_c, part);
   };
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, DEEP ? 1 : 0>;
@@ -606,9 +625,11 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
     }
   };
   // one K-stage: multiply LDS buffer s&1, move stage s+1 from its
-  // registers to the other buffer and load a later stage into them, half way
-  // through this stage's MFMAs so that the wave keeps issuing MFMAs around its
-  // memory instructions.  Nothing here stands under a branch (a stage past the
+  // registers to the other buffer and load a later stage into them, a part after
+  // each k step but the last: the two waves of a SIMD reach their memory
+  // instructions together, and the matrix pipe idles while both issue them (all
+  // after one k step: complex ring 7533^3 41.1 ms, in parts 39.6; real 15.2 and
+  // 13.7).  Nothing here stands under a branch (a stage past the
   // end reads valid elements that are never used): at a branch's end the
   // compiler would wait for every LDS operation in flight.  The stage's one
   // barrier stands before the MFMAs of its last k step, whose fragments are in
@@ -630,10 +651,10 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
       // raise what waits for the loads above them
       __builtin_amdgcn_sched_barrier(0);
       multiply(kq & 1);
-      if (kq == KQ / 2 - 1) {
-        store_lds(s + 1, par ^ 1, set_c);
-        load_data(set_c);           // stage s+AHEAD
-        load_koff(s + AHEAD + 1);
+      if (kq < PARTS) {
+        store_part(s + 1, par ^ 1, set_c, kq);
+        load_part(set_c, kq);  // of stage s+AHEAD
+        if (kq == PARTS - 1) load_koff(s + AHEAD + 1);
       }
     }
   };
