@@ -500,8 +500,9 @@ void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
   auto C = [&](double al, const View &A, const View &B, double be, const View &Cv) {
     E.contract(al, A, B, be, Cv);
   };
-  auto S = [&](double al, const View &A, double be, const View &Cv) {
-    E.sum(al, A, be, Cv);
+  // Cv = al A B + Dv
+  auto CD = [&](double al, const View &A, const View &B, const View &Dv, const View &Cv) {
+    E.contract(al, A, B, 1.0, Cv, &Dv);
   };
   auto Vhhpp = [&w](const std::string &names) { return w.Vhhpp_view.as(names); };
   auto &Vhhhp = w.Vhhhp;
@@ -524,29 +525,25 @@ void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
   C(-2.0, B("cdkl"), A("adkl"), 0.0, w.Kac("ac"));              // :465-466
   C(2.0, B("cdkl"), A("cdil"), 0.0, w.Kki("ki"));               // :472-473
   C(2.0, B("cdkl"), T1.as("dl"), 0.0, w.Kck("ck"));             // :613-614
-  S(1.0, w.Kac("ac"), 0.0, w.Lac("ac"));                        // :468
   C(1.0, gam("hp", "Gkd"), T1.as("dk"), 0.0, w.wG("G"));        // :469
-  C(2.0, gam("pp", "Gac", true), w.wG("G"), 1.0, w.Lac("ac"));
+  CD(2.0, gam("pp", "Gac", true), w.wG("G"), w.Kac("ac"), w.Lac("ac"));  // :468
   C(1.0, gam("pp", "Gad", true), T1.as("dk"), 0.0, w.Zgvo("Gak"));  // :470
   C(-1.0, w.Zgvo("Gak"), gam("hp", "Gkc"), 1.0, w.Lac("ac"));
-  S(1.0, w.Kki("ki"), 0.0, w.Lki("ki"));                        // :476
-  C(2.0, Vhhhp("klic"), T1.as("cl"), 1.0, w.Lki("ki"));         // :477
+  CD(2.0, Vhhhp("klic"), T1.as("cl"), w.Kki("ki"), w.Lki("ki"));  // :476-477
   C(-1.0, Vhhhp("lkic"), T1.as("cl"), 1.0, w.Lki("ki"));        // :478
   C(1.0, w.Lac("ac"), T2.as("cbij"), 0.0, R2);                  // :481
   C(-1.0, w.Lki("ki"), T2.as("abkj"), 1.0, R2);                 // :484
-  S(1.0, gam("ph", "Gai", true), 0.0, w.DGph("Gai"));           // :487
-  C(-1.0, gam("hh", "Gki", true), T1.as("ak"), 1.0, w.DGph("Gai"));  // :488
+  CD(-1.0, gam("hh", "Gki", true), T1.as("ak"), gam("ph", "Gai", true),
+     w.DGph("Gai"));                                            // :487-488
   C(1.0, gam("pp", "Gbc"), T1.as("cj"), 0.0, w.Wgvo("Gbj"));    // :489
   C(1.0, w.DGph("Gai"), w.Wgvo("Gbj"), 1.0, R2);
   // Q_akij = V_akij + V_akic T_cj (:490-491); complex: V_akic = sum_G
   // cTGamma_ph[G,a,i] Gamma_hp[G,k,c] (slice phhp) through G; real: V_akic is V_acik
   if (cplx) {
     C(1.0, gam("hp", "Gkc"), T1.as("cj"), 0.0, w.Zgoo("Gkj"));
-    C(1.0, gam("ph", "Gai", true), w.Zgoo("Gkj"), 0.0, w.Wvooo("akij"));
-    S(1.0, w.Vphhh("akij"), 1.0, w.Wvooo("akij"));
+    CD(1.0, gam("ph", "Gai", true), w.Zgoo("Gkj"), w.Vphhh("akij"), w.Wvooo("akij"));
   } else {
-    C(1.0, Vpphh.as("acik"), T1.as("cj"), 0.0, w.Wvooo("akij"));
-    S(1.0, Vhhhp("jika"), 1.0, w.Wvooo("akij"));
+    CD(1.0, Vpphh.as("acik"), T1.as("cj"), Vhhhp("jika"), w.Wvooo("akij"));
   }
   // the resident ladder (half of it: R2 is symmetrised below) and, with U_kaji
   // in Q_akij, the T1 dressing of its left or right vertex
@@ -555,13 +552,12 @@ void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
   C(-1.0, w.Wvooo("akij"), T1.as("bk"), 1.0, R2);
   // A = T2 + 2 T1 T1
   tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 2.0, o, v);         // :462-463
-  S(1.0, w.Zgvo("Gai"), 1.0, w.DGph("Gai"));                    // :494
+  E.sum(1.0, w.Zgvo("Gai"), 1.0, w.DGph("Gai"));                // :494
   C(-0.5, gam("hp", "Gld", true), A("dail"), 1.0, w.DGph("Gai"));   // :495
   // crossed ring, its intermediate Xakci stored as [a,k,i,c]; A = Z
-  S(1.0, gam("pp", "Gab", true), 0.0, w.DGpp("Gab"));           // :509
-  C(-1.0, gam("hp", "Glc", true), T1.as("al"), 1.0, w.DGpp("Gac"));  // :510
-  S(1.0, gam("hh", "Gij"), 0.0, w.DGhh("Gij"));                 // :511
-  C(1.0, gam("hp", "Gkd"), T1.as("di"), 1.0, w.DGhh("Gki"));    // :512
+  CD(-1.0, gam("hp", "Glc", true), T1.as("al"), gam("pp", "Gac", true),
+     w.DGpp("Gac"));                                            // :509-510
+  CD(1.0, gam("hp", "Gkd"), T1.as("di"), gam("hh", "Gki"), w.DGhh("Gki"));  // :511-512
   C(1.0, w.DGpp("Gac"), w.DGhh("Gki"), 0.0, X("akic"));         // :514
   C(-0.5, Vhhpp("lkcd"), T2.as("dail"), 1.0, X("akic"));        // :515
   C(1.0, X("bkic"), T2.as("ackj"), 0.0, A("abij"));             // :517
@@ -573,12 +569,10 @@ void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
   combine(w.X.v, T2, 2.0, -1.0, 0.0);                           // :500-501
   C(1.0, X("akic"), A("cbkj"), 1.0, R2);                        // :502, :516
   C(1.0, w.Kck("ck"), A("caki"), 0.0, R1);                      // :617-618
-  symmetrize_pairs(st, f, R2.ptr, o, v);                        // :520
-  S(1.0, Vpphh, 1.0, R2);                                       // :529
+  symmetrize_pairs(st, f, R2.ptr, o, v, Vpphh.ptr);             // :520, 529
   // hole ladder; A = tau
   tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 1.0, o, v);
-  S(1.0, w.Vhhhh("klij"), 0.0, w.Xklij("klij"));                // :534
-  C(1.0, Vhhhp("klic"), T1.as("cj"), 1.0, w.Xklij("klij"));     // :535
+  CD(1.0, Vhhhp("klic"), T1.as("cj"), w.Vhhhh("klij"), w.Xklij("klij"));  // :534-535
   C(1.0, Vhhhp("lkjc"), T1.as("ci"), 1.0, w.Xklij("klij"));     // :536
   if (opt_.ppl && !resident) {
     C(1.0, w.Xklij("klij"), A("abkl"), 1.0, R2);                // :538

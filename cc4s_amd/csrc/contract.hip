@@ -23,6 +23,10 @@ struct KArgs {
   double *C;
   double *W;
   const int64_t *rowA, *colA, *rowB, *colB, *rowC, *colC;
+  // C = alpha A B + beta D: D is C itself or another tensor of C's indices
+  const double *D;
+  const int64_t *rowD, *colD;
+  double signD;  // -1 conjugates D
   int64_t M, N, K, kChunk;
   double alpha, beta;
   double signA, signB;  // -1 conjugates the operand's imaginary part
@@ -42,6 +46,22 @@ struct KArgs {
   int fullTiles, tailTiles, tailSplits;
   int64_t tailChunk;
 };
+
+// C[oc] = alpha x + beta D[od]
+__device__ __forceinline__ void store_result(const KArgs &p, double2 x, int64_t oc, int64_t od) {
+  double2 out = make_double2(p.alpha * x.x, p.alpha * x.y);
+  if (p.beta != 0.0) {
+    const double2 old = reinterpret_cast<const double2 *>(p.D)[od];
+    out.x += p.beta * old.x;
+    out.y += p.beta * (p.signD * old.y);
+  }
+  reinterpret_cast<double2 *>(p.C)[oc] = out;
+}
+__device__ __forceinline__ void store_result(const KArgs &p, double x, int64_t oc, int64_t od) {
+  double out = p.alpha * x;
+  if (p.beta != 0.0) out += p.beta * p.D[od];
+  p.C[oc] = out;
+}
 
 // index in a contiguous run of `n` items per XCD: workgroups go round the 8 XCDs
 __device__ __forceinline__ int xcd_run(int g, int n) {
@@ -686,13 +706,14 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
         }
     return;
   }
-  int64_t cCol[NB];
+  int64_t cCol[NB], dCol[NB];
   bool cColOk[NB];
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
     const int64_t n = n0 + wn * WN + j * 16 + (lane & 15);
     cColOk[j] = n < p.N;
     cCol[j] = (cColOk[j] && !p.W) ? p.colC[n] : 0;
+    dCol[j] = (cColOk[j] && !p.W) ? p.colD[n] : 0;
   }
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
@@ -700,43 +721,24 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
     for (int r = 0; r < 4; ++r) {
       const int64_t m = m0 + wm * WM + i * 16 + 4 * r + (lane >> 4);
       if (m >= p.M) continue;
-      const int64_t rc = p.W ? 0 : p.rowC[m];
+      const int64_t rc = p.W ? 0 : p.rowC[m], rd = p.W ? 0 : p.rowD[m];
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
         if (!cColOk[j]) continue;
         const int64_t n = n0 + wn * WN + j * 16 + (lane & 15);
-        if constexpr (CPLX) {
-          double vr = accR[i][j][r];
-          double vi = accI[i][j][r];
-          if constexpr (M3) {
-            const double p1 = vr, p2 = vi;
-            vr = p1 - p2;
-            vi = accS[i][j][r] - (p1 + p2);
-          }
-          if (p.W) {
-            const int64_t o = (static_cast<int64_t>(blockIdx.y) * p.M + m) * p.N + n;
-            reinterpret_cast<double2 *>(p.W)[o] = make_double2(vr, vi);
-          } else {
-            double2 *c = reinterpret_cast<double2 *>(p.C) + rc + cCol[j];
-            double2 out = make_double2(p.alpha * vr, p.alpha * vi);
-            if (p.beta != 0.0) {
-              const double2 old = *c;
-              out.x += p.beta * old.x;
-              out.y += p.beta * old.y;
-            }
-            *c = out;
-          }
+        T x;
+        if constexpr (!CPLX) {
+          x = accR[i][j][r];
+        } else if constexpr (M3) {
+          const double p1 = accR[i][j][r], p2 = accI[i][j][r];
+          x = make_double2(p1 - p2, accS[i][j][r] - (p1 + p2));
         } else {
-          const double vr = accR[i][j][r];
-          if (p.W) {
-            p.W[(static_cast<int64_t>(blockIdx.y) * p.M + m) * p.N + n] = vr;
-          } else {
-            double *c = p.C + rc + cCol[j];
-            double out = p.alpha * vr;
-            if (p.beta != 0.0) out += p.beta * *c;
-            *c = out;
-          }
+          x = make_double2(accR[i][j][r], accI[i][j][r]);
         }
+        if (p.W)
+          reinterpret_cast<T *>(p.W)[(static_cast<int64_t>(blockIdx.y) * p.M + m) * p.N + n] = x;
+        else
+          store_result(p, x, rc + cCol[j], rd + dCol[j]);
       }
     }
   }
@@ -748,14 +750,13 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
 // of splits, four loads in flight per thread; the group sums are added in LDS.
 // Both orders are fixed, so the result is reproducible.
 template <bool CPLX, int G>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(
-    const double *W, double *C, const int64_t *rowC, const int64_t *colC, uint32_t total,
-    uint32_t N, int splits, double alpha, double beta) {
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(KArgs p, int splits) {
+  const uint32_t total = static_cast<uint32_t>(p.M * p.N), N = static_cast<uint32_t>(p.N);
   using T = std::conditional_t<CPLX, double2, double>;
   constexpr uint32_t E = 256 / G;
   __shared__ T part[G][E];
   const uint32_t u = threadIdx.x % E, g = threadIdx.x / E;
-  const T *w = reinterpret_cast<const T *>(W);
+  const T *w = reinterpret_cast<const T *>(p.W);
   for (uint32_t e0 = blockIdx.x * E; e0 < total; e0 += gridDim.x * E) {
     const uint32_t e = e0 + u;
     const uint32_t ec = e < total ? e : total - 1;
@@ -785,21 +786,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(
     }
     if (g == 0 && e < total) {
       const uint32_t m = e / N, n = e - m * N;
-      const int64_t o = rowC[m] + colC[n];
-      T *c = reinterpret_cast<T *>(C) + o;
-      T out;
-      if constexpr (CPLX) {
-        out = make_double2(alpha * acc[0].x, alpha * acc[0].y);
-        if (beta != 0.0) {
-          const T old = *c;
-          out.x += beta * old.x;
-          out.y += beta * old.y;
-        }
-      } else {
-        out = alpha * acc[0];
-        if (beta != 0.0) out += beta * *c;
-      }
-      *c = out;
+      store_result(p, acc[0], p.rowC[m] + p.colC[n], p.rowD[m] + p.colD[n]);
     }
     if constexpr (G > 1) __syncthreads();  // part is written again
   }
@@ -832,20 +819,7 @@ __global__ __launch_bounds__(256) void tail_reduce_kernel(KArgs p, int BM, int B
       acc += x;
     }
   }
-  T *c = reinterpret_cast<T *>(p.C) + p.rowC[m] + p.colC[n];
-  if constexpr (CPLX) {
-    T out = make_double2(p.alpha * acc.x, p.alpha * acc.y);
-    if (p.beta != 0.0) {
-      const T old = *c;
-      out.x += p.beta * old.x;
-      out.y += p.beta * old.y;
-    }
-    *c = out;
-  } else {
-    T out = p.alpha * acc;
-    if (p.beta != 0.0) out += p.beta * *c;
-    *c = out;
-  }
+  store_result(p, acc, p.rowC[m] + p.colC[n], p.rowD[m] + p.colD[n]);
 }
 
 constexpr int kMaxRank = 8;
@@ -977,6 +951,10 @@ std::string gett_variant(const GettLaunch &L) {
   return n;
 }
 
+namespace {
+void reduce_partials(bool cplx, const KArgs &a, int splits, hipStream_t s);
+}
+
 void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
                  hipEvent_t stop) {
   const bool cplx = L.field == Field::Complex;
@@ -993,6 +971,12 @@ void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
   a.W = L.splits > 1 ? static_cast<double *>(L.W) : nullptr;
   a.rowA = L.rowA; a.colA = L.colA; a.rowB = L.rowB; a.colB = L.colB;
   a.rowC = L.rowC; a.colC = L.colC;
+  a.D = L.D ? static_cast<const double *>(L.D) : a.C;
+  a.rowD = L.D ? L.rowD : L.rowC;
+  a.colD = L.D ? L.colD : L.colC;
+  a.signD = L.conjD ? -1.0 : 1.0;
+  CC4S_ASSERT(!L.D || !cplx || g_complex_generation != 1,
+              "the first-generation kernel adds to its own result only");
   a.M = L.M; a.N = L.N; a.K = L.K;
   const int64_t kstages = (L.K + BK - 1) / BK;
   a.kChunk = ((kstages + L.splits - 1) / L.splits) * BK;
@@ -1059,31 +1043,42 @@ void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
       tail_reduce_kernel<false><<<blocks, 256, 0, s>>>(a, BM, BN, GM);
     CC4S_HIP(hipGetLastError());
   }
-  if (L.splits > 1)
-    launch_splitk_reduce(L.field, a.W, a.C, L.rowC, L.colC, L.M, L.N, L.splits,
-                         L.alpha, L.beta, s);
+  if (L.splits > 1) reduce_partials(cplx, a, L.splits, s);
 }
+
+namespace {
+void reduce_partials(bool cplx, const KArgs &a, int splits, hipStream_t s) {
+  CC4S_ASSERT(a.M * a.N < (int64_t(1) << 31), "split-K result too large");
+  const int64_t total = a.M * a.N;
+  auto run = [&](auto kernel, int G) { kernel<<<grid_for(total * G), 256, 0, s>>>(a, splits); };
+  // groups of splits while the elements alone leave the chip idle (under 64 K
+  // threads) and every group still has several splits
+  if (total < 16384 && splits >= 32)
+    cplx ? run(splitk_reduce_kernel<true, 16>, 16) : run(splitk_reduce_kernel<false, 16>, 16);
+  else if (total < 65536 && splits >= 8)
+    cplx ? run(splitk_reduce_kernel<true, 4>, 4) : run(splitk_reduce_kernel<false, 4>, 4);
+  else
+    cplx ? run(splitk_reduce_kernel<true, 1>, 1) : run(splitk_reduce_kernel<false, 1>, 1);
+  CC4S_HIP(hipGetLastError());
+}
+}  // namespace
 
 void launch_splitk_reduce(Field f, const double *W, double *C,
                           const int64_t *rowC, const int64_t *colC, int64_t M,
                           int64_t N, int splits, double alpha, double beta,
                           hipStream_t s) {
-  CC4S_ASSERT(M * N < (int64_t(1) << 31), "split-K result too large");
-  const uint32_t total = static_cast<uint32_t>(M * N), n32 = static_cast<uint32_t>(N);
-  auto run = [&](auto kernel, int G) {
-    kernel<<<grid_for(static_cast<int64_t>(total) * G), 256, 0, s>>>(W, C, rowC, colC, total, n32,
-                                                                   splits, alpha, beta);
-  };
-  // groups of splits while the elements alone leave the chip idle (under 64 K
-  // threads) and every group still has several splits
-  const bool c = f == Field::Complex;
-  if (total < 16384 && splits >= 32)
-    c ? run(splitk_reduce_kernel<true, 16>, 16) : run(splitk_reduce_kernel<false, 16>, 16);
-  else if (total < 65536 && splits >= 8)
-    c ? run(splitk_reduce_kernel<true, 4>, 4) : run(splitk_reduce_kernel<false, 4>, 4);
-  else
-    c ? run(splitk_reduce_kernel<true, 1>, 1) : run(splitk_reduce_kernel<false, 1>, 1);
-  CC4S_HIP(hipGetLastError());
+  KArgs a{};
+  a.W = const_cast<double *>(W);
+  a.C = C;
+  a.D = C;
+  a.rowC = a.rowD = rowC;
+  a.colC = a.colD = colC;
+  a.signD = 1.0;
+  a.M = M;
+  a.N = N;
+  a.alpha = alpha;
+  a.beta = beta;
+  reduce_partials(f == Field::Complex, a, splits, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1098,6 +1093,7 @@ struct GettPlan {
   Tile tile = Tile::Large;
   DeviceBuffer tables;
   const int64_t *rowA, *colA, *rowB, *colB, *rowC, *colC;
+  const int64_t *rowD = nullptr, *colD = nullptr;  // of an added tensor other than C
   // two-segment plans: the second contraction's tables; swap2 tells that
   // its second operand carries the M indices
   bool swap2 = false;
@@ -1304,8 +1300,9 @@ void choose_tile(Field f, int64_t M, int64_t N, int64_t K, size_t max_workspace,
 }  // namespace
 
 GettPlan &ContractionEngine::plan_for(const View &A0, const View &B0,
-                                      const View &C) {
-  const std::string key = plan_key(A0, B0, C);
+                                      const View &C, const View *D) {
+  std::string key = plan_key(A0, B0, C);
+  if (D) key += "+" + plan_key(*D, *D, *D);
   auto it = plans_.find(key);
   if (it != plans_.end()) return *it->second;
 
@@ -1328,6 +1325,11 @@ GettPlan &ContractionEngine::plan_for(const View &A0, const View &B0,
                 std::string("index '") + c + "' only in one operand");
   for (char c : Ki)
     CC4S_ASSERT(A0.len(c) == B0.len(c), std::string("length mismatch of '") + c + "'");
+  if (D) {
+    CC4S_ASSERT(D->rank() == C.rank(), "added tensor has other indices");
+    for (char c : C.idx)
+      CC4S_ASSERT(D->find(c) >= 0 && D->len(c) == C.len(c), "length mismatch (added tensor)");
+  }
   for (char c : Mi) CC4S_ASSERT(A0.len(c) == C.len(c), "length mismatch (A, C)");
   for (char c : Ni) CC4S_ASSERT(B0.len(c) == C.len(c), "length mismatch (B, C)");
 
@@ -1372,6 +1374,13 @@ GettPlan &ContractionEngine::plan_for(const View &A0, const View &B0,
     all.insert(all.end(), v.begin(), v.end());
   };
   append(rowA); append(colA); append(rowB); append(colB); append(rowC); append(colC);
+  std::vector<int64_t> rowD, colD;
+  if (D) {
+    rowD = offsets(*D, Mi, C);
+    colD = offsets(*D, Ni, C);
+    append(rowD);
+    append(colD);
+  }
   plan->tables.allocate(all.size() * sizeof(int64_t));
   CC4S_HIP(hipMemcpy(plan->tables.get(), all.data(), all.size() * sizeof(int64_t),
                      hipMemcpyHostToDevice));
@@ -1381,7 +1390,11 @@ GettPlan &ContractionEngine::plan_for(const View &A0, const View &B0,
   plan->rowB = base; base += rowB.size();
   plan->colB = base; base += colB.size();
   plan->rowC = base; base += rowC.size();
-  plan->colC = base;
+  plan->colC = base; base += colC.size();
+  if (D) {
+    plan->rowD = base; base += rowD.size();
+    plan->colD = base;
+  }
 
   choose_tile(C.field, plan->M, plan->N, plan->K, max_workspace, *plan);
 
@@ -1540,10 +1553,15 @@ void ContractionEngine::contract2(double alpha, const View &A1, const View &B1,
 }
 
 void ContractionEngine::contract(double alpha, const View &A, const View &B,
-                                 double beta, const View &C) {
+                                 double beta, const View &C, const View *D) {
   CC4S_ASSERT(A.field == C.field && B.field == C.field, "mixed scalar fields");
   CC4S_ASSERT(!C.conj, "conjugated result view");
-  GettPlan &P = plan_for(A, B, C);
+  CC4S_ASSERT(!D || (D->field == C.field && !mixed_), "added tensor in a split pass");
+  if (D && C.field == Field::Complex && g_complex_generation == 1) {
+    sum(1.0, *D, 0.0, C);
+    D = nullptr;
+  }
+  GettPlan &P = plan_for(A, B, C, D);
   if (P.M == 0 || P.N == 0) return;
   GettLaunch L;
   L.field = C.field;
@@ -1554,6 +1572,11 @@ void ContractionEngine::contract(double alpha, const View &A, const View &B,
   L.C = C.ptr;
   L.rowA = P.rowA; L.colA = P.colA; L.rowB = P.rowB; L.colB = P.colB;
   L.rowC = P.rowC; L.colC = P.colC;
+  if (D) {
+    L.D = D->ptr;
+    L.conjD = D->conj;
+    L.rowD = P.rowD; L.colD = P.colD;
+  }
   L.M = P.M; L.N = P.N; L.K = P.K;
   L.splits = P.splits;
   L.tile = static_cast<int>(P.tile);

@@ -40,9 +40,11 @@ class ContractionEngine {
   explicit ContractionEngine(hipStream_t s);
   ~ContractionEngine();
 
-  // C = alpha * op(A) op(B) + beta * C, op = conjugation where the view says
+  // C = alpha * op(A) op(B) + beta * op(D), op = conjugation where the view says;
+  // without D, D is C (FP64 passes may name another tensor of C's indices, whose
+  // copy into C it saves)
   void contract(double alpha, const View &A, const View &B, double beta,
-                const View &C);
+                const View &C, const View *D = nullptr);
   // C = alpha * op(A1) op(B1) + alpha2 * op(A2) op(B2) + beta * C for two
   // contractions whose operands split C's indices the same way: one launch
   // with the second contraction as a second K segment, so C is read and
@@ -113,7 +115,7 @@ class ContractionEngine {
   }
 
  private:
-  GettPlan &plan_for(const View &A, const View &B, const View &C);
+  GettPlan &plan_for(const View &A, const View &B, const View &C, const View *D = nullptr);
   GettPlan &plan_for2(const View &A1, const View &B1, const View &A2, const View &B2,
                       const View &C);
   void *reserve_partials(const GettPlan &P, Field f);
@@ -166,6 +168,10 @@ struct GettLaunch {
   int64_t K1 = 0, K1p = 0, K2 = 0;
   double f2 = 1.0;
   bool conjA2 = false, conjB2 = false;
+  // tensor added with beta (null: C)
+  const void *D = nullptr;
+  const int64_t *rowD = nullptr, *colD = nullptr;
+  bool conjD = false;
 };
 // `start`/`stop` (optional) bracket the main kernel, not the reduction
 void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start = nullptr,

@@ -65,12 +65,13 @@ __global__ __launch_bounds__(kBlock) void tau_kernel(typename Sc<CPLX>::T *X,
 // read and written along their contiguous index
 constexpr int kPairTile = 32;
 
-// R_abij <- R_abij + R_baji (old values on the right): one block per
+// R_abij <- R_abij + R_baji (old values on the right) + V_abij (V may be null):
+// one block per
 // unordered pair of tiles {(A, B, i, j), (B, A, j, i)}, taken where
 // (i, tile A) <= (j, tile B); both tiles are read before either is written
 template <bool CPLX>
-__global__ __launch_bounds__(kBlock) void symmetrize_kernel(typename Sc<CPLX>::T *R,
-                                                            int64_t No, int64_t Nv) {
+__global__ __launch_bounds__(kBlock) void symmetrize_kernel(
+    typename Sc<CPLX>::T *R, const typename Sc<CPLX>::T *__restrict__ V, int64_t No, int64_t Nv) {
   using S = Sc<CPLX>;
   using T = typename S::T;
   constexpr int kt = kPairTile;
@@ -94,10 +95,16 @@ __global__ __launch_bounds__(kBlock) void symmetrize_kernel(typename Sc<CPLX>::T
     __syncthreads();
     for (int e = threadIdx.x; e < kt * kt; e += kBlock) {
       const int u = e % kt, w = e / kt;
-      if (a0 + u < Nv && b0 + w < Nv)
-        R[offX + (a0 + u) + Nv * (b0 + w)] = S::add(xs[u][w], ys[w][u]);
-      if (P != Q && b0 + u < Nv && a0 + w < Nv)
-        R[offY + (b0 + u) + Nv * (a0 + w)] = S::add(ys[u][w], xs[w][u]);
+      if (a0 + u < Nv && b0 + w < Nv) {
+        const int64_t o = offX + (a0 + u) + Nv * (b0 + w);
+        const T r = S::add(xs[u][w], ys[w][u]);
+        R[o] = V ? S::add(r, V[o]) : r;
+      }
+      if (P != Q && b0 + u < Nv && a0 + w < Nv) {
+        const int64_t o = offY + (b0 + u) + Nv * (a0 + w);
+        const T r = S::add(ys[u][w], xs[w][u]);
+        R[o] = V ? S::add(r, V[o]) : r;
+      }
     }
   }
 }
@@ -363,11 +370,13 @@ void tau(hipStream_t s, Field f, void *X, const void *T2, const void *T1,
   CC4S_HIP(hipGetLastError());
 }
 
-void symmetrize_pairs(hipStream_t s, Field f, void *R2, int64_t No, int64_t Nv) {
+void symmetrize_pairs(hipStream_t s, Field f, void *R2, int64_t No, int64_t Nv, const void *V) {
   if (f == Field::Complex)
-    symmetrize_kernel<true><<<kReduceBlocks, kBlock, 0, s>>>(static_cast<double2 *>(R2), No, Nv);
+    symmetrize_kernel<true><<<kReduceBlocks, kBlock, 0, s>>>(
+        static_cast<double2 *>(R2), static_cast<const double2 *>(V), No, Nv);
   else
-    symmetrize_kernel<false><<<kReduceBlocks, kBlock, 0, s>>>(static_cast<double *>(R2), No, Nv);
+    symmetrize_kernel<false><<<kReduceBlocks, kBlock, 0, s>>>(
+        static_cast<double *>(R2), static_cast<const double *>(V), No, Nv);
   CC4S_HIP(hipGetLastError());
 }
 

@@ -14,8 +14,10 @@ using cplx = std::complex<double>;
 void tau(hipStream_t s, Field f, void *X, const void *T2, const void *T1,
          double factor, int64_t No, int64_t Nv);
 
-// R_abij += R_baji with the old values on both sides (Ccsd.cxx:256, 520)
-void symmetrize_pairs(hipStream_t s, Field f, void *R2, int64_t No, int64_t Nv);
+// R_abij += R_baji with the old values on both sides (Ccsd.cxx:256, 520), then
+// R_abij += V_abij unless V is null (:263, 529)
+void symmetrize_pairs(hipStream_t s, Field f, void *R2, int64_t No, int64_t Nv,
+                      const void *V = nullptr);
 
 // out_abij = alpha in_abij + beta in_baij + gamma out_abij (gamma 0: out is not
 // read), `in` conjugated first with conj; out and in are different [v,v,o,o]
