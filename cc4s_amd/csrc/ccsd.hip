@@ -41,7 +41,7 @@ struct Ccsd::Work {
   // resident ladder: pair integrals S, A and the products Rp, Rm; formed at
   // the first pass that can use them
   enum class Resident { Unknown, Ready, Off } resident = Resident::Unknown;
-  Tensor VS, VA, Rp, Rm;
+  Tensor VS, VA, Rp, Rm, Tpm;  // Tpm: tau's combinations
   int64_t NGe = 0;  // length of the G index of the real-path vertex views
   bool hermitian = false;
 };
@@ -326,7 +326,8 @@ bool Ccsd::resident_integrals() {
   const int64_t Np = o * (o + 1) / 2, Nm = o * (o - 1) / 2;
   const double es = static_cast<double>(scalar_bytes(f));
   const double need = es * (double(Kp) * double(Kp + o * v) + double(Km) * double(Km + o * v) +
-                            double(Np) * double(Kp + o * v) + double(Nm) * double(Km + o * v));
+                            double(Np) * double(Kp + o * v) + double(Nm) * double(Km + o * v) +
+                            double(Kp) * double(Np) + double(Km) * double(Nm));
   size_t free_b = 0, total_b = 0;
   CC4S_HIP(hipMemGetInfo(&free_b, &total_b));
   const double avail = static_cast<double>(free_b) - 6.0 * (1 << 30);
@@ -344,6 +345,7 @@ bool Ccsd::resident_integrals() {
     w.VA.reset(f, "km", {Km, Km + o * v});
     w.Rp.reset(f, "nm", {Np, Kp + o * v});
     w.Rm.reset(f, "nm", {Nm, Km + o * v});
+    w.Tpm.reset(f, "n", {Kp * Np + Km * Nm});
     slab.reset(f, "cxdy", {v, nx, v, v});
   } catch (const Error &) {  // no room after all
     (void)hipGetLastError();
@@ -351,6 +353,7 @@ bool Ccsd::resident_integrals() {
     w.VA = Tensor();
     w.Rp = Tensor();
     w.Rm = Tensor();
+    w.Tpm = Tensor();
     return false;
   }
   const hipStream_t st = E_.stream();
@@ -376,8 +379,17 @@ bool Ccsd::resident_integrals() {
   return true;
 }
 
-// Rp and Rm of the resident ladder; tau's combinations go to Xakic's buffer
-void Ccsd::resident_products(const View &tauv) {
+// tau's combinations of the resident ladder
+void Ccsd::resident_combinations(const View &tauv) {
+  auto &w = *w_;
+  const int64_t Kp = s_.Nv * (s_.Nv + 1) / 2, Np = s_.No * (s_.No + 1) / 2;
+  void *Tp = w.Tpm.buf.get();
+  ladder_tau_pairs(s_.field, tauv.ptr, Tp, offset_ptr(Tp, Kp * Np, s_.field), 0.5, s_.Nv, s_.No,
+                   E_.stream());
+}
+
+// Rp and Rm of the resident ladder
+void Ccsd::resident_products() {
   auto &w = *w_;
   const Field f = s_.field;
   const int64_t o = s_.No, v = s_.Nv;
@@ -389,9 +401,8 @@ void Ccsd::resident_products(const View &tauv) {
     CC4S_HIP(hipEventCreate(&e1));
     CC4S_HIP(hipEventRecord(e0, E_.stream()));
   }
-  void *Tp = w.Xakic.buf.get();
+  void *Tp = w.Tpm.buf.get();
   void *Tm = offset_ptr(Tp, Kp * Np, f);
-  ladder_tau_pairs(f, tauv.ptr, Tp, Tm, 0.5, v, o, E_.stream());
   const double flops0 = E_.stats.flops;
   E_.contract(1.0, w.VS("km"), dense_view(Tp, f, "kn", {Kp, Np}), 0.0, w.Rp("nm"));
   E_.contract(1.0, w.VA("km"), dense_view(Tm, f, "kn", {Km, Nm}), 0.0, w.Rm("nm"));
@@ -516,89 +527,113 @@ void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
     exchange_combination(st, f, out.ptr, in.ptr, al, be, ga, conj, o, v);
   };
 
-  // A = tau; the resident ladder's products
+  // A = tau, B = Wt
   tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 1.0, o, v);         // :460-461
   const bool resident = opt_.ppl && resident_integrals();
-  if (resident) resident_products(w.X.v);
-  // one-particle intermediates; B = Wt
+  // the hole ladder acts on tau in one product unless the slab ladder follows
+  const bool merged = resident || !opt_.ppl;
+  if (resident) resident_combinations(w.X.v);
+  if (resident && profile) resident_products();  // timed by itself
   combine(Bv, Vpphh, 1.0, -0.5, 0.0, cplx);
-  C(-2.0, B("cdkl"), A("adkl"), 0.0, w.Kac("ac"));              // :465-466
-  C(2.0, B("cdkl"), A("cdil"), 0.0, w.Kki("ki"));               // :472-473
-  C(2.0, B("cdkl"), T1.as("dl"), 0.0, w.Kck("ck"));             // :613-614
-  C(1.0, gam("hp", "Gkd"), T1.as("dk"), 0.0, w.wG("G"));        // :469
-  CD(2.0, gam("pp", "Gac", true), w.wG("G"), w.Kac("ac"), w.Lac("ac"));  // :468
-  C(1.0, gam("pp", "Gad", true), T1.as("dk"), 0.0, w.Zgvo("Gak"));  // :470
-  C(-1.0, w.Zgvo("Gak"), gam("hp", "Gkc"), 1.0, w.Lac("ac"));
-  CD(2.0, Vhhhp("klic"), T1.as("cl"), w.Kki("ki"), w.Lki("ki"));  // :476-477
-  C(-1.0, Vhhhp("lkic"), T1.as("cl"), 1.0, w.Lki("ki"));        // :478
-  C(1.0, w.Lac("ac"), T2.as("cbij"), 0.0, R2);                  // :481
-  C(-1.0, w.Lki("ki"), T2.as("abkj"), 1.0, R2);                 // :484
-  CD(-1.0, gam("hh", "Gki", true), T1.as("ak"), gam("ph", "Gai", true),
-     w.DGph("Gai"));                                            // :487-488
-  C(1.0, gam("pp", "Gbc"), T1.as("cj"), 0.0, w.Wgvo("Gbj"));    // :489
-  C(1.0, w.DGph("Gai"), w.Wgvo("Gbj"), 1.0, R2);
-  // Q_akij = V_akij + V_akic T_cj (:490-491); complex: V_akic = sum_G
-  // cTGamma_ph[G,a,i] Gamma_hp[G,k,c] (slice phhp) through G; real: V_akic is V_acik
-  if (cplx) {
-    C(1.0, gam("hp", "Gkc"), T1.as("cj"), 0.0, w.Zgoo("Gkj"));
-    CD(1.0, gam("ph", "Gai", true), w.Zgoo("Gkj"), w.Vphhh("akij"), w.Wvooo("akij"));
-  } else {
-    CD(1.0, Vpphh.as("acik"), T1.as("cj"), Vhhhp("jika"), w.Wvooo("akij"));
-  }
-  // the resident ladder (half of it: R2 is symmetrised below) and, with U_kaji
-  // in Q_akij, the T1 dressing of its left or right vertex
+  // each group's statements do not depend on each other
+  E.group([&] {
+    if (resident && !profile) resident_products();
+    C(-2.0, B("cdkl"), A("adkl"), 0.0, w.Kac("ac"));              // :465-466
+    C(2.0, B("cdkl"), A("cdil"), 0.0, w.Kki("ki"));               // :472-473
+    C(2.0, B("cdkl"), T1.as("dl"), 0.0, w.Kck("ck"));             // :613-614
+    C(1.0, gam("hp", "Gkd"), T1.as("dk"), 0.0, w.wG("G"));        // :469
+    C(1.0, gam("pp", "Gad", true), T1.as("dk"), 0.0, w.Zgvo("Gak"));  // :470
+    C(1.0, gam("pp", "Gbc"), T1.as("cj"), 0.0, w.Wgvo("Gbj"));    // :489
+    CD(-1.0, gam("hh", "Gki", true), T1.as("ak"), gam("ph", "Gai", true),
+       w.DGph("Gai"));                                            // :487-488
+    CD(-1.0, gam("hp", "Glc", true), T1.as("al"), gam("pp", "Gac", true),
+       w.DGpp("Gac"));                                            // :509-510
+    CD(1.0, gam("hp", "Gkd"), T1.as("di"), gam("hh", "Gki"), w.DGhh("Gki"));  // :511-512
+    CD(1.0, Vhhhp("klic"), T1.as("cj"), w.Vhhhh("klij"), w.Xklij("klij"));    // :534-535
+    // Q_akij = V_akij + V_akic T_cj (:490-491); complex: V_akic = sum_G
+    // cTGamma_ph[G,a,i] Gamma_hp[G,k,c] (slice phhp) through G; real: V_akic is
+    // V_acik
+    if (cplx)
+      C(1.0, gam("hp", "Gkc"), T1.as("cj"), 0.0, w.Zgoo("Gkj"));
+    else
+      CD(1.0, Vpphh.as("acik"), T1.as("cj"), Vhhhp("jika"), w.Wvooo("akij"));
+  });
+  // B = 2 tau - tau~
+  combine(Bv, w.X.v, 2.0, -1.0, 0.0);
+  E.group([&] {
+    CD(2.0, gam("pp", "Gac", true), w.wG("G"), w.Kac("ac"), w.Lac("ac"));  // :468-469
+    CD(2.0, Vhhhp("klic"), T1.as("cl"), w.Kki("ki"), w.Lki("ki"));  // :476-477
+    if (cplx)
+      CD(1.0, gam("ph", "Gai", true), w.Zgoo("Gkj"), w.Vphhh("akij"), w.Wvooo("akij"));
+    C(1.0, Vhhhp("lkjc"), T1.as("ci"), 1.0, w.Xklij("klij"));     // :536
+    C(1.0, w.Kac("ac"), T1.as("ci"), 0.0, R1);                    // :609
+  });
+  E.group([&] {
+    C(-1.0, w.Zgvo("Gak"), gam("hp", "Gkc"), 1.0, w.Lac("ac"));   // :470
+    C(-1.0, Vhhhp("lkic"), T1.as("cl"), 1.0, w.Lki("ki"));        // :478
+    if (merged) C(1.0, Vhhpp("klcd"), A("cdij"), 1.0, w.Xklij("klij"));  // :541
+    // :620, V_akic T_ck = sum_G cTGamma_ph[G,a,i] (sum_kc Gamma_hp[G,k,c] T_ck)
+    C(2.0, gam("ph", "Gai", true), w.wG("G"), 1.0, R1);
+  });
+  E.group([&] {
+    C(1.0, w.Lac("ac"), T2.as("cbij"), 0.0, R2);                  // :481
+    C(-1.0, Vhhhp("klic"), B("ackl"), 1.0, R1);                   // :627-628
+  });
+  E.group([&] {
+    C(-1.0, w.Lki("ki"), T2.as("abkj"), 1.0, R2);                 // :484
+    C(1.0, w.Kck("ck"), T1.as("ci"), -1.0, w.Kki("ki"));          // :610, :619
+  });
+  E.group([&] {
+    C(1.0, w.DGph("Gai"), w.Wgvo("Gbj"), 1.0, R2);                // :489
+    C(1.0, w.Kki("ki"), T1.as("ak"), 1.0, R1);                    // :610, :619
+  });
+  E.group([&] {
+    // half of the hole ladder: R2 is symmetrised below.  Over tau: :542-546
+    // without ppl, or with the dressing T_ak T_bl V_klcd tau_cdij of the resident
+    // ladder
+    if (merged) C(0.5, w.Xklij("klij"), A("abkl"), 1.0, R2);      // :538
+    // :621-625, all of the form cTGamma_pp[G,a,c] W[G,c,i]
+    C(-1.0, gam("hh", "Gki"), T1.as("ck"), 0.0, w.Wgvo("Gci"));
+  });
+  // half of the resident ladder and, with U_kaji in Q_akij, the T1 dressing of
+  // its left or right vertex
   if (resident)
     resident_unpack(f, w.Rp.buf.get(), w.Rm.buf.get(), R2.ptr, w.Wvooo.buf.get(), 0.5, v, o, st);
-  C(-1.0, w.Wvooo("akij"), T1.as("bk"), 1.0, R2);
+  E.group([&] {
+    C(-1.0, w.Wvooo("akij"), T1.as("bk"), 1.0, R2);               // :490-491
+    C(1.0, gam("hp", "Gkd"), B("cdik"), 1.0, w.Wgvo("Gci"));      // :622-625
+  });
   // A = T2 + 2 T1 T1
   tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 2.0, o, v);         // :462-463
   E.sum(1.0, w.Zgvo("Gai"), 1.0, w.DGph("Gai"));                // :494
-  C(-0.5, gam("hp", "Gld", true), A("dail"), 1.0, w.DGph("Gai"));   // :495
-  // crossed ring, its intermediate Xakci stored as [a,k,i,c]; A = Z
-  CD(-1.0, gam("hp", "Glc", true), T1.as("al"), gam("pp", "Gac", true),
-     w.DGpp("Gac"));                                            // :509-510
-  CD(1.0, gam("hp", "Gkd"), T1.as("di"), gam("hh", "Gki"), w.DGhh("Gki"));  // :511-512
-  C(1.0, w.DGpp("Gac"), w.DGhh("Gki"), 0.0, X("akic"));         // :514
+  // the crossed ring's intermediate Xakci, stored as [a,k,i,c], takes B's place
+  E.group([&] {
+    C(-0.5, gam("hp", "Gld", true), A("dail"), 1.0, w.DGph("Gai"));   // :495
+    C(1.0, w.DGpp("Gac"), w.DGhh("Gki"), 0.0, X("akic"));         // :514
+    C(1.0, gam("pp", "Gac", true), w.Wgvo("Gci"), 1.0, R1);       // :621-625
+  });
   C(-0.5, Vhhpp("lkcd"), T2.as("dail"), 1.0, X("akic"));        // :515
-  C(1.0, X("bkic"), T2.as("ackj"), 0.0, A("abij"));             // :517
+  C(1.0, X("bkic"), T2.as("ackj"), 0.0, A("abij"));             // :517, A = Z
   combine(R2, w.X.v, -1.0, -0.5, 1.0);
   // ring over Xakic - 1/2 Xakci; A = Wt, then 2 T - T~
   C(1.0, w.DGph("Gai"), gam("hp", "Gkc"), -0.5, X("akic"));     // :496
   combine(w.X.v, Vpphh, 1.0, -0.5, 0.0, cplx);                  // :497-498
   C(1.0, A("dclk"), T2.as("adil"), 1.0, X("akic"));             // :499
   combine(w.X.v, T2, 2.0, -1.0, 0.0);                           // :500-501
-  C(1.0, X("akic"), A("cbkj"), 1.0, R2);                        // :502, :516
-  C(1.0, w.Kck("ck"), A("caki"), 0.0, R1);                      // :617-618
+  E.group([&] {
+    C(1.0, X("akic"), A("cbkj"), 1.0, R2);                        // :502, :516
+    C(1.0, w.Kck("ck"), A("caki"), 1.0, R1);                      // :617-618
+  });
   symmetrize_pairs(st, f, R2.ptr, o, v, Vpphh.ptr);             // :520, 529
-  // hole ladder; A = tau
-  tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 1.0, o, v);
-  CD(1.0, Vhhhp("klic"), T1.as("cj"), w.Vhhhh("klij"), w.Xklij("klij"));  // :534-535
-  C(1.0, Vhhhp("lkjc"), T1.as("ci"), 1.0, w.Xklij("klij"));     // :536
-  if (opt_.ppl && !resident) {
+  if (!merged) {
+    tau(st, f, w.X.buf.get(), T2.ptr, T1.ptr, 1.0, o, v);
     C(1.0, w.Xklij("klij"), A("abkl"), 1.0, R2);                // :538
     C(1.0, Vhhpp("klcd"), A("cdij"), 0.0, w.Xklij("klij"));     // :541
     C(1.0, w.Xklij("klij"), T2.as("abkl"), 1.0, R2);            // :542-546
     // with Gamma_qp = conj Gamma_pq, Gamma_pp[G,a,b] - Gamma_hp[G,k,b] T_ak
     // (:560-561) equals cTDGamma_pp[G,a,b] of :509-510 term by term
     ladder(w.DGpp.v, w.DGpp.v, w.X.v, R2);                      // :564-600
-  } else {
-    // over tau: :542-546 without ppl, or with the dressing T_ak T_bl V_klcd tau_cdij
-    // of the resident ladder
-    C(1.0, Vhhpp("klcd"), A("cdij"), 1.0, w.Xklij("klij"));     // :541
-    C(1.0, w.Xklij("klij"), A("abkl"), 1.0, R2);                // :538, :542-546
   }
-  // singles; B = 2 tau - tau~
-  combine(Bv, w.X.v, 2.0, -1.0, 0.0);
-  C(1.0, w.Kac("ac"), T1.as("ci"), 1.0, R1);                    // :609
-  C(1.0, w.Kck("ck"), T1.as("ci"), -1.0, w.Kki("ki"));          // :610, :619
-  C(1.0, w.Kki("ki"), T1.as("ak"), 1.0, R1);
-  // :620, V_akic T_ck = sum_G cTGamma_ph[G,a,i] (sum_kc Gamma_hp[G,k,c] T_ck)
-  C(2.0, gam("ph", "Gai", true), w.wG("G"), 1.0, R1);
-  // :621-625, all of the form cTGamma_pp[G,a,c] W[G,c,i]
-  C(-1.0, gam("hh", "Gki"), T1.as("ck"), 0.0, w.Wgvo("Gci"));
-  C(1.0, gam("hp", "Gkd"), B("cdik"), 1.0, w.Wgvo("Gci"));
-  C(1.0, gam("pp", "Gac", true), w.Wgvo("Gci"), 1.0, R1);
-  C(-1.0, Vhhhp("klic"), B("ackl"), 1.0, R1);                   // :627-628
 }
 
 void Ccsd::residuum_complex(const void *Tp, void *Rp) {

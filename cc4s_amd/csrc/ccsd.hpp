@@ -81,7 +81,8 @@ class Ccsd {
   void residuum_drccd(const void *T, void *R);
   void form_slice(Tensor &V, const char *name);
   bool resident_integrals();
-  void resident_products(const View &tauv);
+  void resident_combinations(const View &tauv);
+  void resident_products();
   void ladder(const View &left, const View &right, const View &tauv,
               const View &R2);
   View gam(const char *part, const std::string &names, bool conjT = false) const;

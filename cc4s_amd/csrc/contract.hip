@@ -31,6 +31,15 @@ struct KArgs {
   double alpha, beta;
   double signA, signB;  // -1 conjugates the operand's imaginary part
   int tilesM, tilesN;
+  // tiles [0, fullTiles) run over all of K; the others, the last partial wave of
+  // workgroups, are cut into tailSplits parts of tailChunk k each, whose sums go
+  // to Wt [part][tile][BM][BN] (fullTiles is the tile count where nothing is cut)
+  double *Wt;
+  int fullTiles, tailTiles, tailSplits;
+  int64_t tailChunk;
+};
+
+struct KArgs2 : KArgs {
   // second K segment (SEG2 kernels): k in [K1p, K1p + K2) reads
   // A2[rowA2[m] + colA2[k - K1p]] and B2[rowB2[k - K1p] + colB2[n]], times
   // f2, with its own conjugation signs; the first segment is k < K1 (K1p is
@@ -39,12 +48,6 @@ struct KArgs {
   const int64_t *rowA2, *colA2, *rowB2, *colB2;
   int64_t K1, K1p, K2;
   double f2, signA2, signB2;
-  // tiles [0, fullTiles) run over all of K; the others, the last partial wave of
-  // workgroups, are cut into tailSplits parts of tailChunk k each, whose sums go
-  // to Wt [part][tile][BM][BN] (fullTiles is the tile count where nothing is cut)
-  double *Wt;
-  int fullTiles, tailTiles, tailSplits;
-  int64_t tailChunk;
 };
 
 // C[oc] = alpha x + beta D[od]
@@ -352,10 +355,24 @@ constexpr int kZThreads = 512;
 // SEG2 adds a second K segment with its own operands (two contractions with
 // the same result index partition, e.g. a particle and a hole term of (T),
 // accumulated in one pass over C); a K-stage lies in one segment.
+template <bool CPLX>
+using Scalar = std::conditional_t<CPLX, double2, double>;
+// elements past the end of an LDS row.  Complex: one shifts consecutive k-rows by
+// one 16-byte bank group, so the column-wise stores of K-contiguous operands and
+// the row-wise 128-bit operand reads are both conflict-free per 16-lane pass.
+// Real: a shift of 18 8-byte banks (of 32) spreads the 16 k-rows of a column-wise
+// store over all even banks and leaves two of 32 lanes of a row-wise read in
+// conflict.
+template <bool CPLX>
+constexpr int kRowPad = CPLX ? 1 : 18;
+
+// one workgroup: block `block` of the tiles (and tail parts), part `slice` of K
 template <bool CPLX, int NT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC,
-          bool M3, bool DEEP, int MINW = 1, bool SEG2 = false>
-__global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
-  using T = std::conditional_t<CPLX, double2, double>;
+          bool M3, bool DEEP, bool SEG2>
+__device__ __forceinline__ void gett_tile(
+    const std::conditional_t<SEG2, KArgs2, KArgs> &p, int block, int slice,
+    Scalar<CPLX> (&As)[2][BK][BM + kRowPad<CPLX>], Scalar<CPLX> (&Bs)[2][BK][BN + kRowPad<CPLX>]) {
+  using T = Scalar<CPLX>;
   static_assert(CPLX || (!M3 && !SEG2), "complex forms");
   constexpr int MB = WM / 16, NB = WN / 16;
   constexpr int WAVES_N = BN / WN;
@@ -370,21 +387,9 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
   constexpr int NRA = AKC ? EA : 1;
   constexpr int NKB = BKC ? 1 : EB;
   constexpr int NRB = BKC ? EB : 1;
-  // elements per LDS row.  Complex: BM+1 shifts consecutive k-rows by one
-  // 16-byte bank group, so the column-wise stores of K-contiguous operands
-  // and the row-wise 128-bit operand reads are both conflict-free per
-  // 16-lane pass.  Real: a shift of 18 8-byte banks (of 32) spreads the 16
-  // k-rows of a column-wise store over all even banks and leaves two of 32
-  // lanes of a row-wise read in conflict.
-  constexpr int PAD = CPLX ? 1 : 18;
-  constexpr int LDA = BM + PAD, LDB = BN + PAD;
-
-  __shared__ T As[2][BK][LDA];
-  __shared__ T Bs[2][BK][LDB];
-
   const int t = threadIdx.x;
-  int g = blockIdx.x;
-  int64_t kbeg = static_cast<int64_t>(blockIdx.y) * p.kChunk, klen = p.kChunk;
+  int g = block;
+  int64_t kbeg = static_cast<int64_t>(slice) * p.kChunk, klen = p.kChunk;
   const bool tail = g >= p.fullTiles;
   int part = 0;  // (cut, tile) of a tail workgroup
   if (tail) {
@@ -497,7 +502,8 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
   // factor) applied, elements past K zeroed
   auto store_part = [&](int s, int buf, auto set_c, int part) {
     constexpr int q = decltype(set_c)::value;
-    const bool seg2 = SEG2 && kbeg + static_cast<int64_t>(s) * BK >= p.K1p;
+    bool seg2 = false;
+    if constexpr (SEG2) seg2 = kbeg + static_cast<int64_t>(s) * BK >= p.K1p;
     if (part == 0) {
       int64_t left = p.K - kbeg - static_cast<int64_t>(s) * BK;  // k of this stage within K
       if constexpr (SEG2) left = seg2 ? left : p.K1 - kbeg - static_cast<int64_t>(s) * BK;
@@ -736,11 +742,66 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
           x = make_double2(accR[i][j][r], accI[i][j][r]);
         }
         if (p.W)
-          reinterpret_cast<T *>(p.W)[(static_cast<int64_t>(blockIdx.y) * p.M + m) * p.N + n] = x;
+          reinterpret_cast<T *>(p.W)[(static_cast<int64_t>(slice) * p.M + m) * p.N + n] = x;
         else
           store_result(p, x, rc + cCol[j], rd + dCol[j]);
       }
     }
+  }
+}
+
+template <bool CPLX, int NT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC,
+          bool M3, bool DEEP, int MINW = 1, bool SEG2 = false>
+__global__ __launch_bounds__(NT, MINW) void zgett_kernel(
+    std::conditional_t<SEG2, KArgs2, KArgs> p) {
+  __shared__ Scalar<CPLX> As[2][BK][BM + kRowPad<CPLX>];
+  __shared__ Scalar<CPLX> Bs[2][BK][BN + kRowPad<CPLX>];
+  gett_tile<CPLX, NT, BM, BN, BK, WM, WN, AKC, BKC, M3, DEEP, SEG2>(p, blockIdx.x, blockIdx.y, As,
+                                                                   Bs);
+}
+
+// Several independent contractions with small results in one launch: blocks
+// first[i] ... of the grid are contraction i's tiles times its K splits.  Alone,
+// each is bound by latency (4 to 6 us for a launch, one stage's loads and the
+// stores), which the group pays once.  Always the 32x32 tile: four waves, 34 KB of
+// LDS, so four blocks of different contractions share a CU.  Measured, one
+// iteration, launched one by one -> grouped: complex No=4 Nv=16 455 -> 337 us,
+// No=12 Nv=60 1.82 -> 1.62 ms; eleven real ones, No=8 Nv=40, 10.6 -> 8.7 ms.
+constexpr int kGroup = 16;
+struct GroupArgs {
+  KArgs k[kGroup];
+  int first[kGroup + 1];
+  int orient[kGroup];  // 2 a_kcontig + b_kcontig
+  int count;
+};
+static_assert(sizeof(GroupArgs) <= 4096, "kernel arguments");
+
+__device__ __forceinline__ int group_item(const GroupArgs &g) {
+  int i = 0;
+  while (i + 1 < g.count && static_cast<int>(blockIdx.x) >= g.first[i + 1]) ++i;
+  return i;
+}
+
+template <bool CPLX>
+__global__ __launch_bounds__(256, 4) void gett_group_kernel(GroupArgs g) {
+  __shared__ Scalar<CPLX> As[2][16][32 + kRowPad<CPLX>];
+  __shared__ Scalar<CPLX> Bs[2][16][32 + kRowPad<CPLX>];
+  const int i = group_item(g);
+  const KArgs &p = g.k[i];
+  const int b = static_cast<int>(blockIdx.x) - g.first[i], tiles = p.tilesM * p.tilesN;
+  const int slice = b / tiles, block = b - slice * tiles;
+  switch (g.orient[i]) {
+    case 0:
+      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, false, false, CPLX, false, false>(p, block, slice, As, Bs);
+      break;
+    case 1:
+      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, false, true, CPLX, false, false>(p, block, slice, As, Bs);
+      break;
+    case 2:
+      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, true, false, CPLX, false, false>(p, block, slice, As, Bs);
+      break;
+    default:
+      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, true, true, CPLX, false, false>(p, block, slice, As, Bs);
   }
 }
 
@@ -750,14 +811,15 @@ __global__ __launch_bounds__(NT, MINW) void zgett_kernel(KArgs p) {
 // of splits, four loads in flight per thread; the group sums are added in LDS.
 // Both orders are fixed, so the result is reproducible.
 template <bool CPLX, int G>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(KArgs p, int splits) {
+__device__ __forceinline__ void splitk_reduce(const KArgs &p, int splits, uint32_t block,
+                                              uint32_t blocks) {
   const uint32_t total = static_cast<uint32_t>(p.M * p.N), N = static_cast<uint32_t>(p.N);
   using T = std::conditional_t<CPLX, double2, double>;
   constexpr uint32_t E = 256 / G;
   __shared__ T part[G][E];
   const uint32_t u = threadIdx.x % E, g = threadIdx.x / E;
   const T *w = reinterpret_cast<const T *>(p.W);
-  for (uint32_t e0 = blockIdx.x * E; e0 < total; e0 += gridDim.x * E) {
+  for (uint32_t e0 = block * E; e0 < total; e0 += blocks * E) {
     const uint32_t e = e0 + u;
     const uint32_t ec = e < total ? e : total - 1;
     T acc[4] = {};
@@ -790,6 +852,18 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(KArgs p, int splits)
     }
     if constexpr (G > 1) __syncthreads();  // part is written again
   }
+}
+
+template <bool CPLX, int G>
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(KArgs p, int splits) {
+  splitk_reduce<CPLX, G>(p, splits, blockIdx.x, gridDim.x);
+}
+
+// the reductions of a group's split contractions, 64 elements per block
+template <bool CPLX>
+__global__ __launch_bounds__(256) void group_reduce_kernel(GroupArgs g) {
+  const int i = group_item(g);
+  splitk_reduce<CPLX, 4>(g.k[i], g.orient[i], blockIdx.x - g.first[i], g.first[i + 1] - g.first[i]);
 }
 
 // Results of the tail tiles from their parts, in order.  One block takes 256
@@ -880,7 +954,8 @@ void dispatch_gett(const GettLaunch &L, const KArgs &args, dim3 grid, hipStream_
 
 template <bool CPLX, int NT, int BM, int BN, int BK, int WM, int WN, bool M3,
           bool DEEP = false, int MINW = 1, bool SEG2 = false>
-void dispatch_zgett(const GettLaunch &L, const KArgs &args, dim3 grid, hipStream_t s) {
+void dispatch_zgett(const GettLaunch &L, const std::conditional_t<SEG2, KArgs2, KArgs> &args,
+                    dim3 grid, hipStream_t s) {
   if (L.a_kcontig && L.b_kcontig)
     zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, true, true, M3, DEEP, MINW, SEG2>
         <<<grid, NT, 0, s>>>(args);
@@ -953,18 +1028,12 @@ std::string gett_variant(const GettLaunch &L) {
 
 namespace {
 void reduce_partials(bool cplx, const KArgs &a, int splits, hipStream_t s);
-}
 
-void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
-                 hipEvent_t stop) {
+KArgs2 kernel_args(const GettLaunch &L) {
   const bool cplx = L.field == Field::Complex;
-  const bool seg2 = L.A2 != nullptr;
-  CC4S_ASSERT(!seg2 || (cplx && g_complex_generation == 3),
-              "two-segment contractions need the complex generation-3 kernel");
-  const Tile tile = static_cast<Tile>(L.tile);
-  const TileShape shape = tile_shape(L.field, tile);
+  const TileShape shape = tile_shape(L.field, static_cast<Tile>(L.tile));
   const int BM = shape.BM, BN = shape.BN, BK = kZ3BK;
-  KArgs a;
+  KArgs2 a{};
   a.A = static_cast<const double *>(L.A);
   a.B = static_cast<const double *>(L.B);
   a.C = static_cast<double *>(L.C);
@@ -1002,6 +1071,20 @@ void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
   a.tailChunk = L.tail_splits > 1 ? (kstages + L.tail_splits - 1) / L.tail_splits * BK : 0;
   CC4S_ASSERT(L.tail_splits <= 1 || (L.splits == 1 && L.W && a.fullTiles > 0 && a.tailTiles > 0),
               "tail split without its workspace");
+  return a;
+}
+}  // namespace
+
+void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
+                 hipEvent_t stop) {
+  const bool cplx = L.field == Field::Complex;
+  const bool seg2 = L.A2 != nullptr;
+  CC4S_ASSERT(!seg2 || (cplx && g_complex_generation == 3),
+              "two-segment contractions need the complex generation-3 kernel");
+  const Tile tile = static_cast<Tile>(L.tile);
+  const TileShape shape = tile_shape(L.field, tile);
+  const int BM = shape.BM, BN = shape.BN;
+  const KArgs2 a = kernel_args(L);
   dim3 grid(a.fullTiles + a.tailTiles * std::max(1, L.tail_splits), L.splits);
   if (start) CC4S_HIP(hipEventRecord(start, s));
   if (cplx && g_complex_generation == 3) {
@@ -1584,7 +1667,6 @@ void ContractionEngine::contract(double alpha, const View &A, const View &B,
   L.tail_splits = P.tail_splits;
   L.alpha = alpha; L.beta = beta;
   L.a_kcontig = P.a_kc; L.b_kcontig = P.b_kc;
-  L.W = reserve_partials(P, C.field);
   const double flops = (C.field == Field::Complex ? 8.0 : 2.0) * double(P.M) *
                        double(P.N) * double(P.K);
   if (mixed_ && C.field == Field::Complex && flops >= mixed_min_flops) {
@@ -1593,6 +1675,16 @@ void ContractionEngine::contract(double alpha, const View &A, const View &B,
     stats.launches += 1;
     return;
   }
+  // a small contraction of a group waits for its end
+  if (grouping_ && !profiling_ && P.tile == Tile::Small && P.tail_splits == 1 &&
+      P.M * P.N * P.splits < kGroupElements &&
+      (C.field == Field::Real || g_complex_generation == 3)) {
+    group_.push_back(L);
+    stats.flops += flops;
+    stats.launches += 1;
+    return;
+  }
+  L.W = reserve_partials(P, C.field);
   if (profiling_) {
     Pending p{take_event(), take_event(), gett_variant(L), flops};
     launch_gett(L, stream_, p.start, p.stop);
@@ -1603,6 +1695,56 @@ void ContractionEngine::contract(double alpha, const View &A, const View &B,
   }
   stats.flops += flops;
   stats.launches += 1;
+}
+
+void ContractionEngine::launch_group() {
+  std::vector<GettLaunch> all;
+  all.swap(group_);
+  for (size_t first = 0; first < all.size(); first += kGroup) {
+    const size_t n = std::min<size_t>(kGroup, all.size() - first);
+    size_t bytes = 0;
+    for (size_t i = 0; i < n; ++i)
+      if (all[first + i].splits > 1)
+        bytes += static_cast<size_t>(all[first + i].splits) * all[first + i].M *
+                 all[first + i].N * scalar_bytes(all[first + i].field);
+    workspace_.reserve(bytes);
+    const bool cplx = all[first].field == Field::Complex;
+    GroupArgs g{}, r{};
+    size_t used = 0;
+    for (size_t i = 0; i < n; ++i) {
+      GettLaunch &L = all[first + i];
+      if (L.splits > 1) {
+        L.W = workspace_.as<char>() + used;
+        used += static_cast<size_t>(L.splits) * L.M * L.N * scalar_bytes(L.field);
+      }
+      const KArgs a = kernel_args(L);
+      g.k[i] = a;
+      g.orient[i] = 2 * (L.a_kcontig ? 1 : 0) + (L.b_kcontig ? 1 : 0);
+      g.first[i + 1] = g.first[i] + a.tilesM * a.tilesN * L.splits;
+      if (L.splits > 1) {
+        r.k[r.count] = a;
+        r.orient[r.count] = L.splits;
+        r.first[r.count + 1] = r.first[r.count] + static_cast<int>((L.M * L.N + 63) / 64);
+        ++r.count;
+      }
+    }
+    g.count = static_cast<int>(n);
+    if (n == 1 && !r.count) {
+      launch_gett(all[first], stream_);
+      continue;
+    }
+    if (cplx)
+      gett_group_kernel<true><<<g.first[n], 256, 0, stream_>>>(g);
+    else
+      gett_group_kernel<false><<<g.first[n], 256, 0, stream_>>>(g);
+    CC4S_HIP(hipGetLastError());
+    if (!r.count) continue;
+    if (cplx)
+      group_reduce_kernel<true><<<r.first[r.count], 256, 0, stream_>>>(r);
+    else
+      group_reduce_kernel<false><<<r.first[r.count], 256, 0, stream_>>>(r);
+    CC4S_HIP(hipGetLastError());
+  }
 }
 
 void ContractionEngine::contract_mixed(GettPlan &P, double alpha, const View &A,

@@ -35,6 +35,34 @@ struct KernelTiming {
   double ms = 0, flops = 0;
 };
 
+// kernel-level entry used by the planner and by tests of the kernel itself
+struct GettLaunch {
+  Field field;
+  const void *A, *B;
+  void *C;
+  void *W;  // split-K partials, splits * M * N elements (tail_splits > 1: parts of whole tiles), or null
+  const int64_t *rowA, *colA, *rowB, *colB, *rowC, *colC;
+  int64_t M, N, K;
+  int splits;
+  int64_t full_tiles = 0;  // tiles of whole waves where the others are cut along K
+  int tail_splits = 1;     // parts of each of those others (> 1: partials in W)
+  int tile;  // 0 large, 1 medium (64 x 64), 2 small (32 x 32) workgroup tile
+  double alpha, beta;
+  bool conjA, conjB;
+  bool a_kcontig, b_kcontig;
+  // optional second K segment (complex generation-3 kernel): k in
+  // [K1p, K1p + K2) from A2, B2 and their tables, times f2; K = K1p + K2,
+  // K1p = K1 rounded up to whole K-stages (16)
+  const void *A2 = nullptr, *B2 = nullptr;
+  const int64_t *rowA2 = nullptr, *colA2 = nullptr, *rowB2 = nullptr, *colB2 = nullptr;
+  int64_t K1 = 0, K1p = 0, K2 = 0;
+  double f2 = 1.0;
+  bool conjA2 = false, conjB2 = false;
+  // tensor added with beta (null: C)
+  const void *D = nullptr;
+  const int64_t *rowD = nullptr, *colD = nullptr;
+  bool conjD = false;
+};
 class ContractionEngine {
  public:
   explicit ContractionEngine(hipStream_t s);
@@ -45,6 +73,22 @@ class ContractionEngine {
   // copy into C it saves)
   void contract(double alpha, const View &A, const View &B, double beta,
                 const View &C, const View *D = nullptr);
+  // `statements` contracts in any order: those contractions with small results
+  // run in one launch (and one for their split-K reductions) after the others
+  template <class Statements>
+  void group(Statements &&statements) {
+    group_.clear();
+    grouping_ = true;
+    try {
+      statements();
+    } catch (...) {
+      grouping_ = false;
+      group_.clear();
+      throw;
+    }
+    grouping_ = false;
+    launch_group();
+  }
   // C = alpha * op(A1) op(B1) + alpha2 * op(A2) op(B2) + beta * C for two
   // contractions whose operands split C's indices the same way: one launch
   // with the second contraction as a second K segment, so C is read and
@@ -118,6 +162,12 @@ class ContractionEngine {
   GettPlan &plan_for(const View &A, const View &B, const View &C, const View *D = nullptr);
   GettPlan &plan_for2(const View &A1, const View &B1, const View &A2, const View &B2,
                       const View &C);
+  void launch_group();
+  bool grouping_ = false;
+  std::vector<GettLaunch> group_;
+  // result elements times splits up to which a contraction joins a group: larger
+  // ones fill the chip by themselves
+  static constexpr int64_t kGroupElements = int64_t(1) << 20;
   void *reserve_partials(const GettPlan &P, Field f);
   void contract_mixed(GettPlan &P, double alpha, const View &A, const View &B,
                       double beta, const View &C, double flops);
@@ -145,34 +195,6 @@ class ContractionEngine {
   DeviceBuffer workspace_;
 };
 
-// kernel-level entry used by the planner and by tests of the kernel itself
-struct GettLaunch {
-  Field field;
-  const void *A, *B;
-  void *C;
-  void *W;  // split-K partials, splits * M * N elements (tail_splits > 1: parts of whole tiles), or null
-  const int64_t *rowA, *colA, *rowB, *colB, *rowC, *colC;
-  int64_t M, N, K;
-  int splits;
-  int64_t full_tiles = 0;  // tiles of whole waves where the others are cut along K
-  int tail_splits = 1;     // parts of each of those others (> 1: partials in W)
-  int tile;  // 0 large, 1 medium (64 x 64), 2 small (32 x 32) workgroup tile
-  double alpha, beta;
-  bool conjA, conjB;
-  bool a_kcontig, b_kcontig;
-  // optional second K segment (complex generation-3 kernel): k in
-  // [K1p, K1p + K2) from A2, B2 and their tables, times f2; K = K1p + K2,
-  // K1p = K1 rounded up to whole K-stages (16)
-  const void *A2 = nullptr, *B2 = nullptr;
-  const int64_t *rowA2 = nullptr, *colA2 = nullptr, *rowB2 = nullptr, *colB2 = nullptr;
-  int64_t K1 = 0, K1p = 0, K2 = 0;
-  double f2 = 1.0;
-  bool conjA2 = false, conjB2 = false;
-  // tensor added with beta (null: C)
-  const void *D = nullptr;
-  const int64_t *rowD = nullptr, *colD = nullptr;
-  bool conjD = false;
-};
 // `start`/`stop` (optional) bracket the main kernel, not the reduction
 void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start = nullptr,
                  hipEvent_t stop = nullptr);
