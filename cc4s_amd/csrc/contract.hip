@@ -1174,7 +1174,6 @@ struct GettPlan {
   int splits = 1, tail_splits = 1;
   int64_t full_tiles = 0;
   Tile tile = Tile::Large;
-  DeviceBuffer tables;
   const int64_t *rowA, *colA, *rowB, *colB, *rowC, *colC;
   const int64_t *rowD = nullptr, *colD = nullptr;  // of an added tensor other than C
   // two-segment plans: the second contraction's tables; swap2 tells that
@@ -1278,27 +1277,61 @@ std::string plan_key(const View &A, const View &B, const View &C) {
 // K offset tables are padded with their first entry, a valid offset, to whole
 // K-stages and past them: a kernel reads its table up to four stages ahead
 constexpr int64_t kTablePad = 5 * kZ3BK;
-void pad_k(std::vector<int64_t> &v) {
-  if (v.empty()) return;
-  v.resize((v.size() + kZ3BK - 1) / kZ3BK * kZ3BK + kTablePad, v.front());
-}
 
-// offsets of every multi-index of `group` (first listed index fastest)
-std::vector<int64_t> offsets(const View &v, const std::string &group,
-                             const View &shape) {
-  int64_t n = 1;
-  for (char c : group) n *= shape.len(c);
-  std::vector<int64_t> out(static_cast<size_t>(n), 0);
-  int64_t block = 1;
-  for (char c : group) {
-    const int64_t L = shape.len(c), s = v.stride(c);
-    for (int64_t e = 0; e < n; ++e) out[e] += ((e / block) % L) * s;
-    block *= L;
+// Offset tables of a plan, built where they are read: table t holds the offset of
+// every multi-index of its modes (first mode fastest), entries n[t] ... of a padded
+// one its first offset, which is 0.  One launch instead of an allocation, a host
+// loop over every entry and a blocking copy (25 to 40 us a plan, about 50 plans in
+// a residuum's first pass): that pass took 1378 -> 675 us (complex No=4 Nv=16) and
+// 6.7 -> 3.2 ms (No=12 Nv=60).
+constexpr int kTables = 8, kTableModes = 8;
+struct TableArgs {
+  int64_t *out;
+  int64_t first[kTables + 1];  // table t at out + first[t], padded length by difference
+  int64_t n[kTables], block[kTables];  // entries; entries per step of the first mode here
+  int64_t len[kTables][kTableModes], stride[kTables][kTableModes];
+  int modes[kTables];
+  int count;
+  bool add;  // modes beyond the first kTableModes are added in further launches
+};
+
+__global__ __launch_bounds__(256) void offsets_kernel(TableArgs p) {
+  for (int64_t e = blockIdx.x * int64_t(256) + threadIdx.x; e < p.first[p.count];
+       e += gridDim.x * int64_t(256)) {
+    int t = 0;
+    while (e >= p.first[t + 1]) ++t;
+    const int64_t i = e - p.first[t];
+    int64_t off = 0;
+    if (i < p.n[t]) {
+      int64_t rest = i / p.block[t];
+      for (int m = 0; m < p.modes[t]; ++m) {
+        const int64_t q = rest / p.len[t][m];
+        off += (rest - q * p.len[t][m]) * p.stride[t][m];
+        rest = q;
+      }
+    }
+    p.out[e] = p.add ? p.out[e] + off : off;
   }
-  return out;
 }
 
 }  // namespace
+
+// a table of `group`'s multi-indices (first listed fastest) with v's strides
+struct OffsetTable {
+  const View *v;
+  std::string group;
+  bool padded;
+  const int64_t **out;
+  int64_t entries() const {
+    int64_t n = 1;
+    for (char c : group) n *= v->len(c);
+    return n;
+  }
+  int64_t size() const {
+    const int64_t n = entries();
+    return padded && n ? (n + kZ3BK - 1) / kZ3BK * kZ3BK + kTablePad : n;
+  }
+};
 
 namespace {
 
@@ -1382,6 +1415,48 @@ void choose_tile(Field f, int64_t M, int64_t N, int64_t K, size_t max_workspace,
 
 }  // namespace
 
+// the tables' entries go to the arena; `stream_` builds them and reads them
+void ContractionEngine::build_tables(const OffsetTable *tables, int count) {
+  CC4S_ASSERT(count <= kTables, "too many offset tables");
+  TableArgs a{};
+  a.count = count;
+  size_t rounds = 1;
+  for (int t = 0; t < count; ++t) {
+    a.first[t + 1] = a.first[t] + tables[t].size();
+    a.n[t] = tables[t].entries();
+    a.block[t] = 1;
+    rounds = std::max(rounds, (tables[t].group.size() + kTableModes - 1) / kTableModes);
+  }
+  const int64_t total = a.first[count];
+  const size_t bytes = (static_cast<size_t>(total) * sizeof(int64_t) + 255) / 256 * 256;
+  if (arena_.empty() || arena_used_ + bytes > arena_.back().bytes()) {
+    DeviceBuffer chunk;
+    chunk.allocate(std::max(bytes, kArenaChunk));
+    arena_.push_back(std::move(chunk));
+    arena_used_ = 0;
+  }
+  a.out = reinterpret_cast<int64_t *>(arena_.back().as<char>() + arena_used_);
+  arena_used_ += bytes;
+  for (int t = 0; t < count; ++t) *tables[t].out = a.out + a.first[t];
+  if (total == 0) return;
+  for (size_t r = 0; r < rounds; ++r) {
+    a.add = r > 0;
+    for (int t = 0; t < count; ++t) {
+      const std::string &g = tables[t].group;
+      a.modes[t] = 0;
+      for (size_t m = r * kTableModes; m < std::min(g.size(), (r + 1) * kTableModes); ++m) {
+        a.len[t][a.modes[t]] = std::max<int64_t>(1, tables[t].v->len(g[m]));
+        a.stride[t][a.modes[t]++] = tables[t].v->stride(g[m]);
+      }
+    }
+    const int64_t blocks = std::min<int64_t>((total + 255) / 256, 4096);
+    offsets_kernel<<<static_cast<unsigned>(blocks), 256, 0, stream_>>>(a);
+    CC4S_HIP(hipGetLastError());
+    for (int t = 0; t < count; ++t)
+      for (int m = 0; m < a.modes[t]; ++m) a.block[t] *= a.len[t][m];
+  }
+}
+
 GettPlan &ContractionEngine::plan_for(const View &A0, const View &B0,
                                       const View &C, const View *D) {
   std::string key = plan_key(A0, B0, C);
@@ -1442,42 +1517,20 @@ GettPlan &ContractionEngine::plan_for(const View &A0, const View &B0,
   plan->a_kc = unit(A, Ki) || !unit(A, Mi);
   plan->b_kc = unit(B, Ki) || !unit(B, Ni);
 
-  auto rowA = offsets(A, Mi, C), colA = offsets(A, Ki, A);
-  auto rowB = offsets(B, Ki, A), colB = offsets(B, Ni, C);
-  auto rowC = offsets(C, Mi, C), colC = offsets(C, Ni, C);
-  plan->M = static_cast<int64_t>(rowA.size());
-  plan->N = static_cast<int64_t>(colB.size());
-  plan->K = static_cast<int64_t>(colA.size());
-  if (Ki.empty()) plan->K = 1;  // outer product: one k with offset 0
-
-  pad_k(colA);
-  pad_k(rowB);
-  std::vector<int64_t> all;
-  auto append = [&all](const std::vector<int64_t> &v) {
-    all.insert(all.end(), v.begin(), v.end());
-  };
-  append(rowA); append(colA); append(rowB); append(colB); append(rowC); append(colC);
-  std::vector<int64_t> rowD, colD;
-  if (D) {
-    rowD = offsets(*D, Mi, C);
-    colD = offsets(*D, Ni, C);
-    append(rowD);
-    append(colD);
-  }
-  plan->tables.allocate(all.size() * sizeof(int64_t));
-  CC4S_HIP(hipMemcpy(plan->tables.get(), all.data(), all.size() * sizeof(int64_t),
-                     hipMemcpyHostToDevice));
-  const int64_t *base = plan->tables.as<int64_t>();
-  plan->rowA = base; base += rowA.size();
-  plan->colA = base; base += colA.size();
-  plan->rowB = base; base += rowB.size();
-  plan->colB = base; base += colB.size();
-  plan->rowC = base; base += rowC.size();
-  plan->colC = base; base += colC.size();
-  if (D) {
-    plan->rowD = base; base += rowD.size();
-    plan->colD = base;
-  }
+  const std::vector<OffsetTable> tables = [&] {
+    std::vector<OffsetTable> t = {{&A, Mi, false, &plan->rowA}, {&A, Ki, true, &plan->colA},
+                            {&B, Ki, true, &plan->rowB},  {&B, Ni, false, &plan->colB},
+                            {&C, Mi, false, &plan->rowC}, {&C, Ni, false, &plan->colC}};
+    if (D) {
+      t.push_back({D, Mi, false, &plan->rowD});
+      t.push_back({D, Ni, false, &plan->colD});
+    }
+    return t;
+  }();
+  plan->M = tables[0].entries();
+  plan->N = tables[3].entries();
+  plan->K = tables[1].entries();  // an outer product has one k with offset 0
+  build_tables(tables.data(), static_cast<int>(tables.size()));
 
   choose_tile(C.field, plan->M, plan->N, plan->K, max_workspace, *plan);
 
@@ -1552,30 +1605,15 @@ GettPlan &ContractionEngine::plan_for2(const View &A1, const View &B1, const Vie
   bool a_unit_k = false;
   for (char c : Ki) a_unit_k |= A.stride(c) == 1 && A.len(c) > 1;
   std::stable_sort(Ki.begin(), Ki.end(), a_unit_k ? by(A) : by(B));
-  auto rowA = offsets(A, Mi, C), colA = offsets(A, Ki, A);
-  auto rowB = offsets(B, Ki, A), colB = offsets(B, Ni, C);
-  CC4S_ASSERT(static_cast<int64_t>(rowA.size()) == plan->M &&
-                  static_cast<int64_t>(colB.size()) == plan->N,
-              "the two contractions have different result shapes");
+  const OffsetTable tables[] = {{&A, Mi, false, &plan->rowA2},
+                          {&A, Ki, true, &plan->colA2},
+                          {&B, Ki, true, &plan->rowB2},
+                          {&B, Ni, false, &plan->colB2}};
   plan->K1 = P1.K;
   plan->K1p = (P1.K + kZ3BK - 1) / kZ3BK * kZ3BK;
-  plan->K2 = static_cast<int64_t>(colA.size());
+  plan->K2 = tables[1].entries();
   plan->K = plan->K1p + plan->K2;
-  pad_k(colA);
-  pad_k(rowB);
-  std::vector<int64_t> all;
-  all.insert(all.end(), rowA.begin(), rowA.end());
-  all.insert(all.end(), colA.begin(), colA.end());
-  all.insert(all.end(), rowB.begin(), rowB.end());
-  all.insert(all.end(), colB.begin(), colB.end());
-  plan->tables.allocate(all.size() * sizeof(int64_t));
-  CC4S_HIP(hipMemcpy(plan->tables.get(), all.data(), all.size() * sizeof(int64_t),
-                     hipMemcpyHostToDevice));
-  const int64_t *base = plan->tables.as<int64_t>();
-  plan->rowA2 = base; base += rowA.size();
-  plan->colA2 = base; base += colA.size();
-  plan->rowB2 = base; base += rowB.size();
-  plan->colB2 = base;
+  build_tables(tables, 4);
   plan->rowA = P1.rowA; plan->colA = P1.colA; plan->rowB = P1.rowB; plan->colB = P1.colB;
   plan->rowC = P1.rowC; plan->colC = P1.colC;
   choose_tile(C.field, plan->M, plan->N, plan->K, max_workspace, *plan);

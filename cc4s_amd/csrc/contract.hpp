@@ -63,6 +63,8 @@ struct GettLaunch {
   const int64_t *rowD = nullptr, *colD = nullptr;
   bool conjD = false;
 };
+struct OffsetTable;  // of a plan
+
 class ContractionEngine {
  public:
   explicit ContractionEngine(hipStream_t s);
@@ -192,6 +194,11 @@ class ContractionEngine {
   std::unordered_map<std::string, KernelTiming> timings_;
   hipStream_t stream_;
   std::unordered_map<std::string, std::unique_ptr<GettPlan>> plans_;
+  // the plans' offset tables, kept as long as the plans
+  void build_tables(const OffsetTable *tables, int count);
+  static constexpr size_t kArenaChunk = size_t(2) << 20;
+  std::vector<DeviceBuffer> arena_;
+  size_t arena_used_ = 0;  // of the last chunk
   DeviceBuffer workspace_;
 };
 
