@@ -844,84 +844,47 @@ void Ccsd::residuum_real(const void *Tp, void *Rp) {
 
 namespace cc4s_amd {
 
-namespace {
-
-// `v` with index `c` fixed at `value` (the dimension dropped)
-View fixed(const View &v, char c, int64_t value) {
-  const int d = v.find(c);
-  CC4S_ASSERT(d >= 0 && value >= 0 && value < v.lens[d], "fixed: bad index");
-  View r = v;
-  r.ptr = static_cast<char *>(v.ptr) + value * v.strides[d] * static_cast<int64_t>(scalar_bytes(v.field));
-  r.idx.erase(d, 1);
-  r.lens.erase(r.lens.begin() + d);
-  r.strides.erase(r.strides.begin() + d);
-  return r;
-}
-
-}  // namespace
-
-// (T): for every hole pair (i, j) and chunk of k, the connected amplitudes
-// W_abcijk = sum over the six pair permutations of
-//   T'_{x1x2x3,y1y2y3} = V_{x2 x3 d y3} T_{x1 d y1 y2} - conj(V_{y2 y3 l x3}) T_{x1 x2 y1 l}
-// (PerturbativeTriplesReference.cxx:106-116) are accumulated by twelve
-// contractions into W[a,b,c,k], each reading its operands in place through
-// index-permuted views (no transposes); the energy kernel then adds the
-// disconnected part and the denominator (:118-163).  Only i <= j <= k is
-// formed (the energy kernel adds the other orderings through the symmetry of
-// W), so the particle contractions cost No^3 Nv^4 MACs in total instead of
+// (T) over the hole triples i <= j <= k (the energy kernel adds the other
+// orderings through the symmetry of W), in chunks whose connected amplitudes fit
+// the budget; the particle contractions cost No^3 Nv^4 MACs in total instead of
 // 6 No^3 Nv^4.
 double Ccsd::triples(const void *Tp, const double *eps_h, const double *eps_p) {
   auto &w = *w_;
   auto &E = E_;
   const Field f = s_.field;
-  const bool cplx = f == Field::Complex;
   const int64_t o = s_.No, v = s_.Nv;
   const size_t es = scalar_bytes(f);
   Tensor Vppph;
   form_slice(Vppph, "ppph");                                     // V[b,c,d,k]
-  const View T1 = dense_view(const_cast<void *>(Tp), f, "ai", {v, o});
-  const View T2 = dense_view(offset_ptr(Tp, s_.n1(), f), f, "abij", {v, v, o, o});
-  auto t2 = [&](const char *names) { return T2.as(names); };
-  auto vp = [&](const char *names) { return Vppph.v.as(names); };
-  const View Vh0 = cplx ? w.Vhhhp.v.conjugated() : w.Vhhhp.v;   // conj V_hhhp
-  auto vh = [&](const char *names) { return Vh0.as(names); };
+  const void *T2 = offset_ptr(const_cast<void *>(Tp), s_.n1(), f);
 
-  // bytes of W per hole-triple chunk (CC4S_TRIPLES_W_BYTES overrides)
-  size_t budget = size_t(4) << 30;
-  if (const char *e = std::getenv("CC4S_TRIPLES_W_BYTES")) budget = std::strtoull(e, nullptr, 10);
-  const int64_t per_k = v * v * v * static_cast<int64_t>(es);
-  const int64_t kc = std::max<int64_t>(1, std::min<int64_t>(o, static_cast<int64_t>(budget) / per_k));
-  Tensor Wt(f, "abck", {v, v, v, kc});
+  // Bytes of connected amplitudes per chunk of hole triples
+  // (CC4S_TRIPLES_W_BYTES overrides): a triple's three parts, or their sum, formed
+  // by three launches, where the parts of one triple do not fit.  1 GiB is near
+  // the best (complex No=10, Nv=96: 24.0 ms with 64 MiB, 22.1 with 256, 19.5 with
+  // 1024, 19.0 with 2048).
+  const int64_t per = v * v * v * static_cast<int64_t>(es), all = o * (o + 1) * (o + 2) / 6;
+  int64_t budget = int64_t(1) << 30;
+  size_t free_b = 0, total_b = 0;
+  CC4S_HIP(hipMemGetInfo(&free_b, &total_b));
+  if (3 * per > budget && 3 * per + budget < static_cast<int64_t>(free_b)) budget = 3 * per;
+  if (const char *e = std::getenv("CC4S_TRIPLES_W_BYTES"))
+    budget = static_cast<int64_t>(std::strtoull(e, nullptr, 10));
+  const int parts = budget >= 3 * per ? 3 : 1;
+  const int64_t chunk = triples_chunk(v, all, budget / (per * parts), parts);
+  DeviceBuffer Y(chunk * per * parts);
   DeviceBuffer acc(kTriplesBlocks * sizeof(double));
   CC4S_HIP(hipMemsetAsync(acc.get(), 0, kTriplesBlocks * sizeof(double), E.stream()));
-  for (int64_t i = 0; i < o; ++i) {
-    for (int64_t j = i; j < o; ++j) {
-      for (int64_t k0 = j; k0 < o; k0 += kc) {
-        const int64_t kn = std::min(kc, o - k0);
-        const View W = Wt.v.sliced(3, 0, kn);
-        auto K = [&](const View &x) { return x.sliced(x.find('k'), k0, k0 + kn); };
-        // the six particle terms T'_{abc,ijk}, T'_{bac,jik}, T'_{acb,ikj},
-        // T'_{cba,kji}, T'_{cab,kij}, T'_{bca,jki} (K = d) and the six hole
-        // terms (K = l), each hole term paired with the particle term that
-        // splits W's indices the same way ({a}|{bck}, {b}|{ack}, {ak}|{bc},
-        // {ck}|{ab} twice, {bk}|{ac}): one launch per pair, W read and
-        // written six times instead of twelve
-        E.contract2(1.0, fixed(fixed(t2("adij"), 'i', i), 'j', j), K(vp("bcdk")),
-                    -1.0, K(t2("cbkl")), fixed(fixed(vh("jila"), 'j', j), 'i', i), 0.0, W);
-        E.contract2(1.0, fixed(fixed(t2("bdji"), 'j', j), 'i', i), K(vp("acdk")),
-                    -1.0, K(t2("cakl")), fixed(fixed(vh("ijlb"), 'i', i), 'j', j), 1.0, W);
-        E.contract2(1.0, K(fixed(t2("adik"), 'i', i)), fixed(vp("cbdj"), 'j', j),
-                    -1.0, fixed(t2("bcjl"), 'j', j), K(fixed(vh("kila"), 'i', i)), 1.0, W);
-        E.contract2(1.0, K(fixed(t2("cdkj"), 'j', j)), fixed(vp("badi"), 'i', i),
-                    -1.0, fixed(t2("abil"), 'i', i), K(fixed(vh("jklc"), 'j', j)), 1.0, W);
-        E.contract2(1.0, K(fixed(t2("cdki"), 'i', i)), fixed(vp("abdj"), 'j', j),
-                    -1.0, fixed(t2("bajl"), 'j', j), K(fixed(vh("iklc"), 'i', i)), 1.0, W);
-        E.contract2(1.0, K(fixed(t2("bdjk"), 'j', j)), fixed(vp("cadi"), 'i', i),
-                    -1.0, fixed(t2("acil"), 'i', i), K(fixed(vh("kjlb"), 'j', j)), 1.0, W);
-        triples_energy(E.stream(), f, W.ptr, w.Vpphh.v.ptr, T1.ptr, eps_h, eps_p, o, v, i, j,
-                       k0, kn, acc.as<double>());
-      }
-    }
+  for (int64_t t = 0; t < all; t += chunk) {
+    const int64_t n = std::min(chunk, all - t);
+    for (int part = parts == 3 ? -1 : 0; part < (parts == 3 ? 0 : 3); ++part)
+      triples_product(E.stream(), f, Vppph.buf.get(), T2, w.Vhhhp.buf.get(), Y.get(), o, v, t, n,
+                      part);
+    triples_energy(E.stream(), f, Y.get(), w.Vpphh.v.ptr, offset_ptr(const_cast<void *>(Tp), 0, f),
+                   eps_h, eps_p, o, v, t, n, parts, acc.as<double>());
+    E.stats.flops += (f == Field::Complex ? 8.0 : 2.0) * 6.0 * static_cast<double>(n) * v * v * v *
+                     static_cast<double>(v + o);
+    E.stats.launches += 2;
   }
   std::vector<double> h(kTriplesBlocks);
   CC4S_HIP(hipMemcpyAsync(h.data(), acc.get(), kTriplesBlocks * sizeof(double),

@@ -39,17 +39,6 @@ struct KArgs {
   int64_t tailChunk;
 };
 
-struct KArgs2 : KArgs {
-  // second K segment (SEG2 kernels): k in [K1p, K1p + K2) reads
-  // A2[rowA2[m] + colA2[k - K1p]] and B2[rowB2[k - K1p] + colB2[n]], times
-  // f2, with its own conjugation signs; the first segment is k < K1 (K1p is
-  // K1 rounded up to whole K-stages)
-  const double *A2, *B2;
-  const int64_t *rowA2, *colA2, *rowB2, *colB2;
-  int64_t K1, K1p, K2;
-  double f2, signA2, signB2;
-};
-
 // C[oc] = alpha x + beta D[od]
 __device__ __forceinline__ void store_result(const KArgs &p, double2 x, int64_t oc, int64_t od) {
   double2 out = make_double2(p.alpha * x.x, p.alpha * x.y);
@@ -351,10 +340,6 @@ constexpr int kZThreads = 512;
 // launch bound's minimum of waves per SIMD (2 with 256 threads: two
 // workgroups share a CU, so one's prologue and epilogue overlap the other's
 // multiplies).
-//
-// SEG2 adds a second K segment with its own operands (two contractions with
-// the same result index partition, e.g. a particle and a hole term of (T),
-// accumulated in one pass over C); a K-stage lies in one segment.
 template <bool CPLX>
 using Scalar = std::conditional_t<CPLX, double2, double>;
 // elements past the end of an LDS row.  Complex: one shifts consecutive k-rows by
@@ -368,12 +353,12 @@ constexpr int kRowPad = CPLX ? 1 : 18;
 
 // one workgroup: block `block` of the tiles (and tail parts), part `slice` of K
 template <bool CPLX, int NT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC,
-          bool M3, bool DEEP, bool SEG2>
+          bool M3, bool DEEP>
 __device__ __forceinline__ void gett_tile(
-    const std::conditional_t<SEG2, KArgs2, KArgs> &p, int block, int slice,
+    const KArgs &p, int block, int slice,
     Scalar<CPLX> (&As)[2][BK][BM + kRowPad<CPLX>], Scalar<CPLX> (&Bs)[2][BK][BN + kRowPad<CPLX>]) {
   using T = Scalar<CPLX>;
-  static_assert(CPLX || (!M3 && !SEG2), "complex forms");
+  static_assert(CPLX || !M3, "complex forms");
   constexpr int MB = WM / 16, NB = WN / 16;
   constexpr int WAVES_N = BN / WN;
   static_assert((BM / WM) * (BN / WN) * 64 == NT, "one wave per WM x WN block");
@@ -417,21 +402,17 @@ __device__ __forceinline__ void gett_tile(
 
   // byte addresses of this thread's rows of A and columns of B; one past the
   // edge reads the last row (its products are never stored)
-  const char *aRow[NRA], *aRow2[SEG2 ? NRA : 1];
+  const char *aRow[NRA];
 #pragma unroll
   for (int i = 0; i < NRA; ++i) {
     const int64_t m = min(m0 + a_m(i), p.M - 1);
     aRow[i] = reinterpret_cast<const char *>(p.A) + p.rowA[m] * static_cast<int64_t>(sizeof(T));
-    if constexpr (SEG2)
-      aRow2[i] = reinterpret_cast<const char *>(p.A2) + p.rowA2[m] * static_cast<int64_t>(sizeof(T));
   }
-  const char *bCol[NRB], *bCol2[SEG2 ? NRB : 1];
+  const char *bCol[NRB];
 #pragma unroll
   for (int i = 0; i < NRB; ++i) {
     const int64_t n = min(n0 + b_n(i), p.N - 1);
     bCol[i] = reinterpret_cast<const char *>(p.B) + p.colB[n] * static_cast<int64_t>(sizeof(T));
-    if constexpr (SEG2)
-      bCol2[i] = reinterpret_cast<const char *>(p.B2) + p.colB2[n] * static_cast<int64_t>(sizeof(T));
   }
 
   // K offsets of the next stage to load: its loads take them from the
@@ -460,17 +441,9 @@ __device__ __forceinline__ void gett_tile(
   };
   auto a_off = [&](int i) { return UA ? k_lane(i) : aK[AKC ? 0 : UA ? 0 : i]; };
   auto b_off = [&](int i) { return UB ? k_lane(LA + i) : bK[BKC ? 0 : UB ? 0 : i]; };
-  bool segK = false;  // SEG2: the stage lies in the second segment
   auto load_koff = [&](int s) {
-    int64_t kb = kbeg + static_cast<int64_t>(s) * BK;
+    const int64_t kb = kbeg + static_cast<int64_t>(s) * BK;
     const int64_t *ca = p.colA, *rb = p.rowB;
-    if constexpr (SEG2) {
-      const bool sg = kb >= p.K1p;
-      segK = sg;
-      ca = sg ? p.colA2 : ca;
-      rb = sg ? p.rowB2 : rb;
-      kb = sg ? kb - p.K1p : kb;
-    }
     if constexpr (LANES > 0) kLane = (UA && (!UB || (t & 63) < LA) ? ca : rb)[kb + kIndex];
     if constexpr (!UA) {
 #pragma unroll
@@ -485,23 +458,11 @@ __device__ __forceinline__ void gett_tile(
   // staging registers; DEEP uses two sets, always indexed by constants
   constexpr int NSET = DEEP ? 2 : 1;
   T ra[NSET][EA], rb[NSET][EB];
-  bool segOn = false;  // SEG2: the row pointers are the second segment's
   // the stage's EA + EB elements in PARTS parts, part q in [lo(q), lo(q + 1))
   constexpr int PARTS = BK / 4 - 1;
   auto lo = [](int q) { return q * (EA + EB) / PARTS; };
   auto load_part = [&](auto set_c, int part) {
     constexpr int q = decltype(set_c)::value;
-    if constexpr (SEG2) {
-      if (part == 0) {
-        if (segK && !segOn) {  // once, at the first stage of the second segment
-          segOn = true;
-#pragma unroll
-          for (int i = 0; i < NRA; ++i) aRow[i] = aRow2[i];
-#pragma unroll
-          for (int i = 0; i < NRB; ++i) bCol[i] = bCol2[i];
-        }
-      }
-    }
 #pragma unroll
     for (int i = 0; i < EA; ++i)
       if (i >= lo(part) && i < lo(part + 1))
@@ -522,15 +483,11 @@ __device__ __forceinline__ void gett_tile(
   auto flip = [](double x, int mask) {
     return __hiloint2double(__double2hiint(x) ^ mask, __double2loint(x));
   };
-  // stage s from its registers to LDS: conjugation (and the second segment's
-  // factor) applied, elements past K zeroed
+  // stage s from its registers to LDS: conjugation applied, elements past K zeroed
   auto store_part = [&](int s, int buf, auto set_c, int part) {
     constexpr int q = decltype(set_c)::value;
-    bool seg2 = false;
-    if constexpr (SEG2) seg2 = kbeg + static_cast<int64_t>(s) * BK >= p.K1p;
     if (part == 0) {
-      int64_t left = p.K - kbeg - static_cast<int64_t>(s) * BK;  // k of this stage within K
-      if constexpr (SEG2) left = seg2 ? left : p.K1 - kbeg - static_cast<int64_t>(s) * BK;
+      const int64_t left = p.K - kbeg - static_cast<int64_t>(s) * BK;  // k of this stage within K
       if (left < BK) {
 #pragma unroll
         for (int i = 0; i < EA; ++i)
@@ -540,23 +497,11 @@ __device__ __forceinline__ void gett_tile(
           if (b_k(i) >= left) rb[q][i] = T{};
       }
     }
-    int fa = flipA, fb = flipB, fx = 0;
-    if constexpr (SEG2) {
-      // the second segment's factor: its sign as bits, its size where it is not 1
-      fx = seg2 && p.f2 < 0.0 ? static_cast<int>(0x80000000u) : 0;
-      fa = fx ^ (seg2 ? (p.signA2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fa);
-      fb = seg2 ? (p.signB2 < 0.0 ? static_cast<int>(0x80000000u) : 0) : fb;
-      const double f = fabs(p.f2);
-      if (part == 0 && seg2 && f != 1.0)
-#pragma unroll
-        for (int i = 0; i < EA; ++i) ra[q][i] = make_double2(f * ra[q][i].x, f * ra[q][i].y);
-    }
 #pragma unroll
     for (int i = 0; i < EA; ++i)
       if (i >= lo(part) && i < lo(part + 1)) {
         if constexpr (CPLX)
-          As[buf][a_k(i)][a_m(i)] = make_double2(SEG2 ? flip(ra[q][i].x, fx) : ra[q][i].x,
-                                                 flip(ra[q][i].y, fa));
+          As[buf][a_k(i)][a_m(i)] = make_double2(ra[q][i].x, flip(ra[q][i].y, flipA));
         else
           As[buf][a_k(i)][a_m(i)] = ra[q][i];
       }
@@ -564,7 +509,7 @@ __device__ __forceinline__ void gett_tile(
     for (int i = 0; i < EB; ++i)
       if (EA + i >= lo(part) && EA + i < lo(part + 1)) {
         if constexpr (CPLX)
-          Bs[buf][b_k(i)][b_n(i)] = make_double2(rb[q][i].x, flip(rb[q][i].y, fb));
+          Bs[buf][b_k(i)][b_n(i)] = make_double2(rb[q][i].x, flip(rb[q][i].y, flipB));
         else
           Bs[buf][b_k(i)][b_n(i)] = rb[q][i];
       }
@@ -775,12 +720,12 @@ __device__ __forceinline__ void gett_tile(
 }
 
 template <bool CPLX, int NT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC,
-          bool M3, bool DEEP, int MINW = 1, bool SEG2 = false>
+          bool M3, bool DEEP, int MINW = 1>
 __global__ __launch_bounds__(NT, MINW) void zgett_kernel(
-    std::conditional_t<SEG2, KArgs2, KArgs> p) {
+    KArgs p) {
   __shared__ Scalar<CPLX> As[2][BK][BM + kRowPad<CPLX>];
   __shared__ Scalar<CPLX> Bs[2][BK][BN + kRowPad<CPLX>];
-  gett_tile<CPLX, NT, BM, BN, BK, WM, WN, AKC, BKC, M3, DEEP, SEG2>(p, blockIdx.x, blockIdx.y, As,
+  gett_tile<CPLX, NT, BM, BN, BK, WM, WN, AKC, BKC, M3, DEEP>(p, blockIdx.x, blockIdx.y, As,
                                                                    Bs);
 }
 
@@ -816,16 +761,16 @@ __global__ __launch_bounds__(256, 4) void gett_group_kernel(GroupArgs g) {
   const int slice = b / tiles, block = b - slice * tiles;
   switch (g.orient[i]) {
     case 0:
-      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, false, false, CPLX, false, false>(p, block, slice, As, Bs);
+      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, false, false, CPLX, false>(p, block, slice, As, Bs);
       break;
     case 1:
-      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, false, true, CPLX, false, false>(p, block, slice, As, Bs);
+      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, false, true, CPLX, false>(p, block, slice, As, Bs);
       break;
     case 2:
-      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, true, false, CPLX, false, false>(p, block, slice, As, Bs);
+      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, true, false, CPLX, false>(p, block, slice, As, Bs);
       break;
     default:
-      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, true, true, CPLX, false, false>(p, block, slice, As, Bs);
+      gett_tile<CPLX, 256, 32, 32, 16, 16, 16, true, true, CPLX, false>(p, block, slice, As, Bs);
   }
 }
 
@@ -977,20 +922,20 @@ void dispatch_gett(const GettLaunch &L, const KArgs &args, dim3 grid, hipStream_
 }
 
 template <bool CPLX, int NT, int BM, int BN, int BK, int WM, int WN, bool M3,
-          bool DEEP = false, int MINW = 1, bool SEG2 = false>
-void dispatch_zgett(const GettLaunch &L, const std::conditional_t<SEG2, KArgs2, KArgs> &args,
+          bool DEEP = false, int MINW = 1>
+void dispatch_zgett(const GettLaunch &L, const KArgs &args,
                     dim3 grid, hipStream_t s) {
   if (L.a_kcontig && L.b_kcontig)
-    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, true, true, M3, DEEP, MINW, SEG2>
+    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, true, true, M3, DEEP, MINW>
         <<<grid, NT, 0, s>>>(args);
   else if (L.a_kcontig)
-    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, true, false, M3, DEEP, MINW, SEG2>
+    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, true, false, M3, DEEP, MINW>
         <<<grid, NT, 0, s>>>(args);
   else if (L.b_kcontig)
-    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, false, true, M3, DEEP, MINW, SEG2>
+    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, false, true, M3, DEEP, MINW>
         <<<grid, NT, 0, s>>>(args);
   else
-    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, false, false, M3, DEEP, MINW, SEG2>
+    zgett_kernel<CPLX, NT, BM, BN, BK, WM, WN, false, false, M3, DEEP, MINW>
         <<<grid, NT, 0, s>>>(args);
 }
 
@@ -1046,18 +991,17 @@ std::string gett_variant(const GettLaunch &L) {
   n += L.b_kcontig ? "_bk" : "_bn";
   if (L.tile == 1) n += "_t64";
   if (L.tile == 2) n += "_t32";
-  if (L.A2) n += "_seg2";
   return n;
 }
 
 namespace {
 void reduce_partials(bool cplx, const KArgs &a, int splits, hipStream_t s);
 
-KArgs2 kernel_args(const GettLaunch &L) {
+KArgs kernel_args(const GettLaunch &L) {
   const bool cplx = L.field == Field::Complex;
   const TileShape shape = tile_shape(L.field, static_cast<Tile>(L.tile));
   const int BM = shape.BM, BN = shape.BN, BK = kZ3BK;
-  KArgs2 a{};
+  KArgs a{};
   a.A = static_cast<const double *>(L.A);
   a.B = static_cast<const double *>(L.B);
   a.C = static_cast<double *>(L.C);
@@ -1080,13 +1024,6 @@ KArgs2 kernel_args(const GettLaunch &L) {
   a.tilesN = static_cast<int>((L.N + BN - 1) / BN);
   CC4S_ASSERT(static_cast<int64_t>(a.tilesM) * a.tilesN < (int64_t(1) << 31),
               "contraction too large for one launch");
-  a.A2 = static_cast<const double *>(L.A2);
-  a.B2 = static_cast<const double *>(L.B2);
-  a.rowA2 = L.rowA2; a.colA2 = L.colA2; a.rowB2 = L.rowB2; a.colB2 = L.colB2;
-  a.K1 = L.K1; a.K1p = L.K1p; a.K2 = L.K2;
-  a.f2 = L.f2;
-  a.signA2 = L.conjA2 ? -1.0 : 1.0;
-  a.signB2 = L.conjB2 ? -1.0 : 1.0;
   const int ntiles = a.tilesM * a.tilesN;
   a.fullTiles = L.tail_splits > 1 ? static_cast<int>(L.full_tiles) : ntiles;
   a.tailTiles = ntiles - a.fullTiles;
@@ -1102,23 +1039,14 @@ KArgs2 kernel_args(const GettLaunch &L) {
 void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
                  hipEvent_t stop) {
   const bool cplx = L.field == Field::Complex;
-  const bool seg2 = L.A2 != nullptr;
-  CC4S_ASSERT(!seg2 || (cplx && g_complex_generation == 3),
-              "two-segment contractions need the complex generation-3 kernel");
   const Tile tile = static_cast<Tile>(L.tile);
   const TileShape shape = tile_shape(L.field, tile);
   const int BM = shape.BM, BN = shape.BN;
-  const KArgs2 a = kernel_args(L);
+  const KArgs a = kernel_args(L);
   dim3 grid(a.fullTiles + a.tailTiles * std::max(1, L.tail_splits), L.splits);
   if (start) CC4S_HIP(hipEventRecord(start, s));
   if (cplx && g_complex_generation == 3) {
-    if (seg2 && tile == Tile::Large)
-      dispatch_zgett<true, 512, 128, 64, 16, 32, 32, true, false, 1, true>(L, a, grid, s);
-    else if (seg2 && tile == Tile::Medium)
-      dispatch_zgett<true, 256, 64, 64, 16, 32, 32, true, false, 2, true>(L, a, grid, s);
-    else if (seg2)
-      dispatch_zgett<true, 256, 32, 32, 16, 16, 16, true, false, 4, true>(L, a, grid, s);
-    else if (tile == Tile::Large)
+    if (tile == Tile::Large)
       dispatch_zgett<true, 512, 128, 64, 16, 32, 32, true>(L, a, grid, s);
     else if (tile == Tile::Medium)
       dispatch_zgett<true, 256, 64, 64, 16, 32, 32, true, false, 2>(L, a, grid, s);
@@ -1200,11 +1128,6 @@ struct GettPlan {
   Tile tile = Tile::Large;
   const int64_t *rowA, *colA, *rowB, *colB, *rowC, *colC;
   const int64_t *rowD = nullptr, *colD = nullptr;  // of an added tensor other than C
-  // two-segment plans: the second contraction's tables; swap2 tells that
-  // its second operand carries the M indices
-  bool swap2 = false;
-  int64_t K1 = 0, K1p = 0, K2 = 0;
-  const int64_t *rowA2 = nullptr, *colA2 = nullptr, *rowB2 = nullptr, *colB2 = nullptr;
 };
 
 ContractionEngine::ContractionEngine(hipStream_t s) : stream_(s) { apply_env_overrides(); }
@@ -1576,125 +1499,6 @@ void *ContractionEngine::reserve_partials(const GettPlan &P, Field f) {
   if (elements == 0) return nullptr;
   workspace_.reserve(elements * scalar_bytes(f));
   return workspace_.get();
-}
-
-GettPlan &ContractionEngine::plan_for2(const View &A1, const View &B1, const View &A2,
-                                       const View &B2, const View &C) {
-  const std::string key = "2|" + plan_key(A1, B1, C) + "|" + plan_key(A2, B2, C);
-  auto it = plans_.find(key);
-  if (it != plans_.end()) return *it->second;
-  // the first contraction's plan fixes the M and N orders and the swap
-  const GettPlan &P1 = plan_for(A1, B1, C);
-  auto plan = std::make_unique<GettPlan>();
-  plan->M = P1.M;
-  plan->N = P1.N;
-  plan->swap = P1.swap;
-  plan->a_kc = P1.a_kc;
-  plan->b_kc = P1.b_kc;
-  // M indices: C's indices carried by the first contraction's A-role operand,
-  // in the order of its strides (as plan_for orders them)
-  const View &Aop = P1.swap ? B1 : A1;
-  std::string Mi, Ni;
-  for (char c : C.idx) (Aop.find(c) >= 0 ? Mi : Ni) += c;
-  auto by = [](const View &v) {
-    return [&v](char x, char y) { return v.stride(x) < v.stride(y); };
-  };
-  std::stable_sort(Mi.begin(), Mi.end(), by(Aop));
-  std::stable_sort(Ni.begin(), Ni.end(), by(C));
-  auto c_set = [&C](const View &v) {
-    std::string s;
-    for (char c : v.idx)
-      if (C.find(c) >= 0) s += c;
-    std::sort(s.begin(), s.end());
-    return s;
-  };
-  std::string ms = Mi, ns = Ni;
-  std::sort(ms.begin(), ms.end());
-  std::sort(ns.begin(), ns.end());
-  CC4S_ASSERT((c_set(A2) == ms && c_set(B2) == ns) || (c_set(A2) == ns && c_set(B2) == ms),
-              "the two contractions split the result indices differently");
-  plan->swap2 = c_set(A2) != ms;
-  const View &A = plan->swap2 ? B2 : A2;
-  const View &B = plan->swap2 ? A2 : B2;
-  std::string Ki;
-  for (char c : A.idx) {
-    if (C.find(c) >= 0) continue;
-    CC4S_ASSERT(B.find(c) >= 0 && A.len(c) == B.len(c),
-                std::string("index '") + c + "' of the second contraction");
-    Ki += c;
-  }
-  CC4S_ASSERT(!Ki.empty(), "the second contraction has no summed index");
-  for (char c : Mi) CC4S_ASSERT(A.len(c) == C.len(c), "length mismatch (A2, C)");
-  for (char c : Ni) CC4S_ASSERT(B.len(c) == C.len(c), "length mismatch (B2, C)");
-  bool a_unit_k = false;
-  for (char c : Ki) a_unit_k |= A.stride(c) == 1 && A.len(c) > 1;
-  std::stable_sort(Ki.begin(), Ki.end(), a_unit_k ? by(A) : by(B));
-  const OffsetTable tables[] = {{&A, Mi, false, &plan->rowA2},
-                          {&A, Ki, true, &plan->colA2},
-                          {&B, Ki, true, &plan->rowB2},
-                          {&B, Ni, false, &plan->colB2}};
-  plan->K1 = P1.K;
-  plan->K1p = (P1.K + kZ3BK - 1) / kZ3BK * kZ3BK;
-  plan->K2 = tables[1].entries();
-  plan->K = plan->K1p + plan->K2;
-  build_tables(tables, 4);
-  plan->rowA = P1.rowA; plan->colA = P1.colA; plan->rowB = P1.rowB; plan->colB = P1.colB;
-  plan->rowC = P1.rowC; plan->colC = P1.colC;
-  choose_tile(C.field, plan->M, plan->N, plan->K, max_workspace, *plan);
-  auto &ref = *plan;
-  plans_.emplace(key, std::move(plan));
-  return ref;
-}
-
-void ContractionEngine::contract2(double alpha, const View &A1, const View &B1,
-                                  double alpha2, const View &A2, const View &B2,
-                                  double beta, const View &C) {
-  CC4S_ASSERT(A1.field == C.field && B1.field == C.field && A2.field == C.field &&
-                  B2.field == C.field,
-              "mixed scalar fields");
-  if (C.field != Field::Complex || g_complex_generation != 3 || mixed_ || alpha == 0.0) {
-    contract(alpha, A1, B1, beta, C);
-    contract(alpha2, A2, B2, 1.0, C);
-    return;
-  }
-  CC4S_ASSERT(!C.conj, "conjugated result view");
-  GettPlan &P = plan_for2(A1, B1, A2, B2, C);
-  if (P.M == 0 || P.N == 0) return;
-  GettLaunch L;
-  L.field = C.field;
-  L.A = P.swap ? B1.ptr : A1.ptr;
-  L.B = P.swap ? A1.ptr : B1.ptr;
-  L.conjA = P.swap ? B1.conj : A1.conj;
-  L.conjB = P.swap ? A1.conj : B1.conj;
-  L.A2 = P.swap2 ? B2.ptr : A2.ptr;
-  L.B2 = P.swap2 ? A2.ptr : B2.ptr;
-  L.conjA2 = P.swap2 ? B2.conj : A2.conj;
-  L.conjB2 = P.swap2 ? A2.conj : B2.conj;
-  L.C = C.ptr;
-  L.rowA = P.rowA; L.colA = P.colA; L.rowB = P.rowB; L.colB = P.colB;
-  L.rowA2 = P.rowA2; L.colA2 = P.colA2; L.rowB2 = P.rowB2; L.colB2 = P.colB2;
-  L.rowC = P.rowC; L.colC = P.colC;
-  L.M = P.M; L.N = P.N; L.K = P.K;
-  L.K1 = P.K1; L.K1p = P.K1p; L.K2 = P.K2;
-  L.f2 = alpha2 / alpha;
-  L.splits = P.splits;
-  L.tile = static_cast<int>(P.tile);
-  L.full_tiles = P.full_tiles;
-  L.tail_splits = P.tail_splits;
-  L.alpha = alpha; L.beta = beta;
-  L.a_kcontig = P.a_kc; L.b_kcontig = P.b_kc;
-  L.W = reserve_partials(P, C.field);
-  const double flops = 8.0 * double(P.M) * double(P.N) * double(P.K1 + P.K2);
-  if (profiling_) {
-    Pending p{take_event(), take_event(), gett_variant(L), flops};
-    launch_gett(L, stream_, p.start, p.stop);
-    pending_.push_back(p);
-    if (pending_.size() > 4096) (void)timings();
-  } else {
-    launch_gett(L, stream_);
-  }
-  stats.flops += flops;
-  stats.launches += 1;
 }
 
 void ContractionEngine::contract(double alpha, const View &A, const View &B,

@@ -50,14 +50,6 @@ struct GettLaunch {
   double alpha, beta;
   bool conjA, conjB;
   bool a_kcontig, b_kcontig;
-  // optional second K segment (complex generation-3 kernel): k in
-  // [K1p, K1p + K2) from A2, B2 and their tables, times f2; K = K1p + K2,
-  // K1p = K1 rounded up to whole K-stages (16)
-  const void *A2 = nullptr, *B2 = nullptr;
-  const int64_t *rowA2 = nullptr, *colA2 = nullptr, *rowB2 = nullptr, *colB2 = nullptr;
-  int64_t K1 = 0, K1p = 0, K2 = 0;
-  double f2 = 1.0;
-  bool conjA2 = false, conjB2 = false;
   // tensor added with beta (null: C)
   const void *D = nullptr;
   const int64_t *rowD = nullptr, *colD = nullptr;
@@ -91,12 +83,6 @@ class ContractionEngine {
     grouping_ = false;
     launch_group();
   }
-  // C = alpha * op(A1) op(B1) + alpha2 * op(A2) op(B2) + beta * C for two
-  // contractions whose operands split C's indices the same way: one launch
-  // with the second contraction as a second K segment, so C is read and
-  // written once (complex FP64 passes; otherwise two launches)
-  void contract2(double alpha, const View &A1, const View &B1, double alpha2,
-                 const View &A2, const View &B2, double beta, const View &C);
   // C = alpha * op(A) + beta * C, A's indices are a permutation of C's
   void sum(double alpha, const View &A, double beta, const View &C);
   // C = beta * C
@@ -162,8 +148,6 @@ class ContractionEngine {
 
  private:
   GettPlan &plan_for(const View &A, const View &B, const View &C, const View *D = nullptr);
-  GettPlan &plan_for2(const View &A1, const View &B1, const View &A2, const View &B2,
-                      const View &C);
   void launch_group();
   bool grouping_ = false;
   std::vector<GettLaunch> group_;

@@ -1,8 +1,13 @@
-// Energy kernel of the (T) correction.  For one hole pair (i, j) and a chunk
-// of k, W[a,b,c,k] holds the six-fold symmetrised connected triples
-// amplitude W_abcijk (PerturbativeTriplesReference.cxx:106-116, formed by
-// contractions on the MFMA engine); this kernel adds the disconnected part,
-// the spin-adapted combination and the denominator (:118-163):
+// The (T) correction.  The connected triples amplitude of a hole triple
+// i <= j <= k, the six-fold symmetrised W_abcijk
+// (PerturbativeTriplesReference.cxx:106-116), comes as three parts that the
+// first kernel forms:
+//   W_abc = Y_i[a;b,c] + Y_j[b;a,c] + Y_k[c;a,b],
+//   Y_i[a;b,c] = sum_d V_bcdk T_adij + V_cbdj T_adik
+//              - sum_l T_bcjl conj(V_kila) + T_cbkl conj(V_jila)
+// (Y_j and Y_k with the holes and particles exchanged likewise).  The energy
+// kernel adds them up, and the disconnected part, the spin-adapted combination
+// and the denominator (:118-163):
 //   S_x   = W_x + T1_{x1 i} V_{x2 x3 j k} + T1_{x2 j} V_{x1 x3 i k} + T1_{x3 k} V_{x1 x2 i j}
 //   Z     = 4/3 S_abc - 2 S_acb + 2/3 S_bca
 //   E    += Re(W_abc Z) / (e_i + e_j + e_k - e_a - e_b - e_c).
@@ -19,6 +24,7 @@
 // most CUs idle while it runs).
 #include "triples.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace cc4s_amd {
@@ -27,6 +33,17 @@ namespace {
 
 constexpr int kBlock = 512;
 constexpr int kComplexBlocks = 512;
+
+using dbl4 = double __attribute__((ext_vector_type(4)));
+
+// hole triple number n: tetrahedral(k) + triangular(j) + i, i <= j <= k
+__device__ __forceinline__ void hole_triple(int64_t n, int64_t (&h)[3]) {
+  h[2] = h[1] = 0;
+  while ((h[2] + 1) * (h[2] + 2) * (h[2] + 3) / 6 <= n) ++h[2];
+  n -= h[2] * (h[2] + 1) * (h[2] + 2) / 6;
+  while ((h[1] + 1) * (h[1] + 2) / 2 <= n) ++h[1];
+  h[0] = n - h[1] * (h[1] + 1) / 2;
+}
 
 template <bool CPLX>
 struct TS;
@@ -50,6 +67,262 @@ struct TS<true> {
   }
   __device__ static T plus(T a, T b) { return make_double2(a.x + b.x, a.y + b.y); }
 };
+
+// Y_y1[x1; x2, x3] of the hole triples t0 ... and of their parts part0 ..., one
+// after the other.  As a product it has M = (x2, x3), N = x1 and K in four
+// segments, d twice and l twice; every address is affine in m, n and k, so there
+// are no tables.  Bound by the matrix pipe where 2 Nv is long against the
+// prologue and the epilogue, and next by the traffic of Y: each of the three parts
+// is written once and read once by the energy kernel (as six contractions into one
+// W it was written six times and read five times between), in one launch for all
+// hole triples (330 launches, most too small for the chip).  M is walked in blocks
+// of 8 x 8 (x2, x3): V_x2x3 and V_x3x2 are then both read in whole 128-byte lines.
+// 128 rows by BN = 96 or 64 columns, whichever leaves fewer columns of padding
+// (Nv = 96 on tiles of 64 would multiply 1.33 times as much); eight waves of 32 x
+// BN / 2, in stages of 16 k that are loaded two stages ahead, in parts between the
+// MFMAs.  Measured with the energy at complex No=10, Nv=96: 28.2 -> 19.4 ms.
+struct ProductArgs {
+  const void *V, *T, *H;  // V[x2,x3,d,k], T[a,b,i,j], H = V_hhhp[i,j,l,a]
+  void *Y;
+  int64_t No, Nv, t0;  // first hole triple
+  int64_t blocks;      // workgroups
+  int parts, part0;    // parts per triple, the first of them
+  bool add;            // one part: Y += in W's order [a, b, c]
+};
+
+template <bool CPLX, int BN>
+__global__ __launch_bounds__(512, CPLX ? 2 : 4) void triples_product_kernel(ProductArgs p) {
+  using T = typename TS<CPLX>::T;
+  constexpr int NT = 512, BM = 128, BK = 16, MB = 2, NB = BN / 32;
+  constexpr int EA = BM * BK / NT, EB = BN * BK / NT, PARTS = BK / 4 - 1;
+  constexpr int PAD = CPLX ? 1 : 18;  // as in the contraction engine
+  static_assert(BN % 32 == 0 && BN * BK % NT == 0, "whole subtiles and elements");
+  __shared__ T As[2][BK][BM + PAD];
+  __shared__ T Bs[2][BK][BN + PAD];
+  const int t = threadIdx.x;
+  const int64_t v = p.Nv, o = p.No;
+  // consecutive workgroups are dealt to the 8 XCDs in turn: give each XCD a run of
+  // tiles, which share V or T in its L2
+  int64_t g = blockIdx.x;
+  const int64_t per = p.blocks / 8, rest = p.blocks % 8, xcd = g % 8;
+  g = xcd * per + min(xcd, rest) + g / 8;
+  const int64_t nb = (v + 7) / 8;  // blocks of 8 along x2 and x3
+  const int64_t tilesM = (nb * nb + 1) / 2, tilesN = (v + BN - 1) / BN;
+  const int64_t batch = g / (tilesM * tilesN);
+  g -= batch * (tilesM * tilesN);
+  const int64_t tm = g / tilesN, n0 = (g - tm * tilesN) * BN;
+  const int64_t triple = batch / p.parts;
+  const int part = p.part0 + static_cast<int>(batch - triple * p.parts);
+  int64_t h[3];
+  hole_triple(p.t0 + triple, h);
+  const int64_t y1 = part == 0 ? h[0] : part == 1 ? h[1] : h[2], y2 = part == 0 ? h[1] : h[0],
+                y3 = part == 2 ? h[1] : h[2];
+
+  // (x2, x3) of row m of the tile; past the edge the last is read
+  auto row = [&](int m, int64_t &x2, int64_t &x3) {
+    const int64_t q = min(tm * 2 + (m >> 6), nb * nb - 1);
+    x3 = q / nb;
+    x2 = (q - x3 * nb) * 8 + (m & 7);
+    x3 = x3 * 8 + ((m >> 3) & 7);
+    return tm * 2 + (m >> 6) < nb * nb && x2 < v && x3 < v;
+  };
+  int64_t row23, row32;  // of (x2, x3) and of (x3, x2)
+  {
+    int64_t x2, x3;
+    row(t % BM, x2, x3);
+    x2 = min(x2, v - 1);
+    x3 = min(x3, v - 1);
+    row23 = x2 + v * x3;
+    row32 = x3 + v * x2;
+  }
+  const int kA = t / BM;  // k of element i: kA + 4 i, one over a wave
+  int nB[EB], kB[EB];
+#pragma unroll
+  for (int i = 0; i < EB; ++i) {
+    nB[i] = static_cast<int>(min(n0 + (t + NT * i) % BN, v - 1));
+    kB[i] = (t + NT * i) / BN;
+  }
+  // Operands of segments 0 and 1 (V T) by base, the others' (T V_hhhp) and the
+  // second of each pair by what they add: choices between variables would keep
+  // them, and the registers' arrays with them, in memory
+  const char *A0 = static_cast<const char *>(p.V), *B0 = static_cast<const char *>(p.T);
+  const int64_t toHoleA = static_cast<const char *>(p.T) - A0,
+                toHoleB = static_cast<const char *>(p.H) - B0;
+  const int64_t holeK = o - v, holeSA = v * v * o - v * v, holeSB = o * o - v,
+                holeSN = o * o * o - 1, v2 = v * v;
+  const int64_t dy = y2 - y3, drow = row32 - row23;
+  const int stD = static_cast<int>((v + BK - 1) / BK), stL = static_cast<int>((o + BK - 1) / BK);
+  const int nstages = 2 * (stD + stL);
+  // segment 0 to 3 of stage s and its first k: V T, V~ T, T V_hhhp, T~ V_hhhp
+  auto segment = [&](int s, int &seg) {
+    const int d = s < stD ? 0 : s < 2 * stD ? 1 : s < 2 * stD + stL ? 2 : 3;
+    seg = d;
+    return (s - (d > 0 ? stD : 0) - (d > 1 ? stD : 0) - (d > 2 ? stL : 0)) * BK;
+  };
+  T ra[EA], rb[EB];
+  auto lo = [](int q) { return q * (EA + EB) / PARTS; };
+  // a part of stage s to registers; past a segment's K, and past the last stage,
+  // valid elements are read
+  auto load_part = [&](int s, auto part_c) {
+    constexpr int part_ = decltype(part_c)::value;
+    int seg;
+    const int kb = segment(min(s, nstages - 1), seg);
+    const bool hole = seg >= 2;
+    // y3 (segments 0, 3) or y2, and the other
+    const int64_t m0 = seg == 0 || seg == 3 ? 0 : dy, yA = y3 + m0, yB = y2 - m0;
+    const int64_t K = v + (hole ? holeK : 0), sA = v2 + (hole ? holeSA : 0),
+                  sB = v + (hole ? holeSB : 0), sN = 1 + (hole ? holeSN : 0);
+    const T *A = reinterpret_cast<const T *>(A0 + (hole ? toHoleA : 0)) +
+                 v2 * (hole ? yA : v * yA) + row23 + (seg & 1 ? drow : 0);
+    const T *B = reinterpret_cast<const T *>(B0 + (hole ? toHoleB : 0)) +
+                 (hole ? yB + o * y1 : v2 * (y1 + o * yB));
+#pragma unroll
+    for (int i = 0; i < EA; ++i)
+      if (i >= lo(part_) && i < lo(part_ + 1))
+        ra[i] = A[min(static_cast<int64_t>(kb + __builtin_amdgcn_readfirstlane(kA) + 4 * i),
+                       K - 1) * sA];
+#pragma unroll
+    for (int i = 0; i < EB; ++i)
+      if (EA + i >= lo(part_) && EA + i < lo(part_ + 1))
+        rb[i] = B[nB[i] * sN + min(static_cast<int64_t>(kb + kB[i]), K - 1) * sB];
+  };
+  auto sign = [](double x, int mask) {
+    return __hiloint2double(__double2hiint(x) ^ mask, __double2loint(x));
+  };
+  // and to LDS: zero past K, - conj(V_hhhp)
+  auto store_part = [&](int s, int buf, auto part_c) {
+    constexpr int part_ = decltype(part_c)::value;
+    int seg;
+    const int kb = segment(min(s, nstages - 1), seg);
+    const int left = static_cast<int>(v + (seg >= 2 ? holeK : 0)) - kb;
+    const int neg = seg >= 2 ? static_cast<int>(0x80000000u) : 0;
+#pragma unroll
+    for (int i = 0; i < EA; ++i)
+      if (i >= lo(part_) && i < lo(part_ + 1)) {
+        if (kA + 4 * i >= left) ra[i] = T{};
+        As[buf][kA + 4 * i][t % BM] = ra[i];
+      }
+#pragma unroll
+    for (int i = 0; i < EB; ++i)
+      if (EA + i >= lo(part_) && EA + i < lo(part_ + 1)) {
+        if (kB[i] >= left) rb[i] = T{};
+        if constexpr (CPLX)
+          rb[i].x = sign(rb[i].x, neg);
+        else
+          rb[i] = sign(rb[i], neg);
+        Bs[buf][kB[i]][(t + NT * i) % BN] = rb[i];
+      }
+  };
+
+  const int lane = t & 63, w = t >> 6, wm = w >> 1, wn = w & 1;
+  // three products per complex one: re re, im im, (re + im)(re + im)
+  dbl4 acc[CPLX ? 3 : 1][MB][NB];
+#pragma unroll
+  for (int c = 0; c < (CPLX ? 3 : 1); ++c)
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[c][i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+  T fa[2][MB], fb[2][NB];
+  auto load_frag = [&](int buf, int kq, auto q_c) {
+    constexpr int q = decltype(q_c)::value;
+    const int kr = kq * 4 + (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) fa[q][i] = As[buf][kr][wm * 32 + i * 16 + (lane & 15)];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) fb[q][j] = Bs[buf][kr][wn * (BN / 2) + j * 16 + (lane & 15)];
+  };
+  auto multiply = [&](auto q_c) {
+    constexpr int q = decltype(q_c)::value;
+    auto mma = [&](dbl4(&c)[MB][NB], auto of) {
+      double x[MB], y[NB];
+#pragma unroll
+      for (int i = 0; i < MB; ++i) x[i] = of(fa[q][i]);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) y[j] = of(fb[q][j]);
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          c[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i], y[j], c[i][j], 0, 0, 0);
+    };
+    if constexpr (CPLX) {
+      mma(acc[0], [](T z) { return z.x; });
+      mma(acc[1], [](T z) { return z.y; });
+      mma(acc[2], [](T z) { return z.x + z.y; });
+    } else {
+      mma(acc[0], [](T z) { return z; });
+    }
+  };
+
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I3 = std::integral_constant<int, 3>;
+  static_assert(PARTS == 3, "three parts, four k steps");
+  load_part(0, I0{}), load_part(0, I1{}), load_part(0, I2{});
+  store_part(0, 0, I0{}), store_part(0, 0, I1{}), store_part(0, 0, I2{});
+  load_part(1, I0{}), load_part(1, I1{}), load_part(1, I2{});
+  __syncthreads();
+  load_frag(0, 0, I0{});
+  // multiply LDS buffer s & 1, move stage s + 1 from the registers to the other
+  // one and load stage s + 2, a part after each k step but the last; the barrier
+  // stands before the last k step, whose fragments are in registers, so that the
+  // next stage's first are read under its MFMAs
+  auto step = [&](int s, auto par_c, auto kq_c) {
+    constexpr int par = decltype(par_c)::value, kq = decltype(kq_c)::value;
+    constexpr std::integral_constant<int, kq & 1> q;
+    constexpr std::integral_constant<int, (kq + 1) & 1> next;
+    if constexpr (kq < PARTS) {
+      load_frag(par, kq + 1, next);
+    } else {
+      __syncthreads();
+      load_frag(par ^ 1, 0, next);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(q);
+    if constexpr (kq < PARTS) {
+      store_part(s + 1, par ^ 1, kq_c);
+      load_part(s + 2, kq_c);
+    }
+  };
+  auto stage = [&](int s, auto par) {
+    step(s, par, I0{}), step(s, par, I1{}), step(s, par, I2{}), step(s, par, I3{});
+  };
+  for (int s = 0; s < nstages; s += 2) {  // an even number
+    stage(s, I0{});
+    stage(s + 1, I1{});
+  }
+
+  // element (x1, x2, x3) of a part of its own, or of W[a, b, c]
+  int64_t s1 = 1, s2 = v, s3 = v * v;
+  T *Y = static_cast<T *>(p.Y) + batch * v * v * v;
+  if (p.parts == 1) {
+    s1 = part == 0 ? 1 : part == 1 ? v : v * v;
+    s2 = part == 0 ? v : 1;
+    s3 = part == 2 ? v : v * v;
+  }
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      int64_t x2, x3;
+      if (!row(wm * 32 + i * 16 + 4 * r + (lane >> 4), x2, x3)) continue;
+      T *out = Y + s2 * x2 + s3 * x3;
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int64_t x1 = n0 + wn * (BN / 2) + j * 16 + (lane & 15);
+        if (x1 >= v) continue;
+        T x;
+        if constexpr (CPLX)
+          x = make_double2(acc[0][i][j][r] - acc[1][i][j][r],
+                           acc[2][i][j][r] - (acc[0][i][j][r] + acc[1][i][j][r]));
+        else
+          x = acc[0][i][j][r];
+        out[s1 * x1] = p.add ? TS<CPLX>::plus(out[s1 * x1], x) : x;
+      }
+    }
+}
 
 // The particle triples are taken in tiles of kTile^3 (a, b, c).  A block
 // takes a canonical tile triple tA <= tB <= tC and forms S at the six
@@ -86,14 +359,15 @@ __device__ __forceinline__ void six(F &&f) {
 // there once, keeps it in registers for the energy of the same element, and its
 // reads of W, V and T1 are in flight together (two blocks per CU with 128
 // registers; three with 80 spill and take 4.1 ms below).  Blocks walk the
-// canonical triples only, so they share them evenly.  Measured over the 55
-// launches of (T) at No=10, Nv=96: 5.6 -> 2.4 ms.
+// canonical triples only, so they share them evenly.  Measured over (T) at
+// No=10, Nv=96: 5.6 -> 2.4 ms, and 3.6 with the sum of three parts, which the
+// products used to form.
 template <bool CPLX>
 __global__ __launch_bounds__(kBlock, 4) void triples_energy_kernel(
     const typename TS<CPLX>::T *__restrict__ W, const typename TS<CPLX>::T *__restrict__ V,
     const typename TS<CPLX>::T *__restrict__ T1, const double *__restrict__ eh,
-    const double *__restrict__ ep, int64_t No, int64_t Nv, int64_t i, int64_t j,
-    int64_t k0, int64_t kc, double *acc) {
+    const double *__restrict__ ep, int64_t No, int64_t Nv, int64_t t0, int64_t count,
+    int parts, double *acc) {
   using S = TS<CPLX>;
   using T = typename S::T;
   // S at the six orderings of the canonical tile triple's index ranges
@@ -103,9 +377,8 @@ __global__ __launch_bounds__(kBlock, 4) void triples_energy_kernel(
   const int64_t v = Nv, o = No;
   const int64_t nt = (v + kTile - 1) / kTile;
   const int64_t nc = nt * (nt + 1) * (nt + 2) / 6;  // canonical tile triples
-  const int64_t ntiles = nc * kc;
+  const int64_t ntiles = nc * count;
   // V_pphh[p,q,s,r] at p + v (q + v (s + o r)); T1[a,i] at a + v i
-  const T *Vjk = V + v * v * j, *Vij = V + v * v * (i + o * j);
   const int t = threadIdx.x;
   const int l[3] = {t % kTile, (t / kTile) % kTile, t / (kTile * kTile)};
   double sum = 0.0;
@@ -120,9 +393,12 @@ __global__ __launch_bounds__(kBlock, 4) void triples_energy_kernel(
     const int64_t tA = r - tB * (tB + 1) / 2;
     const int64_t ti[3] = {tA, tB, tC};
     const int64_t r0[3] = {tA * kTile, tB * kTile, tC * kTile};
-    const int64_t base = v * v * v * kl;
-    const int64_t k = k0 + kl;
-    const T *Vik = V + v * v * (i + o * k), *Vjkk = Vjk + v * v * o * k;
+    const int64_t v3 = v * v * v, base = v3 * kl * parts;
+    int64_t hole[3];
+    hole_triple(t0 + kl, hole);
+    const int64_t i = hole[0], j = hole[1], k = hole[2];
+    const T *Vij = V + v * v * (i + o * j), *Vik = V + v * v * (i + o * k),
+            *Vjkk = V + v * v * (j + o * k);
     __syncthreads();  // the previous tile's LDS reads are done
     // S at the ordering (x1, x2, x3) and the holes (i, j, k): W plus the
     // disconnected part; x1 runs fastest, so the V and T1 reads along x1 are
@@ -136,6 +412,9 @@ __global__ __launch_bounds__(kBlock, 4) void triples_energy_kernel(
       const bool in = y1 < v && y2 < v && y3 < v;
       const int64_t x1 = min(y1, v - 1), x2 = min(y2, v - 1), x3 = min(y3, v - 1);
       w[p] = W[base + x1 + v * (x2 + v * x3)];
+      if (parts == 3)
+        w[p] = S::plus(w[p], S::plus(W[base + v3 + x2 + v * (x1 + v * x3)],
+                                     W[base + 2 * v3 + x3 + v * (x1 + v * x2)]));
       const T s = S::plus(w[p], S::plus(S::mul(T1[x1 + v * i], Vjkk[x2 + v * x3]),
                                         S::plus(S::mul(T1[x2 + v * j], Vik[x1 + v * x3]),
                                                 S::mul(T1[x3 + v * k], Vij[x1 + v * x2]))));
@@ -182,20 +461,73 @@ __global__ __launch_bounds__(kBlock, 4) void triples_energy_kernel(
 
 }  // namespace
 
+namespace {
+// columns of a tile: whichever leaves fewer columns of padding
+int64_t tile_columns(int64_t Nv) {
+  return (Nv + 95) / 96 * 96 <= (Nv + 63) / 64 * 64 ? 96 : 64;
+}
+// tiles of one part of one hole triple
+int64_t tiles_of(int64_t Nv) {
+  const int64_t nb = (Nv + 7) / 8, BN = tile_columns(Nv);
+  return (nb * nb + 1) / 2 * ((Nv + BN - 1) / BN);
+}
+}  // namespace
+
+int64_t triples_chunk(int64_t Nv, int64_t all, int64_t most, int parts) {
+  most = std::max<int64_t>(1, std::min(all, most));
+  // between half the most and the most, the number whose last wave of
+  // workgroups (one per CU) is fullest
+  const int64_t tiles = tiles_of(Nv) * parts;
+  auto loss = [&](int64_t n) {
+    const int64_t slots = (n * tiles + 255) / 256 * 256;
+    return static_cast<double>(slots - n * tiles) / static_cast<double>(slots);
+  };
+  int64_t best = most;
+  if (most < all)
+    for (int64_t n = most; n > most / 2 && n > most - 64; --n)
+      if (loss(n) < loss(best)) best = n;
+  return best;
+}
+
+void triples_product(hipStream_t s, Field f, const void *Vppph, const void *T2, const void *Vhhhp,
+                     void *Y, int64_t No, int64_t Nv, int64_t t0, int64_t count, int part) {
+  CC4S_ASSERT(No > 0 && Nv > 0 && t0 >= 0 && count > 0 && part < 3 &&
+                  t0 + count <= No * (No + 1) * (No + 2) / 6,
+              "triples: hole triples out of range");
+  const bool wide = tile_columns(Nv) == 96;
+  const int64_t parts = part < 0 ? 3 : 1, tiles = tiles_of(Nv) * parts;
+  // launches of less than 2^32 threads
+  const int64_t per = ((int64_t(1) << 32) / 512 - 1) / tiles;
+  CC4S_ASSERT(per > 0, "triples: too many tiles for one launch");
+  for (int64_t t = 0; t < count; t += per) {
+    const int64_t n = std::min(per, count - t);
+    ProductArgs a{Vppph, T2, Vhhhp,
+                  static_cast<char *>(Y) + t * parts * Nv * Nv * Nv * scalar_bytes(f),
+                  No, Nv, t0 + t, tiles * n, static_cast<int>(parts), std::max(part, 0), part > 0};
+    auto run = [&](auto kernel) {
+      kernel<<<static_cast<unsigned>(a.blocks), 512, 0, s>>>(a);
+      CC4S_HIP(hipGetLastError());
+    };
+    if (f == Field::Complex)
+      wide ? run(triples_product_kernel<true, 96>) : run(triples_product_kernel<true, 64>);
+    else
+      wide ? run(triples_product_kernel<false, 96>) : run(triples_product_kernel<false, 64>);
+  }
+}
+
 void triples_energy(hipStream_t s, Field f, const void *W, const void *Vpphh,
                     const void *T1, const double *eps_h, const double *eps_p,
-                    int64_t No, int64_t Nv, int64_t i, int64_t j, int64_t k0,
-                    int64_t kc, double *acc) {
-  CC4S_ASSERT(i >= 0 && i <= j && j < No && k0 >= j && kc > 0 && k0 + kc <= No,
-              "triples: hole indices out of range (needs i <= j <= k)");
+                    int64_t No, int64_t Nv, int64_t t0, int64_t count, int parts, double *acc) {
+  CC4S_ASSERT(t0 >= 0 && count > 0 && t0 + count <= No * (No + 1) * (No + 2) / 6,
+              "triples: hole triples out of range");
   if (f == Field::Complex)
     triples_energy_kernel<true><<<kComplexBlocks, kBlock, 0, s>>>(
         static_cast<const double2 *>(W), static_cast<const double2 *>(Vpphh),
-        static_cast<const double2 *>(T1), eps_h, eps_p, No, Nv, i, j, k0, kc, acc);
+        static_cast<const double2 *>(T1), eps_h, eps_p, No, Nv, t0, count, parts, acc);
   else
     triples_energy_kernel<false><<<kTriplesBlocks, kBlock, 0, s>>>(
         static_cast<const double *>(W), static_cast<const double *>(Vpphh),
-        static_cast<const double *>(T1), eps_h, eps_p, No, Nv, i, j, k0, kc, acc);
+        static_cast<const double *>(T1), eps_h, eps_p, No, Nv, t0, count, parts, acc);
   CC4S_HIP(hipGetLastError());
 }
 

@@ -303,6 +303,35 @@ def test_triples_parity(field, shape):
     assert abs(e - ref) <= 1e-12 * abs(ref)
 
 
+# (shape, bytes of connected amplitudes per chunk): Nv on both sides of the 8 x 8
+# blocks of (x2, x3), of the 64- and 96-column tiles and of two of them; all hole
+# triples in one launch, one triple in three parts, one triple part by part
+TRIPLES_CASES = [((2, 3, 5), None), ((3, 8, 9), None), ((17, 18, 9), None), ((2, 64, 10), None),
+                 ((2, 65, 10), None), ((2, 96, 10), None), ((2, 97, 10), None),
+                 ((3, 33, 20), "three"), ((3, 33, 20), "one"), ((3, 66, 10), "one")]
+
+
+@pytest.mark.parametrize("field", ["complex", "real"])
+@pytest.mark.parametrize("shape,chunk", TRIPLES_CASES)
+def test_triples_tile_edges_and_chunks(field, shape, chunk, monkeypatch):
+    """As test_triples_parity: sums of 2 (Nv + No) products per amplitude, same
+    1e-12 relative."""
+    No, Nv, NG = shape
+    print(f"triples {field} {shape} {chunk}", flush=True)
+    if chunk:
+        part = Nv ** 3 * (16 if field == "complex" else 8)
+        monkeypatch.setenv("CC4S_TRIPLES_W_BYTES", str({"three": 3, "one": 1}[chunk] * part))
+    inp = syn.generate(No, Nv, NG, field, 31)
+    T = _amps(No, Nv, field, 37, scale=0.1)
+    with api.CoupledCluster(No, Nv, NG, field=field) as cc:
+        cc.set_inputs(inp.gamma, inp.eps)
+        cc.set_amplitudes(*T)
+        e = cc.triples()
+        assert e == cc.triples()
+    ref = O.perturbative_triples(inp.gamma, inp.eps, No, field, T)
+    assert abs(e - ref) <= 1e-12 * abs(ref)
+
+
 def test_ueg_triples_of_the_reference_test_suite():
     """(T) of the GPU CCSD amplitudes of the uniform electron gas rs=1, No=7,
     Nv=26 equals the reference's recorded PerturbativeTriplesReference
