@@ -857,6 +857,8 @@ double Ccsd::triples(const void *Tp, const double *eps_h, const double *eps_p) {
   Tensor Vppph;
   form_slice(Vppph, "ppph");                                     // V[b,c,d,k]
   const void *T2 = offset_ptr(const_cast<void *>(Tp), s_.n1(), f);
+  Tensor H(f, "alji", {v, o, o, o});  // - conj(V_ijla), a fastest as in T2
+  E.sum(-1.0, f == Field::Complex ? w.Vhhhp("ijla").conjugated() : w.Vhhhp("ijla"), 0.0, H("alji"));
 
   // Bytes of connected amplitudes per chunk of hole triples
   // (CC4S_TRIPLES_W_BYTES overrides): a triple's three parts, or their sum, formed
@@ -878,7 +880,7 @@ double Ccsd::triples(const void *Tp, const double *eps_h, const double *eps_p) {
   for (int64_t t = 0; t < all; t += chunk) {
     const int64_t n = std::min(chunk, all - t);
     for (int part = parts == 3 ? -1 : 0; part < (parts == 3 ? 0 : 3); ++part)
-      triples_product(E.stream(), f, Vppph.buf.get(), T2, w.Vhhhp.buf.get(), Y.get(), o, v, t, n,
+      triples_product(E.stream(), f, Vppph.buf.get(), T2, H.buf.get(), Y.get(), o, v, t, n,
                       part);
     triples_energy(E.stream(), f, Y.get(), w.Vpphh.v.ptr, offset_ptr(const_cast<void *>(Tp), 0, f),
                    eps_h, eps_p, o, v, t, n, parts, acc.as<double>());

@@ -71,7 +71,8 @@ struct TS<true> {
 // Y_y1[x1; x2, x3] of the hole triples t0 ... and of their parts part0 ..., one
 // after the other.  As a product it has M = (x2, x3), N = x1 and K in four
 // segments, d twice and l twice; every address is affine in m, n and k, so there
-// are no tables.  Bound by the matrix pipe where 2 Nv is long against the
+// are no tables, and with H in T's order only bases, a stride and K differ between
+// the segments.  Bound by the matrix pipe where 2 Nv is long against the
 // prologue and the epilogue, and next by the traffic of Y: each of the three parts
 // is written once and read once by the energy kernel (as six contractions into one
 // W it was written six times and read five times between), in one launch for all
@@ -80,15 +81,23 @@ struct TS<true> {
 // 128 rows by BN = 96 or 64 columns, whichever leaves fewer columns of padding
 // (Nv = 96 on tiles of 64 would multiply 1.33 times as much); eight waves of 32 x
 // BN / 2, in stages of 16 k that are loaded two stages ahead, in parts between the
-// MFMAs.  Measured with the energy at complex No=10, Nv=96: 28.2 -> 19.4 ms.
+// MFMAs.  Measured with the energy at complex No=10, Nv=96: 28.2 -> 18.3 ms.
 struct ProductArgs {
-  const void *V, *T, *H;  // V[x2,x3,d,k], T[a,b,i,j], H = V_hhhp[i,j,l,a]
+  const void *V, *T, *H;  // V[x2,x3,d,k], T[a,b,i,j], H[a,l,j,i] = -conj(V_ijla)
   void *Y;
   int64_t No, Nv, t0;  // first hole triple
-  int64_t blocks;      // workgroups
+  int tiles;           // of all the parts and triples
   int parts, part0;    // parts per triple, the first of them
   bool add;            // one part: Y += in W's order [a, b, c]
 };
+
+typedef double dbl2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void store_stream(double *p, double x) {
+  __builtin_nontemporal_store(x, p);
+}
+__device__ __forceinline__ void store_stream(double2 *p, double2 x) {
+  __builtin_nontemporal_store(dbl2{x.x, x.y}, reinterpret_cast<dbl2 *>(p));
+}
 
 template <bool CPLX, int BN>
 __global__ __launch_bounds__(512, CPLX ? 2 : 4) void triples_product_kernel(ProductArgs p) {
@@ -101,128 +110,129 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void triples_product_kernel(Prod
   __shared__ T Bs[2][BK][BN + PAD];
   const int t = threadIdx.x;
   const int64_t v = p.Nv, o = p.No;
-  // consecutive workgroups are dealt to the 8 XCDs in turn: give each XCD a run of
-  // tiles, which share V or T in its L2
-  int64_t g = blockIdx.x;
-  const int64_t per = p.blocks / 8, rest = p.blocks % 8, xcd = g % 8;
-  g = xcd * per + min(xcd, rest) + g / 8;
-  const int64_t nb = (v + 7) / 8;  // blocks of 8 along x2 and x3
-  const int64_t tilesM = (nb * nb + 1) / 2, tilesN = (v + BN - 1) / BN;
-  const int64_t batch = g / (tilesM * tilesN);
-  g -= batch * (tilesM * tilesN);
-  const int64_t tm = g / tilesN, n0 = (g - tm * tilesN) * BN;
-  const int64_t triple = batch / p.parts;
-  const int part = p.part0 + static_cast<int>(batch - triple * p.parts);
-  int64_t h[3];
-  hole_triple(p.t0 + triple, h);
-  const int64_t y1 = part == 0 ? h[0] : part == 1 ? h[1] : h[2], y2 = part == 0 ? h[1] : h[0],
-                y3 = part == 2 ? h[1] : h[2];
-
-  // (x2, x3) of row m of the tile; past the edge the last is read
-  auto row = [&](int m, int64_t &x2, int64_t &x3) {
-    const int64_t q = min(tm * 2 + (m >> 6), nb * nb - 1);
-    x3 = q / nb;
-    x2 = (q - x3 * nb) * 8 + (m & 7);
-    x3 = x3 * 8 + ((m >> 3) & 7);
-    return tm * 2 + (m >> 6) < nb * nb && x2 < v && x3 < v;
+  const int64_t v2 = v * v;
+  // a run of consecutive tiles per workgroup; consecutive workgroups are dealt to
+  // the 8 XCDs in turn, so that an XCD's runs follow each other and share V or T
+  // in its L2
+  const int grid = gridDim.x, place = (blockIdx.x & 7) * (grid >> 3) + (blockIdx.x >> 3);
+  const int first = static_cast<int>(static_cast<int64_t>(p.tiles) * place / grid);
+  const int last = static_cast<int>(static_cast<int64_t>(p.tiles) * (place + 1) / grid);
+  if (first == last) return;
+  const int nb = static_cast<int>((v + 7) / 8);  // blocks of 8 along x2 and x3
+  const int tilesM = (nb * nb + 1) / 2, tilesN = static_cast<int>((v + BN - 1) / BN);
+  struct Tile {
+    int batch, part, n0;
+    int x2, x3, d2, d3;  // of its first block of (x2, x3), and to its second
+    int two;             // whether there is a second (else the first again)
+    int64_t y1, y2, y3;
   };
-  int64_t row23, row32;  // of (x2, x3) and of (x3, x2)
-  {
-    int64_t x2, x3;
-    row(t % BM, x2, x3);
-    x2 = min(x2, v - 1);
-    x3 = min(x3, v - 1);
-    row23 = x2 + v * x3;
-    row32 = x3 + v * x2;
-  }
-  const int kA = t / BM;  // k of element i: kA + 4 i, one over a wave
-  int nB[EB], kB[EB];
+  auto locate = [&](int g) {
+    Tile c;
+    c.batch = g / (tilesM * tilesN);
+    g -= c.batch * (tilesM * tilesN);
+    const int tm = g / tilesN, triple = c.batch / p.parts;
+    c.n0 = (g - tm * tilesN) * BN;
+    c.part = p.part0 + c.batch - triple * p.parts;
+    c.two = 2 * tm + 1 < nb * nb;
+    const int q = c.two ? 2 * tm + 1 : 2 * tm, r2 = 2 * tm / nb, r3 = q / nb;
+    c.x3 = r2 * 8;
+    c.x2 = (2 * tm - r2 * nb) * 8;
+    c.d3 = r3 * 8 - c.x3;
+    c.d2 = (q - r3 * nb) * 8 - c.x2;
+    int64_t h[3];
+    hole_triple(p.t0 + triple, h);
+    c.y1 = c.part == 0 ? h[0] : c.part == 1 ? h[1] : h[2];
+    c.y2 = c.part == 0 ? h[1] : h[0];
+    c.y3 = c.part == 2 ? h[1] : h[2];
+    return c;
+  };
+  // what this thread loads of the tile in the load pipeline, in bytes: the row of
+  // (x2, x3), what (x3, x2) adds to it, the columns; past the edge the last are read
+  constexpr int ES = sizeof(T);
+  uint32_t row23, drow, nB[EB];
+  int64_t y1, y2, y3;
+  auto load_from = [&](const Tile &c) {
+    const bool k = t & 64;
+    const int x2 = min(c.x2 + (k ? c.d2 : 0) + (t & 7), static_cast<int>(v) - 1),
+              x3 = min(c.x3 + (k ? c.d3 : 0) + ((t >> 3) & 7), static_cast<int>(v) - 1);
+    row23 = static_cast<uint32_t>(x2 + v * x3) * ES;
+    drow = static_cast<uint32_t>(x3 + v * x2) * ES - row23;
+    y1 = c.y1;
+    y2 = c.y2;
+    y3 = c.y3;
 #pragma unroll
-  for (int i = 0; i < EB; ++i) {
-    nB[i] = static_cast<int>(min(n0 + (t + NT * i) % BN, v - 1));
-    kB[i] = (t + NT * i) / BN;
-  }
-  // Operands of segments 0 and 1 (V T) by base, the others' (T V_hhhp) and the
-  // second of each pair by what they add: choices between variables would keep
-  // them, and the registers' arrays with them, in memory
+    for (int i = 0; i < EB; ++i)
+      nB[i] = static_cast<uint32_t>(min(c.n0 + (t + NT * i) % BN, static_cast<int>(v) - 1)) * ES;
+  };
+  const int kA = __builtin_amdgcn_readfirstlane(t / BM);  // k of element i: kA + 4 i
+  int kB[EB];
+#pragma unroll
+  for (int i = 0; i < EB; ++i) kB[i] = (t + NT * i) / BN;
+  const int stD = static_cast<int>((v + BK - 1) / BK), stL = static_cast<int>((o + BK - 1) / BK);
+  const int nstages = 2 * (stD + stL);
+  // segment 0 to 3 of stage s and its first k: V T, V~ T, T H, T~ H (~: x2, x3
+  // exchanged).  Sums of conditions and masks, here and below: choices would
+  // become branches, at whose ends the compiler waits for every LDS operation
+  auto segment = [&](int s, int &d1, int &d2, int &d3) {
+    d1 = s >= stD;
+    d2 = s >= 2 * stD;
+    d3 = s >= 2 * stD + stL;
+    return (s - stD * (d1 + d2) - stL * d3) * BK;
+  };
+  // the stage being loaded
+  const char *A, *B;  // of its first k
+  int64_t sA;         // A's bytes per k; B's are v elements
+  int left;           // k to the end of the segment
+  uint32_t rowA;
   const char *A0 = static_cast<const char *>(p.V), *B0 = static_cast<const char *>(p.T);
   const int64_t toHoleA = static_cast<const char *>(p.T) - A0,
                 toHoleB = static_cast<const char *>(p.H) - B0;
-  const int64_t holeK = o - v, holeSA = v * v * o - v * v, holeSB = o * o - v,
-                holeSN = o * o * o - 1, v2 = v * v;
-  const int64_t dy = y2 - y3, drow = row32 - row23;
-  const int stD = static_cast<int>((v + BK - 1) / BK), stL = static_cast<int>((o + BK - 1) / BK);
-  const int nstages = 2 * (stD + stL);
-  // segment 0 to 3 of stage s and its first k: V T, V~ T, T V_hhhp, T~ V_hhhp
-  auto segment = [&](int s, int &seg) {
-    const int d = s < stD ? 0 : s < 2 * stD ? 1 : s < 2 * stD + stL ? 2 : 3;
-    seg = d;
-    return (s - (d > 0 ? stD : 0) - (d > 1 ? stD : 0) - (d > 2 ? stL : 0)) * BK;
+  auto begin_load = [&](int s) {
+    int d1, d2, d3;
+    const int64_t kb = segment(s, d1, d2, d3);
+    const int64_t hole = -static_cast<int64_t>(d2), other = -static_cast<int64_t>(d1 ^ d3);
+    const int64_t dy = (y2 - y3) & other, K = v + ((o - v) & hole);
+    sA = ES * (v2 + ((v2 * o - v2) & hole));
+    A = A0 + (toHoleA & hole) + ES * v2 * (y3 + dy) * (v + ((1 - v) & hole)) + kb * sA;
+    B = B0 + (toHoleB & hole) + ES * v * (K * (y1 + o * (y2 - dy)) + kb);
+    left = static_cast<int>(K - kb);
+    rowA = row23 + (drow & -static_cast<uint32_t>((d1 + d2 + d3) & 1));
   };
   T ra[EA], rb[EB];
   auto lo = [](int q) { return q * (EA + EB) / PARTS; };
-  // a part of stage s to registers; past a segment's K, and past the last stage,
-  // valid elements are read
-  auto load_part = [&](int s, auto part_c) {
+  // a part of it to registers; past a segment's K valid elements are read
+  auto load_part = [&](auto part_c) {
     constexpr int part_ = decltype(part_c)::value;
-    int seg;
-    const int kb = segment(min(s, nstages - 1), seg);
-    const bool hole = seg >= 2;
-    // y3 (segments 0, 3) or y2, and the other
-    const int64_t m0 = seg == 0 || seg == 3 ? 0 : dy, yA = y3 + m0, yB = y2 - m0;
-    const int64_t K = v + (hole ? holeK : 0), sA = v2 + (hole ? holeSA : 0),
-                  sB = v + (hole ? holeSB : 0), sN = 1 + (hole ? holeSN : 0);
-    const T *A = reinterpret_cast<const T *>(A0 + (hole ? toHoleA : 0)) +
-                 v2 * (hole ? yA : v * yA) + row23 + (seg & 1 ? drow : 0);
-    const T *B = reinterpret_cast<const T *>(B0 + (hole ? toHoleB : 0)) +
-                 (hole ? yB + o * y1 : v2 * (y1 + o * yB));
 #pragma unroll
     for (int i = 0; i < EA; ++i)
       if (i >= lo(part_) && i < lo(part_ + 1))
-        ra[i] = A[min(static_cast<int64_t>(kb + __builtin_amdgcn_readfirstlane(kA) + 4 * i),
-                       K - 1) * sA];
+        ra[i] = *reinterpret_cast<const T *>(A + min(kA + 4 * i, left - 1) * sA + rowA);
 #pragma unroll
     for (int i = 0; i < EB; ++i)
       if (EA + i >= lo(part_) && EA + i < lo(part_ + 1))
-        rb[i] = B[nB[i] * sN + min(static_cast<int64_t>(kb + kB[i]), K - 1) * sB];
+        rb[i] = *reinterpret_cast<const T *>(
+            B + (nB[i] + static_cast<uint32_t>(min(kB[i], left - 1)) *
+                             static_cast<uint32_t>(v * ES)));
   };
-  auto sign = [](double x, int mask) {
-    return __hiloint2double(__double2hiint(x) ^ mask, __double2loint(x));
-  };
-  // and to LDS: zero past K, - conj(V_hhhp)
+  // a part of stage s to LDS, zero past K
   auto store_part = [&](int s, int buf, auto part_c) {
     constexpr int part_ = decltype(part_c)::value;
-    int seg;
-    const int kb = segment(min(s, nstages - 1), seg);
-    const int left = static_cast<int>(v + (seg >= 2 ? holeK : 0)) - kb;
-    const int neg = seg >= 2 ? static_cast<int>(0x80000000u) : 0;
+    int d1, d2, d3;
+    const int kb = segment(s, d1, d2, d3);
+    const int within = static_cast<int>(v + ((o - v) & -static_cast<int64_t>(d2))) - kb;
 #pragma unroll
     for (int i = 0; i < EA; ++i)
-      if (i >= lo(part_) && i < lo(part_ + 1)) {
-        if (kA + 4 * i >= left) ra[i] = T{};
-        As[buf][kA + 4 * i][t % BM] = ra[i];
-      }
+      if (i >= lo(part_) && i < lo(part_ + 1))
+        As[buf][kA + 4 * i][t % BM] = kA + 4 * i < within ? ra[i] : T{};
 #pragma unroll
     for (int i = 0; i < EB; ++i)
-      if (EA + i >= lo(part_) && EA + i < lo(part_ + 1)) {
-        if (kB[i] >= left) rb[i] = T{};
-        if constexpr (CPLX)
-          rb[i].x = sign(rb[i].x, neg);
-        else
-          rb[i] = sign(rb[i], neg);
-        Bs[buf][kB[i]][(t + NT * i) % BN] = rb[i];
-      }
+      if (EA + i >= lo(part_) && EA + i < lo(part_ + 1))
+        Bs[buf][kB[i]][(t + NT * i) % BN] = kB[i] < within ? rb[i] : T{};
   };
 
   const int lane = t & 63, w = t >> 6, wm = w >> 1, wn = w & 1;
   // three products per complex one: re re, im im, (re + im)(re + im)
   dbl4 acc[CPLX ? 3 : 1][MB][NB];
-#pragma unroll
-  for (int c = 0; c < (CPLX ? 3 : 1); ++c)
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-      for (int j = 0; j < NB; ++j) acc[c][i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
   T fa[2][MB], fb[2][NB];
   auto load_frag = [&](int buf, int kq, auto q_c) {
     constexpr int q = decltype(q_c)::value;
@@ -260,15 +270,24 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void triples_product_kernel(Prod
   using I2 = std::integral_constant<int, 2>;
   using I3 = std::integral_constant<int, 3>;
   static_assert(PARTS == 3, "three parts, four k steps");
-  load_part(0, I0{}), load_part(0, I1{}), load_part(0, I2{});
+  Tile cur = locate(first);
+  load_from(cur);
+  begin_load(0);
+  load_part(I0{}), load_part(I1{}), load_part(I2{});
   store_part(0, 0, I0{}), store_part(0, 0, I1{}), store_part(0, 0, I2{});
-  load_part(1, I0{}), load_part(1, I1{}), load_part(1, I2{});
+  begin_load(1);
+  load_part(I0{}), load_part(I1{}), load_part(I2{});
   __syncthreads();
   load_frag(0, 0, I0{});
   // multiply LDS buffer s & 1, move stage s + 1 from the registers to the other
   // one and load stage s + 2, a part after each k step but the last; the barrier
   // stands before the last k step, whose fragments are in registers, so that the
-  // next stage's first are read under its MFMAs
+  // next stage's first are read under its MFMAs.  The stages of a run's tiles follow
+  // each other without a gap: a tile's first two are loaded under the last two of
+  // the tile before (one workgroup fits a CU, so nothing else would cover a tile's
+  // first loads: complex No=10, Nv=96 19.4 -> 18.3 ms, 0.2 of it by the streaming
+  // stores)
+  auto wrap = [&](int s) { return s - (nstages & -static_cast<int>(s >= nstages)); };
   auto step = [&](int s, auto par_c, auto kq_c) {
     constexpr int par = decltype(par_c)::value, kq = decltype(kq_c)::value;
     constexpr std::integral_constant<int, kq & 1> q;
@@ -282,46 +301,67 @@ __global__ __launch_bounds__(512, CPLX ? 2 : 4) void triples_product_kernel(Prod
     __builtin_amdgcn_sched_barrier(0);
     multiply(q);
     if constexpr (kq < PARTS) {
-      store_part(s + 1, par ^ 1, kq_c);
-      load_part(s + 2, kq_c);
+      store_part(wrap(s + 1), par ^ 1, kq_c);
+      if constexpr (kq == 0) begin_load(wrap(s + 2));
+      load_part(kq_c);
     }
   };
   auto stage = [&](int s, auto par) {
     step(s, par, I0{}), step(s, par, I1{}), step(s, par, I2{}), step(s, par, I3{});
   };
-  for (int s = 0; s < nstages; s += 2) {  // an even number
-    stage(s, I0{});
-    stage(s + 1, I1{});
-  }
-
-  // element (x1, x2, x3) of a part of its own, or of W[a, b, c]
-  int64_t s1 = 1, s2 = v, s3 = v * v;
-  T *Y = static_cast<T *>(p.Y) + batch * v * v * v;
-  if (p.parts == 1) {
-    s1 = part == 0 ? 1 : part == 1 ? v : v * v;
-    s2 = part == 0 ? v : 1;
-    s3 = part == 2 ? v : v * v;
-  }
+  for (int g = first; g < last; ++g) {
 #pragma unroll
-  for (int i = 0; i < MB; ++i)
+    for (int c = 0; c < (CPLX ? 3 : 1); ++c)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      int64_t x2, x3;
-      if (!row(wm * 32 + i * 16 + 4 * r + (lane >> 4), x2, x3)) continue;
-      T *out = Y + s2 * x2 + s3 * x3;
+      for (int i = 0; i < MB; ++i)
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        const int64_t x1 = n0 + wn * (BN / 2) + j * 16 + (lane & 15);
-        if (x1 >= v) continue;
-        T x;
-        if constexpr (CPLX)
-          x = make_double2(acc[0][i][j][r] - acc[1][i][j][r],
-                           acc[2][i][j][r] - (acc[0][i][j][r] + acc[1][i][j][r]));
-        else
-          x = acc[0][i][j][r];
-        out[s1 * x1] = p.add ? TS<CPLX>::plus(out[s1 * x1], x) : x;
+        for (int j = 0; j < NB; ++j) acc[c][i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+    Tile next = cur;
+    for (int s = 0; s < nstages; s += 2) {  // an even number
+      if (s + 2 == nstages) {               // past the last tile its own are loaded
+        next = locate(min(g + 1, last - 1));
+        load_from(next);
       }
+      stage(s, I0{});
+      stage(s + 1, I1{});
     }
+
+    // element (x1, x2, x3) of a part of its own, or of W[a, b, c]
+    int64_t s1 = 1, s2 = v, s3 = v2;
+    T *Y = static_cast<T *>(p.Y) + cur.batch * v2 * v;
+    if (p.parts == 1) {
+      s1 = cur.part == 0 ? 1 : cur.part == 1 ? v : v2;
+      s2 = cur.part == 0 ? v : 1;
+      s3 = cur.part == 2 ? v : v2;
+    }
+    const bool second = wm >= 2;  // the wave's rows lie in one block of 64
+    const int b2 = cur.x2 + (second ? cur.d2 : 0), b3 = cur.x3 + (second ? cur.d3 : 0);
+    if (!second || cur.two) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = wm * 32 + i * 16 + 4 * r + (lane >> 4);
+          const int x2 = b2 + (m & 7), x3 = b3 + ((m >> 3) & 7);
+          if (x2 >= v || x3 >= v) continue;
+          T *out = Y + s2 * x2 + s3 * x3;
+#pragma unroll
+          for (int j = 0; j < NB; ++j) {
+            const int64_t x1 = cur.n0 + wn * (BN / 2) + j * 16 + (lane & 15);
+            if (x1 >= v) continue;
+            T x;
+            if constexpr (CPLX)
+              x = make_double2(acc[0][i][j][r] - acc[1][i][j][r],
+                               acc[2][i][j][r] - (acc[0][i][j][r] + acc[1][i][j][r]));
+            else
+              x = acc[0][i][j][r];
+            if (p.add) x = TS<CPLX>::plus(out[s1 * x1], x);
+            store_stream(out + s1 * x1, x);
+          }
+        }
+    }
+    cur = next;
+  }
 }
 
 // The particle triples are taken in tiles of kTile^3 (a, b, c).  A block
@@ -489,29 +529,31 @@ int64_t triples_chunk(int64_t Nv, int64_t all, int64_t most, int parts) {
   return best;
 }
 
-void triples_product(hipStream_t s, Field f, const void *Vppph, const void *T2, const void *Vhhhp,
+void triples_product(hipStream_t s, Field f, const void *Vppph, const void *T2, const void *H,
                      void *Y, int64_t No, int64_t Nv, int64_t t0, int64_t count, int part) {
   CC4S_ASSERT(No > 0 && Nv > 0 && t0 >= 0 && count > 0 && part < 3 &&
                   t0 + count <= No * (No + 1) * (No + 2) / 6,
               "triples: hole triples out of range");
   const bool wide = tile_columns(Nv) == 96;
   const int64_t parts = part < 0 ? 3 : 1, tiles = tiles_of(Nv) * parts;
-  // launches of less than 2^32 threads
-  const int64_t per = ((int64_t(1) << 32) / 512 - 1) / tiles;
-  CC4S_ASSERT(per > 0, "triples: too many tiles for one launch");
+  const int64_t per = ((int64_t(1) << 31) - 1) / tiles;  // a launch counts tiles in 32 bits
+  CC4S_ASSERT(per > 0 && Nv < 16384, "triples: too many tiles for one launch");
   for (int64_t t = 0; t < count; t += per) {
     const int64_t n = std::min(per, count - t);
-    ProductArgs a{Vppph, T2, Vhhhp,
+    ProductArgs a{Vppph, T2, H,
                   static_cast<char *>(Y) + t * parts * Nv * Nv * Nv * scalar_bytes(f),
-                  No, Nv, t0 + t, tiles * n, static_cast<int>(parts), std::max(part, 0), part > 0};
-    auto run = [&](auto kernel) {
-      kernel<<<static_cast<unsigned>(a.blocks), 512, 0, s>>>(a);
+                  No, Nv, t0 + t, static_cast<int>(tiles * n), static_cast<int>(parts),
+                  std::max(part, 0), part > 0};
+    // as many workgroups as are resident at once: one per CU (complex) or two
+    auto run = [&](auto kernel, int grid) {
+      kernel<<<grid, 512, 0, s>>>(a);
       CC4S_HIP(hipGetLastError());
     };
     if (f == Field::Complex)
-      wide ? run(triples_product_kernel<true, 96>) : run(triples_product_kernel<true, 64>);
+      wide ? run(triples_product_kernel<true, 96>, 256) : run(triples_product_kernel<true, 64>, 256);
     else
-      wide ? run(triples_product_kernel<false, 96>) : run(triples_product_kernel<false, 64>);
+      wide ? run(triples_product_kernel<false, 96>, 512)
+           : run(triples_product_kernel<false, 64>, 512);
   }
 }
 

@@ -18,8 +18,8 @@ int64_t triples_chunk(int64_t Nv, int64_t all, int64_t most, int parts);
 // tetrahedral(k) + triangular(j) + i, i <= j <= k), in three parts that add up
 // (triples.hip): all of them, Y[x1,x2,x3,part,triple], or (part >= 0) one of them
 // in W[a,b,c,triple], written (0) or added (1, 2).  Dense operands V_ppph[b,c,d,k],
-// T2[a,b,i,j], V_hhhp[i,j,l,a].
-void triples_product(hipStream_t s, Field f, const void *Vppph, const void *T2, const void *Vhhhp,
+// T2[a,b,i,j], H[a,l,j,i] = -conj(V_ijla).
+void triples_product(hipStream_t s, Field f, const void *Vppph, const void *T2, const void *H,
                      void *Y, int64_t No, int64_t Nv, int64_t t0, int64_t count, int part);
 
 // acc[block] += partial sums of the weighted Re(W Zs)/D over those hole triples;
