@@ -1674,10 +1674,15 @@ void ContractionEngine::contract_mixed(GettPlan &P, double alpha, const View &A,
       cache_eb_[slot] = eb;
     }
   }
-  if (mixed_half && !cacheA)
+  auto known = [&](const View &v) { return !nine && max_ptr_ && v.ptr == max_ptr_; };
+  if (mixed_half && !cacheA && known(Aop))
+    launch_split_scale_of(maxima_, max_count_, scA, stream_);
+  else if (mixed_half && !cacheA)
     launch_split_scale(static_cast<const double *>(Aop.ptr), P.rowA, P.colA, P.M, P.K,
                        P.a_kc, nine, scPart, scA, stream_);
-  if (mixed_half && !cacheB)
+  if (mixed_half && !cacheB && known(Bop))
+    launch_split_scale_of(maxima_, max_count_, scB, stream_);
+  else if (mixed_half && !cacheB)
     launch_split_scale(static_cast<const double *>(Bop.ptr), P.colB, P.rowB, P.N, P.K,
                        P.b_kc, nine, scPart, scB, stream_);
   const double *useScA = mixed_half ? (cacheA ? scC : scA) : nullptr;

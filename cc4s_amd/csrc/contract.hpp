@@ -112,6 +112,13 @@ class ContractionEngine {
   // split parts in IEEE half with per-operand power-of-two scaling (about
   // 22 significant bits per real part) instead of bf16 (about 16)
   bool mixed_half = false;
+  // The next contraction's operand at `ptr` has its largest |Re|, |Im| already, in
+  // `count` parts: a split contraction then does not read it for its scale (null: none)
+  void set_operand_max(const void *ptr, const double *maxima, int count) {
+    max_ptr_ = ptr;
+    maxima_ = maxima;
+    max_count_ = count;
+  }
   // 16-bit products per complex multiply-add of the split kernel: 12 (the
   // hi*hi, hi*lo and lo*hi products of both real parts) or 16 (also lo*lo,
   // which lies 2^-22 below the product, under the FP32 sums' rounding), or,
@@ -149,6 +156,9 @@ class ContractionEngine {
  private:
   GettPlan &plan_for(const View &A, const View &B, const View &C, const View *D = nullptr);
   void launch_group();
+  const void *max_ptr_ = nullptr;
+  const double *maxima_ = nullptr;
+  int max_count_ = 0;
   bool grouping_ = false;
   std::vector<GettLaunch> group_;
   // result elements times splits up to which a contraction joins a group: larger
@@ -232,6 +242,8 @@ void launch_pack(const double *X, const int64_t *offMN, const int64_t *offK,
 void launch_split_scale(const double *X, const int64_t *offMN, const int64_t *offK,
                         int64_t MN, int64_t K, bool kcontig, bool sumabs,
                         double *partials, double *scale, hipStream_t s);
+// the same from `count` parts of the maximum
+void launch_split_scale_of(const double *maxima, int count, double *scale, hipStream_t s);
 size_t split_scale_partials_bytes();
 // C = alpha * sum_s W[s] / (scaleA[0] scaleB[0]) + beta * C over the FP32
 // partials of launch_bgemm (scales null: bf16 parts, no scaling)

@@ -35,14 +35,16 @@ double ladder_fused(const View &left, const View &right, const View &tau,
 //   ladder_tau_pairs:    tau [c,d,i,j] dense -> tau+ [Kp][Np] (its c = d
 //                        elements times `diag`), tau- [Km][Nm]
 //   ladder_vertex_pairs: slab [c,x,d,y] dense (v, cx, v, Ny) -> Vp [Kp][x][y],
-//                        Vm [Km][x][y]
+//                        Vm [Km][x][y]; `maxima` (or null) takes the largest
+//                        |Re| and |Im| of Vp in kLadderMaxima parts, and of Vm
 //   ladder_unpack_pairs: Rp [xy][Np], Rm [xy][Nm] -> R [xy][i][j]
 // with Kp = v(v+1)/2, Km = v(v-1)/2, Np = o(o+1)/2, Nm = o(o-1)/2, k or xy
 // fastest.
 void ladder_tau_pairs(Field f, const void *tau, void *Tp, void *Tm, double diag, int64_t v,
                       int64_t o, hipStream_t s);
+constexpr int kLadderMaxima = 64;
 void ladder_vertex_pairs(const void *slab, void *Vp, void *Vm, int64_t v, int64_t cx,
-                         int64_t Ny, hipStream_t s);
+                         int64_t Ny, double *maxima, hipStream_t s);
 void ladder_unpack_pairs(const void *Rp, const void *Rm, void *R, int64_t nxy, int64_t o,
                          hipStream_t s);
 

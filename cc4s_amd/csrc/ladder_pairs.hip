@@ -113,7 +113,8 @@ constexpr int kT = 32;  // (c, d) tile of the vertex fold
 // grid (tiles, cx * Ny)
 __global__ __launch_bounds__(256) void vertex_pairs_kernel(const double2 *slab, double2 *Vp,
                                                            double2 *Vm, int64_t v, int64_t cx,
-                                                           int64_t Kp, int64_t Km) {
+                                                           int64_t Kp, int64_t Km,
+                                                           unsigned long long *maxima) {
   __shared__ double2 t1[kT][kT + 1];  // [d][c]: V_xycd
   __shared__ double2 t2[kT][kT + 1];  // [c][d]: V_xydc
   int64_t cb, db;
@@ -135,6 +136,8 @@ __global__ __launch_bounds__(256) void vertex_pairs_kernel(const double2 *slab, 
   }
   __syncthreads();
   const int64_t ox = xy;  // (x, y) column of Vp / Vm
+  double mp = 0.0, mm = 0.0;
+  auto larger = [](double m, double2 z) { return fmax(m, fmax(fabs(z.x), fabs(z.y))); };
   for (int e = t; e < kT * kT; e += 256) {
     const int a = e % kT, b = e / kT;
     const int64_t c = c0 + a, d = d0 + b;
@@ -142,11 +145,24 @@ __global__ __launch_bounds__(256) void vertex_pairs_kernel(const double2 *slab, 
     const double2 vcd = t1[b][a];
     if (c == d) {
       Vp[c + d * (d + 1) / 2 + Kp * ox] = vcd;
+      mp = larger(mp, vcd);
     } else {
-      const double2 vdc = t2[a][b];
-      Vp[c + d * (d + 1) / 2 + Kp * ox] = add2(vcd, vdc);
-      Vm[c + d * (d - 1) / 2 + Km * ox] = sub2(vcd, vdc);
+      const double2 vdc = t2[a][b], p = add2(vcd, vdc), m = sub2(vcd, vdc);
+      Vp[c + d * (d + 1) / 2 + Kp * ox] = p;
+      Vm[c + d * (d - 1) / 2 + Km * ox] = m;
+      mp = larger(mp, p);
+      mm = larger(mm, m);
     }
+  }
+  if (!maxima) return;
+  // magnitudes order as their bits do
+  mp = wave_max(mp);
+  mm = wave_max(mm);
+  if ((t & 63) == 0) {
+    const int slot = (blockIdx.x + gridDim.x * blockIdx.y) % kLadderMaxima;
+    atomicMax(maxima + slot, static_cast<unsigned long long>(__double_as_longlong(mp)));
+    atomicMax(maxima + kLadderMaxima + slot,
+              static_cast<unsigned long long>(__double_as_longlong(mm)));
   }
 }
 
@@ -365,14 +381,16 @@ void resident_unpack(Field f, const void *Rp, const void *Rm, void *R2, void *Q,
 }
 
 void ladder_vertex_pairs(const void *slab, void *Vp, void *Vm, int64_t v, int64_t cx,
-                         int64_t Ny, hipStream_t s) {
+                         int64_t Ny, double *maxima, hipStream_t s) {
   const int64_t Kp = v * (v + 1) / 2, Km = v * (v - 1) / 2;
   const int64_t nb = (v + kT - 1) / kT;
+  if (maxima) CC4S_HIP(hipMemsetAsync(maxima, 0, 2 * kLadderMaxima * sizeof(double), s));
   CC4S_ASSERT(cx * Ny < 65536, "paired ladder: slab chunk out of range");
   const dim3 grid(static_cast<unsigned>(nb * (nb + 1) / 2), static_cast<unsigned>(cx * Ny));
   vertex_pairs_kernel<<<grid, 256, 0, s>>>(static_cast<const double2 *>(slab),
                                            static_cast<double2 *>(Vp),
-                                           static_cast<double2 *>(Vm), v, cx, Kp, Km);
+                                           static_cast<double2 *>(Vm), v, cx, Kp, Km,
+                                           reinterpret_cast<unsigned long long *>(maxima));
   CC4S_HIP(hipGetLastError());
 }
 

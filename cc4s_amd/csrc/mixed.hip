@@ -789,6 +789,11 @@ void launch_split_scale(const double *X, const int64_t *offMN, const int64_t *of
   CC4S_HIP(hipGetLastError());
 }
 
+void launch_split_scale_of(const double *maxima, int count, double *scale, hipStream_t s) {
+  scale_kernel<<<1, 256, 0, s>>>(maxima, count, scale);
+  CC4S_HIP(hipGetLastError());
+}
+
 size_t split_scale_partials_bytes() { return kMaxBlocks * sizeof(double); }
 
 void launch_split_reduce(const void *W, double *C, const int64_t *rowC,
