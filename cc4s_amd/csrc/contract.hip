@@ -324,9 +324,11 @@ __global__ __launch_bounds__(kThreads, 2) void gett_kernel(KArgs p) {
 // past K are zeroed in their one stage only, 35 vector instructions per stage
 // and wave of 32 x 32 instead of 82; and LDS reads and stores waited for in
 // place (fragments one k step ahead, no branch around the stores).  Measured
-// before -> after: complex ring (8192^3) 55.2 -> 51.9 ms, 85 TFLOP/s of 8 flops
-// per complex MAC; real ring (7533^3), which ran on a single-buffered kernel
-// with loads under branches, 19.8 -> 15.6 ms (55 TFLOP/s).
+// before -> after: complex ring (8192^3) 55.2 -> 51.9 ms; real ring (7533^3), which
+// ran on a single-buffered kernel with loads under branches, 19.8 -> 15.6 ms.
+// With memory instructions spread over a stage and K offsets by lane (below)
+// 7533^3 takes 39.5 ms complex (86 TFLOP/s of 8 flops per complex MAC) and 13.1
+// real (65).
 //
 // M3 selects the three-product complex multiply (Gauss/Karatsuba):
 //   P1 = ar br, P2 = ai bi, P3 = (ar + ai)(br + bi),
@@ -335,11 +337,6 @@ __global__ __launch_bounds__(kThreads, 2) void gett_kernel(KArgs p) {
 // the four-product one with |ar|+|ai| and |br|+|bi| in place of |a|, |b|.
 constexpr int kZThreads = 512;
 
-// DEEP keeps two stages of global loads in flight (two register sets): the
-// loads for stage s+3 are issued while stage s is multiplied.  MINW is the
-// launch bound's minimum of waves per SIMD (2 with 256 threads: two
-// workgroups share a CU, so one's prologue and epilogue overlap the other's
-// multiplies).
 template <bool CPLX>
 using Scalar = std::conditional_t<CPLX, double2, double>;
 // elements past the end of an LDS row.  Complex: one shifts consecutive k-rows by
@@ -351,7 +348,12 @@ using Scalar = std::conditional_t<CPLX, double2, double>;
 template <bool CPLX>
 constexpr int kRowPad = CPLX ? 1 : 18;
 
-// one workgroup: block `block` of the tiles (and tail parts), part `slice` of K
+// One workgroup: block `block` of the tiles (and tail parts), part `slice` of K.
+// DEEP keeps two stages of global loads in flight (two register sets): the
+// loads for stage s+3 are issued while stage s is multiplied.  MINW (below) is
+// the launch bound's minimum of waves per SIMD (2 with 256 threads: two
+// workgroups share a CU, so one's prologue and epilogue overlap the other's
+// multiplies).
 template <bool CPLX, int NT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC,
           bool M3, bool DEEP>
 __device__ __forceinline__ void gett_tile(
@@ -422,10 +424,10 @@ __device__ __forceinline__ void gett_tile(
   // the offset of the wave's element i (A's, then B's), one load and two registers
   // instead of one and two per element, and the loads take it through scalar
   // registers (real 7533^3, both operands so: 14.5 -> 13.1 ms; complex 40.1 ->
-  // 39.7, 720^3 66 -> 64 us).  The K tables are padded with
-  // a valid offset (kTablePad entries past whole stages), so neither these loads
-  // nor the operand loads they address need a bound; what lies past K is zeroed
-  // when it is stored to LDS, in the one stage that holds K's end
+  // 39.7, 720^3 66 -> 64 us).  The K tables are padded with a valid offset
+  // (kTablePad entries past whole stages), so neither these loads nor the operand
+  // loads they address need a bound; what lies past K is zeroed when it is stored
+  // to LDS, in the one stage that holds K's end
   constexpr bool UA = !AKC && BM % 64 == 0, UB = !BKC && BN % 64 == 0;
   constexpr int LA = UA ? EA : 0, LANES = LA + (UB ? EB : 0);
   static_assert(LANES <= 64, "one lane per element");
