@@ -18,6 +18,7 @@ CSRC = HERE / "csrc"
 OBJ = HERE / "_build"
 LIB = HERE / "libcc4s_ccsd.so"
 BENCH = HERE / "gett_bench"
+CHECK = HERE / "native_check"
 DRIVER = HERE / "cc4s_ccsd"
 DRIVER_SOURCES = ["main.cpp", "yaml.cpp", "tensor_io.cpp"]
 SOURCES = ["contract.hip", "mixed.hip", "elementwise.hip", "adjoint.hip", "triples.hip", "ccsd.hip",
@@ -70,6 +71,16 @@ def build(jobs: int = 8, verbose: bool = True) -> pathlib.Path:
         raise RuntimeError(f"benchmark build failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
     if verbose:
         print(f"built {BENCH}")
+    # test program that defines some of the runtime's functions: its symbols stand
+    # before the runtime's for the library too
+    cmd = [HIPCC, *COMMON, "-x", "hip", str(ROOT / "tests" / "native" / "native_check.cpp"),
+           "-o", str(CHECK), f"-L{HERE}", "-lcc4s_ccsd", "-ldl", "-rdynamic",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"test program build failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    if verbose:
+        print(f"built {CHECK}")
     # host drop-in driver for cc4s operation files (host C++ over the C ABI)
     drv = CSRC / "driver"
     cmd = [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-Wall",

@@ -273,24 +273,24 @@ void Ccsd::ladder(const View &left, const View &right, const View &tauv,
           // finds as it writes (No=24, Nv=192: 83 us of reading per slab less, 14 more
           // in the fold; a residuum 97.8 -> 96.0 ms)
           double *maxima = nullptr;
-          if (E_.mixed()) {
+          if (E_.uses_operand_max()) {
             w.maxima.reserve(2 * kLadderMaxima * sizeof(double));
             maxima = w.maxima.as<double>();
           }
           ladder_vertex_pairs(slab.ptr, Vp, Vm, v, cx, Ny, maxima, E_.stream());
           const double fl0 = E_.stats.flops;
-          if (maxima) E_.set_operand_max(Vp, maxima, kLadderMaxima);
+          const OperandMax maxp{maxima, kLadderMaxima},
+              maxm{maxima ? maxima + kLadderMaxima : nullptr, kLadderMaxima};
           E_.contract(1.0, dense_view(Vp, f, "kxy", {Kp, cx, Ny}),
                       dense_view(Tp, f, "kn", {Kp, Np}), 0.0,
-                      dense_view(Rp, f, "xyn", {cx, Ny, Np}));
+                      dense_view(Rp, f, "xyn", {cx, Ny, Np}), nullptr, maxima ? &maxp : nullptr);
           const View RmV = dense_view(Rm, f, "xyn", {cx, Ny, Nm});
-          if (maxima) E_.set_operand_max(Vm, maxima + kLadderMaxima, kLadderMaxima);
           if (Nm > 0 && Km > 0)
             E_.contract(1.0, dense_view(Vm, f, "kxy", {Km, cx, Ny}),
-                        dense_view(Tm, f, "kn", {Km, Nm}), 0.0, RmV);
+                        dense_view(Tm, f, "kn", {Km, Nm}), 0.0, RmV, nullptr,
+                        maxima ? &maxm : nullptr);
           else if (Nm > 0)
             E_.scale(0.0, RmV);
-          E_.set_operand_max(nullptr, nullptr, 0);
           // credited as the slab contraction it replaces (8 flops per complex
           // MAC over Nv^2 k and No^2 columns), the convention of the others
           E_.stats.flops = fl0 + 8.0 * static_cast<double>(cx * Ny) * v * v * o * o;

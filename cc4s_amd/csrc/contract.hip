@@ -1506,7 +1506,8 @@ void *ContractionEngine::reserve_partials(const GettPlan &P, Field f) {
 }
 
 void ContractionEngine::contract(double alpha, const View &A, const View &B,
-                                 double beta, const View &C, const View *D) {
+                                 double beta, const View &C, const View *D,
+                                 const OperandMax *maxA) {
   CC4S_ASSERT(A.field == C.field && B.field == C.field, "mixed scalar fields");
   CC4S_ASSERT(!C.conj, "conjugated result view");
   CC4S_ASSERT(!D || (D->field == C.field && !mixed_), "added tensor in a split pass");
@@ -1540,7 +1541,7 @@ void ContractionEngine::contract(double alpha, const View &A, const View &B,
   const double flops = (C.field == Field::Complex ? 8.0 : 2.0) * double(P.M) *
                        double(P.N) * double(P.K);
   if (mixed_ && C.field == Field::Complex && flops >= mixed_min_flops) {
-    contract_mixed(P, alpha, A, B, beta, C, flops);
+    contract_mixed(P, alpha, A, B, beta, C, flops, maxA);
     stats.flops += flops;
     stats.launches += 1;
     return;
@@ -1619,7 +1620,7 @@ void ContractionEngine::launch_group() {
 
 void ContractionEngine::contract_mixed(GettPlan &P, double alpha, const View &A,
                                        const View &B, double beta, const View &C,
-                                       double flops) {
+                                       double flops, const OperandMax *maxA) {
   // 9 products per complex MAC: half parts plus a third plane of Re + Im
   const bool nine = mixed_half && mixed_terms == 9;
   const int terms = mixed_terms == 9 && !mixed_half ? 12 : mixed_terms;
@@ -1676,14 +1677,14 @@ void ContractionEngine::contract_mixed(GettPlan &P, double alpha, const View &A,
       cache_eb_[slot] = eb;
     }
   }
-  auto known = [&](const View &v) { return !nine && max_ptr_ && v.ptr == max_ptr_; };
-  if (mixed_half && !cacheA && known(Aop))
-    launch_split_scale_of(maxima_, max_count_, scA, stream_);
+  const OperandMax *known = uses_operand_max() ? maxA : nullptr;  // of A, Bop where P.swap
+  if (mixed_half && !cacheA && known && !P.swap)
+    launch_split_scale_of(known->parts, known->count, scA, stream_);
   else if (mixed_half && !cacheA)
     launch_split_scale(static_cast<const double *>(Aop.ptr), P.rowA, P.colA, P.M, P.K,
                        P.a_kc, nine, scPart, scA, stream_);
-  if (mixed_half && !cacheB && known(Bop))
-    launch_split_scale_of(maxima_, max_count_, scB, stream_);
+  if (mixed_half && !cacheB && known && P.swap)
+    launch_split_scale_of(known->parts, known->count, scB, stream_);
   else if (mixed_half && !cacheB)
     launch_split_scale(static_cast<const double *>(Bop.ptr), P.colB, P.rowB, P.N, P.K,
                        P.b_kc, nine, scPart, scB, stream_);

@@ -57,6 +57,12 @@ struct GettLaunch {
 };
 struct OffsetTable;  // of a plan
 
+// largest |Re| and |Im| of an operand, in parts (device memory)
+struct OperandMax {
+  const double *parts;
+  int count;
+};
+
 class ContractionEngine {
  public:
   explicit ContractionEngine(hipStream_t s);
@@ -64,9 +70,11 @@ class ContractionEngine {
 
   // C = alpha * op(A) op(B) + beta * op(D), op = conjugation where the view says;
   // without D, D is C (FP64 passes may name another tensor of C's indices, whose
-  // copy into C it saves)
+  // copy into C it saves).  `maxA` (or null) holds A's largest |Re| and |Im|, found
+  // by whoever wrote A: a contraction that uses_operand_max() does not read A for
+  // its scale then
   void contract(double alpha, const View &A, const View &B, double beta,
-                const View &C, const View *D = nullptr);
+                const View &C, const View *D = nullptr, const OperandMax *maxA = nullptr);
   // `statements` contracts in any order: those contractions with small results
   // run in one launch (and one for their split-K reductions) after the others
   template <class Statements>
@@ -112,19 +120,15 @@ class ContractionEngine {
   // split parts in IEEE half with per-operand power-of-two scaling (about
   // 22 significant bits per real part) instead of bf16 (about 16)
   bool mixed_half = false;
-  // The next contraction's operand at `ptr` has its largest |Re|, |Im| already, in
-  // `count` parts: a split contraction then does not read it for its scale (null: none)
-  void set_operand_max(const void *ptr, const double *maxima, int count) {
-    max_ptr_ = ptr;
-    maxima_ = maxima;
-    max_count_ = count;
-  }
   // 16-bit products per complex multiply-add of the split kernel: 12 (the
   // hi*hi, hi*lo and lo*hi products of both real parts) or 16 (also lo*lo,
   // which lies 2^-22 below the product, under the FP32 sums' rounding), or,
   // with half parts, 9 (three real products per complex multiply-add: Re Re,
   // Im Im and (Re + Im)(Re + Im), each split in three)
   int mixed_terms = 12;
+  // whether contractions scale their operands by the largest |Re| and |Im| (the
+  // 9-product form scales by |Re| + |Im|, bf16 parts not at all)
+  bool uses_operand_max() const { return mixed_ && mixed_half && mixed_terms != 9; }
   // CC4S_MIXED_SPLIT, CC4S_MIXED_MAX_K, CC4S_MIXED_TERMS and
   // CC4S_GETT_GENERATION, when set, replace the settings above and the
   // complex kernel generation
@@ -156,9 +160,6 @@ class ContractionEngine {
  private:
   GettPlan &plan_for(const View &A, const View &B, const View &C, const View *D = nullptr);
   void launch_group();
-  const void *max_ptr_ = nullptr;
-  const double *maxima_ = nullptr;
-  int max_count_ = 0;
   bool grouping_ = false;
   std::vector<GettLaunch> group_;
   // result elements times splits up to which a contraction joins a group: larger
@@ -166,7 +167,7 @@ class ContractionEngine {
   static constexpr int64_t kGroupElements = int64_t(1) << 20;
   void *reserve_partials(const GettPlan &P, Field f);
   void contract_mixed(GettPlan &P, double alpha, const View &A, const View &B,
-                      double beta, const View &C, double flops);
+                      double beta, const View &C, double flops, const OperandMax *maxA);
   bool mixed_ = false;
   DeviceBuffer pack_;
   DeviceBuffer cache_[kCacheSlots];

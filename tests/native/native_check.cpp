@@ -1,0 +1,249 @@
+// Checks of the library that need control over the runtime's allocations and
+// copies: this program defines hipMalloc and a few other functions itself, so that
+// the library's calls come here first, can be counted, and can be made to fail on
+// the host as they do when the device is full.  Nothing is launched that the
+// library would not launch.
+//
+//   native_check SCENARIO
+//
+// prints its steps and, if every one holds, "ok SCENARIO" (status 0).
+#include "cc4s_ccsd.h"
+
+#include <dlfcn.h>
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <complex>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <mutex>
+#include <random>
+#include <string>
+#include <utility>
+#include <vector>
+
+// ---------------------------------------------------------------------------
+// the runtime's functions
+// ---------------------------------------------------------------------------
+
+namespace {
+std::mutex g_lock;
+std::map<void *, size_t> g_sizes;
+size_t g_held = 0;           // bytes of device memory
+size_t g_total = 0;          // bytes the device has; 0: what it really has
+long g_fail_at = 0;          // the allocation that fails, counted from arm(); 0: none
+long g_count = 0;
+bool g_failed = false;
+
+template <typename F>
+F real(const char *name) {
+  return reinterpret_cast<F>(dlsym(RTLD_NEXT, name));
+}
+
+void arm(long fail_at) {
+  std::lock_guard<std::mutex> l(g_lock);
+  g_fail_at = fail_at;
+  g_count = 0;
+  g_failed = false;
+}
+size_t held() {
+  std::lock_guard<std::mutex> l(g_lock);
+  return g_held;
+}
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t bytes) {
+  static const auto f = real<hipError_t (*)(void **, size_t)>("hipMalloc");
+  {
+    std::lock_guard<std::mutex> l(g_lock);
+    ++g_count;
+    if ((g_fail_at && g_count == g_fail_at) || (g_total && g_held + bytes > g_total)) {
+      g_failed = true;
+      *p = nullptr;
+      return hipErrorOutOfMemory;
+    }
+  }
+  const hipError_t e = f(p, bytes);
+  if (e == hipSuccess) {
+    std::lock_guard<std::mutex> l(g_lock);
+    g_sizes[*p] = bytes;
+    g_held += bytes;
+  }
+  return e;
+}
+hipError_t hipFree(void *p) {
+  static const auto f = real<hipError_t (*)(void *)>("hipFree");
+  const hipError_t e = f(p);
+  std::lock_guard<std::mutex> l(g_lock);
+  auto it = g_sizes.find(p);
+  if (it != g_sizes.end()) {
+    g_held -= it->second;
+    g_sizes.erase(it);
+  }
+  return e;
+}
+hipError_t hipMemGetInfo(size_t *free_bytes, size_t *total_bytes) {
+  static const auto f = real<hipError_t (*)(size_t *, size_t *)>("hipMemGetInfo");
+  std::lock_guard<std::mutex> l(g_lock);
+  if (!g_total) return f(free_bytes, total_bytes);
+  *free_bytes = g_total > g_held ? g_total - g_held : 0;
+  *total_bytes = g_total;
+  return hipSuccess;
+}
+}
+
+namespace {
+
+// ---------------------------------------------------------------------------
+// problems
+// ---------------------------------------------------------------------------
+
+#define CHECK(cond)                                                        \
+  do {                                                                     \
+    if (!(cond)) {                                                         \
+      std::printf("FAILED %s:%d %s\n", __FILE__, __LINE__, #cond);         \
+      std::fflush(stdout);                                                 \
+      std::exit(1);                                                        \
+    }                                                                      \
+  } while (0)
+
+void step(const std::string &what) {
+  std::printf("%s\n", what.c_str());
+  std::fflush(stdout);
+}
+
+struct Problem {
+  bool cplx;
+  int64_t o, v, G;
+  std::vector<double> gamma, eps, T1, T2;  // complex interleaved where complex
+  int es() const { return cplx ? 2 : 1; }
+  size_t n1() const { return size_t(o) * v * es(); }
+  size_t n2() const { return size_t(o) * o * v * v * es(); }
+};
+
+// a Hermitian (real field: symmetric) vertex and amplitudes with T_abij = T_baji,
+// both exactly
+Problem problem(bool cplx, int64_t o, int64_t v, int64_t G, unsigned seed) {
+  Problem p{cplx, o, v, G, {}, {}, {}, {}};
+  const int64_t n = o + v;
+  std::mt19937_64 rng(seed);
+  std::normal_distribution<double> d;
+  p.gamma.assign(2 * G * n * n, 0.0);
+  for (int64_t q = 0; q < n; ++q)
+    for (int64_t r = 0; r <= q; ++r)
+      for (int64_t g = 0; g < G; ++g) {
+        const double re = 0.1 * d(rng) / std::sqrt(double(G)), im = 0.1 * d(rng) / std::sqrt(double(G));
+        double *x = &p.gamma[2 * (g + G * (q + n * r))], *y = &p.gamma[2 * (g + G * (r + n * q))];
+        x[0] = y[0] = re;
+        x[1] = q == r && cplx ? 0.0 : im;
+        y[1] = cplx ? -x[1] : x[1];
+      }
+  for (int64_t q = 0; q < n; ++q) p.eps.push_back(q < o ? -1.0 - 0.1 * q : 0.5 + 0.05 * q);
+  for (size_t k = 0; k < p.n1(); ++k) p.T1.push_back(0.05 * d(rng));
+  p.T2.assign(p.n2(), 0.0);
+  const int es = p.es();
+  for (int64_t a = 0; a < v; ++a)
+    for (int64_t b = 0; b < v; ++b)
+      for (int64_t i = 0; i < o; ++i)
+        for (int64_t j = 0; j < o; ++j)
+          for (int c = 0; c < es; ++c) {
+            double &x = p.T2[es * (a + v * (b + v * (i + o * j))) + c];
+            double &y = p.T2[es * (b + v * (a + v * (j + o * i))) + c];
+            if (a + v * i <= b + v * j) x = y = 0.05 * d(rng);
+          }
+  return p;
+}
+
+struct Context {
+  cc4s_ccsd_context *c = nullptr;
+  Context(const Problem &p, const std::function<void(cc4s_ccsd_params &)> &set = {}) {
+    cc4s_ccsd_params q;
+    cc4s_ccsd_default_params(&q);
+    q.field = p.cplx ? CC4S_FIELD_COMPLEX : CC4S_FIELD_REAL;
+    q.No = p.o;
+    q.Nv = p.v;
+    q.NG = p.G;
+    if (set) set(q);
+    CHECK(cc4s_ccsd_create(&q, &c) == 0);
+  }
+  ~Context() { cc4s_ccsd_destroy(c); }
+  operator cc4s_ccsd_context *() const { return c; }
+};
+
+using Out = std::pair<std::vector<double>, std::vector<double>>;  // R1, R2
+
+int residuum(cc4s_ccsd_context *c, const Problem &p, Out &r) {
+  r.first.assign(p.n1(), 0.0);
+  r.second.assign(p.n2(), 0.0);
+  return cc4s_ccsd_residuum(c, p.T1.data(), p.T2.data(), r.first.data(), r.second.data());
+}
+double rel(const std::vector<double> &a, const std::vector<double> &b) {
+  double d = 0, m = 0;
+  for (size_t k = 0; k < a.size(); ++k) {
+    if (!std::isfinite(a[k])) return HUGE_VAL;
+    d = std::max(d, std::fabs(a[k] - b[k]));
+    m = std::max(m, std::fabs(b[k]));
+  }
+  return d / m;
+}
+
+// several slices of the ladder, the last one short
+Problem mixed_problem() { return problem(true, 5, 23, 40, 3); }
+void mixed(cc4s_ccsd_params &q) { q.precision = CC4S_PRECISION_MIXED; }
+
+// ---------------------------------------------------------------------------
+// scenarios
+// ---------------------------------------------------------------------------
+
+// A split residuum in which one allocation after the other fails leaves nothing
+// behind: the next one on the same context is that of a fresh context, bit for bit.
+void failed_split_pass() {
+  setenv("CC4S_MIXED_MIN_FLOPS", "0", 1);  // every contraction is split
+  const Problem p = mixed_problem();
+  Problem other = p;  // what the failing pass is given: large dressed vertices
+  for (double &x : other.T1) x *= 1e3;
+  Out ref, r;
+  {
+    Context c(p, mixed);
+    CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+    CHECK(residuum(c, p, ref) == 0);
+  }
+  long n = 0;
+  for (bool failed = true; failed;) {
+    Context c(p, mixed);
+    CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+    arm(++n);
+    const int rc = residuum(c, other, r);
+    failed = g_failed;
+    arm(0);
+    if (!failed) break;
+    step("allocation " + std::to_string(n) + (rc ? ": " : " passed over") +
+         (rc ? cc4s_ccsd_last_error(c) : ""));
+    CHECK(residuum(c, p, r) == 0);
+    CHECK(r.first == ref.first && r.second == ref.second);
+  }
+  CHECK(n > 10);
+}
+
+const std::map<std::string, void (*)()> kScenarios = {
+    {"failed_split_pass", failed_split_pass},
+};
+
+}  // namespace
+
+int main(int argc, char **argv) {
+  const auto it = kScenarios.find(argc > 1 ? argv[1] : "");
+  if (it == kScenarios.end()) {
+    for (const auto &s : kScenarios) std::printf("%s\n", s.first.c_str());
+    return 2;
+  }
+  it->second();
+  std::printf("ok %s\n", argv[1]);
+  return 0;
+}

@@ -1,0 +1,19 @@
+"""Checks that need control over the runtime's allocations and copies, in a program
+that stands between the library and the HIP runtime (tests/native/native_check.cpp):
+what a call leaves behind when device memory runs out under it."""
+
+import pathlib
+import subprocess
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+PROGRAM = pathlib.Path(__file__).resolve().parent.parent / "cc4s_amd" / "native_check"
+
+
+@pytest.mark.parametrize("scenario", ["failed_split_pass"])
+def test_native(scenario):
+    print(f"native {scenario}", flush=True)
+    r = subprocess.run([str(PROGRAM), scenario], capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0 and f"ok {scenario}" in r.stdout, r.stdout[-4000:] + r.stderr[-2000:]
