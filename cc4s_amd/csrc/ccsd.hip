@@ -241,6 +241,7 @@ void Ccsd::ladder(const View &left, const View &right, const View &tauv,
   }
   // tau (or its two combinations) is read unchanged by every slab
   // contraction: in split mode it is packed once for all of them
+  const OperandCacheScope cached(E_);
   if (E_.mixed() && paired) {
     E_.set_operand_cache(Tp, 0, "kn");
     E_.set_operand_cache(Tm, 2, "kn");
@@ -307,7 +308,6 @@ void Ccsd::ladder(const View &left, const View &right, const View &tauv,
       }
     }
   }
-  E_.clear_operand_cache();
   if (profile) {
     CC4S_HIP(hipEventRecord(e1, E_.stream()));
     CC4S_HIP(hipEventSynchronize(e1));

@@ -1656,6 +1656,7 @@ void ContractionEngine::contract_mixed(GettPlan &P, double alpha, const View &A,
   if (cacheA || cacheB) {
     const int64_t rows = cacheA ? Mp : Np;
     if (cache_plan_[slot] != &P || cache_is_a_[slot] != cacheA || cache_eb_[slot] != eb) {
+      cache_plan_[slot] = nullptr;  // not that plan's operand any more
       cache_[slot].reserve(static_cast<size_t>(rows) * Kfull * eb);
       char *cs = nine ? cache_[slot].as<char>() + static_cast<size_t>(rows) * Kfull * 8
                       : nullptr;

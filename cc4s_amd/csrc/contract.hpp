@@ -197,6 +197,29 @@ class ContractionEngine {
   DeviceBuffer workspace_;
 };
 
+// Split contractions in a scope, and packed operands kept in one: both are state of
+// the engine that other calls on it must not meet, also after an exception.
+class SplitScope {
+ public:
+  SplitScope(ContractionEngine &E, bool on) : E_(E) { E_.set_mixed(on); }
+  ~SplitScope() { E_.set_mixed(false); }
+  SplitScope(const SplitScope &) = delete;
+  SplitScope &operator=(const SplitScope &) = delete;
+
+ private:
+  ContractionEngine &E_;
+};
+class OperandCacheScope {
+ public:
+  explicit OperandCacheScope(ContractionEngine &E) : E_(E) {}
+  ~OperandCacheScope() { E_.clear_operand_cache(); }
+  OperandCacheScope(const OperandCacheScope &) = delete;
+  OperandCacheScope &operator=(const OperandCacheScope &) = delete;
+
+ private:
+  ContractionEngine &E_;
+};
+
 // `start`/`stop` (optional) bracket the main kernel, not the reduction
 void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start = nullptr,
                  hipEvent_t stop = nullptr);

@@ -450,9 +450,10 @@ IterationReport CoupledCluster::iterate() {
     // pair); the pass itself continues with R64 and a DIIS history that
     // holds no split residua
     defect_.reserve(packed_set_size(s.No, s.Nv) * scalar_bytes(s.field));
-    engine_->set_mixed(true);
-    ccsd_->get_residuum(T, R_.get(), symmetric_);
-    engine_->set_mixed(false);
+    {
+      const SplitScope split(*engine_, true);
+      ccsd_->get_residuum(T, R_.get(), symmetric_);
+    }
     pack_axpby(stream_, s.field, R_.get(), -1.0, defect_.get(), 0.0, s.No, s.Nv);
     ccsd_->get_residuum(T, R_.get(), symmetric_);                   // :136
     pack_axpby(stream_, s.field, R_.get(), 1.0, defect_.get(), 1.0, s.No, s.Nv);
@@ -462,9 +463,10 @@ IterationReport CoupledCluster::iterate() {
   } else {
     rep.mixed = phase_ == Phase::Mixed || phase_ == Phase::Corrected;
     rep.kind = phase_ == Phase::Mixed ? 1 : phase_ == Phase::Corrected ? 3 : 0;
-    engine_->set_mixed(rep.mixed);
-    ccsd_->get_residuum(T, R_.get(), symmetric_);                   // :136
-    engine_->set_mixed(false);
+    {
+      const SplitScope split(*engine_, rep.mixed);
+      ccsd_->get_residuum(T, R_.get(), symmetric_);                   // :136
+    }
     if (phase_ == Phase::Corrected)
       unpack_accumulate(stream_, s.field, defect_.get(), 0, packed_set_size(s.No, s.Nv),
                         1.0, false, R_.get(), s.No, s.Nv);
@@ -572,9 +574,10 @@ void CoupledCluster::residuum(const double *T1, const double *T2, double *R1,
   }
   const bool symmetric = T && pairs_symmetric(T);
   // a context created for mixed precision evaluates its residuum that way
-  engine_->set_mixed(p_.mixed);
-  ccsd_->get_residuum(T, R_.get(), symmetric);
-  engine_->set_mixed(false);
+  {
+    const SplitScope split(*engine_, p_.mixed);
+    ccsd_->get_residuum(T, R_.get(), symmetric);
+  }
   download_set(R_.get(), R1, R2);
 }
 

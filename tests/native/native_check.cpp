@@ -231,7 +231,30 @@ void failed_split_pass() {
   CHECK(n > 10);
 }
 
+// After a split pass that failed, the FP64 gradient is that of a fresh context.
+void failed_split_pass_then_gradient() {
+  setenv("CC4S_MIXED_MIN_FLOPS", "0", 1);
+  const Problem p = mixed_problem();
+  const size_t n = size_t(2) * p.G * (p.o + p.v) * (p.o + p.v);
+  std::vector<double> ref(n), grad(n);
+  Out r;
+  for (long fail_at : {0L, 1L, 4L, 9L}) {
+    Context c(p, mixed);
+    CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+    CHECK(cc4s_ccsd_set_amplitudes(c, p.T1.data(), p.T2.data()) == 0);
+    arm(fail_at);
+    const int rc = fail_at % 2 ? cc4s_ccsd_iterate(c, nullptr) : residuum(c, p, r);
+    CHECK(rc == (g_failed ? 1 : 0) && g_failed == (fail_at > 0));
+    arm(0);
+    step("allocation " + std::to_string(fail_at));
+    CHECK(cc4s_ccsd_energy_grad_backward(c, nullptr, 0, (fail_at ? grad : ref).data(), 0, nullptr,
+                                         CC4S_PRECISION_FP64) == 0);
+    if (fail_at) CHECK(grad == ref);
+  }
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"failed_split_pass_then_gradient", failed_split_pass_then_gradient},
     {"failed_split_pass", failed_split_pass},
 };
 
