@@ -970,12 +970,10 @@ constexpr TileShape kRealTiles[3] = {
 constexpr int kCBM = 128, kCBN = 64, kCBK = 16, kCWM = 64, kCWN = 32;
 constexpr int kZBM = 128, kZBN = 128, kZBK = 16, kZWM = 64, kZWN = 32;
 
-int g_complex_generation = 3;
-
-TileShape tile_shape(Field f, Tile t) {
+TileShape tile_shape(Field f, Tile t, int generation) {
   if (f == Field::Real) return kRealTiles[static_cast<int>(t)];
-  if (g_complex_generation == 2) return {kZBM, kZBN, 1, 6.6, 6.6, 0.0, 10.0};
-  if (g_complex_generation == 1) return {kCBM, kCBN, 2, 4.0, 4.0, 0.0, 10.0};
+  if (generation == 2) return {kZBM, kZBN, 1, 6.6, 6.6, 0.0, 10.0};
+  if (generation == 1) return {kCBM, kCBN, 2, 4.0, 4.0, 0.0, 10.0};
   return kComplexTiles[static_cast<int>(t)];
 }
 
@@ -984,10 +982,6 @@ inline int grid_for(int64_t n) {
 }
 
 }  // namespace
-
-void set_complex_gett_generation(int g) {
-  g_complex_generation = (g >= 1 && g <= 5) ? g : 3;
-}
 
 std::string gett_variant(const GettLaunch &L) {
   std::string n = L.field == Field::Complex ? "gett_c64" : "gett_f64";
@@ -1003,7 +997,7 @@ void reduce_partials(bool cplx, const KArgs &a, int splits, hipStream_t s);
 
 KArgs kernel_args(const GettLaunch &L) {
   const bool cplx = L.field == Field::Complex;
-  const TileShape shape = tile_shape(L.field, static_cast<Tile>(L.tile));
+  const TileShape shape = tile_shape(L.field, static_cast<Tile>(L.tile), L.generation);
   const int BM = shape.BM, BN = shape.BN, BK = kZ3BK;
   KArgs a{};
   a.A = static_cast<const double *>(L.A);
@@ -1016,7 +1010,7 @@ KArgs kernel_args(const GettLaunch &L) {
   a.rowD = L.D ? L.rowD : L.rowC;
   a.colD = L.D ? L.colD : L.colC;
   a.signD = L.conjD ? -1.0 : 1.0;
-  CC4S_ASSERT(!L.D || !cplx || g_complex_generation != 1,
+  CC4S_ASSERT(!L.D || !cplx || L.generation != 1,
               "the first-generation kernel adds to its own result only");
   a.M = L.M; a.N = L.N; a.K = L.K;
   const int64_t kstages = (L.K + BK - 1) / BK;
@@ -1044,23 +1038,23 @@ void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start,
                  hipEvent_t stop) {
   const bool cplx = L.field == Field::Complex;
   const Tile tile = static_cast<Tile>(L.tile);
-  const TileShape shape = tile_shape(L.field, tile);
+  const TileShape shape = tile_shape(L.field, tile, L.generation);
   const int BM = shape.BM, BN = shape.BN;
   const KArgs a = kernel_args(L);
   dim3 grid(a.fullTiles + a.tailTiles * std::max(1, L.tail_splits), L.splits);
   if (start) CC4S_HIP(hipEventRecord(start, s));
-  if (cplx && g_complex_generation == 3) {
+  if (cplx && L.generation == 3) {
     if (tile == Tile::Large)
       dispatch_zgett<true, 512, 128, 64, 16, 32, 32, true>(L, a, grid, s);
     else if (tile == Tile::Medium)
       dispatch_zgett<true, 256, 64, 64, 16, 32, 32, true, false, 2>(L, a, grid, s);
     else
       dispatch_zgett<true, 256, 32, 32, 16, 16, 16, true, false, 4>(L, a, grid, s);
-  } else if (cplx && g_complex_generation == 2) {
+  } else if (cplx && L.generation == 2) {
     dispatch_zgett<true, kZThreads, kZBM, kZBN, kZBK, kZWM, kZWN, false>(L, a, grid, s);
-  } else if (cplx && g_complex_generation == 4) {
+  } else if (cplx && L.generation == 4) {
     dispatch_zgett<true, 256, 128, 64, 16, 64, 32, true>(L, a, grid, s);
-  } else if (cplx && g_complex_generation == 5) {
+  } else if (cplx && L.generation == 5) {
     dispatch_zgett<true, 512, 128, 64, 16, 32, 32, true, true>(L, a, grid, s);
   } else if (cplx) {
     dispatch_gett<kCBM, kCBN, kCBK, kCWM, kCWN>(L, a, grid, s);
@@ -1125,6 +1119,7 @@ void launch_splitk_reduce(Field f, const double *W, double *C,
 // ---------------------------------------------------------------------------
 
 struct GettPlan {
+  int generation = 3;  // kernel that tile, splits and tail are for
   int64_t M = 0, N = 0, K = 0;
   bool swap = false, a_kc = true, b_kc = true;
   int splits = 1, tail_splits = 1;
@@ -1144,9 +1139,11 @@ void ContractionEngine::apply_env_overrides() {
     CC4S_ASSERT(v == "half" || v == "bf16", "CC4S_MIXED_SPLIT must be half or bf16");
     mixed_half = v == "half";
   }
-  // CC4S_GETT_GENERATION selects the complex FP64 kernel (plans made later)
-  if (const char *e = std::getenv("CC4S_GETT_GENERATION"))
-    set_complex_gett_generation(std::atoi(e));
+  // CC4S_GETT_GENERATION selects the complex FP64 kernel of this engine
+  if (const char *e = std::getenv("CC4S_GETT_GENERATION")) {
+    const int v = std::atoi(e);
+    complex_generation = v >= 1 && v <= 5 ? v : 3;
+  }
   if (const char *e = std::getenv("CC4S_MIXED_TERMS")) {
     const int v = std::atoi(e);
     CC4S_ASSERT(v == 9 || v == 12 || v == 16, "CC4S_MIXED_TERMS must be 9, 12 or 16");
@@ -1304,6 +1301,7 @@ namespace {
 //     ms; energy and gradient of No=24, Nv=192, NG=1100 (4608 x 1100 x 4608) 9.2
 //     -> 8.2 ms.
 void choose_tile(Field f, int64_t M, int64_t N, int64_t K, size_t max_workspace, GettPlan &plan) {
+  const int generation = plan.generation;
   constexpr double kReduce = 3.5, kBytesPerUs = 4e6;
   plan.tile = Tile::Large;
   plan.splits = plan.tail_splits = 1;
@@ -1311,10 +1309,10 @@ void choose_tile(Field f, int64_t M, int64_t N, int64_t K, size_t max_workspace,
   if (M <= 0 || N <= 0 || K <= 0) return;
   const int64_t kstages = (K + kZ3BK - 1) / kZ3BK;
   const double es = static_cast<double>(scalar_bytes(f));
-  const bool fixed_tile = f == Field::Complex && g_complex_generation != 3;
+  const bool fixed_tile = f == Field::Complex && generation != 3;
   double best = -1;
   for (int t = 0; t < (fixed_tile ? 1 : 3); ++t) {
-    const TileShape s = tile_shape(f, static_cast<Tile>(t));
+    const TileShape s = tile_shape(f, static_cast<Tile>(t), generation);
     const int64_t tiles = ((M + s.BM - 1) / s.BM) * ((N + s.BN - 1) / s.BN);
     if (tiles >= (int64_t(1) << 31)) continue;
     const int64_t per = 256 * s.cap;
@@ -1412,10 +1410,12 @@ GettPlan &ContractionEngine::plan_for(const View &A0, const View &B0,
                                       const View &C, const View *D) {
   std::string key = plan_key(A0, B0, C);
   if (D) key += "+" + plan_key(*D, *D, *D);
+  if (C.field == Field::Complex) key += "g" + std::to_string(complex_generation);
   auto it = plans_.find(key);
   if (it != plans_.end()) return *it->second;
 
   auto plan = std::make_unique<GettPlan>();
+  plan->generation = complex_generation;
   std::string Mi, Ni, Ki;
   for (char c : C.idx) {
     const bool inA = A0.find(c) >= 0, inB = B0.find(c) >= 0;
@@ -1496,7 +1496,7 @@ void *ContractionEngine::reserve_partials(const GettPlan &P, Field f) {
   if (P.splits > 1) {
     elements = static_cast<size_t>(P.splits) * P.M * P.N;
   } else if (P.tail_splits > 1) {
-    const TileShape t = tile_shape(f, P.tile);
+    const TileShape t = tile_shape(f, P.tile, P.generation);
     const int64_t tiles = ((P.M + t.BM - 1) / t.BM) * ((P.N + t.BN - 1) / t.BN);
     elements = static_cast<size_t>(P.tail_splits) * (tiles - P.full_tiles) * t.BM * t.BN;
   }
@@ -1511,7 +1511,7 @@ void ContractionEngine::contract(double alpha, const View &A, const View &B,
   CC4S_ASSERT(A.field == C.field && B.field == C.field, "mixed scalar fields");
   CC4S_ASSERT(!C.conj, "conjugated result view");
   CC4S_ASSERT(!D || (D->field == C.field && !mixed_), "added tensor in a split pass");
-  if (D && C.field == Field::Complex && g_complex_generation == 1) {
+  if (D && C.field == Field::Complex && complex_generation == 1) {
     sum(1.0, *D, 0.0, C);
     D = nullptr;
   }
@@ -1534,6 +1534,7 @@ void ContractionEngine::contract(double alpha, const View &A, const View &B,
   L.M = P.M; L.N = P.N; L.K = P.K;
   L.splits = P.splits;
   L.tile = static_cast<int>(P.tile);
+  L.generation = P.generation;
   L.full_tiles = P.full_tiles;
   L.tail_splits = P.tail_splits;
   L.alpha = alpha; L.beta = beta;
@@ -1549,7 +1550,7 @@ void ContractionEngine::contract(double alpha, const View &A, const View &B,
   // a small contraction of a group waits for its end
   if (grouping_ && !profiling_ && P.tile == Tile::Small && P.tail_splits == 1 &&
       P.M * P.N * P.splits < kGroupElements &&
-      (C.field == Field::Real || g_complex_generation == 3)) {
+      (C.field == Field::Real || P.generation == 3)) {
     group_.push_back(L);
     stats.flops += flops;
     stats.launches += 1;

@@ -46,6 +46,7 @@ struct GettLaunch {
   int splits;
   int64_t full_tiles = 0;  // tiles of whole waves where the others are cut along K
   int tail_splits = 1;     // parts of each of those others (> 1: partials in W)
+  int generation = 3;      // complex kernel (ContractionEngine::complex_generation)
   int tile;  // 0 large, 1 medium (64 x 64), 2 small (32 x 32) workgroup tile
   double alpha, beta;
   bool conjA, conjB;
@@ -129,6 +130,12 @@ class ContractionEngine {
   // whether contractions scale their operands by the largest |Re| and |Im| (the
   // 9-product form scales by |Re| + |Im|, bf16 parts not at all)
   bool uses_operand_max() const { return mixed_ && mixed_half && mixed_terms != 9; }
+  // Complex FP64 kernel: 3 128x64, 64x64 and 32x32 tiles chosen per plan, three
+  // products per complex MAC; 1 four waves, 128x64 tile, single LDS buffer; 2 eight
+  // waves, 128x128 tile, double-buffered LDS, four products per complex MAC; 4 as 3,
+  // always 128x64 with four waves of 64x32; 5 as 3, always 128x64 with the loads two
+  // stages ahead.  A plan belongs to the kernel that it was made for.
+  int complex_generation = 3;
   // CC4S_MIXED_SPLIT, CC4S_MIXED_MAX_K, CC4S_MIXED_TERMS and
   // CC4S_GETT_GENERATION, when set, replace the settings above and the
   // complex kernel generation
@@ -225,13 +232,6 @@ void launch_gett(const GettLaunch &L, hipStream_t s, hipEvent_t start = nullptr,
                  hipEvent_t stop = nullptr);
 // name of the kernel variant launch_gett uses for L
 std::string gett_variant(const GettLaunch &L);
-// selects the complex kernel generation (1: 4 waves, 128x64 tile, single
-// LDS buffer; 2: 8 waves, 128x128 tile, double-buffered LDS, four MFMA
-// products per complex MAC; 3 (default): 128x64, 64x64 and 32x32 tiles chosen
-// per plan, three products per complex MAC; 4: as 3, always 128x64 with 4 waves
-// of 64x32; 5: as 3, always 128x64 with the loads two stages ahead); plans
-// created afterwards use its tile shapes
-void set_complex_gett_generation(int generation);
 
 // split-K reduction shared by both kernel families:
 // C[rowC[m] + colC[n]] = alpha * sum_s W[s][m][n] + beta * C

@@ -94,10 +94,9 @@ int main(int argc, char **argv) {
   try {
     hipStream_t st;
     CC4S_HIP(hipStreamCreate(&st));
-    set_complex_gett_generation(2);
-    ContractionEngine Eref(st);
-    set_complex_gett_generation(engine_gen);
-    ContractionEngine E(st);
+    ContractionEngine Eref(st), E(st);
+    Eref.complex_generation = 2;
+    E.complex_generation = engine_gen;
     E.set_profiling(true);
     if (gen == 3) {
       E.set_mixed(true);
@@ -114,10 +113,8 @@ int main(int argc, char **argv) {
         // relative Frobenius difference to the four-product kernel
         const size_t n = C.size() * 2;
         std::vector<double> ref(n), got(n);
-        set_complex_gett_generation(2);
         Eref.contract(1.0, A.v, B.v, 0.0, C.v);
         CC4S_HIP(hipMemcpyAsync(ref.data(), C.buf.get(), n * 8, hipMemcpyDeviceToHost, st));
-        set_complex_gett_generation(engine_gen);
         E.contract(1.0, A.v, B.v, 0.0, C.v);
         CC4S_HIP(hipMemcpyAsync(got.data(), C.buf.get(), n * 8, hipMemcpyDeviceToHost, st));
         CC4S_HIP(hipStreamSynchronize(st));
