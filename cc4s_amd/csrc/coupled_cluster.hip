@@ -361,6 +361,7 @@ CoupledCluster::~CoupledCluster() {
 void CoupledCluster::set_inputs(const double *gamma, bool on_device,
                                 const double *eps) {
   CC4S_HIP(hipSetDevice(device_));
+  inputs_set_ = false;  // until the new ones are complete: the former vertex goes first
   const auto &s = p_.shape;
   const size_t gbytes = static_cast<size_t>(s.NG) * s.Np() * s.Np() * 16;
   gamma_.allocate(gbytes);

@@ -208,6 +208,7 @@ struct Tensor {
   void reset(Field f, const std::string &idx, const std::vector<int64_t> &lens) {
     int64_t n = 1;
     for (auto l : lens) n *= l;
+    v = View();  // the former memory is gone, also if the allocation fails
     buf.allocate(static_cast<size_t>(n) * scalar_bytes(f));
     v = dense_view(buf.get(), f, idx, lens);
   }

@@ -253,7 +253,39 @@ void failed_split_pass_then_gradient() {
   }
 }
 
+// New inputs whose allocations fail leave a context that refuses to go on, and takes
+// inputs again.
+void failed_inputs() {
+  const Problem p = problem(true, 3, 9, 12, 4), q = problem(true, 3, 9, 12, 5);
+  Out ref, r;
+  {
+    Context c(p);
+    CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+    CHECK(residuum(c, p, ref) == 0);
+  }
+  long n = 0;
+  for (bool failed = true; failed;) {
+    Context c(p);
+    CHECK(cc4s_ccsd_set_inputs(c, q.gamma.data(), q.eps.data()) == 0);
+    CHECK(residuum(c, q, r) == 0);
+    arm(++n);
+    const int rc = cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data());
+    failed = g_failed;
+    arm(0);
+    CHECK(rc == (failed ? 1 : 0));
+    if (!failed) break;
+    step("allocation " + std::to_string(n));
+    CHECK(residuum(c, p, r) == 1);
+    CHECK(cc4s_ccsd_iterate(c, nullptr) == 1);
+    CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+    CHECK(residuum(c, p, r) == 0);
+    CHECK(r == ref);
+  }
+  CHECK(n > 10);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"failed_inputs", failed_inputs},
     {"failed_split_pass_then_gradient", failed_split_pass_then_gradient},
     {"failed_split_pass", failed_split_pass},
 };

@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 PROGRAM = pathlib.Path(__file__).resolve().parent.parent / "cc4s_amd" / "native_check"
 
 
-@pytest.mark.parametrize("scenario", ["failed_split_pass", "failed_split_pass_then_gradient"])
+@pytest.mark.parametrize("scenario", ["failed_split_pass", "failed_split_pass_then_gradient",
+                                      "failed_inputs"])
 def test_native(scenario):
     print(f"native {scenario}", flush=True)
     r = subprocess.run([str(PROGRAM), scenario], capture_output=True, text=True, timeout=110)
