@@ -882,6 +882,7 @@ double Ccsd::triples(const void *Tp, const double *eps_h, const double *eps_p) {
   size_t free_b = 0, total_b = 0;
   CC4S_HIP(hipMemGetInfo(&free_b, &total_b));
   if (3 * per > budget && 3 * per + budget < static_cast<int64_t>(free_b)) budget = 3 * per;
+  budget = std::min(budget, static_cast<int64_t>(free_b / 2));  // on a device that is nearly full
   if (const char *e = std::getenv("CC4S_TRIPLES_W_BYTES"))
     budget = static_cast<int64_t>(std::strtoull(e, nullptr, 10));
   const int parts = budget >= 3 * per ? 3 : 1;

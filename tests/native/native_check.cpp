@@ -284,7 +284,31 @@ void failed_inputs() {
   CHECK(n > 10);
 }
 
+// sizes at which the resident pair integrals are most of what a context holds (about
+// 160 MB complex, 80 real, against 30 and 15 without them)
+Problem resident_problem(bool cplx) { return problem(cplx, 5, 64, 24, 6); }
+constexpr size_t kMiB = size_t(1) << 20;
+void slabs(cc4s_ccsd_params &q) { q.integrals_slice_size = q.No; }  // the default's slices
+constexpr double kTol = 1e-12;  // of one FP64 residuum in two orders of summation
+
+// (T) goes on with fewer hole triples at a time where little memory is free.
+void triples_little_memory() {
+  const Problem p = resident_problem(true);
+  double ref = 0, e = 0;
+  for (size_t room : {size_t(0), 60 * kMiB, 40 * kMiB}) {
+    Context c(p, slabs);
+    CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+    CHECK(cc4s_ccsd_set_amplitudes(c, p.T1.data(), p.T2.data()) == 0);
+    g_total = room ? held() + room : 0;  // the ppph integrals take 20 MiB of it
+    step("room " + std::to_string(room / kMiB));
+    CHECK(cc4s_ccsd_triples(c, room ? &e : &ref) == 0);
+    if (room) CHECK(std::fabs(e - ref) <= kTol * std::fabs(ref));
+    g_total = 0;
+  }
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"triples_little_memory", triples_little_memory},
     {"failed_inputs", failed_inputs},
     {"failed_split_pass_then_gradient", failed_split_pass_then_gradient},
     {"failed_split_pass", failed_split_pass},
