@@ -23,7 +23,7 @@ DRIVER = HERE / "cc4s_ccsd"
 DRIVER_SOURCES = ["main.cpp", "yaml.cpp", "tensor_io.cpp"]
 SOURCES = ["contract.hip", "mixed.hip", "elementwise.hip", "adjoint.hip", "triples.hip", "ccsd.hip",
            "coupled_cluster.hip", "finite_size.hip", "abi.hip", "noalloc.hip", "ladder.hip", "ladder_pairs.hip",
-           "host_transfer.hip"]
+           "host_transfer.hip", "device_memory.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("CC4S_OFFLOAD_ARCH", "gfx950")

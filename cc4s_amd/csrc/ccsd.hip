@@ -45,6 +45,12 @@ struct Ccsd::Work {
   Tensor VS, VA, Rp, Rm, Tpm;  // Tpm: tau's combinations
   int64_t NGe = 0;  // length of the G index of the real-path vertex views
   bool hermitian = false;
+  // the resident ladder's memory; the slabs serve where it was given back
+  void drop_resident() {
+    for (Tensor *t : {&VS, &VA, &Rp, &Rm, &Tpm}) *t = Tensor();
+    resident = Resident::Off;
+  }
+  SpareMemory spare{[this] { drop_resident(); }};
 };
 
 Ccsd::Ccsd(ContractionEngine &E, const CcsdShape &shape, const CcsdOptions &opt,
@@ -174,7 +180,7 @@ void Ccsd::get_residuum(const void *T, void *R, bool symmetric) {
   if (opt_.method == Method::Drccd)
     residuum_drccd(T, R);
   else if (T && symmetric && w_->hermitian && !E_.mixed())
-    residuum_symmetric(T, R);
+    residuum_symmetric_or_slabs(T, R);
   else if (s_.field == Field::Complex)
     residuum_complex(T, R);
   else
@@ -321,12 +327,28 @@ void Ccsd::ladder(const View &left, const View &right, const View &tauv,
   }
 }
 
+bool Ccsd::release_resident() { return w_->spare.release(); }
+
+// A pass that finds the device full goes on with the slab ladder, which a context
+// of the same size has room for.
+void Ccsd::residuum_symmetric_or_slabs(const void *T, void *R) {
+  const double flops0 = E_.stats.flops;
+  try {
+    residuum_symmetric(T, R);
+  } catch (const OutOfMemory &) {
+    if (!release_resident()) throw;
+    E_.stats.flops = flops0;
+    residuum_symmetric(T, R);
+  }
+}
+
 // The ladder's pair integrals S and A (ladder_pairs.hip), formed from Gamma on
 // first use and kept for the run like the other integral slices.  They are kept
 // when they take at most half of the device memory that is free then (less what
-// the pass itself may still allocate), so that other contexts and the caller
-// keep room; other runs use the slab ladder.  An explicit integralsSliceSize
-// asks for the slab, whose memory it bounds, and so do the other ladder modes.
+// the pass itself may still allocate), so that the caller keeps room, and are
+// given back when an allocation of this or another context finds the device full;
+// other runs use the slab ladder.  An explicit integralsSliceSize asks for the
+// slab, whose memory it bounds, and so do the other ladder modes.
 bool Ccsd::resident_integrals() {
   auto &w = *w_;
   if (w.resident != Work::Resident::Unknown) return w.resident == Work::Resident::Ready;
@@ -351,23 +373,31 @@ bool Ccsd::resident_integrals() {
   if (fit < 1 || v > 65535) return false;
   const int64_t nx = std::min(std::min<int64_t>(fit, std::max<int64_t>(16, v / 16)), 65535 / v);
   if (nx < 1) return false;
-  Tensor slab;
   try {
     w.VS.reset(f, "km", {Kp, Kp + o * v});
     w.VA.reset(f, "km", {Km, Km + o * v});
     w.Rp.reset(f, "nm", {Np, Kp + o * v});
     w.Rm.reset(f, "nm", {Nm, Km + o * v});
     w.Tpm.reset(f, "n", {Kp * Np + Km * Nm});
-    slab.reset(f, "cxdy", {v, nx, v, v});
-  } catch (const Error &) {  // no room after all
-    (void)hipGetLastError();
-    w.VS = Tensor();
-    w.VA = Tensor();
-    w.Rp = Tensor();
-    w.Rm = Tensor();
-    w.Tpm = Tensor();
+    form_resident(nx);
+  } catch (const OutOfMemory &) {  // no room after all
+    w.drop_resident();
     return false;
+  } catch (...) {
+    w.drop_resident();
+    throw;
   }
+  w.resident = Work::Resident::Ready;
+  w.spare.set_held(true);
+  return true;
+}
+
+void Ccsd::form_resident(int64_t nx) {
+  auto &w = *w_;
+  const Field f = s_.field;
+  const int64_t o = s_.No, v = s_.Nv;
+  const int64_t Kp = v * (v + 1) / 2, Km = v * (v - 1) / 2;
+  Tensor slab(f, "cxdy", {v, nx, v, v});
   const hipStream_t st = E_.stream();
   const View left = gam("pp", "Gxc", true), right = gam("pp", "Gyd");
   for (int64_t x0 = 0; x0 < v; x0 += nx) {
@@ -387,8 +417,6 @@ bool Ccsd::resident_integrals() {
     resident_fold(f, false, V.ptr, w.VS.buf.get(), w.VA.buf.get(), v, cx, v, x0, v, st);
   }
   CC4S_HIP(hipStreamSynchronize(st));  // the slab is released here
-  w.resident = Work::Resident::Ready;
-  return true;
 }
 
 // tau's combinations of the resident ladder
@@ -510,6 +538,7 @@ void Ccsd::residuum_drccd(const void *Tp, void *Rp) {
 // statements: residuum_complex and residuum_real.
 void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
   auto &w = *w_;
+  const SpareMemory::Use resident_in_use(w.spare);
   auto &E = E_;
   const Field f = s_.field;
   const bool cplx = f == Field::Complex;
@@ -879,10 +908,9 @@ double Ccsd::triples(const void *Tp, const double *eps_h, const double *eps_p) {
   // 1024, 19.0 with 2048).
   const int64_t per = v * v * v * static_cast<int64_t>(es), all = o * (o + 1) * (o + 2) / 6;
   int64_t budget = int64_t(1) << 30;
-  size_t free_b = 0, total_b = 0;
-  CC4S_HIP(hipMemGetInfo(&free_b, &total_b));
-  if (3 * per > budget && 3 * per + budget < static_cast<int64_t>(free_b)) budget = 3 * per;
-  budget = std::min(budget, static_cast<int64_t>(free_b / 2));  // on a device that is nearly full
+  const int64_t free_b = static_cast<int64_t>(device_free_bytes(std::max(3 * per, budget) + budget));
+  if (3 * per > budget && 3 * per + budget < free_b) budget = 3 * per;
+  budget = std::min(budget, free_b / 2);  // on a device that is nearly full
   if (const char *e = std::getenv("CC4S_TRIPLES_W_BYTES"))
     budget = static_cast<int64_t>(std::strtoull(e, nullptr, 10));
   const int parts = budget >= 3 * per ? 3 : 1;

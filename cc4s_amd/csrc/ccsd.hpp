@@ -71,16 +71,20 @@ class Ccsd {
   // Gamma^G_qp == conj(Gamma^G_pq) (real field: == Gamma^G_pq) bit for bit
   // (checked on the device)
   bool vertex_is_hermitian() const;
+  // gives the resident pair integrals back; whether there were any
+  bool release_resident();
   CcsdTimings timings;
   bool profile = false;
 
  private:
   void residuum_symmetric(const void *T, void *R);
+  void residuum_symmetric_or_slabs(const void *T, void *R);
   void residuum_complex(const void *T, void *R);
   void residuum_real(const void *T, void *R);
   void residuum_drccd(const void *T, void *R);
   void form_slice(Tensor &V, const char *name);
   bool resident_integrals();
+  void form_resident(int64_t nx);
   void resident_combinations(const View &tauv);
   void resident_products();
   void ladder(const View &left, const View &right, const View &tauv,

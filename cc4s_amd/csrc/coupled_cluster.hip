@@ -311,8 +311,6 @@ CoupledCluster::CoupledCluster(const CoupledClusterParams &p, int device)
 // (override with CC4S_DIIS_PLACEMENT=device|host|host_all).
 void CoupledCluster::create_mixer() {
   const auto &s = p_.shape;
-  size_t free_b = 0, total_b = 0;
-  CC4S_HIP(hipMemGetInfo(&free_b, &total_b));
   // room kept for buffers allocated on first use (ladder slab and block,
   // operand packs, split-K partials; in mixed mode the packed tau of the
   // ladder, Nv^2 x No^2 rounded to the kernel tile, 8 bytes each)
@@ -324,7 +322,6 @@ void CoupledCluster::create_mixer() {
     if (p_.mixed_refine)
       reserve += static_cast<size_t>(packed_set_size(s.No, s.Nv)) * scalar_bytes(s.field);
   }
-  const size_t avail = free_b > reserve ? free_b - reserve : 0;
   const char *env = std::getenv("CC4S_DIIS_PLACEMENT");
   const std::string placement = env ? env : "auto";
   auto need = [&](DiisPlacement w) {
@@ -340,6 +337,9 @@ void CoupledCluster::create_mixer() {
   } else {
     CC4S_ASSERT(placement == "auto",
                 "CC4S_DIIS_PLACEMENT must be auto, device, host or host_all");
+    // a history on the device goes before other contexts' resident integrals
+    const size_t free_b = device_free_bytes(reserve + need(DiisPlacement::Device));
+    const size_t avail = free_b > reserve ? free_b - reserve : 0;
     if (need(DiisPlacement::Device) <= avail)
       where = DiisPlacement::Device;
     else if (need(DiisPlacement::AmplitudesOnHost) <= avail)
@@ -362,6 +362,7 @@ void CoupledCluster::set_inputs(const double *gamma, bool on_device,
                                 const double *eps) {
   CC4S_HIP(hipSetDevice(device_));
   inputs_set_ = false;  // until the new ones are complete: the former vertex goes first
+  if (ccsd_) ccsd_->release_resident();  // of the former vertex
   const auto &s = p_.shape;
   const size_t gbytes = static_cast<size_t>(s.NG) * s.Np() * s.Np() * 16;
   gamma_.allocate(gbytes);

@@ -8,7 +8,7 @@
 // of Ccsd.cxx:431-436 are views of the same memory, never copies.
 #pragma once
 
-#include "common.hpp"
+#include "device_memory.hpp"
 
 #include <string>
 #include <utility>
@@ -41,7 +41,7 @@ class DeviceBuffer {
   void allocate(size_t bytes) {
     release();
     if (bytes == 0) return;
-    CC4S_HIP(hipMalloc(&p_, bytes));
+    p_ = device_malloc(bytes);
     bytes_ = bytes;
   }
   // grow-only reallocation, contents are not preserved

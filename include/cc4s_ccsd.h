@@ -109,9 +109,12 @@ typedef struct {
                                      Gamma_qp = conj(Gamma_pq) (real field: Gamma_pq) and
                                      amplitudes with T_abij = T_baji, FP64 passes of both
                                      fields keep the pair integrals of the ladder on the
-                                     device instead (about Nv^4 scalars), formed in the
-                                     first such pass, where they take at most half of the
-                                     free device memory.  The real field otherwise uses
+                                     device instead (about Nv^4/2 + No Nv^3 scalars), formed
+                                     in the first such pass where they take at most half
+                                     of the free device memory, and given back when an
+                                     allocation of any context finds the device full.
+                                     integrals_slice_size No asks for the slabs of 0
+                                     without them.  The real field otherwise uses
                                      the slab. */
 } cc4s_ccsd_params;
 

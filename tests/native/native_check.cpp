@@ -24,6 +24,7 @@
 #include <mutex>
 #include <random>
 #include <string>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -109,7 +110,7 @@ namespace {
     if (!(cond)) {                                                         \
       std::printf("FAILED %s:%d %s\n", __FILE__, __LINE__, #cond);         \
       std::fflush(stdout);                                                 \
-      std::exit(1);                                                        \
+      std::_Exit(1);                                                       \
     }                                                                      \
   } while (0)
 
@@ -288,8 +289,68 @@ void failed_inputs() {
 // 160 MB complex, 80 real, against 30 and 15 without them)
 Problem resident_problem(bool cplx) { return problem(cplx, 5, 64, 24, 6); }
 constexpr size_t kMiB = size_t(1) << 20;
+constexpr size_t kReserve = size_t(6) << 30;  // what the library leaves free for a pass
 void slabs(cc4s_ccsd_params &q) { q.integrals_slice_size = q.No; }  // the default's slices
 constexpr double kTol = 1e-12;  // of one FP64 residuum in two orders of summation
+
+// device memory one residuum leaves a context with, and the residuum
+size_t held_after(const Problem &p, const std::function<void(cc4s_ccsd_params &)> &set, Out &r) {
+  Context c(p, set);
+  CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+  CHECK(residuum(c, p, r) == 0);
+  return held();
+}
+
+// Where the resident integrals do not fit, the slab ladder gives what it gives where
+// it is asked for.
+void small_device() {
+  for (bool cplx : {true, false}) {
+    const Problem p = resident_problem(cplx);
+    Out resident, slab, r;
+    const size_t with = held_after(p, {}, resident), without = held_after(p, slabs, slab);
+    step("held with " + std::to_string(with / kMiB) + " MiB, without " +
+         std::to_string(without / kMiB));
+    CHECK(with > 2 * without && rel(resident.first, slab.first) < kTol &&
+          rel(resident.second, slab.second) < kTol);
+    g_total = kReserve + with;  // less than twice what they need is free
+    CHECK(held_after(p, {}, r) <= without);
+    g_total = 0;
+    CHECK(r == slab);
+  }
+}
+
+// An allocation that fails while the resident integrals are formed, or later in the
+// pass, costs the integrals and not the pass, and nothing of them stays allocated.
+void failed_formation() {
+  for (bool cplx : {true, false}) {
+    const Problem p = resident_problem(cplx);
+    Out ref, r;
+    const size_t without = held_after(p, slabs, ref);
+    bool started = false;
+    long n = 0, done = 0;
+    for (bool failed = true; failed;) {
+      Context c(p);
+      CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+      arm(++n);
+      int rc = residuum(c, p, r);
+      failed = g_failed;
+      arm(0);
+      if (!failed) break;
+      step("allocation " + std::to_string(n) + (rc ? " fails" : " passed over"));
+      if (rc) {
+        CHECK(!started);  // before the first of the integrals' only
+        continue;
+      }
+      started = true;
+      ++done;
+      CHECK(rel(r.first, ref.first) < kTol && rel(r.second, ref.second) < kTol);
+      CHECK(held() <= without + 16 * kMiB);
+      CHECK(residuum(c, p, r) == 0);
+      CHECK(rel(r.first, ref.first) < kTol && rel(r.second, ref.second) < kTol);
+    }
+    CHECK(done > 6);
+  }
+}
 
 // (T) goes on with fewer hole triples at a time where little memory is free.
 void triples_little_memory() {
@@ -307,7 +368,128 @@ void triples_little_memory() {
   }
 }
 
+// The integrals that one context keeps do not take room from another context's
+// history or from the context's own later calls: they are given back.
+void given_back() {
+  const Problem p = resident_problem(true);
+  const size_t n = size_t(2) * p.G * (p.o + p.v) * (p.o + p.v);
+  Out ref, r;
+  double triples_ref = 0, triples = 0;
+  std::vector<double> grad_ref(n), grad(n);
+  {
+    Context c(p, slabs);
+    CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+    CHECK(cc4s_ccsd_set_amplitudes(c, p.T1.data(), p.T2.data()) == 0);
+    CHECK(residuum(c, p, ref) == 0);
+    CHECK(cc4s_ccsd_triples(c, &triples_ref) == 0);
+    CHECK(cc4s_ccsd_energy_grad_backward(c, nullptr, 0, grad_ref.data(), 0, nullptr,
+                                         CC4S_PRECISION_FP64) == 0);
+  }
+  auto right = [&](cc4s_ccsd_context *c) {
+    CHECK(residuum(c, p, r) == 0);
+    CHECK(rel(r.first, ref.first) < kTol && rel(r.second, ref.second) < kTol);
+  };
+  auto resident = [&](cc4s_ccsd_context *c) {  // a pass that forms them
+    g_total = 0;
+    CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+    CHECK(cc4s_ccsd_set_amplitudes(c, p.T1.data(), p.T2.data()) == 0);
+    const size_t before = held();
+    right(c);
+    CHECK(held() > before + 100 * kMiB);
+  };
+  Context a(p);
+  resident(a);
+  step("another context's history");
+  {
+    const size_t before = held();
+    size_t other = 0;
+    {
+      Context b(p);
+      CHECK(cc4s_ccsd_set_inputs(b, p.gamma.data(), p.eps.data()) == 0);
+      other = held() - before;
+    }
+    g_total = before + kReserve + other - kMiB;  // the history is short of 1 MiB
+    Context b(p);
+    CHECK(cc4s_ccsd_set_inputs(b, p.gamma.data(), p.eps.data()) == 0);
+    cc4s_ccsd_iteration it;
+    CHECK(cc4s_ccsd_iterate(b, &it) == 0);
+    CHECK(it.diis_placement == 0 && held() < before);
+    right(a);
+    right(b);
+  }
+  resident(a);
+  step("new inputs");
+  g_total = held() + 40 * kMiB;
+  CHECK(cc4s_ccsd_set_inputs(a, p.gamma.data(), p.eps.data()) == 0);
+  right(a);
+  resident(a);
+  step("(T)");
+  g_total = held() + 4 * kMiB;  // the ppph integrals take 20 MiB
+  CHECK(cc4s_ccsd_triples(a, &triples) == 0);
+  CHECK(std::fabs(triples - triples_ref) <= kTol * std::fabs(triples_ref));
+  right(a);
+  resident(a);
+  step("gradient");
+  g_total = held() + kMiB / 4;
+  CHECK(cc4s_ccsd_energy_grad_backward(a, nullptr, 0, grad.data(), 0, nullptr,
+                                       CC4S_PRECISION_FP64) == 0);
+  CHECK(rel(grad, grad_ref) < kTol);
+  right(a);
+  g_total = 0;
+}
+
+// A context that forms its integrals again and again on one thread, and on another
+// thread contexts whose history needs their room: both stay right.
+void given_back_between_threads() {
+  const Problem p = problem(true, 4, 40, 16, 7), q = problem(true, 10, 40, 16, 8);
+  auto long_history = [](cc4s_ccsd_params &x) { x.max_residua = 11; };
+  Out refp, refq, r;
+  const size_t base = held();
+  const size_t without = held_after(p, slabs, refp);
+  const size_t resident = held_after(p, {}, r) - without;
+  held_after(q, slabs, refq);
+  size_t other = 0;
+  {
+    Context b(q, long_history);
+    CHECK(cc4s_ccsd_set_inputs(b, q.gamma.data(), q.eps.data()) == 0);
+    other = held() - base;
+  }
+  step("integrals " + std::to_string(resident / kMiB) + " MiB, the other context " +
+       std::to_string(other / kMiB));
+  CHECK(other > resident + 4 * kMiB);
+  // the history is short of 3 MiB beside the integrals; on the host it has room also
+  // while they are formed (16 MiB more)
+  g_total = kReserve + without + resident + other - 3 * kMiB;
+  std::thread first([&] {
+    Context a(p);
+    Out x;
+    for (int n = 0; n < 12; ++n) {
+      CHECK(cc4s_ccsd_set_inputs(a, p.gamma.data(), p.eps.data()) == 0);
+      for (int k = 0; k < 3; ++k) {
+        CHECK(residuum(a, p, x) == 0);
+        CHECK(rel(x.first, refp.first) < kTol && rel(x.second, refp.second) < kTol);
+      }
+    }
+  });
+  std::thread second([&] {
+    Out x;
+    for (int n = 0; n < 12; ++n) {
+      Context b(q, long_history);
+      if (cc4s_ccsd_set_inputs(b, q.gamma.data(), q.eps.data())) step(cc4s_ccsd_last_error(b));
+      CHECK(residuum(b, q, x) == 0);
+      CHECK(rel(x.first, refq.first) < kTol && rel(x.second, refq.second) < kTol);
+    }
+  });
+  first.join();
+  second.join();
+  g_total = 0;
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"given_back_between_threads", given_back_between_threads},
+    {"small_device", small_device},
+    {"failed_formation", failed_formation},
+    {"given_back", given_back},
     {"triples_little_memory", triples_little_memory},
     {"failed_inputs", failed_inputs},
     {"failed_split_pass_then_gradient", failed_split_pass_then_gradient},
