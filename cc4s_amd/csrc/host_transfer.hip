@@ -89,6 +89,14 @@ void slice_of(size_t bytes, int slice, int slices, size_t &begin, size_t &end) {
   end = std::min(bytes, pages * (slice + 1) / slices * 4096);
 }
 
+// memory the runtime knows (pinned, managed, a device's) is no matter of the ring
+bool pageable(const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();  // memory it has never seen
+  return true;
+}
+
 }  // namespace
 
 HostTransfer::~HostTransfer() {
@@ -108,11 +116,11 @@ bool HostTransfer::ring() {
 }
 
 void HostTransfer::download(void *host, const void *device, size_t bytes, hipStream_t s) {
-  if (bytes < kStagedBytes || !ring()) {
+  auto direct = [&] {
     CC4S_HIP(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, s));
     CC4S_HIP(hipStreamSynchronize(s));
-    return;
-  }
+  };
+  if (bytes < kStagedBytes || !pageable(host) || !ring()) return direct();
   const size_t n = (bytes + kChunk - 1) / kChunk;
   auto len = [&](size_t c) { return std::min(kChunk, bytes - c * kChunk); };
   Copiers copiers(n, [&](size_t c, int slice, int slices) {
@@ -140,11 +148,11 @@ void HostTransfer::download(void *host, const void *device, size_t bytes, hipStr
 }
 
 void HostTransfer::upload(void *device, const void *host, size_t bytes, hipStream_t s) {
-  if (bytes < kStagedBytes || !ring()) {
+  auto direct = [&] {
     CC4S_HIP(hipMemcpyAsync(device, host, bytes, hipMemcpyHostToDevice, s));
     CC4S_HIP(hipStreamSynchronize(s));
-    return;
-  }
+  };
+  if (bytes < kStagedBytes || !pageable(host) || !ring()) return direct();
   const size_t n = (bytes + kChunk - 1) / kChunk;
   auto len = [&](size_t c) { return std::min(kChunk, bytes - c * kChunk); };
   {

@@ -40,6 +40,12 @@ size_t g_total = 0;          // bytes the device has; 0: what it really has
 long g_fail_at = 0;          // the allocation that fails, counted from arm(); 0: none
 long g_count = 0;
 bool g_failed = false;
+struct Copy {
+  const void *dst, *src;
+  size_t bytes;
+};
+bool g_record = false;
+std::vector<Copy> g_copies;  // while g_record
 
 template <typename F>
 F real(const char *name) {
@@ -88,6 +94,16 @@ hipError_t hipFree(void *p) {
     g_sizes.erase(it);
   }
   return e;
+}
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKind kind,
+                          hipStream_t stream) {
+  static const auto f =
+      real<hipError_t (*)(void *, const void *, size_t, hipMemcpyKind, hipStream_t)>("hipMemcpyAsync");
+  {
+    std::lock_guard<std::mutex> l(g_lock);
+    if (g_record) g_copies.push_back({dst, src, bytes});
+  }
+  return f(dst, src, bytes, kind, stream);
 }
 hipError_t hipMemGetInfo(size_t *free_bytes, size_t *total_bytes) {
   static const auto f = real<hipError_t (*)(size_t *, size_t *)>("hipMemGetInfo");
@@ -485,7 +501,42 @@ void given_back_between_threads() {
   g_total = 0;
 }
 
+// 17 MiB of amplitudes, any bytes: over the ring's threshold, a short last chunk
+Problem transfer_problem() {
+  Problem p{true, 7, 151, 2, {}, {}, {}, {}};
+  std::mt19937_64 rng(9);
+  for (size_t k = 0; k < p.n1(); ++k) p.T1.push_back(double(rng()));
+  for (size_t k = 0; k < p.n2(); ++k) p.T2.push_back(double(rng()));
+  return p;
+}
+
+// The caller's pinned memory is copied at once, not through the ring.
+void pinned_copies() {
+  const Problem p = transfer_problem();
+  const size_t b1 = p.n1() * 8, b2 = p.n2() * 8;
+  double *h1 = nullptr, *h2 = nullptr;
+  CHECK(hipHostMalloc(reinterpret_cast<void **>(&h1), b1, hipHostMallocDefault) == hipSuccess);
+  CHECK(hipHostMalloc(reinterpret_cast<void **>(&h2), b2, hipHostMallocDefault) == hipSuccess);
+  std::memcpy(h1, p.T1.data(), b1);
+  std::memcpy(h2, p.T2.data(), b2);
+  Context c(p);
+  g_record = true;
+  CHECK(cc4s_ccsd_set_amplitudes(c, h1, h2) == 0);
+  std::memset(h2, 0, b2);
+  CHECK(cc4s_ccsd_get_amplitudes(c, h1, h2) == 0);
+  g_record = false;
+  int up = 0, down = 0;
+  for (const Copy &x : g_copies) {
+    up += x.src == h2 && x.bytes == b2;
+    down += x.dst == h2 && x.bytes == b2;
+  }
+  CHECK(up == 1 && down == 1);
+  CHECK(std::memcmp(h1, p.T1.data(), b1) == 0 && std::memcmp(h2, p.T2.data(), b2) == 0);
+  CHECK(hipHostFree(h1) == hipSuccess && hipHostFree(h2) == hipSuccess);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"pinned_copies", pinned_copies},
     {"given_back_between_threads", given_back_between_threads},
     {"small_device", small_device},
     {"failed_formation", failed_formation},
