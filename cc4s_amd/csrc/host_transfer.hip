@@ -7,6 +7,7 @@
 #include <cstring>
 #include <functional>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -15,20 +16,28 @@ namespace cc4s_amd {
 namespace {
 
 // Worker threads that copy their slice of chunk 0, 1, ... n-1 as the chunks are
-// opened, and count it done.  The destructor ends and joins them.
+// opened, and count it done.  As many as the system grants: the slices are those of
+// the threads there are, which is settled before the first chunk is opened.  The
+// destructor ends and joins them.
 class Copiers {
  public:
   Copiers(size_t n, std::function<void(size_t chunk, int slice, int slices)> copy)
       : n_(n), copy_(std::move(copy)), done_(n, 0) {
     const unsigned hw = std::thread::hardware_concurrency();
-    count_ = static_cast<int>(std::min(8u, std::max(1u, hw / 2)));
+    const int want = static_cast<int>(std::min(8u, std::max(1u, hw / 2)));
+    threads_.reserve(want);
     try {
-      for (int t = 0; t < count_; ++t) threads_.emplace_back([this, t] { work(t); });
+      while (count_ < want) {
+        threads_.emplace_back([this, t = count_] { work(t); });
+        ++count_;
+      }
+    } catch (const std::system_error &) {  // no more of them
     } catch (...) {
       end();
       throw;
     }
   }
+  int count() const { return count_; }
   ~Copiers() { end(); }
   // chunks [0, upto) may be copied
   void open(size_t upto) {
@@ -73,7 +82,7 @@ class Copiers {
   size_t n_;
   std::function<void(size_t, int, int)> copy_;
   std::vector<int> done_;
-  int count_ = 1;
+  int count_ = 0;  // workers read it after the first chunk was opened
   size_t open_ = 0;
   bool end_ = false;
   std::mutex m_;
@@ -130,6 +139,7 @@ void HostTransfer::download(void *host, const void *device, size_t bytes, hipStr
       std::memcpy(static_cast<char *>(host) + c * kChunk + b,
                   static_cast<const char *>(buf_[c % kRing].get()) + b, e - b);
   });
+  if (!copiers.count()) return direct();
   size_t issued = 0;
   for (size_t c = 0; c < n; ++c) {
     // one buffer less than the ring in flight: the wait for a free one is for a
@@ -163,6 +173,7 @@ void HostTransfer::upload(void *device, const void *host, size_t bytes, hipStrea
         std::memcpy(static_cast<char *>(buf_[c % kRing].get()) + b,
                     static_cast<const char *>(host) + c * kChunk + b, e - b);
     });
+    if (!copiers.count()) return direct();
     copiers.open(kRing);
     for (size_t c = 0; c < n; ++c) {
       copiers.wait(c);

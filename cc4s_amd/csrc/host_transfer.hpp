@@ -15,7 +15,7 @@ namespace cc4s_amd {
 // Nv=256 (1.1 GB) 541 -> 466 ms, No=17, Nv=131 (79 MB) 21.8 -> 15.5 ms, real
 // Drccd No=24, Nv=160 (118 MB) 16.5 -> 8.0 ms; smaller transfers take under 2 ms
 // either way and keep the runtime's path, and so does a call that gets no pinned
-// memory.  The ring belongs to one context, is
+// memory or no thread.  The ring belongs to one context, is
 // made on its first large transfer and freed with it.  Both calls return when
 // the data has arrived.
 class HostTransfer {

@@ -10,7 +10,9 @@
 #include "cc4s_ccsd.h"
 
 #include <dlfcn.h>
+#include <errno.h>
 #include <hip/hip_runtime.h>
+#include <pthread.h>
 
 #include <algorithm>
 #include <atomic>
@@ -40,6 +42,7 @@ size_t g_total = 0;          // bytes the device has; 0: what it really has
 long g_fail_at = 0;          // the allocation that fails, counted from arm(); 0: none
 long g_count = 0;
 bool g_failed = false;
+long g_threads = -1;         // threads that may still be created; -1: any number
 struct Copy {
   const void *dst, *src;
   size_t bytes;
@@ -104,6 +107,16 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKin
     if (g_record) g_copies.push_back({dst, src, bytes});
   }
   return f(dst, src, bytes, kind, stream);
+}
+int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*run)(void *), void *arg) noexcept {
+  static const auto f = real<int (*)(pthread_t *, const pthread_attr_t *, void *(*)(void *), void *)>(
+      "pthread_create");
+  {
+    std::lock_guard<std::mutex> l(g_lock);
+    if (g_threads == 0) return EAGAIN;
+    if (g_threads > 0) --g_threads;
+  }
+  return f(t, a, run, arg);
 }
 hipError_t hipMemGetInfo(size_t *free_bytes, size_t *total_bytes) {
   static const auto f = real<hipError_t (*)(size_t *, size_t *)>("hipMemGetInfo");
@@ -535,8 +548,28 @@ void pinned_copies() {
   CHECK(hipHostFree(h1) == hipSuccess && hipHostFree(h2) == hipSuccess);
 }
 
+// Copies of pageable memory with the threads that the system grants, and with none.
+void copies_without_threads() {
+  const Problem p = transfer_problem();
+  Context c(p);
+  std::vector<double> T1(p.n1()), T2(p.n2());
+  for (long granted : {-1L, 0L, 1L, 3L}) {
+    for (int up = 0; up < 2; ++up) {
+      step(std::to_string(granted) + (up ? " up" : " down"));
+      T2.assign(p.n2(), 0.0);
+      g_threads = up ? granted : -1;
+      CHECK(cc4s_ccsd_set_amplitudes(c, p.T1.data(), p.T2.data()) == 0);
+      g_threads = up ? -1 : granted;
+      CHECK(cc4s_ccsd_get_amplitudes(c, T1.data(), T2.data()) == 0);
+      g_threads = -1;
+      CHECK(T1 == p.T1 && T2 == p.T2);
+    }
+  }
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
     {"pinned_copies", pinned_copies},
+    {"copies_without_threads", copies_without_threads},
     {"given_back_between_threads", given_back_between_threads},
     {"small_device", small_device},
     {"failed_formation", failed_formation},
