@@ -395,6 +395,7 @@ void CoupledCluster::upload_set(void *dst, const double *T1, const double *T2) {
   const size_t es = scalar_bytes(s.field);
   transfer_.upload(dst, T1, s.n1() * es, stream_);
   transfer_.upload(static_cast<char *>(dst) + s.n1() * es, T2, s.n2() * es, stream_);
+  CC4S_HIP(hipStreamSynchronize(stream_));
 }
 
 void CoupledCluster::download_set(const void *src, double *T1, double *T2) {
@@ -403,19 +404,21 @@ void CoupledCluster::download_set(const void *src, double *T1, double *T2) {
   if (T1) transfer_.download(T1, src, s.n1() * es, stream_);
   if (T2)
     transfer_.download(T2, static_cast<const char *>(src) + s.n1() * es, s.n2() * es, stream_);
+  CC4S_HIP(hipStreamSynchronize(stream_));
 }
 
 bool CoupledCluster::pairs_symmetric(const void *T) {
   const auto &s = p_.shape;
+  if (p_.ccsd.method == Method::Drccd) return false;  // does not ask
   return cc4s_amd::pairs_symmetric(
       stream_, s.field, static_cast<const char *>(T) + s.n1() * scalar_bytes(s.field), s.No,
-      s.Nv);
+      s.Nv, energy_partials_.get());
 }
 
 void CoupledCluster::set_amplitudes(const double *T1, const double *T2) {
   CC4S_HIP(hipSetDevice(device_));
+  symmetry_known_ = false;  // a pass will ask
   upload_set(T_.get(), T1, T2);
-  symmetric_ = pairs_symmetric(T_.get());
   have_amplitudes_ = true;
 }
 
@@ -445,6 +448,10 @@ IterationReport CoupledCluster::iterate() {
   IterationReport rep;
   rep.iteration = iterations_done + 1;
   const void *T = have_amplitudes_ ? T_.get() : nullptr;
+  if (T && !symmetry_known_) {
+    symmetric_ = pairs_symmetric(T);
+    symmetry_known_ = true;
+  }
   if (phase_ == Phase::Anchor && T) {
     // the split residuum and the FP64 residuum at the same amplitudes:
     // d = R64(T) - Rsplit(T), kept pair-packed (both residua satisfy
@@ -481,7 +488,7 @@ IterationReport CoupledCluster::iterate() {
   const bool is_second_order = !have_amplitudes_;
   mixer_->append(T_.get());                             // :145-147
   have_amplitudes_ = true;
-  symmetric_ = true;  // the mixer's history is pair-packed
+  symmetric_ = symmetry_known_ = true;  // the mixer's history is pair-packed
   CC4S_HIP(hipStreamSynchronize(stream_));
   const auto t2 = std::chrono::steady_clock::now();
   rep.residuum_seconds = std::chrono::duration<double>(t1 - t0).count();

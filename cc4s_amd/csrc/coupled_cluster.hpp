@@ -179,7 +179,10 @@ class CoupledCluster {
   // transition structure factor: singular vectors, grid vertex blocks, Y
   DeviceBuffer fsc_u_, fsc_ph_, fsc_hp_, fsc_y_;
   bool have_amplitudes_ = false;
-  bool symmetric_ = true;  // T_ satisfies T_abij = T_baji (set_amplitudes may not)
+  // T_ satisfies T_abij = T_baji: the iteration's own amplitudes do, those of
+  // set_amplitudes are looked at by the first pass (by set_amplitudes itself No=4,
+  // Nv=16 40 -> 66 us, which (T), gradients and Drccd do not need)
+  bool symmetric_ = true, symmetry_known_ = true;
   bool inputs_set_ = false;
   enum class Phase { Fp64, Mixed, Anchor, Corrected };
   Phase phase_ = Phase::Fp64;

@@ -968,9 +968,9 @@ bool is_hermitian(hipStream_t s, Field f, const void *gamma, int64_t NG, int64_t
   return finish_count(s, p) == 0.0;
 }
 
-bool pairs_symmetric(hipStream_t s, Field f, const void *T2, int64_t No, int64_t Nv) {
-  DeviceBuffer part((kReduceBlocks + 1) * sizeof(double2));
-  double2 *p = part.as<double2>();
+bool pairs_symmetric(hipStream_t s, Field f, const void *T2, int64_t No, int64_t Nv,
+                     void *partials) {
+  double2 *p = static_cast<double2 *>(partials);
   if (f == Field::Complex)
     asymmetry_kernel<true><<<kReduceBlocks, kBlock, 0, s>>>(static_cast<const double2 *>(T2),
                                                             No, Nv, p);

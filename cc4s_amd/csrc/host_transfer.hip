@@ -127,7 +127,6 @@ bool HostTransfer::ring() {
 void HostTransfer::download(void *host, const void *device, size_t bytes, hipStream_t s) {
   auto direct = [&] {
     CC4S_HIP(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, s));
-    CC4S_HIP(hipStreamSynchronize(s));
   };
   if (bytes < kStagedBytes || !pageable(host) || !ring()) return direct();
   const size_t n = (bytes + kChunk - 1) / kChunk;
@@ -160,7 +159,6 @@ void HostTransfer::download(void *host, const void *device, size_t bytes, hipStr
 void HostTransfer::upload(void *device, const void *host, size_t bytes, hipStream_t s) {
   auto direct = [&] {
     CC4S_HIP(hipMemcpyAsync(device, host, bytes, hipMemcpyHostToDevice, s));
-    CC4S_HIP(hipStreamSynchronize(s));
   };
   if (bytes < kStagedBytes || !pageable(host) || !ring()) return direct();
   const size_t n = (bytes + kChunk - 1) / kChunk;

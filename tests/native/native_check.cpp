@@ -567,7 +567,29 @@ void copies_without_threads() {
   }
 }
 
+// Calls repeated on a context allocate nothing on the device.
+void no_allocations() {
+  const Problem p = problem(true, 3, 9, 12, 4), q2 = problem(true, 3, 9, 12, 5);
+  for (int method : {CC4S_METHOD_CCSD, CC4S_METHOD_DRCCD}) {
+    Context c(p, [&](cc4s_ccsd_params &q) { q.method = method; });
+    Out r;
+    std::vector<double> T1(p.n1()), T2(p.n2());
+    CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+    for (int n = 0; n < 2; ++n) {
+      arm(0);  // counts from here
+      const Problem &t = n ? q2 : p;
+      CHECK(cc4s_ccsd_set_amplitudes(c, t.T1.data(), t.T2.data()) == 0);
+      CHECK(cc4s_ccsd_iterate(c, nullptr) == 0);
+      CHECK(residuum(c, t, r) == 0);
+      CHECK(cc4s_ccsd_get_amplitudes(c, T1.data(), T2.data()) == 0);
+      step("method " + std::to_string(method) + ": " + std::to_string(g_count) + " allocations");
+    }
+    CHECK(g_count == 0);
+  }
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"no_allocations", no_allocations},
     {"pinned_copies", pinned_copies},
     {"copies_without_threads", copies_without_threads},
     {"given_back_between_threads", given_back_between_threads},

@@ -16,7 +16,7 @@ PROGRAM = pathlib.Path(__file__).resolve().parent.parent / "cc4s_amd" / "native_
                                       "failed_inputs", "triples_little_memory", "small_device",
                                       "failed_formation", "given_back",
                                       "given_back_between_threads", "pinned_copies",
-                                      "copies_without_threads"])
+                                      "copies_without_threads", "no_allocations"])
 def test_native(scenario):
     print(f"native {scenario}", flush=True)
     r = subprocess.run([str(PROGRAM), scenario], capture_output=True, text=True, timeout=110)
