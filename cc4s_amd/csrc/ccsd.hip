@@ -373,6 +373,7 @@ bool Ccsd::resident_integrals() {
   if (fit < 1 || v > 65535) return false;
   const int64_t nx = std::min(std::min<int64_t>(fit, std::max<int64_t>(16, v / 16)), 65535 / v);
   if (nx < 1) return false;
+  w.spare.set_held(true);
   try {
     w.VS.reset(f, "km", {Kp, Kp + o * v});
     w.VA.reset(f, "km", {Km, Km + o * v});
@@ -381,14 +382,15 @@ bool Ccsd::resident_integrals() {
     w.Tpm.reset(f, "n", {Kp * Np + Km * Nm});
     form_resident(nx);
   } catch (const OutOfMemory &) {  // no room after all
+    w.spare.set_held(false);
     w.drop_resident();
     return false;
   } catch (...) {
+    w.spare.set_held(false);
     w.drop_resident();
     throw;
   }
   w.resident = Work::Resident::Ready;
-  w.spare.set_held(true);
   return true;
 }
 
