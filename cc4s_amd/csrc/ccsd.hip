@@ -175,14 +175,14 @@ void Ccsd::form_integrals() {
 
 bool Ccsd::vertex_is_hermitian() const { return w_->hermitian; }
 
-void Ccsd::get_residuum(const void *T, void *R, bool symmetric) {
+void Ccsd::get_residuum(const void *T, void *R, PairSymmetry pairs) {
   auto t0 = std::chrono::steady_clock::now();
   if (opt_.method == Method::Drccd)
     residuum_drccd(T, R);
-  else if (T && symmetric && w_->hermitian && !E_.mixed())
+  else if (T && pairs == PairSymmetry::Exact && w_->hermitian && !E_.mixed())
     residuum_symmetric_or_slabs(T, R);
   else if (s_.field == Field::Complex)
-    residuum_complex(T, R);
+    residuum_complex(T, R, pairs);
   else
     residuum_real(T, R);
   if (profile) {
@@ -200,17 +200,18 @@ void Ccsd::get_residuum(const void *T, void *R, bool symmetric) {
 // With ladder_fused (FP64 complex passes) one kernel forms V in LDS and
 // contracts it, and no slab exists.
 void Ccsd::ladder(const View &left, const View &right, const View &tauv,
-                  const View &R2) {
+                  const View &R2, PairSymmetry pairs) {
   auto &w = *w_;
   const Field f = s_.field;
   const int64_t v = s_.Nv, o = s_.No, s = opt_.integrals_slice_size;
   const int64_t ns = (v + s - 1) / s;
   const size_t es = scalar_bytes(f);
   const bool fused = opt_.ladder_fused && f == Field::Complex && !E_.mixed();
-  // paired: tau's combinations go to Y's buffer (v^2 o^2 elements, unused
+  // paired, for a tau with the pairs' symmetry: its combinations go to Y's buffer (v^2 o^2 elements, unused
   // after the ring terms) and each chunk's Vp, Vm to Xakic's (free after the
   // crossed ring terms): cx * Ny * v^2 <= v^2 o^2
   const bool paired = !fused && opt_.ladder_paired && f == Field::Complex &&
+                      pairs != PairSymmetry::None &&
                       w.Y.size() > 0 && std::min(s, v) <= o * o;
   const size_t slab_budget = size_t(2) << 30;
   const int64_t per_x = v * v * std::min(s, v) * static_cast<int64_t>(es);
@@ -675,11 +676,11 @@ void Ccsd::residuum_symmetric(const void *Tp, void *Rp) {
     C(1.0, w.Xklij("klij"), T2.as("abkl"), 1.0, R2);            // :542-546
     // with Gamma_qp = conj Gamma_pq, Gamma_pp[G,a,b] - Gamma_hp[G,k,b] T_ak
     // (:560-561) equals cTDGamma_pp[G,a,b] of :509-510 term by term
-    ladder(w.DGpp.v, w.DGpp.v, w.X.v, R2);                      // :564-600
+    ladder(w.DGpp.v, w.DGpp.v, w.X.v, R2, PairSymmetry::Exact); // :564-600
   }
 }
 
-void Ccsd::residuum_complex(const void *Tp, void *Rp) {
+void Ccsd::residuum_complex(const void *Tp, void *Rp, PairSymmetry pairs) {
   auto &w = *w_;
   auto &E = E_;
   const Field f = Field::Complex;
@@ -761,11 +762,11 @@ void Ccsd::residuum_complex(const void *Tp, void *Rp) {
     if (w.hermitian) {
       // with Gamma_qp = conj Gamma_pq exactly, Gamma_pp[G,a,b] - Gamma_hp[G,k,b]
       // T_ak (:560-561) equals cTDGamma_pp[G,a,b] of :509-510 term by term
-      ladder(w.DGpp.v, w.DGpp.v, X.v, R2);                      // :564-600
+      ladder(w.DGpp.v, w.DGpp.v, X.v, R2, pairs);               // :564-600
     } else {
       S(1.0, gam("pp", "Gab"), 0.0, w.Dpp("Gab"));              // :560
       C(-1.0, gam("hp", "Gkb"), T1.as("ak"), 1.0, w.Dpp("Gab"));  // :561
-      ladder(w.DGpp.v, w.Dpp.v, X.v, R2);                       // :564-600
+      ladder(w.DGpp.v, w.Dpp.v, X.v, R2, pairs);                // :564-600
     }
   }
   C(1.0, w.Kac("ac"), T1.as("ci"), 0.0, R1);                    // :609
@@ -863,7 +864,7 @@ void Ccsd::residuum_real(const void *Tp, void *Rp) {
   C(1.0, w.Xklij("klij"), X("abkl"), 1.0, R2);                   // :273
   C(1.0, Vp("cdkl"), X("cdij"), 0.0, w.Xklij("klij"));           // :275
   C(1.0, w.Xklij("klij"), opt_.ppl ? T2.as("abkl") : X("abkl"), 1.0, R2);  // :276-280
-  if (opt_.ppl) ladder(w.DGpp.v, w.DGpp.v, X.v, R2);             // :283-333
+  if (opt_.ppl) ladder(w.DGpp.v, w.DGpp.v, X.v, R2, PairSymmetry::None);  // :283-333
   C(1.0, w.Kac("ac"), T1.as("ci"), 0.0, R1);                     // :341
   C(-1.0, w.Kki("ki"), T1.as("ak"), 1.0, R1);                    // :342
   C(2.0, Vp("cdkl"), T1.as("dl"), 0.0, w.Kck("ck"));             // :345

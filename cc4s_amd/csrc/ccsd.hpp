@@ -6,6 +6,7 @@
 #pragma once
 
 #include "contract.hpp"
+#include "elementwise.hpp"
 
 #include <memory>
 
@@ -58,9 +59,9 @@ class Ccsd {
   void form_integrals();
 
   // R = residuum(T); T == nullptr is the first iteration (R1 = 0, R2 = V).
-  // `symmetric` tells that T_abij = T_baji holds exactly (the iteration's own
-  // amplitudes always satisfy it).
-  void get_residuum(const void *T, void *R, bool symmetric);
+  // `pairs` tells how T_abij = T_baji holds (exactly for the iteration's own
+  // amplitudes).
+  void get_residuum(const void *T, void *R, PairSymmetry pairs);
 
   const View &Vpphh() const;
 
@@ -79,7 +80,7 @@ class Ccsd {
  private:
   void residuum_symmetric(const void *T, void *R);
   void residuum_symmetric_or_slabs(const void *T, void *R);
-  void residuum_complex(const void *T, void *R);
+  void residuum_complex(const void *T, void *R, PairSymmetry pairs);
   void residuum_real(const void *T, void *R);
   void residuum_drccd(const void *T, void *R);
   void form_slice(Tensor &V, const char *name);
@@ -88,7 +89,7 @@ class Ccsd {
   void resident_combinations(const View &tauv);
   void resident_products();
   void ladder(const View &left, const View &right, const View &tauv,
-              const View &R2);
+              const View &R2, PairSymmetry pairs);
   View gam(const char *part, const std::string &names, bool conjT = false) const;
 
   ContractionEngine &E_;

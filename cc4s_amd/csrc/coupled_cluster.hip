@@ -407,17 +407,17 @@ void CoupledCluster::download_set(const void *src, double *T1, double *T2) {
   CC4S_HIP(hipStreamSynchronize(stream_));
 }
 
-bool CoupledCluster::pairs_symmetric(const void *T) {
+PairSymmetry CoupledCluster::pair_symmetry(const void *T) {
   const auto &s = p_.shape;
-  if (p_.ccsd.method == Method::Drccd) return false;  // does not ask
-  return cc4s_amd::pairs_symmetric(
+  if (p_.ccsd.method == Method::Drccd) return PairSymmetry::None;  // does not ask
+  return cc4s_amd::pair_symmetry(
       stream_, s.field, static_cast<const char *>(T) + s.n1() * scalar_bytes(s.field), s.No,
       s.Nv, energy_partials_.get());
 }
 
 void CoupledCluster::set_amplitudes(const double *T1, const double *T2) {
   CC4S_HIP(hipSetDevice(device_));
-  symmetry_known_ = false;  // a pass will ask
+  pairs_known_ = false;  // a pass will ask
   upload_set(T_.get(), T1, T2);
   have_amplitudes_ = true;
 }
@@ -448,9 +448,9 @@ IterationReport CoupledCluster::iterate() {
   IterationReport rep;
   rep.iteration = iterations_done + 1;
   const void *T = have_amplitudes_ ? T_.get() : nullptr;
-  if (T && !symmetry_known_) {
-    symmetric_ = pairs_symmetric(T);
-    symmetry_known_ = true;
+  if (T && !pairs_known_) {
+    pairs_ = pair_symmetry(T);
+    pairs_known_ = true;
   }
   if (phase_ == Phase::Anchor && T) {
     // the split residuum and the FP64 residuum at the same amplitudes:
@@ -461,10 +461,10 @@ IterationReport CoupledCluster::iterate() {
     defect_.reserve(packed_set_size(s.No, s.Nv) * scalar_bytes(s.field));
     {
       const SplitScope split(*engine_, true);
-      ccsd_->get_residuum(T, R_.get(), symmetric_);
+      ccsd_->get_residuum(T, R_.get(), pairs_);
     }
     pack_axpby(stream_, s.field, R_.get(), -1.0, defect_.get(), 0.0, s.No, s.Nv);
-    ccsd_->get_residuum(T, R_.get(), symmetric_);                   // :136
+    ccsd_->get_residuum(T, R_.get(), pairs_);                   // :136
     pack_axpby(stream_, s.field, R_.get(), 1.0, defect_.get(), 1.0, s.No, s.Nv);
     mixer_->restart(0);
     rep.mixed = false;
@@ -474,7 +474,7 @@ IterationReport CoupledCluster::iterate() {
     rep.kind = phase_ == Phase::Mixed ? 1 : phase_ == Phase::Corrected ? 3 : 0;
     {
       const SplitScope split(*engine_, rep.mixed);
-      ccsd_->get_residuum(T, R_.get(), symmetric_);                   // :136
+      ccsd_->get_residuum(T, R_.get(), pairs_);                   // :136
     }
     if (phase_ == Phase::Corrected)
       unpack_accumulate(stream_, s.field, defect_.get(), 0, packed_set_size(s.No, s.Nv),
@@ -488,7 +488,8 @@ IterationReport CoupledCluster::iterate() {
   const bool is_second_order = !have_amplitudes_;
   mixer_->append(T_.get());                             // :145-147
   have_amplitudes_ = true;
-  symmetric_ = symmetry_known_ = true;  // the mixer's history is pair-packed
+  pairs_ = PairSymmetry::Exact;  // the mixer's history is pair-packed
+  pairs_known_ = true;
   CC4S_HIP(hipStreamSynchronize(stream_));
   const auto t2 = std::chrono::steady_clock::now();
   rep.residuum_seconds = std::chrono::duration<double>(t1 - t0).count();
@@ -581,11 +582,11 @@ void CoupledCluster::residuum(const double *T1, const double *T2, double *R1,
     upload_set(scratch_.get(), T1, T2);
     T = scratch_.get();
   }
-  const bool symmetric = T && pairs_symmetric(T);
+  const PairSymmetry pairs = T ? pair_symmetry(T) : PairSymmetry::Exact;
   // a context created for mixed precision evaluates its residuum that way
   {
     const SplitScope split(*engine_, p_.mixed);
-    ccsd_->get_residuum(T, R_.get(), symmetric);
+    ccsd_->get_residuum(T, R_.get(), pairs);
   }
   download_set(R_.get(), R1, R2);
 }

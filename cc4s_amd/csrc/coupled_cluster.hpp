@@ -157,7 +157,7 @@ class CoupledCluster {
 
  private:
   void energy(const void *T, cplx *E, cplx *D, cplx *X);
-  bool pairs_symmetric(const void *T);
+  PairSymmetry pair_symmetry(const void *T);
   void upload_set(void *dst, const double *T1, const double *T2);
   void download_set(const void *src, double *T1, double *T2);
   void create_mixer();
@@ -179,10 +179,11 @@ class CoupledCluster {
   // transition structure factor: singular vectors, grid vertex blocks, Y
   DeviceBuffer fsc_u_, fsc_ph_, fsc_hp_, fsc_y_;
   bool have_amplitudes_ = false;
-  // T_ satisfies T_abij = T_baji: the iteration's own amplitudes do, those of
+  // how T_ satisfies T_abij = T_baji: the iteration's own amplitudes do, those of
   // set_amplitudes are looked at by the first pass (by set_amplitudes itself No=4,
   // Nv=16 40 -> 66 us, which (T), gradients and Drccd do not need)
-  bool symmetric_ = true, symmetry_known_ = true;
+  PairSymmetry pairs_ = PairSymmetry::Exact;
+  bool pairs_known_ = true;
   bool inputs_set_ = false;
   enum class Phase { Fp64, Mixed, Anchor, Corrected };
   Phase phase_ = Phase::Fp64;

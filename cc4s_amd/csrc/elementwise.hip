@@ -906,12 +906,13 @@ __global__ __launch_bounds__(kBlock) void hermitian_kernel(const double2 *g, dou
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
-// per-block count of elements with T_abij != T_baji: tile pairs
-// {(A, B, i, j), (B, A, j, i)} through LDS, as symmetrize_kernel
+// per block, `stride` apart: the count of elements with T_abij != T_baji, the largest
+// |Re| and |Im| of their differences and of T; tile pairs {(A, B, i, j), (B, A, j, i)}
+// through LDS, as symmetrize_kernel
 template <bool CPLX>
 __global__ __launch_bounds__(kBlock) void asymmetry_kernel(const typename Sc<CPLX>::T *T2,
                                                            int64_t No, int64_t Nv,
-                                                           double2 *partials) {
+                                                           double *partials, int stride) {
   using S = Sc<CPLX>;
   using T = typename S::T;
   constexpr int kt = kPairTile;
@@ -919,7 +920,7 @@ __global__ __launch_bounds__(kBlock) void asymmetry_kernel(const typename Sc<CPL
   __shared__ T ys[kt][kt + 1];
   const int64_t nt = (Nv + kt - 1) / kt;
   const int64_t ntiles = nt * nt * No * No;
-  double bad = 0.0;
+  double bad = 0.0, diff = 0.0, largest = 0.0;
   for (int64_t tid = blockIdx.x; tid < ntiles; tid += gridDim.x) {
     const int64_t ta = tid % nt, tb = (tid / nt) % nt, ij = tid / (nt * nt);
     const int64_t i = ij % No, j = ij / No;
@@ -938,13 +939,58 @@ __global__ __launch_bounds__(kBlock) void asymmetry_kernel(const typename Sc<CPL
       const T x = T2[offX + (a0 + u) + Nv * (b0 + w)], y = ys[w][u];
       if constexpr (CPLX) {
         if (!(x.x == y.x && x.y == y.y)) bad += 1.0;
+        diff = fmax(diff, fmax(fabs(x.x - y.x), fabs(x.y - y.y)));
+        largest = fmax(largest, fmax(fabs(x.x), fabs(x.y)));
       } else {
         if (!(x == y)) bad += 1.0;
+        diff = fmax(diff, fabs(x - y));
+        largest = fmax(largest, fabs(x));
       }
     }
   }
   const double2 s = block_sum(make_double2(bad, 0.0), sh);
-  if (threadIdx.x == 0) partials[blockIdx.x] = s;
+  diff = wave_max(diff);
+  largest = wave_max(largest);
+  __syncthreads();
+  if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = make_double2(diff, largest);
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int w = 1; w < kBlock / 64; ++w) {
+    diff = fmax(diff, sh[w].x);
+    largest = fmax(largest, sh[w].y);
+  }
+  partials[blockIdx.x] = s.x;
+  partials[stride + blockIdx.x] = diff;
+  partials[2 * stride + blockIdx.x] = largest;
+}
+
+// the sum and the two maxima of n blocks' partials to partials[3 n] ...
+__global__ __launch_bounds__(kBlock) void asymmetry_finish_kernel(double *partials, int n) {
+  __shared__ double sh[3][kBlock / 64];
+  double bad = 0.0, diff = 0.0, largest = 0.0;
+  for (int k = threadIdx.x; k < n; k += kBlock) {
+    bad += partials[k];
+    diff = fmax(diff, partials[n + k]);
+    largest = fmax(largest, partials[2 * n + k]);
+  }
+  bad = wave_sum(bad);
+  diff = wave_max(diff);
+  largest = wave_max(largest);
+  if (threadIdx.x % 64 == 0) {
+    sh[0][threadIdx.x / 64] = bad;
+    sh[1][threadIdx.x / 64] = diff;
+    sh[2][threadIdx.x / 64] = largest;
+  }
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int w = 1; w < kBlock / 64; ++w) {
+    bad += sh[0][w];
+    diff = fmax(diff, sh[1][w]);
+    largest = fmax(largest, sh[2][w]);
+  }
+  partials[3 * n] = bad;
+  partials[3 * n + 1] = diff;
+  partials[3 * n + 2] = largest;
 }
 
 // sums kReduceBlocks partials and reads the total back
@@ -968,17 +1014,25 @@ bool is_hermitian(hipStream_t s, Field f, const void *gamma, int64_t NG, int64_t
   return finish_count(s, p) == 0.0;
 }
 
-bool pairs_symmetric(hipStream_t s, Field f, const void *T2, int64_t No, int64_t Nv,
-                     void *partials) {
-  double2 *p = static_cast<double2 *>(partials);
+PairSymmetry pair_symmetry(hipStream_t s, Field f, const void *T2, int64_t No, int64_t Nv,
+                           void *partials) {
+  double *p = static_cast<double *>(partials);
+  static_assert(3 * kReduceBlocks + 3 <= 2 * (2 * kReduceBlocks + 2), "the energy's scratch");
   if (f == Field::Complex)
     asymmetry_kernel<true><<<kReduceBlocks, kBlock, 0, s>>>(static_cast<const double2 *>(T2),
-                                                            No, Nv, p);
+                                                            No, Nv, p, kReduceBlocks);
   else
     asymmetry_kernel<false><<<kReduceBlocks, kBlock, 0, s>>>(static_cast<const double *>(T2),
-                                                             No, Nv, p);
+                                                             No, Nv, p, kReduceBlocks);
   CC4S_HIP(hipGetLastError());
-  return finish_count(s, p) == 0.0;
+  asymmetry_finish_kernel<<<1, kBlock, 0, s>>>(p, kReduceBlocks);
+  CC4S_HIP(hipGetLastError());
+  double h[3];  // count, largest difference, largest element
+  CC4S_HIP(hipMemcpyAsync(h, p + 3 * kReduceBlocks, sizeof(h), hipMemcpyDeviceToHost, s));
+  CC4S_HIP(hipStreamSynchronize(s));
+  return h[0] == 0.0                      ? PairSymmetry::Exact
+         : h[1] <= kPairRounding * h[2] ? PairSymmetry::Rounded
+                                        : PairSymmetry::None;
 }
 
 void copy(hipStream_t s, void *y, const void *x, size_t bytes) {

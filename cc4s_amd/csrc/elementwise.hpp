@@ -26,10 +26,14 @@ void symmetrize_pairs(hipStream_t s, Field f, void *R2, int64_t No, int64_t Nv,
 void exchange_combination(hipStream_t s, Field f, void *out, const void *in, double alpha,
                           double beta, double gamma, bool conj, int64_t No, int64_t Nv);
 
-// T_abij == T_baji for every element, exactly; `partials` is device scratch of
-// energy_partials_size()
-bool pairs_symmetric(hipStream_t s, Field f, const void *T2, int64_t No, int64_t Nv,
-                     void *partials);
+// How T_abij = T_baji holds: exactly in every element, or within kPairRounding of the
+// largest |Re| and |Im|, what an amplitude file of another program can be off by (sums
+// of some thousand products in two orders), or not.
+enum class PairSymmetry { None, Rounded, Exact };
+constexpr double kPairRounding = 0x1p-46;
+// `partials` is device scratch of energy_partials_size()
+PairSymmetry pair_symmetry(hipStream_t s, Field f, const void *T2, int64_t No, int64_t Nv,
+                           void *partials);
 
 // New amplitudes and amplitude change of one amplitude set [T1; T2]
 // (CoupledCluster.cxx:137-144, 255-317):

@@ -1,8 +1,8 @@
 // Paired particle-particle ladder: the slab contraction of Ccsd.cxx:590 over
 // pairs c <= d and i <= j (complex).
 //
-// tau has the pair symmetry tau_cdij = tau_dcji (T2 and T1 x T1 both have
-// it), so with
+// tau has the pair symmetry tau_cdij = tau_dcji (T1 x T1 has it, and T2 where it
+// holds to rounding; other amplitudes take the slab contraction), so with
 //   tau+_cd(ij) = (tau_cdij + tau_cdji) / 2   symmetric in (c, d),
 //   tau-_cd(ij) = (tau_cdij - tau_cdji) / 2   antisymmetric in (c, d),
 // the slab contraction R_xyij = sum_cd V_xycd tau_cdij becomes

@@ -104,7 +104,8 @@ typedef struct {
                                      CC4S_LADDER_PAIRED (default: the slab contraction over
                                      pairs c <= d, i <= j of tau's symmetric and
                                      antisymmetric combinations, half its multiply-adds;
-                                     FP64 and split passes); same results to rounding.
+                                     FP64 and split passes; amplitudes without T_abij =
+                                     T_baji take the slab); same results to rounding.
                                      With PAIRED, integrals_slice_size 0, a vertex with
                                      Gamma_qp = conj(Gamma_pq) (real field: Gamma_pq) and
                                      amplitudes with T_abij = T_baji, FP64 passes of both

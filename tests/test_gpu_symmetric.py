@@ -73,3 +73,90 @@ def test_real_vertex_without_symmetry(shape):
         R1, R2 = cc.residuum(T)
     assert rel_err(R1, Q1) < R_TOL
     assert rel_err(R2, Q2) < R_TOL
+
+
+def _asymmetric(No, Nv, field, scale=1e-2):
+    T1, T2 = syn.random_amplitudes(No, Nv, field, 13, t1_scale=0.05, t2_scale=0.05)
+    rng = np.random.default_rng(No + Nv)
+    d = rng.standard_normal(T2.shape)
+    if field == "complex":
+        d = d + 1j * rng.standard_normal(T2.shape)
+    return T1, np.asfortranarray(T2 + scale * d)
+
+
+# complex: the slab contraction, of the statements of a Hermitian vertex and of another;
+# differences at the level of rounding keep the paired one, which is off by no more
+@pytest.mark.parametrize("ladder", ["paired", "slab", "fused"])
+@pytest.mark.parametrize("scale", [1e-2, 1e-16], ids=["asymmetric", "rounded"])
+@pytest.mark.parametrize("hermitian", [True, False], ids=["herm", "nonherm"])
+@pytest.mark.parametrize("shape", [(3, 9, 12), (4, 33, 20)])
+def test_complex_amplitudes_without_pair_symmetry(shape, hermitian, scale, ladder):
+    print(f"complex amplitudes without pair symmetry {shape} {hermitian} {scale} {ladder}",
+          flush=True)
+    No, Nv, NG = shape
+    T = _asymmetric(No, Nv, "complex", scale)
+    inp = syn.generate(No, Nv, NG, "complex", 21)
+    g = inp.gamma
+    if not hermitian:
+        rng = np.random.default_rng(4)
+        g = g + 0.003 * (rng.standard_normal(g.shape) + 1j * rng.standard_normal(g.shape))
+    P = O.CcsdProblem(g, inp.eps, No, "complex")
+    Q1, Q2 = P.residuum(T)
+    with api.CoupledCluster(No, Nv, NG, field="complex", ladder=ladder) as cc:
+        cc.set_inputs(g, inp.eps)
+        for _ in range(2):
+            R1, R2 = cc.residuum(T)
+            assert rel_err(R1, Q1) < R_TOL
+            assert rel_err(R2, Q2) < R_TOL
+
+
+def test_split_residuum_of_amplitudes_without_pair_symmetry(monkeypatch):
+    """The bound of the split residuum with half parts, as for symmetric amplitudes."""
+    monkeypatch.setenv("CC4S_MIXED_MIN_FLOPS", "0")
+    No, Nv, NG = 4, 33, 20
+    T = _asymmetric(No, Nv, "complex")
+    inp = syn.generate(No, Nv, NG, "complex", 21)
+    Q1, Q2 = O.CcsdProblem(inp.gamma, inp.eps, No, "complex").residuum(T)
+    with api.CoupledCluster(No, Nv, NG, field="complex", precision=api.PRECISION_MIXED) as cc:
+        cc.set_inputs(inp.gamma, inp.eps)
+        R1, R2 = cc.residuum(T)
+    assert rel_err(R1, Q1) < 1e-5
+    assert rel_err(R2, Q2) < 1e-5
+
+
+@pytest.mark.parametrize("field", ["complex", "real"])
+@pytest.mark.parametrize("shape", [(3, 9, 12), (4, 33, 20)])
+def test_iteration_from_amplitudes_with_and_without_pair_symmetry(shape, field):
+    """set_amplitudes decides which statements the next pass takes: without the
+    symmetry, with it, without it again, and the pass after that.  maxResidua 1 makes
+    a pass T' = -R / Delta; the history keeps one element of each pair."""
+    print(f"iteration from set amplitudes {field} {shape}", flush=True)
+    No, Nv, NG = shape
+    inp = syn.generate(No, Nv, NG, field, 21)
+    P = O.CcsdProblem(inp.gamma, inp.eps, No, field)
+    unsymmetric = _asymmetric(No, Nv, field)
+    symmetric = syn.random_amplitudes(No, Nv, field, 17, t1_scale=0.05, t2_scale=0.05)
+    with api.CoupledCluster(No, Nv, NG, field=field, maxResidua=1) as cc:
+        cc.set_inputs(inp.gamma, inp.eps)
+        for T in (unsymmetric, symmetric, unsymmetric, None):
+            if T is None:
+                T = cc.amplitudes()
+            else:
+                cc.set_amplitudes(*T)
+            N1, N2 = O.residuum_to_amplitudes(P, P.residuum(T), T)
+            cc.iterate()
+            S1, S2 = cc.amplitudes()
+            assert rel_err(S1, N1) < R_TOL
+            assert np.array_equal(S2, S2.transpose(1, 0, 3, 2))
+            off = np.minimum(abs(S2 - N2), abs(S2 - N2.transpose(1, 0, 3, 2)))
+            assert np.max(off) < R_TOL * np.max(abs(N2))
+
+
+@pytest.mark.parametrize("field", ["complex", "real"])
+@pytest.mark.parametrize("shape,size", [((3, 9, 12), 2), ((4, 33, 20), 5), ((7, 50, 33), 7),
+                                        ((3, 40, 20), 64)])
+def test_symmetric_residuum_with_the_slab_ladder(field, shape, size):
+    """A slice size of its own takes the slabs under the symmetric statements."""
+    print(f"symmetric residuum, slabs {field} {shape} {size}", flush=True)
+    T = syn.random_amplitudes(shape[0], shape[1], field, 13, t1_scale=0.05, t2_scale=0.05)
+    _check(field, shape, T, integralsSliceSize=size)
