@@ -8,6 +8,7 @@
 //
 // prints its steps and, if every one holds, "ok SCENARIO" (status 0).
 #include "cc4s_ccsd.h"
+#include "contract.hpp"
 
 #include <dlfcn.h>
 #include <errno.h>
@@ -49,6 +50,7 @@ struct Copy {
 };
 bool g_record = false;
 std::vector<Copy> g_copies;  // while g_record
+std::vector<size_t> g_allocations;  // while g_record
 
 template <typename F>
 F real(const char *name) {
@@ -73,6 +75,7 @@ hipError_t hipMalloc(void **p, size_t bytes) {
   {
     std::lock_guard<std::mutex> l(g_lock);
     ++g_count;
+    if (g_record) g_allocations.push_back(bytes);
     if ((g_fail_at && g_count == g_fail_at) || (g_total && g_held + bytes > g_total)) {
       g_failed = true;
       *p = nullptr;
@@ -590,7 +593,249 @@ void no_allocations() {
   }
 }
 
+// ---------------------------------------------------------------------------
+// contraction kernels
+// ---------------------------------------------------------------------------
+
+using namespace cc4s_amd;
+using Z = std::complex<double>;
+
+// C = alpha op(A) op(B) + beta op(D) on the host for some rows
+struct Product {
+  bool cplx;
+  int64_t M, N, K;
+  std::vector<Z> A, B, D;  // [m][k], [n][k], [m][n]
+  Product(bool c, int64_t m, int64_t n, int64_t k) : cplx(c), M(m), N(n), K(k) {
+    std::mt19937_64 rng(m + 3 * n + 7 * k);
+    std::uniform_real_distribution<double> d(-1, 1);
+    for (std::vector<Z> *x : {&A, &B, &D}) {
+      x->resize(x == &A ? M * K : x == &B ? N * K : M * N);
+      for (Z &z : *x) z = Z(d(rng), c ? d(rng) : 0.0);
+    }
+  }
+  Z at(int64_t m, int64_t n, double alpha, bool conjA, bool conjB, double beta, bool conjD) const {
+    const double fa = conjA ? -1 : 1, fb = conjB ? -1 : 1;
+    const Z *a = &A[m * K], *b = &B[n * K];
+    double re = 0, im = 0;
+    for (int64_t k = 0; k < K; ++k) {
+      re += a[k].real() * b[k].real() - fa * fb * a[k].imag() * b[k].imag();
+      im += fb * a[k].real() * b[k].imag() + fa * a[k].imag() * b[k].real();
+    }
+    const Z d = beta == 0.0 ? Z() : conjD ? std::conj(D[m * N + n]) : D[m * N + n];
+    return Z(alpha * re, alpha * im) + beta * d;
+  }
+  // Largest error of C over every `step`-th row and the last, in units of what
+  // rounding allows: partial sums of K products of numbers up to one grow as sqrt(K)
+  // / 3, their sqrt(K) roundings come to about K 2^-53 / 5, the largest of 10^5
+  // elements to four or five times that, two orders of summation and the three-product
+  // form's larger terms to four times more; and a few roundings at the end.
+  double error(const std::vector<Z> &C, int64_t ld, int64_t step, double alpha, bool conjA,
+               bool conjB, double beta, bool conjD) const {
+    double e = 0;
+    for (int64_t m = 0; m < M; m = m == M - 1 ? M : std::min(m + step, M - 1))
+      for (int64_t n = 0; n < N; ++n) {
+        const double x = std::abs(C[m * ld + n] - at(m, n, alpha, conjA, conjB, beta, conjD));
+        if (!(x < HUGE_VAL)) return HUGE_VAL;
+        e = std::max(e, x);
+      }
+    return e / ((8.0 * K + 16.0) * 0x1p-53);
+  }
+};
+std::vector<double> packed(const std::vector<Z> &x, bool cplx) {
+  std::vector<double> r;
+  for (const Z &z : x) {
+    r.push_back(z.real());
+    if (cplx) r.push_back(z.imag());
+  }
+  return r;
+}
+template <typename T>
+DeviceBuffer upload(const std::vector<T> &x) {
+  DeviceBuffer b(x.size() * sizeof(T));
+  CHECK(hipMemcpy(b.get(), x.data(), x.size() * sizeof(T), hipMemcpyHostToDevice) == hipSuccess);
+  return b;
+}
+
+// Every tile of the GETT kernel, in every orientation, whole, with K split and with
+// the last tiles cut along K (the fourth part of four then has no k left), at sizes
+// that are no multiple of any tile, rows longer than what is used of them.
+void gett_tiles() {
+  const int64_t M = 323, N = 261;
+  const int tiles[2][3][2] = {{{128, 128}, {64, 64}, {32, 32}}, {{128, 64}, {64, 64}, {32, 32}}};
+  hipStream_t st;
+  CHECK(hipStreamCreate(&st) == hipSuccess);
+  for (int64_t K : {131, 70, 17, 1})
+    for (bool cplx : {false, true}) {
+      const Product P(cplx, M, N, K);
+      const int64_t Kpad = (K + 15) / 16 * 16 + 80;  // whole stages, and five further
+      const int64_t lk = K + 3, lm = M + 5, ln = N + 7;
+      auto spread = [&](const std::vector<Z> &x, int64_t rows, int64_t cols, int64_t ld, bool turn) {
+        std::vector<Z> r((turn ? cols : rows) * ld, Z(NAN, NAN));
+        for (int64_t i = 0; i < rows; ++i)
+          for (int64_t j = 0; j < cols; ++j) r[turn ? j * ld + i : i * ld + j] = x[i * cols + j];
+        return packed(r, cplx);
+      };
+      auto table = [&](int64_t n, int64_t pad, int64_t stride) {
+        std::vector<int64_t> t(std::max(n, pad), 0);
+        for (int64_t i = 0; i < n; ++i) t[i] = i * stride;
+        return upload(t);
+      };
+      const DeviceBuffer D = upload(spread(P.D, M, N, ln, false));
+      const DeviceBuffer rowC = table(M, 0, ln), colC = table(N, 0, 1);
+      for (int orient = 0; orient < 4; ++orient) {
+        const bool ak = orient & 2, bk = orient & 1;
+        const DeviceBuffer A = upload(spread(P.A, M, K, ak ? lk : lm, !ak)),
+                           B = upload(spread(P.B, N, K, bk ? lk : ln, !bk));
+        const DeviceBuffer rowA = table(M, 0, ak ? lk : 1), colA = table(K, Kpad, ak ? 1 : lm),
+                           rowB = table(K, Kpad, bk ? 1 : ln), colB = table(N, 0, bk ? lk : 1);
+        double worst = 0;
+        for (int t = 0; t < 3; ++t) {
+          const int64_t BM = tiles[cplx][t][0], BN = tiles[cplx][t][1];
+          const int64_t count = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+          struct Mode {
+            int splits, cut;
+            bool add, other;  // beta, to another tensor
+          };
+          for (const Mode mode : {Mode{1, 1, false, false}, Mode{1, 1, true, false},
+                                  Mode{3, 1, true, true}, Mode{1, 2, true, false},
+                                  Mode{1, 4, true, true}, Mode{40, 1, false, false}}) {
+            const int64_t full = count - count / 3;
+            GettLaunch L;
+            L.field = cplx ? Field::Complex : Field::Real;
+            L.A = A.get();
+            L.B = B.get();
+            // C starts as D where that is added in place, as NaN where it is not read
+            DeviceBuffer C = upload(mode.add && !mode.other
+                                        ? spread(P.D, M, N, ln, false)
+                                        : std::vector<double>(M * ln * (cplx ? 2 : 1), NAN));
+            L.C = C.get();
+            L.rowA = rowA.as<int64_t>();
+            L.colA = colA.as<int64_t>();
+            L.rowB = rowB.as<int64_t>();
+            L.colB = colB.as<int64_t>();
+            L.rowC = rowC.as<int64_t>();
+            L.colC = colC.as<int64_t>();
+            L.M = M;
+            L.N = N;
+            L.K = K;
+            L.splits = mode.splits;
+            L.tile = t;
+            if (mode.cut > 1) {
+              L.full_tiles = full;
+              L.tail_splits = mode.cut;
+            }
+            const size_t parts = mode.splits > 1 ? size_t(mode.splits) * M * N
+                                 : mode.cut > 1  ? size_t(mode.cut) * (count - full) * BM * BN
+                                                 : 0;
+            DeviceBuffer W = upload(std::vector<double>(parts * (cplx ? 2 : 1) + 1, NAN));
+            L.W = W.get();
+            L.alpha = 0.75;
+            L.beta = mode.add ? -0.5 : 0.0;
+            L.conjA = cplx && t != 1;
+            L.conjB = cplx && mode.add;
+            L.a_kcontig = ak;
+            L.b_kcontig = bk;
+            if (mode.other) {
+              L.D = D.get();
+              L.rowD = rowC.as<int64_t>();
+              L.colD = colC.as<int64_t>();
+              L.conjD = cplx;
+            }
+            launch_gett(L, st);
+            std::vector<double> h(M * ln * (cplx ? 2 : 1));
+            CHECK(hipStreamSynchronize(st) == hipSuccess);
+            CHECK(hipMemcpy(h.data(), C.get(), h.size() * 8, hipMemcpyDeviceToHost) == hipSuccess);
+            std::vector<Z> z(M * ln);
+            for (int64_t i = 0; i < M * ln; ++i) z[i] = cplx ? Z(h[2 * i], h[2 * i + 1]) : Z(h[i], 0);
+            const double e = P.error(z, ln, 7, L.alpha, L.conjA, L.conjB, L.beta, L.conjD);
+            if (e > 1.0)
+              step("tile " + std::to_string(t) + " splits " + std::to_string(mode.splits) + " cut " +
+                   std::to_string(mode.cut) + " error " + std::to_string(e));
+            worst = std::max(worst, e);
+          }
+        }
+        std::printf("K %d %s orientation %d: %.2f\n", int(K), cplx ? "complex" : "real", orient, worst);
+        std::fflush(stdout);
+        CHECK(worst <= 1.0);
+      }
+    }
+  CHECK(hipStreamDestroy(st) == hipSuccess);
+}
+
+// Sizes that the planner sends to each tile, whole, split and cut, in every
+// orientation: that it does, and the products.
+void gett_planner() {
+  enum { Whole, Split, Cut };
+  struct Size {
+    bool cplx;
+    int64_t M, N, K;
+    const char *tile;
+    int mode;
+  };
+  hipStream_t st;
+  CHECK(hipStreamCreate(&st) == hipSuccess);
+  for (const Size &x : std::vector<Size>{{false, 1677, 3921, 40, "", Whole},
+                                         {false, 3861, 2128, 695, "", Cut},
+                                         {false, 3512, 304, 40, "_t64", Whole},
+                                         {false, 679, 366, 502, "_t64", Split},
+                                         {false, 3886, 798, 183, "_t64", Cut},
+                                         {false, 442, 357, 44, "_t32", Whole},
+                                         {false, 365, 314, 999, "_t32", Split},
+                                         {true, 2058, 748, 574, "", Whole},
+                                         {true, 2226, 329, 1159, "", Split},
+                                         {true, 2400, 1089, 755, "", Cut},
+                                         {true, 864, 1187, 40, "_t64", Whole},
+                                         {true, 565, 478, 655, "_t64", Split},
+                                         {true, 1111, 1862, 185, "_t64", Cut},
+                                         {true, 352, 546, 53, "_t32", Whole},
+                                         {true, 307, 335, 709, "_t32", Split},
+                                         {true, 305, 3310, 194, "_t32", Cut}}) {
+    const Field f = x.cplx ? Field::Complex : Field::Real;
+    const Product P(x.cplx, x.M, x.N, x.K);
+    const size_t result = size_t(x.M) * x.N * scalar_bytes(f);
+    auto turned = [&](const std::vector<Z> &y, int64_t rows) {
+      std::vector<Z> r(y.size());
+      const int64_t cols = y.size() / rows;
+      for (int64_t i = 0; i < rows; ++i)
+        for (int64_t j = 0; j < cols; ++j) r[j * rows + i] = y[i * cols + j];
+      return packed(r, x.cplx);
+    };
+    for (int orient = 0; orient < 4; ++orient) {
+      const bool ak = orient & 2, bk = orient & 1;
+      // first index fastest: "km" is k-contiguous; C is "nm", n-contiguous
+      DeviceBuffer A = upload(ak ? packed(P.A, x.cplx) : turned(P.A, x.M)),
+                   B = upload(bk ? packed(P.B, x.cplx) : turned(P.B, x.N)), C(result);
+      const View a = ak ? dense_view(A.get(), f, "km", {x.K, x.M}) : dense_view(A.get(), f, "mk", {x.M, x.K}),
+                 b = bk ? dense_view(B.get(), f, "kn", {x.K, x.N}) : dense_view(B.get(), f, "nk", {x.N, x.K});
+      ContractionEngine E(st);
+      E.set_profiling(true);
+      g_allocations.clear();
+      g_record = true;
+      E.contract(0.75, a, b, 0.0, dense_view(C.get(), f, "nm", {x.N, x.M}));
+      g_record = false;
+      const std::string name = std::string("gett_") + (x.cplx ? "c64" : "f64") + (ak ? "_ak" : "_am") +
+                               (bk ? "_bk" : "_bn") + x.tile;
+      CHECK(E.timings().size() == 1 && E.timings().count(name) == 1);
+      // the offset tables' chunk, and the partial sums if there are any: of whole
+      // results, or of whole tiles
+      CHECK(g_allocations.size() == (x.mode == Whole ? 1 : 2));
+      if (x.mode != Whole) CHECK((g_allocations[1] % result == 0) == (x.mode == Split));
+      std::vector<double> h(size_t(x.M) * x.N * (x.cplx ? 2 : 1));
+      CHECK(hipMemcpy(h.data(), C.get(), result, hipMemcpyDeviceToHost) == hipSuccess);
+      std::vector<Z> z(size_t(x.M) * x.N);
+      for (size_t i = 0; i < z.size(); ++i) z[i] = x.cplx ? Z(h[2 * i], h[2 * i + 1]) : Z(h[i], 0);
+      const double e = P.error(z, x.N, x.M / 40, 0.75, false, false, 0.0, false);
+      std::printf("%s %d x %d x %d: %.2f\n", name.c_str(), int(x.M), int(x.N), int(x.K), e);
+      std::fflush(stdout);
+      CHECK(e <= 1.0);
+    }
+  }
+  CHECK(hipStreamDestroy(st) == hipSuccess);
+}
+
 const std::map<std::string, void (*)()> kScenarios = {
+    {"gett_tiles", gett_tiles},
+    {"gett_planner", gett_planner},
     {"no_allocations", no_allocations},
     {"pinned_copies", pinned_copies},
     {"copies_without_threads", copies_without_threads},
