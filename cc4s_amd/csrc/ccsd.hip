@@ -371,7 +371,8 @@ bool Ccsd::resident_integrals() {
   // d < x1 than the triangle needs, narrower ones launch more
   const double per_x = es * double(v) * double(v) * double(v);
   const int64_t fit = static_cast<int64_t>((2.0 * (1 << 30)) / per_x);
-  if (fit < 1 || v > 65535) return false;
+  // grids of the resident kernels; the slabs of the real field know no such bounds
+  if (fit < 1 || v + o > 65535 || Np > 65535) return false;
   const int64_t nx = std::min(std::min<int64_t>(fit, std::max<int64_t>(16, v / 16)), 65535 / v);
   if (nx < 1) return false;
   w.spare.set_held(true);

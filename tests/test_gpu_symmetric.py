@@ -160,3 +160,13 @@ def test_symmetric_residuum_with_the_slab_ladder(field, shape, size):
     print(f"symmetric residuum, slabs {field} {shape} {size}", flush=True)
     T = syn.random_amplitudes(shape[0], shape[1], field, 13, t1_scale=0.05, t2_scale=0.05)
     _check(field, shape, T, integralsSliceSize=size)
+
+
+@pytest.mark.parametrize("field", ["complex", "real"])
+@pytest.mark.parametrize("shape", [(2, 1, 1), (2, 2, 1), (3, 1, 4), (5, 2, 3)])
+def test_symmetric_residuum_of_one_or_two_particles(field, shape):
+    """No pairs c < d, or one."""
+    print(f"symmetric residuum {field} {shape}", flush=True)
+    T = syn.random_amplitudes(shape[0], shape[1], field, 13, t1_scale=0.05, t2_scale=0.05)
+    _check(field, shape, T)
+    _check(field, shape, T, ppl=False)
