@@ -147,20 +147,21 @@ void Ccsd::form_slice(Tensor &V, const char *name) {
   }
 }
 
-void Ccsd::form_integrals() {
+void Ccsd::form_integrals(void *scratch) {
   auto &w = *w_;
   const Field f = s_.field;
   const int64_t v = s_.Nv;
   auto make = [&](Tensor &V, const char *name) { form_slice(V, name); };
+  hermitian_test(E_.stream(), f, gamma_, s_.NG, s_.Np(), scratch);
   make(w.Vpphh, "pphh");
   make(w.Vhhhh, "hhhh");
   make(w.Vhhhp, "hhhp");
-  w.hermitian = is_hermitian(E_.stream(), f, gamma_, s_.NG, s_.Np());
+  if (f == Field::Complex) make(w.Vphhh, "phhh");
+  w.hermitian = hermitian_result(E_.stream(), scratch);
   // conj(V_cdkl) = sum_G Gamma[G,k,c] conj Gamma[G,d,l]
   //             = sum_G conj(Gamma[G,c,k]) Gamma[G,l,d] = V_klcd
   if (w.hermitian) w.Vhhpp_view = w.Vpphh.v.transposed({2, 3, 0, 1});
   if (f == Field::Complex) {
-    make(w.Vphhh, "phhh");
     if (w.hermitian) {
       w.Vhhpp_view = w.Vhhpp_view.conjugated();
     } else {

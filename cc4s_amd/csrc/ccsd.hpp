@@ -55,8 +55,8 @@ class Ccsd {
   ~Ccsd();
 
   // Coulomb integral slices from Gamma, once per run
-  // (VertexCoulombIntegrals.cxx:55-197)
-  void form_integrals();
+  // (VertexCoulombIntegrals.cxx:55-197); `scratch` of energy_partials_size()
+  void form_integrals(void *scratch);
 
   // R = residuum(T); T == nullptr is the first iteration (R1 = 0, R2 = V).
   // `pairs` tells how T_abij = T_baji holds (exactly for the iteration's own

@@ -384,7 +384,7 @@ void CoupledCluster::set_inputs(const double *gamma, bool on_device,
   CC4S_HIP(hipMemcpyAsync(eps_p_.get(), eps + s.No, s.Nv * sizeof(double),
                           hipMemcpyHostToDevice, stream_));
   ccsd_.reset(new Ccsd(*engine_, s, p_.ccsd, gamma_.get(), gamma_real));
-  ccsd_->form_integrals();
+  ccsd_->form_integrals(energy_partials_.get());
   CC4S_HIP(hipStreamSynchronize(stream_));
   if (!mixer_) create_mixer();
   inputs_set_ = true;

@@ -993,25 +993,24 @@ __global__ __launch_bounds__(kBlock) void asymmetry_finish_kernel(double *partia
   partials[3 * n + 2] = largest;
 }
 
-// sums kReduceBlocks partials and reads the total back
-double finish_count(hipStream_t s, double2 *p) {
-  finish_kernel<<<1, kBlock, 0, s>>>(p, 1, kReduceBlocks, p + kReduceBlocks);
-  CC4S_HIP(hipGetLastError());
-  double2 h;
-  CC4S_HIP(hipMemcpyAsync(&h, p + kReduceBlocks, sizeof(h), hipMemcpyDeviceToHost, s));
-  CC4S_HIP(hipStreamSynchronize(s));
-  return h.x;
-}
-
 }  // namespace
 
-bool is_hermitian(hipStream_t s, Field f, const void *gamma, int64_t NG, int64_t Np) {
-  DeviceBuffer part((kReduceBlocks + 1) * sizeof(double2));
-  double2 *p = part.as<double2>();
+void hermitian_test(hipStream_t s, Field f, const void *gamma, int64_t NG, int64_t Np,
+                    void *partials) {
+  double2 *p = static_cast<double2 *>(partials);
   hermitian_kernel<<<kReduceBlocks, kBlock, 0, s>>>(
       static_cast<const double2 *>(gamma), f == Field::Complex ? -1.0 : 1.0, NG, Np, p);
   CC4S_HIP(hipGetLastError());
-  return finish_count(s, p) == 0.0;
+  finish_kernel<<<1, kBlock, 0, s>>>(p, 1, kReduceBlocks, p + kReduceBlocks);
+  CC4S_HIP(hipGetLastError());
+}
+
+bool hermitian_result(hipStream_t s, const void *partials) {
+  double2 h;
+  CC4S_HIP(hipMemcpyAsync(&h, static_cast<const double2 *>(partials) + kReduceBlocks, sizeof(h),
+                          hipMemcpyDeviceToHost, s));
+  CC4S_HIP(hipStreamSynchronize(s));
+  return h.x == 0.0;
 }
 
 PairSymmetry pair_symmetry(hipStream_t s, Field f, const void *T2, int64_t No, int64_t Nv,

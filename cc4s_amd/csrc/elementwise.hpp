@@ -107,8 +107,12 @@ double norm_packed_range(hipStream_t s, Field f, const void *const *R,
 
 // true when the vertex [NG, Np, Np] satisfies Gamma[G,q,p] == conj(Gamma[G,p,q])
 // (complex field) or Gamma[G,q,p] == Gamma[G,p,q] (real field: the real and the
-// imaginary part are two real vertices) exactly for every G, p, q
-bool is_hermitian(hipStream_t s, Field f, const void *gamma, int64_t NG, int64_t Np);
+// imaginary part are two real vertices) exactly for every G, p, q.  hermitian_test
+// enqueues the comparison, hermitian_result waits for it; `partials` is device
+// scratch of energy_partials_size() that both are given
+void hermitian_test(hipStream_t s, Field f, const void *gamma, int64_t NG, int64_t Np,
+                    void *partials);
+bool hermitian_result(hipStream_t s, const void *partials);
 
 // y = x (device copy on the stream)
 void copy(hipStream_t s, void *y, const void *x, size_t bytes);

@@ -572,6 +572,19 @@ void copies_without_threads() {
   }
 }
 
+// New inputs allocate nothing that they do not keep.
+void inputs_keep_what_they_allocate() {
+  for (bool cplx : {true, false}) {
+    const Problem p = problem(cplx, 2, 5, 4, 4);  // no partial sums, whose buffer grows
+    Context c(p);
+    const size_t before = g_sizes.size();
+    arm(0);
+    CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+    step(std::to_string(g_count) + " allocations, " + std::to_string(g_sizes.size() - before) + " kept");
+    CHECK(size_t(g_count) == g_sizes.size() - before);
+  }
+}
+
 // Calls repeated on a context allocate nothing on the device.
 void no_allocations() {
   const Problem p = problem(true, 3, 9, 12, 4), q2 = problem(true, 3, 9, 12, 5);
@@ -837,6 +850,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"gett_tiles", gett_tiles},
     {"gett_planner", gett_planner},
     {"no_allocations", no_allocations},
+    {"inputs_keep_what_they_allocate", inputs_keep_what_they_allocate},
     {"pinned_copies", pinned_copies},
     {"copies_without_threads", copies_without_threads},
     {"given_back_between_threads", given_back_between_threads},
