@@ -707,15 +707,17 @@ void CoupledCluster::gradient_blocks(const void *gamma, bool hp, bool ph) {
   const int64_t G = cplx_field ? s.NG : 2 * s.NG;
   energy_weights(stream_, s.field, T_.get(), No, Nv, R_.get());
   const View Z = dense_view(R_.get(), s.field, "abij", {Nv, Nv, No, No});
-  if (hp)
-    engine_->contract(1.0, vertex_block(gamma, false, "Gbj"), Z.conjugated(), 0.0,
-                      dense_view(adj_hp_.get(), s.field, "Gia", {G, No, Nv}));
-  if (ph && cplx_field)
-    engine_->contract(1.0, vertex_block(gamma, true, "Gia"), Z, 0.0,
-                      dense_view(adj_ph_.get(), s.field, "Gbj", {G, Nv, No}));
-  else if (ph)
-    engine_->contract(1.0, vertex_block(gamma, false, "Gbj"), Z, 0.0,
-                      dense_view(adj_ph_.get(), s.field, "Gai", {G, Nv, No}));
+  engine_->group([&] {  // small blocks share a launch
+    if (hp)
+      engine_->contract(1.0, vertex_block(gamma, false, "Gbj"), Z.conjugated(), 0.0,
+                        dense_view(adj_hp_.get(), s.field, "Gia", {G, No, Nv}));
+    if (ph && cplx_field)
+      engine_->contract(1.0, vertex_block(gamma, true, "Gia"), Z, 0.0,
+                        dense_view(adj_ph_.get(), s.field, "Gbj", {G, Nv, No}));
+    else if (ph)
+      engine_->contract(1.0, vertex_block(gamma, false, "Gbj"), Z, 0.0,
+                        dense_view(adj_ph_.get(), s.field, "Gai", {G, Nv, No}));
+  });
 }
 
 // E = sum_G Re sum_ia conj(Gamma^G_ia) g^G_ia (complex), or 1/2 sum_G sum_ai

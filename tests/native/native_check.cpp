@@ -51,6 +51,7 @@ struct Copy {
 bool g_record = false;
 std::vector<Copy> g_copies;  // while g_record
 std::vector<size_t> g_allocations;  // while g_record
+std::atomic<long> g_launches{0};
 
 template <typename F>
 F real(const char *name) {
@@ -110,6 +111,13 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKin
     if (g_record) g_copies.push_back({dst, src, bytes});
   }
   return f(dst, src, bytes, kind, stream);
+}
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t lds,
+                           hipStream_t stream) {
+  static const auto r =
+      real<hipError_t (*)(const void *, dim3, dim3, void **, size_t, hipStream_t)>("hipLaunchKernel");
+  ++g_launches;
+  return r(f, grid, block, args, lds, stream);
 }
 int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*run)(void *), void *arg) noexcept {
   static const auto f = real<int (*)(pthread_t *, const pthread_attr_t *, void *(*)(void *), void *)>(
@@ -572,6 +580,25 @@ void copies_without_threads() {
   }
 }
 
+// A small gradient takes its two products in one launch, beside the weights and the
+// dots of two blocks in two launches each.
+void gradient_launches() {
+  const Problem p = problem(true, 3, 12, 30, 4);
+  const size_t n = size_t(2) * p.G * (p.o + p.v) * (p.o + p.v);
+  std::vector<double> grad(n), S(p.G);
+  Context c(p);
+  CHECK(cc4s_ccsd_set_inputs(c, p.gamma.data(), p.eps.data()) == 0);
+  CHECK(cc4s_ccsd_set_amplitudes(c, p.T1.data(), p.T2.data()) == 0);
+  long before = 0;
+  for (int k = 0; k < 2; ++k) {  // the second call has its plans
+    before = g_launches;
+    CHECK(cc4s_ccsd_energy_grad_backward(c, nullptr, 0, grad.data(), 0, S.data(),
+                                         CC4S_PRECISION_FP64) == 0);
+  }
+  step(std::to_string(g_launches - before) + " launches");
+  CHECK(g_launches - before > 0 && g_launches - before <= 6);
+}
+
 // New inputs allocate nothing that they do not keep.
 void inputs_keep_what_they_allocate() {
   for (bool cplx : {true, false}) {
@@ -850,6 +877,7 @@ const std::map<std::string, void (*)()> kScenarios = {
     {"gett_tiles", gett_tiles},
     {"gett_planner", gett_planner},
     {"no_allocations", no_allocations},
+    {"gradient_launches", gradient_launches},
     {"inputs_keep_what_they_allocate", inputs_keep_what_they_allocate},
     {"pinned_copies", pinned_copies},
     {"copies_without_threads", copies_without_threads},

@@ -18,7 +18,7 @@ PROGRAM = pathlib.Path(__file__).resolve().parent.parent / "cc4s_amd" / "native_
                                       "failed_formation", "given_back",
                                       "given_back_between_threads", "pinned_copies",
                                       "copies_without_threads", "no_allocations",
-                                      "inputs_keep_what_they_allocate",
+                                      "inputs_keep_what_they_allocate", "gradient_launches",
                                       "gett_tiles", "gett_planner"])
 def test_native(scenario):
     print(f"native {scenario}", flush=True)
