@@ -1,10 +1,11 @@
 // CCSD residuum on the GPU.  Each statement below is one tcc statement of
 // Ccsd.cxx (cited by line); three-factor products are split into two
 // pairwise contractions in the cheaper order.  Conjugate transposes and
-// slices of Gamma are strided views (no copies); the particle-particle
-// ladder forms V_xycd slabs from the dressed vertices (or, as an option,
-// forms V tiles in LDS inside one fused kernel) and never holds the full v^4
-// tensor.
+// slices of Gamma are strided views (no copies).  The particle-particle ladder
+// keeps the pair combinations of V_xycd, about v^4 / 2 + o v^3 scalars, where they
+// fit and their symmetries hold; else it forms V_xycd slabs from the dressed
+// vertices (or, as an option, V tiles in LDS inside one fused kernel) and holds
+// no v^4 tensor.
 #include "ccsd.hpp"
 #include "elementwise.hpp"
 #include "ladder.hpp"

@@ -72,12 +72,12 @@ __device__ __forceinline__ void tile_of(int g, int tilesM, int tilesN, int GM, i
   tn = (g % per_group) / gsize;
 }
 
-// Complex GETT, first generation: workgroup tile BM x BN, K staged BK at a time through LDS; 4 waves in a
-// (BM/WM) x (BN/WN) grid, each owning WM x WN of C as 16x16 MFMA blocks.
-// A is read either along K (AKC: consecutive lanes -> consecutive k) or along
-// M; B along K (BKC) or along N.  LDS holds A as [k][m] and B as [k][n] (one
-// plane per real/imaginary part), which is exactly the lane order of the
-// MFMA operands (lane l reads row l%16 at k = l/16).
+// Complex GETT, first generation: workgroup tile BM x BN, K staged BK at a time
+// through LDS; 4 waves in a (BM/WM) x (BN/WN) grid, each owning WM x WN of C as
+// 16x16 MFMA blocks.  A is read either along K (AKC: consecutive lanes ->
+// consecutive k) or along M; B along K (BKC) or along N.  LDS holds A as [k][m] and
+// B as [k][n] (one plane per real/imaginary part), which is exactly the lane order
+// of the MFMA operands (lane l reads row l%16 at k = l/16).
 template <int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC>
 __global__ __launch_bounds__(kThreads, 2) void gett_kernel(KArgs p) {
   constexpr int NPL = 2;

@@ -65,9 +65,8 @@ __global__ __launch_bounds__(kBlock) void tau_kernel(typename Sc<CPLX>::T *X,
 // read and written along their contiguous index
 constexpr int kPairTile = 32;
 
-// R_abij <- R_abij + R_baji (old values on the right) + V_abij (V may be null):
-// one block per
-// unordered pair of tiles {(A, B, i, j), (B, A, j, i)}, taken where
+// R_abij <- R_abij + R_baji (old values on the right) + V_abij (V may be null): one
+// block per unordered pair of tiles {(A, B, i, j), (B, A, j, i)}, taken where
 // (i, tile A) <= (j, tile B); both tiles are read before either is written
 template <bool CPLX>
 __global__ __launch_bounds__(kBlock) void symmetrize_kernel(

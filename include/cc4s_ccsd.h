@@ -248,7 +248,7 @@ int cc4s_ccsd_energy_grad_forward(cc4s_ccsd_context *ctx, const double *gamma,
  * precision: CC4S_PRECISION_FP64 (FP64 MFMA) or CC4S_PRECISION_FP32 (FP32
  * MFMA operands and sums).  FP64 products read the energy weights 2 tau_abij -
  * tau_baij from the residuum's buffer, FP32 ones rebuild them from the amplitudes
- * tile by tile. */
+ * tile by tile, which takes longer (No=16, Nv=100, NG=300: 0.31 ms FP64, 0.75 FP32). */
 int cc4s_ccsd_energy_grad_backward(cc4s_ccsd_context *ctx, const double *gamma,
                                    int gamma_on_device, double *grad,
                                    int grad_on_device, double *structure_factor,

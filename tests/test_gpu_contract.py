@@ -34,8 +34,8 @@ LENS = {"a": 13, "b": 13, "c": 13, "d": 13, "i": 5, "j": 5, "k": 5, "l": 5,
         "G": 37, "x": 7, "y": 6}
 
 
-# longer contracted lengths: every case below has K > 256 (the complex kernel
-# for K <= 256 is a 64x64-tile variant; longer K takes the 128x64 tile)
+# longer contracted lengths, K > 256 in every case below: many K-stages, and K split
+# (the planner sends them to the 32x32 tile; test_gpu_native.py has every tile)
 LENS_LONG = {"a": 21, "b": 19, "c": 23, "d": 17, "i": 6, "j": 5, "k": 12, "l": 16,
              "G": 300, "x": 9, "y": 6}
 CASES_LONG = [
@@ -119,14 +119,14 @@ def test_contract_rejects_bad_indices():
 
 
 # M, N, K at the edges of the 32, 64 and 128 workgroup tiles and of the 16-k
-# stage, one stage and fewer, split-K with few and with many result elements,
-# and sizes at which the planner takes each tile.  Tolerance: K products of
+# stage, one stage and fewer, split-K with few and with many result elements (the
+# planner's choices among all tiles are in test_gpu_native.py).  Tolerance: K products of
 # standard normals in two summation orders, sqrt(K) 2^-53 relative to the
 # largest element's sqrt(K): 1e-13 as above.
 TILE_CASES = [(1, 1, 1), (2, 3, 15), (31, 33, 16), (32, 32, 17), (65, 31, 33), (63, 65, 64),
               (129, 127, 48), (1, 700, 31), (700, 1, 257), (5, 6, 40000), (40, 33, 9000),
               (257, 130, 2000), (1030, 1100, 100), (2000, 2100, 33),
-              # whole waves of tiles and a partial one that is cut along K
+              # whole waves of tiles and a partial one, cut along K in the complex field
               (1650, 1601, 700), (2300, 1111, 1000)]
 
 
